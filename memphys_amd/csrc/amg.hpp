@@ -24,6 +24,9 @@ struct AmgMat {
     DevBuf<int> ptr_b, col_b;
     DevBuf<uint16_t> val_b;  // BF16 values (round to nearest even)
     DevBuf<uint16_t> val2_b; // a second value array in the same slots (composed restriction)
+    DevBuf<uint16_t> col16_b;  // compressed columns of its own (T_0)
+    DevBuf<int> cbase_b;
+    long slots = 0, nnz16 = 0; // T_0: slots, those of slices with 16-bit columns
     const int* ptr = nullptr;
     const int* col = nullptr;
     const uint16_t* val = nullptr;
@@ -36,9 +39,9 @@ struct AmgLevelDev {
     int n = 0;
     AmgMat A;      // operator of this level
     AmgMat P, R;   // prolongation from / restriction to the next level
-    // composed steps (three or more levels): Q = R_{l-1} - A D R_{l-1} (values)
-    // with R_{l-1} in the same slots (levels 2 .. L-2), T = P - D A P (levels
-    // 1 .. L-2)
+    // composed steps: T = P - D A P (levels 0 .. L-2); with three or more
+    // levels also Q = R_{l-1} - A D R_{l-1} (values) with R_{l-1} in the same
+    // slots (levels 2 .. L-2)
     AmgMat Q, T;
     DevBuf<float> dinv;  // omega / a_ii
     DevBuf<float> b, x, res, y;
@@ -57,15 +60,15 @@ struct AmgDevice {
     std::vector<long> nnz;
     std::string layout;  // chosen layout per matrix, for reports
     double setup_seconds = 0.0;
-    // host copies of the hierarchy (A[0] stays empty) and of the T_l, for
-    // re-tuning layouts
+    // host copies of the hierarchy (A[0] stays empty) and of the T_l, l >= 1,
+    // for re-tuning layouts
     std::vector<mp_amg::Csr> hA, hP, hR, hT;
-    // Three or more levels: the cycle below level 1 runs from the composed
-    // matrices (Q_l, T_l and the coarsest solve times R_{L-2}, row-dense BF16
-    // in cr_val: row r's size[r] entries at cr_data[r] act on the level-(L-2)
-    // vector from row cr_first[r]).  plain_cycle runs the level-by-level
-    // cycle instead (the same map, for comparisons).
-    bool composed = false;
+    // The cycle runs from the composed matrices (T_l on the way up; with three
+    // or more levels, deep, also Q_l and the coarsest solve times R_{L-2},
+    // row-dense BF16 in cr_val: row r's size[r] entries at cr_data[r] act on
+    // the level-(L-2) vector from row cr_first[r]).  plain_cycle runs the
+    // level-by-level cycle instead (the same map, for comparisons).
+    bool deep = false;
     bool plain_cycle = false;
     DevBuf<uint16_t> cr_val;
     DevBuf<int> cr_first, cr_size;

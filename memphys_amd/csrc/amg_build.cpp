@@ -333,6 +333,7 @@ Hierarchy build(const Csr& A0, const Options& opt, bool bordered) {
         Csr AP = multiply(*cur, P, opt.threads);
         Csr Ac = multiply(R, AP, opt.threads);
         if (opt.drop > 0.0) Ac = sparsify(Ac, opt.drop);
+        if (h.P.empty()) h.AP0 = std::move(AP);
         h.P.push_back(std::move(P));
         h.R.push_back(std::move(R));
         h.A.push_back(std::move(Ac));

@@ -42,6 +42,7 @@ struct Hierarchy {
     // A[0] is left empty (the caller owns the finest operator); A[l] for
     // l >= 1 are the Galerkin operators.  P[l], R[l] map between l and l+1.
     std::vector<Csr> A, P, R;
+    Csr AP0;                         // A_0 P_0 (columns sorted), from the Galerkin product
     std::vector<double> coarse_inv;  // nc x nc, row-major
     int nc = 0;
     int levels() const { return (int)A.size(); }

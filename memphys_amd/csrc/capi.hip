@@ -423,37 +423,6 @@ namespace {
 // Uploads nprob clouds given back to back in caller order (problem q owns
 // caller nodes [off_q, off_q + nvp[q]); its stencils may only reference its
 // own nodes).  One problem is the ordinary single-cloud case.
-// 16-bit column form of the SELL slots: per slice, the sorted distinct
-// columns are covered greedily by windows of 2^CW_BITS ids; a slice needing
-// at most CW_COUNT windows stores (window << CW_BITS) | (column - base) per
-// slot, any other keeps its 32-bit columns (first base -1).
-void compress_columns(const std::vector<int>& sptr, const std::vector<int>& col, int nslices,
-                      std::vector<uint16_t>& c16, std::vector<int>& cb) {
-    c16.assign(col.size(), 0);
-    cb.assign((size_t)nslices * CW_COUNT, -1);
-    std::vector<int> u;
-    for (int sl = 0; sl < nslices; ++sl) {
-        u.assign(col.begin() + sptr[sl], col.begin() + sptr[sl + 1]);
-        if (u.empty()) continue;
-        std::sort(u.begin(), u.end());
-        int base[CW_COUNT];
-        int nw = 0;
-        for (size_t i = 0; i < u.size() && nw <= CW_COUNT;) {
-            if (nw < CW_COUNT) base[nw] = u[i];
-            ++nw;
-            const int end = u[i] + (1 << CW_BITS);
-            while (i < u.size() && u[i] < end) ++i;
-        }
-        if (nw > CW_COUNT) continue;
-        for (int w = 0; w < CW_COUNT; ++w) cb[(size_t)sl * CW_COUNT + w] = base[std::min(w, nw - 1)];
-        for (int t = sptr[sl]; t < sptr[sl + 1]; ++t) {
-            int w = nw - 1;
-            while (base[w] > col[t]) --w;
-            c16[t] = (uint16_t)((w << CW_BITS) | (col[t] - base[w]));
-        }
-    }
-}
-
 int upload_clouds(mp_ctx* c, const char* fn, int nprob, const int* nvp, int dim,
                   const double* xyz, const uint8_t* boundary, const double* normal,
                   const int* row_ptr, const int* col_idx) {

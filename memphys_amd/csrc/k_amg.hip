@@ -13,23 +13,29 @@
 // the FP64 result; the border unknown of the full-Neumann system passes
 // through unchanged.
 //
-// With three or more levels the cycle below level 1 runs from matrices that
-// compose its steps, built at set-up (the same linear map, one rounding of
-// the composed values instead of one per factor), so each coarse level costs
-// one product on the way down and one on the way up:
+// The cycle runs from matrices that compose these steps, built at set-up (the
+// same linear map, one rounding of the composed values instead of one per
+// factor), so each level below level 1 costs one product on the way down and
+// every level one on the way up:
 //   restrict + pre-smooth  b_l = R_{l-1} res_{l-1},  res_l = Q_l res_{l-1},
 //                          Q_l = R_{l-1} - A_l D_l R_{l-1}        (levels 2 .. L-2)
-//   coarsest solve         y_{L-1} = (G R_{L-2}) res_{L-2}        (dense rows; one
-//                          problem: a batch's many small problems keep
-//                          R_{L-2} and the block-diagonal G, fewer bytes)
+//   coarsest solve         y_{L-1} = (G R_{L-2}) res_{L-2}        (dense rows; three
+//                          or more levels, one problem: a batch's many small
+//                          problems keep R_{L-2} and the block-diagonal G,
+//                          fewer bytes)
 //   prolong + post-smooth  y_l = D_l (b_l + res_l) + T_l y_{l+1},
-//                          T_l = P_l - D_l A_l P_l                (levels 1 .. L-2)
+//                          T_l = P_l - D_l A_l P_l                (levels 0 .. L-2)
 // (with x_l = D_l b_l after pre-smoothing: x_l + P_l y + D_l (b_l - A_l (x_l +
 // P_l y)) = D_l b_l + D_l res_l + (P_l - D_l A_l P_l) y).  Levels 0 and 1 keep
 // the separate restriction and pre-smoothing (Q_1 would be about 25 times
-// denser than A_1), and level 0 the separate prolongation and post-smoothing.  A matrix is SELL-64x4 (one wavefront per slice of 64
-// rows, four neighbours of a row side by side, padding slots with value 0)
-// or CSR with several lanes per row, whichever suits its row lengths.
+// denser than A_1).  T_0 has half as many entries as A_0 (9 against 30 per row
+// on 2D stencils, 20-22 against 43-46 on 3D ones) and gathers from the 12 times
+// smaller level-1 vector: at 1M nodes it takes 36 us, where the separate
+// prolongation and post-smoothing by A_0 took 17 + 56 us (64 2D cavities of 665k
+// nodes: 16 against 10 + 26 us).
+// A matrix is SELL-64x4 (one wavefront per slice of 64 rows, four neighbours
+// of a row side by side, padding slots with value 0) or CSR with several lanes
+// per row, whichever suits its row lengths.
 #include "amg.hpp"
 #include "krylov.hpp"
 
@@ -188,7 +194,9 @@ __global__ __launch_bounds__(BLOCK) void k_amg_op(MatView m, const float* __rest
         xout[i] = acc2;
         res[i] = acc;
     } else if constexpr (OP == OP_TPOST) {
-        out[i] = (TO)(dinv[i] * ((float)b[i] + base[i]) + acc);
+        const float y = dinv[i] * ((float)b[i] + base[i]) + acc;
+        out[i] = (TO)y;
+        if (out32) out32[i] = y;
     } else {
         const float y = xin[i] + dinv[i] * ((float)b[i] - acc);
         out[i] = (TO)y;
@@ -387,6 +395,83 @@ void upload_mat(AmgMat& d, const mp_amg::Csr& M, int g, hipStream_t st) {
     d.val = d.val_b.p;
 }
 
+// T_0 = P_0 - D_0 A_0 P_0 of every problem (device rows row0[q] .., columns
+// from col0[q]) as one SELL-64x4 matrix of n rows with 16-bit columns where
+// they fit.  A_0's rows hold their diagonal, so A_0 P_0 has every entry of P_0
+// and T_0 takes its pattern; both come with sorted columns.
+void upload_t0(AmgMat& d, const std::vector<mp_amg::Hierarchy>& hs,
+               const std::vector<std::pair<int, int>>& blocks, const std::vector<int>& row0,
+               const std::vector<int>& col0, const std::vector<float>& dinv, int n,
+               hipStream_t st) {
+    std::vector<int> prob(n, -1);
+    for (size_t q = 0; q < blocks.size(); ++q)
+        std::fill(prob.begin() + row0[q], prob.begin() + row0[q] + blocks[q].second, (int)q);
+    const int ns = (n + SLICE - 1) / SLICE;
+    std::vector<int> sptr(ns + 1, 0);
+    d.nnz = 0;
+    for (int s = 0; s < ns; ++s) {
+        int w = 0;
+        for (int r = s * SLICE; r < std::min(n, (s + 1) * SLICE); ++r) {
+            if (prob[r] < 0) continue;
+            const mp_amg::Csr& M = hs[prob[r]].AP0;
+            const int len = M.ptr[r - row0[prob[r]] + 1] - M.ptr[r - row0[prob[r]]];
+            w = std::max(w, len);
+            d.nnz += len;
+        }
+        sptr[s + 1] = sptr[s] + sell_width4(w) * SLICE;
+    }
+    std::vector<int> col(sptr[ns], 0), cb;
+    std::vector<uint16_t> val(sptr[ns], 0), c16;
+    parallel_for(ns, [&](int s) {
+        const int w = (sptr[s + 1] - sptr[s]) / SLICE;
+        int pad = 0;  // padding slots: value 0 at the slice's first column
+        for (int l = SLICE - 1; l >= 0; --l) {
+            const int r = s * SLICE + l;
+            if (r < n && prob[r] >= 0) {
+                const mp_amg::Csr& M = hs[prob[r]].AP0;
+                const int i = r - row0[prob[r]];
+                if (M.ptr[i + 1] > M.ptr[i]) pad = col0[prob[r]] + M.col[M.ptr[i]];
+            }
+        }
+        for (int l = 0; l < SLICE; ++l) {
+            const int r = s * SLICE + l, base = sptr[s] + l * SGROUP;
+            int j = 0;
+            if (r < n && prob[r] >= 0) {
+                const int q = prob[r], i = r - row0[q];
+                const mp_amg::Csr &M = hs[q].AP0, &P = hs[q].P[0];
+                int t = P.ptr[i];
+                for (int e = M.ptr[i]; e < M.ptr[i + 1]; ++e, ++j) {
+                    double v = -(double)dinv[r] * M.val[e];
+                    while (t < P.ptr[i + 1] && P.col[t] < M.col[e]) ++t;
+                    if (t < P.ptr[i + 1] && P.col[t] == M.col[e]) v += P.val[t];
+                    col[base + sell_off(j)] = col0[q] + M.col[e];
+                    val[base + sell_off(j)] = f2bf((float)v);
+                }
+            }
+            for (; j < w; ++j) col[base + sell_off(j)] = pad;
+        }
+    });
+    compress_columns(sptr, col, ns, c16, cb);
+    d.n = n;
+    d.g = 0;
+    d.nslices = ns;
+    d.nnz16 = 0;
+    for (int s = 0; s < ns; ++s)
+        if (cb[(size_t)s * CW_COUNT] >= 0) d.nnz16 += sptr[s + 1] - sptr[s];
+    d.slots = sptr[ns];
+    put(d.ptr_b, sptr, st);
+    put(d.col_b, col, st);
+    put(d.val_b, val, st);
+    put(d.col16_b, c16, st);
+    put(d.cbase_b, cb, st);
+    MP_HIP(hipStreamSynchronize(st));  // (the host arrays end here)
+    d.ptr = d.ptr_b.p;
+    d.col = d.col_b.p;
+    d.val = d.val_b.p;
+    d.col16 = d.col16_b.p;
+    d.cbase = d.cbase_b.p;
+}
+
 // Reads n4 float4s (grid-stride), so that a product timed after it finds its
 // matrix and vector outside the caches, as inside a V-cycle, where the finest
 // level's passes evict them between two uses.
@@ -566,6 +651,35 @@ mp_amg::Csr minus_scaled(const mp_amg::Csr& X, const std::vector<float>* d, cons
 
 }  // namespace
 
+void compress_columns(const std::vector<int>& sptr, const std::vector<int>& col, int nslices,
+                      std::vector<uint16_t>& c16, std::vector<int>& cb) {
+    // per slice, the sorted distinct columns are covered greedily by windows of
+    // 2^CW_BITS ids
+    c16.assign(col.size(), 0);
+    cb.assign((size_t)nslices * CW_COUNT, -1);
+    parallel_for(nslices, [&](int sl) {
+        std::vector<int> u(col.begin() + sptr[sl], col.begin() + sptr[sl + 1]);
+        if (u.empty()) return;
+        std::sort(u.begin(), u.end());
+        int base[CW_COUNT];
+        int nw = 0;
+        for (size_t i = 0; i < u.size() && nw <= CW_COUNT;) {
+            if (nw < CW_COUNT) base[nw] = u[i];
+            ++nw;
+            const int end = u[i] + (1 << CW_BITS);
+            while (i < u.size() && u[i] < end) ++i;
+        }
+        if (nw > CW_COUNT) return;
+        for (int w = 0; w < CW_COUNT; ++w)
+            cb[(size_t)sl * CW_COUNT + w] = base[std::min(w, nw - 1)];
+        for (int t = sptr[sl]; t < sptr[sl + 1]; ++t) {
+            int w = nw - 1;
+            while (base[w] > col[t]) --w;
+            c16[t] = (uint16_t)((w << CW_BITS) | (col[t] - base[w]));
+        }
+    });
+}
+
 void AmgDevice::setup(hipStream_t st, const SellView& sv, const double* val64_dev,
                       const SellView& sv_apply, const float* val32_dev,
                       const std::vector<std::pair<int, int>>& blocks,
@@ -734,11 +848,12 @@ void AmgDevice::setup(hipStream_t st, const SellView& sv, const double* val64_de
         }
     }
     put(cinv, g, st);
-    // composed steps below level 1 (three or more levels)
-    composed = L >= 3;
+    // T_0, and the composed steps below level 1 (three or more levels)
+    upload_t0(lv[0].T, hs, blocks, off[0], off[1], dvs[0], n0, st);
+    deep = L >= 3;
     plain_cycle = false;
     hT.assign(L, mp_amg::Csr());
-    if (composed) {
+    if (deep) {
         for (int l = 1; l <= L - 2; ++l) {
             const mp_amg::Csr AP = mp_amg::multiply(Ab[l], Pb[l], opt.threads);
             hT[l] = minus_scaled(Pb[l], &dvs[l], AP, nullptr);
@@ -802,7 +917,7 @@ void AmgDevice::setup(hipStream_t st, const SellView& sv, const double* val64_de
         std::snprintf(buf, sizeof(buf), "A%d:%d P%d:%d R%d:%d ", l, lv[l].A.g, l, lv[l].P.g, l,
                       lv[l].R.g);
         layout += buf;
-        if (composed && l >= 1) {
+        if (deep && l >= 1) {
             std::snprintf(buf, sizeof(buf), "T%d:%d ", l, lv[l].T.g);
             layout += buf;
             if (l >= 2) {
@@ -838,22 +953,18 @@ void AmgDevice::retune(hipStream_t st) {
     try {
         for (int l = 0; l + 1 < L; ++l) {
             AmgLevelDev& d = lv[l];
-            // the composed cycle uses A_1, P_0, R_0, the T_l (the Q_l keep
-            // their CSR layout) and, in a batch, R_{L-2}; the plain cycle
-            // every A_l, P_l, R_l
-            const bool useA = l > 0 && (!composed || l == 1);
-            const bool useP = !composed || l == 0;
-            const bool useR = !composed || l == 0 || (blocked && l == L - 2);
+            // the cycle uses A_1, R_0, the T_l (T_0 and the Q_l keep their
+            // layouts) and, in a batch, R_{L-2}; the plain cycle every A_l,
+            // P_l, R_l
+            const bool useA = l == 1;
+            const bool useR = l == 0 || (blocked && l == L - 2);
             if (useA)
                 upload_tuned(d.A, hA[l], st, tx.p, ty.p, e0, e1, fl, layout,
                              ("A" + std::to_string(l)).c_str());
-            if (useP)
-                upload_tuned(d.P, hP[l], st, tx.p, ty.p, e0, e1, fl, layout,
-                             ("P" + std::to_string(l)).c_str());
             if (useR)
                 upload_tuned(d.R, hR[l], st, tx.p, ty.p, e0, e1, fl, layout,
                              ("R" + std::to_string(l)).c_str());
-            if (composed && l >= 1)
+            if (deep && l >= 1)
                 upload_tuned(d.T, hT[l], st, tx.p, ty.p, e0, e1, fl, layout,
                              ("T" + std::to_string(l)).c_str());
         }
@@ -913,28 +1024,34 @@ void AmgDevice::vcycle(hipStream_t st, const TI* in, TO* out, const double* bin,
             launch_op<OP_PRE, TI, float>(st, lv[0].A, lv[0].dinv.p, in, nullptr, nullptr,
                                              lv[0].x.p, lv[0].res.p, (float*)nullptr, bin, bout,
                                              done);
-        if (composed && !plain_cycle) {
-            // level 0 -> 1 and level 1's pre-smoothing as below; then one
-            // composed product per coarse level down, the composed coarsest
-            // solve, one composed product per level up to level 1
+        if (!plain_cycle) {
+            // level 0 -> 1; then level 1's pre-smoothing, one composed product
+            // per coarser level and the composed coarsest solve (or, with two
+            // levels, the coarsest solve at once), and one composed product
+            // per level up to level 0
             launch_op<OP_SPMV, float, float>(st, lv[0].R, nullptr, (const float*)nullptr,
                                              lv[0].res.p, nullptr, nullptr, nullptr, lv[1].b.p,
                                              nullptr, nullptr, done);
-            launch_op<OP_PRE, float, float>(st, lv[1].A, lv[1].dinv.p, lv[1].b.p, nullptr,
-                                            nullptr, lv[1].x.p, lv[1].res.p, (float*)nullptr,
-                                            nullptr, nullptr, done);
-            for (int l = 2; l <= L - 2; ++l)
-                launch_op<OP_RQ, float, float>(st, lv[l].Q, nullptr, (const float*)nullptr,
-                                               lv[l - 1].res.p, nullptr, lv[l].b.p, lv[l].res.p,
-                                               (float*)nullptr, nullptr, nullptr, done);
-            if (!blocked) {
+            if (deep) {
+                launch_op<OP_PRE, float, float>(st, lv[1].A, lv[1].dinv.p, lv[1].b.p, nullptr,
+                                                nullptr, lv[1].x.p, lv[1].res.p, (float*)nullptr,
+                                                nullptr, nullptr, done);
+                for (int l = 2; l <= L - 2; ++l)
+                    launch_op<OP_RQ, float, float>(st, lv[l].Q, nullptr, (const float*)nullptr,
+                                                   lv[l - 1].res.p, nullptr, lv[l].b.p,
+                                                   lv[l].res.p, (float*)nullptr, nullptr, nullptr,
+                                                   done);
+            }
+            if (deep && !blocked) {
                 hipLaunchKernelGGL(k_amg_rowdense, dim3(nc), dim3(RD_THREADS), 0, st, nc,
                                    cr_val.p, cr_first.p, cr_size.p, cr_data.p,
                                    (const float*)lv[L - 2].res.p, lv[L - 1].y.p, done);
             } else {
-                launch_op<OP_SPMV, float, float>(st, lv[L - 2].R, nullptr, (const float*)nullptr,
-                                                 lv[L - 2].res.p, nullptr, nullptr, nullptr,
-                                                 lv[L - 1].b.p, nullptr, nullptr, done);
+                if (deep)
+                    launch_op<OP_SPMV, float, float>(st, lv[L - 2].R, nullptr,
+                                                     (const float*)nullptr, lv[L - 2].res.p,
+                                                     nullptr, nullptr, nullptr, lv[L - 1].b.p,
+                                                     nullptr, nullptr, done);
                 coarse((const float*)lv[L - 1].b.p, lv[L - 1].y.p, (float*)nullptr,
                        (const double*)nullptr, (double*)nullptr);
             }
@@ -942,13 +1059,9 @@ void AmgDevice::vcycle(hipStream_t st, const TI* in, TO* out, const double* bin,
                 launch_op<OP_TPOST, float, float>(st, lv[l].T, lv[l].dinv.p, lv[l].b.p,
                                                   lv[l + 1].y.p, lv[l].res.p, nullptr, nullptr,
                                                   lv[l].y.p, nullptr, nullptr, done);
-            AmgLevelDev& f = lv[0];
-            launch_op<OP_SPMV, float, float>(st, f.P, nullptr, (const float*)nullptr, lv[1].y.p,
-                                             f.x.p, nullptr, nullptr, f.x.p, nullptr, nullptr,
-                                             done);
             if (post_timer) post_timer->begin(st);
-            launch_op<OP_POST, TI, TO>(st, f.A, f.dinv.p, in, f.x.p, nullptr, nullptr, nullptr,
-                                       out, nullptr, nullptr, done, out32);
+            launch_op<OP_TPOST, TI, TO>(st, lv[0].T, lv[0].dinv.p, in, lv[1].y.p, lv[0].res.p,
+                                        nullptr, nullptr, out, nullptr, nullptr, done, out32);
             if (post_timer) post_timer->end(st);
             return;
         }

@@ -132,7 +132,7 @@ struct PpeSolver {
     int gm_hint = 0;
     long fp64_fallbacks = 0;
     KernelTimer spmv_timer;
-    KernelTimer smooth_timer;         // the multigrid's level-0 post-smoothing product
+    KernelTimer smooth_timer;         // the multigrid's level-0 post-smoothing product (T_0)
     bool use_graphs = true;           // replay each chunk of iterations from a hipGraph
     std::vector<ChunkGraph> graphs;
     long total_iterations = 0, total_solves = 0;
@@ -149,7 +149,7 @@ struct PpeSolver {
     // seg_stats).
     SolveStats solve(hipStream_t s, const double* b_dev, double* x_dev);
     double spmv_bytes(int fp32) const;
-    // algorithmic bytes of the level-0 post-smoothing product (BF16 values)
+    // algorithmic bytes of the level-0 prolongation and post-smoothing product (T_0)
     double smooth_bytes() const;
     // r = b - A x (FP64, unscaled operator incl. border) into `tmp`; returns tmp.p
     double* residual_of(hipStream_t s, const double* b_dev, const double* x_dev);

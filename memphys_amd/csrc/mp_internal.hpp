@@ -2,8 +2,10 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/memphys_hip.h"
@@ -231,6 +233,25 @@ struct SellView {
     const uint16_t* col16 = nullptr;  // [slots] compressed column ids (or null)
     const int* cbase = nullptr;       // [nslices*CW_COUNT] window bases
 };
+
+// Host: the compressed columns of slots sptr/col (see CW_BITS above): c16 per
+// slot, cb CW_COUNT window bases per slice (-1: the slice keeps 32-bit columns).
+void compress_columns(const std::vector<int>& sptr, const std::vector<int>& col, int nslices,
+                      std::vector<uint16_t>& c16, std::vector<int>& cb);
+
+// Host: f(i) for i in [0, n) on up to 16 threads, contiguous ranges.
+template <typename F>
+void parallel_for(int n, F&& f) {
+    const int t = (int)std::max(1u, std::min({16u, std::thread::hardware_concurrency(),
+                                              (unsigned)(n / 64 + 1)}));
+    std::vector<std::thread> pool;
+    for (int q = 1; q < t; ++q)
+        pool.emplace_back([&, q]() {
+            for (int i = (int)((long)n * q / t); i < (int)((long)n * (q + 1) / t); ++i) f(i);
+        });
+    for (int i = 0; i < (int)((long)n / t); ++i) f(i);
+    for (auto& w : pool) w.join();
+}
 
 // Device-side Krylov scalars (FP64) of one system.  Written only by the
 // single-block finishing kernels, read by every block of the following kernels.

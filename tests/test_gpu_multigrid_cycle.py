@@ -1,8 +1,8 @@
 """The multigrid V(1,1)-cycle that preconditions the pressure solve, applied on
-its own through mp_precond_apply: with three or more levels the solver's cycle
-runs the levels below level 1 from composed matrices (Q_l = R_{l-1} - A_l D_l
-R_{l-1}, T_l = P_l - D_l A_l P_l, and the coarsest solve times the restriction
-to it), which is the same linear map as the level-by-level cycle; only the
+its own through mp_precond_apply: the solver's cycle runs from composed
+matrices (T_l = P_l - D_l A_l P_l on the way up; with three or more levels also
+Q_l = R_{l-1} - A_l D_l R_{l-1} below level 1 and the coarsest solve times the
+restriction to it), which is the same linear map as the level-by-level cycle; only the
 BF16 rounding of the stored values differs (one rounding of each composed
 entry instead of one per factor).  A wrong sign, a dropped term or a wrong
 level offset in the composed steps moves the result by O(1); the rounding
@@ -97,6 +97,30 @@ def test_composed_cycle_batch(ctx):
     _print("batch hierarchy", info)
     assert info["levels"] >= 3
     _check_cycles(ctx, ctx.n_sys, cat.nv, True, 13)
+
+
+@pytest.mark.parametrize("dim,sizes", [(2, (24,)), (2, (29, 24)), (3, (9,)), (3, (14, 11))])
+def test_composed_cycle_two_levels(ctx, dim, sizes):
+    """Two levels (coarse solve right below level 0): only T_0 is composed.
+    Row counts off the slice and block sizes, one problem and batches, whose
+    padding rows T_0 holds no entries for."""
+    import memphys_amd as M
+    kw = dict(k_interior=30) if dim == 2 else dict(k_interior=40, k_layers=(60, 55, 50))
+    clouds = [M.box_cloud(dim=dim, n=n, jitter=0.25, seed=n, **kw) for n in sizes]
+    cat = clouds[0]
+    if len(clouds) > 1:
+        cat = ctx.upload_batch(clouds)
+    else:
+        ctx.upload(cat)
+    ctx.weights(3, 3, download=False)
+    u_dir, p_dir, _ = M.lid_conditions(cat)
+    ctx.fs_create(1.0, 0.01, 1e-4, 2, 1e-10, 2000, u_dir, u_dir, u_dir if dim == 3 else None,
+                  p_dir, precision=M.MP_PREC_MIXED, precond=M.MP_PRECOND_AMG,
+                  krylov=M.MP_KRYLOV_GMRES)
+    info = ctx.precond_info()
+    _print("two-level hierarchy", info)
+    assert info["levels"] == 2
+    _check_cycles(ctx, ctx.n_sys, cat.nv, True, 14)
 
 
 def test_autotune_leaves_fields_and_keeps_accuracy(ctx, cavity2d):
