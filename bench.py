@@ -71,8 +71,7 @@ def measured_traffic(n: int, kernel_index: int = 0,
     """HBM bytes per launch measured with rocprofv3 FETCH_SIZE and WRITE_SIZE runs on
     the 100^3 workload, read from a committed summary: the `kernel_index`-th
     `traffic_bytes_per_launch` line (PPE SpMV summary: 0 the headline form's
-    FP32-operator GMRES product, 1 the FP64 form's product; multigrid summary: 0 the
-    level-0 post-smoothing product); None for other workloads."""
+    FP32-operator GMRES product, 1 the FP64 form's product); None for other workloads."""
     path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles", summary)
     if n != 100 or not os.path.exists(path):
         return None
@@ -328,10 +327,29 @@ def cavity2d_c1(M, O, steps=20, warmup=5, with_cpu=True):
     return out
 
 
-def smooth_roofline(t, copy_gbps, gmres: bool = True):
+def level0_traffic(n: int, bytes_l: float, summary: str = "amg_level0_traffic_cavity3d_1M.md"):
+    """Measured HBM bytes per launch of the multigrid level-0 product whose
+    algorithmic bytes per launch (given in the summary before each figure) are
+    bytes_l within 1 %; None for other products and workloads."""
+    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles", summary)
+    if n != 100 or not os.path.exists(path):
+        return None
+    alg = None
+    for line in open(path):
+        if line.startswith("algorithmic_bytes_per_launch"):
+            alg = float(line.split("=")[1])
+        elif line.startswith("traffic_bytes_per_launch") and alg:
+            if abs(bytes_l / alg - 1.0) < 0.01:
+                return float(line.split("=")[1])
+            alg = None
+    return None
+
+
+def smooth_roofline(t, copy_gbps, n_lattice: int = 0, gmres: bool = True):
     """Roofline entry of the multigrid's level-0 prolongation and post-smoothing
     (the composed T_0 product): algorithmic bytes per launch over its mean
-    HIP-event duration, launches that did the work."""
+    HIP-event duration, launches that did the work; `traffic` is its measured
+    HBM bytes per launch on the 100^3 workload (None on others)."""
     if not t or t[1] <= 0:
         return None
     n, ms, bytes_l, all_l = t
@@ -342,7 +360,8 @@ def smooth_roofline(t, copy_gbps, gmres: bool = True):
     return {"kernel": name,
             "bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": ach / HBM_PEAK_GBS, "frac_of_copy": ach / copy_gbps, "bytes_per_launch": bytes_l,
-            "mean_ms": ms, "launches": n, "launches_returned_early": all_l - n}
+            "mean_ms": ms, "launches": n, "launches_returned_early": all_l - n,
+            "traffic": level0_traffic(n_lattice, bytes_l) if gmres else None}
 
 
 def stream_copy_gbps(mib: int = 1024, reps: int = 10) -> float:
@@ -790,7 +809,7 @@ def main():
                                "bytes_per_launch": b64, "mean_ms": ms64, "launches": n64,
                                "launches_returned_early": all64 - n64,
                                "traffic": measured_traffic(args.n, 1)},
-        "amg_level0_roofline": smooth_roofline(head.get("smooth"), copy_gbps, bool(kry)),
+        "amg_level0_roofline": smooth_roofline(head.get("smooth"), copy_gbps, args.n, bool(kry)),
         "step_kernels": step_kernels(head, copy_gbps),
         "cloud_setup": setup,
         "weights_kernel_ms": wk[1],
