@@ -17,6 +17,7 @@ namespace mp {
 //   g  > 0: CSR with g lanes per row and a g-lane reduction (long rows of
 //           the coarse operators and restrictions; ptr = row pointers).
 struct KernelTimer;
+struct GmNorm;
 
 struct AmgMat {
     int n = 0, nslices = 0, g = 0;
@@ -106,9 +107,11 @@ struct AmgDevice {
                bool prescaled = false, float* out32 = nullptr);
     // out = M^-1 in on the node block for a Krylov basis vector (FP32 or
     // FP64 values; the border unknown is not touched), written in FP32; the
-    // smoother input w D^-1 in is already in prescaled_input().
+    // smoother input w D^-1 in is already in prescaled_input().  norm: GMRES's
+    // norm step of the previous iteration, run beside the first product.
     template <typename TI>
-    void apply_basis(hipStream_t s, const TI* in, float* out, const int* done_flag);
+    void apply_basis(hipStream_t s, const TI* in, float* out, const int* done_flag,
+                     const GmNorm& norm);
     KernelTimer* post_timer = nullptr;  // times the level-0 post-smoothing product when set
     float* prescaled_input() { return lv.size() > 1 ? lv[0].x.p : nullptr; }
     const float* level0_dinv() const { return lv.empty() ? nullptr : lv[0].dinv.p; }
@@ -116,7 +119,7 @@ struct AmgDevice {
   private:
     template <typename TI, typename TO>
     void vcycle(hipStream_t s, const TI* in, TO* out, const double* border_in, double* border_out,
-                const int* done_flag, bool prescaled, float* out32);
+                const int* done_flag, bool prescaled, float* out32, const GmNorm& norm);
 };
 
 }  // namespace mp

@@ -37,7 +37,7 @@
 // of a row side by side, padding slots with value 0) or CSR with several lanes
 // per row, whichever suits its row lengths.
 #include "amg.hpp"
-#include "krylov.hpp"
+#include "krylov_device.hpp"
 
 #include <chrono>
 #include <cstring>
@@ -47,7 +47,7 @@ namespace mp {
 
 namespace {
 
-enum { OP_PRE = 0, OP_SPMV = 1, OP_POST = 2, OP_PRES = 3, OP_RQ = 4, OP_TPOST = 5 };
+enum { OP_PRE = 0, OP_SPMV = 1, OP_POST = 2, OP_RQ = 4, OP_TPOST = 5 };
 
 __host__ __device__ inline int nblk_rows(int nslices) { return (nslices * SLICE + BLOCK - 1) / BLOCK; }
 
@@ -93,15 +93,15 @@ __device__ __forceinline__ float gathered(int c, const TB* __restrict__ b, const
 // One multigrid product with its epilogue, in either layout (G == 0: SELL-64x4,
 // else CSR with G lanes per row):
 //   OP_PRE : xout = D^-1 b,  res = b - A (D^-1 b)
-//   OP_PRES: res = b - A xin, with xin = D^-1 b already formed
 //   OP_SPMV: out = base + M xin (base may be null and may alias out)
 //   OP_POST: out = xin + D^-1 (b - A xin)
 //   OP_RQ  : xout = M2 xin, res = M xin (M = Q_l in val, M2 = R_{l-1} in val2;
 //            CSR layouts only)
 //   OP_TPOST: out = D^-1 (b + base) + M xin (M = T_l, base = res_l)
 // Level 0 also copies the border unknown (border_in -> border_out).
-template <int G, int OP, typename TB, typename TO>
-__global__ __launch_bounds__(BLOCK) void k_amg_op(MatView m, const float* __restrict__ dinv,
+// WS: wavefronts per slice in the SELL layout (sell4_block).
+template <int G, int OP, typename TB, typename TO, int WS = 1>
+__global__ __launch_bounds__(BLOCK * WS) void k_amg_op(MatView m, const float* __restrict__ dinv,
                                                   const TB* __restrict__ b, const float* xin,
                                                   const float* base, float* __restrict__ xout,
                                                   float* __restrict__ res, TO* out,
@@ -117,12 +117,11 @@ __global__ __launch_bounds__(BLOCK) void k_amg_op(MatView m, const float* __rest
         if (lb < 0) return;
         if (border_out && lb == 0 && threadIdx.x == 0) *border_out = *border_in;
         i = lb * BLOCK + threadIdx.x;
-        const int s = __builtin_amdgcn_readfirstlane(i >> 6);
-        if (s >= m.nslices) return;
-        acc = sell4_accumulate<4, float>(
-            m.ptr, m.col, m.col16, m.cbase, m.val, s, threadIdx.x & 63, [](uint16_t v) { return bf2f(v); },
+        acc = sell4_block<WS, 4, float>(
+            m.nslices, m.ptr, m.col, m.col16, m.cbase, m.val, lb,
+            [](uint16_t v) { return bf2f(v); },
             [=](int c) { return gathered<OP>(c, b, xin, dinv); });
-        if (i >= m.n) return;
+        if (threadIdx.x >= BLOCK || i >= m.n) return;
     } else {
         constexpr int RPB = BLOCK / G;
         const int lb = xcd_block((m.n + RPB - 1) / RPB);
@@ -186,8 +185,6 @@ __global__ __launch_bounds__(BLOCK) void k_amg_op(MatView m, const float* __rest
         const float bi = (float)b[i];
         xout[i] = dinv[i] * bi;
         res[i] = bi - acc;
-    } else if constexpr (OP == OP_PRES) {
-        res[i] = (float)b[i] - acc;
     } else if constexpr (OP == OP_SPMV) {
         out[i] = (TO)(base ? base[i] + acc : acc);
     } else if constexpr (OP == OP_RQ) {
@@ -202,6 +199,41 @@ __global__ __launch_bounds__(BLOCK) void k_amg_op(MatView m, const float* __rest
         out[i] = (TO)y;
         if (out32) out32[i] = y;  // the same values in FP32 (gathered by the Krylov products)
     }
+}
+
+// Level 0's residual res = b - A xin with xin = D^-1 b already formed, in the
+// SELL layout.  The first nx blocks (a multiple of 8, so that the rows keep
+// their XCDs) run GMRES's norm step of the iteration before, a block per
+// system: its 4-6 us of latency then hide behind the product instead of
+// being a launch.  The stop flag the step may raise is read once per block;
+// a block that misses it works on a stopped system, whose V-cycle is ignored.
+template <typename TB, int WS>
+__global__ __launch_bounds__(BLOCK * WS) void k_amg_pres(MatView m, const TB* __restrict__ b,
+                                                         const float* __restrict__ xin,
+                                                         float* __restrict__ res,
+                                                         const double* __restrict__ border_in,
+                                                         double* __restrict__ border_out,
+                                                         const int* done, GmNorm norm, int nx) {
+    if ((int)blockIdx.x < nx) {
+        if ((int)blockIdx.x < norm.sg.nseg)
+            gm_norm_step<BLOCK * WS>(norm.sg, (int)blockIdx.x, norm.partial, norm.gm, norm.fl,
+                                     norm.m);
+        return;
+    }
+    const int lb = xcd_block(nblk_rows(m.nslices), (int)blockIdx.x - nx);
+    if (lb < 0) return;
+    __shared__ int stop;
+    if (threadIdx.x == 0)
+        stop = done ? __hip_atomic_load(done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+    __syncthreads();
+    if (stop) return;
+    if (border_out && lb == 0 && threadIdx.x == 0) *border_out = *border_in;
+    const float acc = sell4_block<WS, 4, float>(
+        m.nslices, m.ptr, m.col, m.col16, m.cbase, m.val, lb, [](uint16_t v) { return bf2f(v); },
+        [xin](int c) { return xin[c]; });
+    const int i = lb * BLOCK + threadIdx.x;
+    if (threadIdx.x >= BLOCK || i >= m.n) return;
+    res[i] = (float)b[i] - acc;
 }
 
 // y = G b on the coarsest level: one wavefront per row.
@@ -301,10 +333,17 @@ void launch_g(hipStream_t st, const AmgMat& M, const float* dinv, const TB* b, c
               double* bout, const int* done, float* out32) {
     const MatView v{M.n, M.nslices, M.ptr, M.col, M.val, M.col16, M.cbase, M.val2};
     int nb;
-    if constexpr (G == 0)
+    if constexpr (G == 0) {
         nb = nblk_rows(M.nslices);
-    else
+        if (nb <= SPLIT_MAX_BLOCKS) {
+            hipLaunchKernelGGL((k_amg_op<0, OP, TB, TO, 4>), dim3(grid_xcd(nb)), dim3(4 * BLOCK),
+                               0, st, v, dinv, b, xin, base, xout, res, out, bin, bout, done,
+                               out32);
+            return;
+        }
+    } else {
         nb = (M.n + BLOCK / G - 1) / (BLOCK / G);
+    }
     hipLaunchKernelGGL((k_amg_op<G, OP, TB, TO>), dim3(grid_xcd(nb)), dim3(BLOCK), 0, st, v, dinv,
                        b, xin, base, xout, res, out, bin, bout, done, out32);
 }
@@ -326,6 +365,19 @@ void launch_op(hipStream_t st, const AmgMat& M, const float* dinv, const TB* b, 
         case 32: launch_g<32, OP>(st, M, dinv, b, xin, base, xout, res, out, bin, bout, done, out32); break;
         default: launch_g<64, OP>(st, M, dinv, b, xin, base, xout, res, out, bin, bout, done, out32); break;
     }
+}
+
+template <typename TB>
+void launch_pres(hipStream_t st, const AmgMat& M, const TB* b, const float* xin, float* res,
+                 const double* bin, double* bout, const int* done, const GmNorm& norm) {
+    const MatView v{M.n, M.nslices, M.ptr, M.col, M.val, M.col16, M.cbase, M.val2};
+    const int nb = nblk_rows(M.nslices), nx = grid_xcd(norm.sg.nseg);
+    if (nb <= SPLIT_MAX_BLOCKS)
+        hipLaunchKernelGGL((k_amg_pres<TB, 4>), dim3(nx + grid_xcd(nb)), dim3(4 * BLOCK), 0, st, v,
+                           b, xin, res, bin, bout, done, norm, nx);
+    else
+        hipLaunchKernelGGL((k_amg_pres<TB, 1>), dim3(nx + grid_xcd(nb)), dim3(BLOCK), 0, st, v, b,
+                           xin, res, bin, bout, done, norm, nx);
 }
 
 struct HostSell {
@@ -985,7 +1037,7 @@ void AmgDevice::apply(hipStream_t st, const double* in, double* out, int bordere
     // a batch copies every border unknown at the end
     const double* bin = (bordered && !blocked) ? in + nv : nullptr;
     double* bout = (bordered && !blocked) ? out + nv : nullptr;
-    vcycle(st, in, out, bin, bout, done, prescaled, out32);
+    vcycle(st, in, out, bin, bout, done, prescaled, out32, GmNorm{});
     if (bordered && blocked && border_rows.n > 0)
         hipLaunchKernelGGL(k_border_copy, dim3((border_rows.n + 63) / 64), dim3(64), 0, st,
                            (int)border_rows.n, border_rows.p, in, out);
@@ -993,16 +1045,19 @@ void AmgDevice::apply(hipStream_t st, const double* in, double* out, int bordere
 }
 
 template <typename TI>
-void AmgDevice::apply_basis(hipStream_t st, const TI* in, float* out, const int* done) {
-    vcycle(st, in, out, nullptr, nullptr, done, true, nullptr);
+void AmgDevice::apply_basis(hipStream_t st, const TI* in, float* out, const int* done,
+                            const GmNorm& norm) {
+    vcycle(st, in, out, nullptr, nullptr, done, true, nullptr, norm);
     MP_HIP(hipGetLastError());
 }
-template void AmgDevice::apply_basis<float>(hipStream_t, const float*, float*, const int*);
-template void AmgDevice::apply_basis<double>(hipStream_t, const double*, float*, const int*);
+template void AmgDevice::apply_basis<float>(hipStream_t, const float*, float*, const int*,
+                                            const GmNorm&);
+template void AmgDevice::apply_basis<double>(hipStream_t, const double*, float*, const int*,
+                                             const GmNorm&);
 
 template <typename TI, typename TO>
 void AmgDevice::vcycle(hipStream_t st, const TI* in, TO* out, const double* bin, double* bout,
-                       const int* done, bool prescaled, float* out32) {
+                       const int* done, bool prescaled, float* out32, const GmNorm& norm) {
     const int L = (int)lv.size();
     auto coarse = [&](const auto* b, auto* y, float* y32, const double* cbin, double* cbout) {
         using TB = std::remove_cv_t<std::remove_pointer_t<decltype(b)>>;
@@ -1017,9 +1072,7 @@ void AmgDevice::vcycle(hipStream_t st, const TI* in, TO* out, const double* bin,
     {  // (setup builds at least two levels)
         // downward: level 0 from the input (FP64, or an FP32 basis vector)
         if (prescaled)
-            launch_op<OP_PRES, TI, float>(st, lv[0].A, nullptr, in, lv[0].x.p, nullptr,
-                                          nullptr, lv[0].res.p, (float*)nullptr, bin, bout,
-                                          done);
+            launch_pres<TI>(st, lv[0].A, in, lv[0].x.p, lv[0].res.p, bin, bout, done, norm);
         else
             launch_op<OP_PRE, TI, float>(st, lv[0].A, lv[0].dinv.p, in, nullptr, nullptr,
                                              lv[0].x.p, lv[0].res.p, (float*)nullptr, bin, bout,

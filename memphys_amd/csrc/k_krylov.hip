@@ -26,67 +26,16 @@
 // term: the rows of a system add x[b] (b = row0 + nv, its border unknown);
 // row b is sum_j D^-1_j x_j over the system's rows, formed by the finishing
 // kernel.
-#include "krylov.hpp"
+#include "krylov_device.hpp"
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstring>
 
 namespace mp {
 
 namespace {
-
-constexpr int FIN = 1024;  // threads of the finishing kernels (one block per system)
-
-// Block sums of NV values stored at partial[q * nb + lb] (lb: logical block)
-// (plain stores: no atomics, the finishing kernel runs after the grid).
-template <int NV>
-__device__ __forceinline__ void block_store(double (&v)[NV], double* __restrict__ partial, int lb,
-                                            int nb) {
-    __shared__ double sh[NV][BLOCK / 64];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-    for (int q = 0; q < NV; ++q)
-        for (int off = 32; off > 0; off >>= 1) v[q] += __shfl_xor(v[q], off);
-    if (lane == 0)
-#pragma unroll
-        for (int q = 0; q < NV; ++q) sh[q][wid] = v[q];
-    __syncthreads();
-    if (threadIdx.x < NV) {
-        const int q = threadIdx.x;
-        double s = sh[q][0];
-        for (int t = 1; t < BLOCK / 64; ++t) s += sh[q][t];
-        partial[(size_t)q * nb + lb] = s;
-    }
-}
-
-// Sum of the partials of blocks [b0, b0 + cnt) per value (stride nb), in a
-// fixed order; every thread of the block receives the totals.
-template <int NV>
-__device__ __forceinline__ void finish_sum(const double* __restrict__ partial, int nb, int b0,
-                                           int cnt, double (&tot)[NV]) {
-    __shared__ double sh[NV][FIN / 64];
-    double acc[NV];
-#pragma unroll
-    for (int q = 0; q < NV; ++q) acc[q] = 0.0;
-    for (int b = threadIdx.x; b < cnt; b += FIN)
-#pragma unroll
-        for (int q = 0; q < NV; ++q) acc[q] += partial[(size_t)q * nb + b0 + b];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-    for (int q = 0; q < NV; ++q)
-        for (int off = 32; off > 0; off >>= 1) acc[q] += __shfl_xor(acc[q], off);
-    if (lane == 0)
-#pragma unroll
-        for (int q = 0; q < NV; ++q) sh[q][wid] = acc[q];
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < NV; ++q) {
-        double s = sh[q][0];
-        for (int t = 1; t < FIN / 64; ++t) s += sh[q][t];
-        tot[q] = s;
-    }
-}
 
 // Loop head of Eigen's BiCGSTAB: convergence / iteration-cap test, then
 // rho_old = rho, rho = r0.r, restart test, beta.  A non-finite residual or a
@@ -118,13 +67,12 @@ __device__ void loop_top(KScalars* sc, double rr, double r0r) {
     sc->beta = (sc->rho / sc->rho_old) * (sc->alpha / sc->omega);
 }
 
-// Row of the SELL-64x4 product A x for slice s, lane = slice row: the slice
-// width is uniform across the wavefront, so the neighbour loop runs in
-// lockstep.  Padding slots hold a zero value and a valid column, which leaves
-// the fma chain unchanged.
-template <typename T, typename TM, typename TX>
+// Rows of the SELL-64x4 product A x over logical block lb (thread t < BLOCK:
+// row lb * BLOCK + t; see sell4_block).  Padding slots hold a zero value and a
+// valid column, which leaves the fma chains unchanged.
+template <int WS, typename T, typename TM, typename TX>
 __device__ __forceinline__ T sell_dot(const SellView& sv, const TM* __restrict__ a,
-                                      const TX* __restrict__ x, int s, int lane) {
+                                      const TX* __restrict__ x, int lb) {
     // FP64 values (stencil order, 32-bit columns): two groups per iteration
     // keep the register count at eight waves per SIMD, and decoding 16-bit
     // columns there would make the compiler serialise the gathers.  FP32
@@ -132,14 +80,16 @@ __device__ __forceinline__ T sell_dot(const SellView& sv, const TM* __restrict__
     // and the 16-bit columns of the view.  x may be an FP32 copy of a vector
     // whose values are FP32 numbers (the V-cycle's output): same sums.
     constexpr bool wide = sizeof(TM) == 8;
-    return sell4_accumulate<(wide ? 2 : 4), T>(
-        sv.sptr, sv.col, wide ? nullptr : sv.col16, sv.cbase, a, s, lane,
+    return sell4_block<WS, (wide ? 2 : 4), T>(
+        sv.nslices, sv.sptr, sv.col, wide ? nullptr : sv.col16, sv.cbase, a, lb,
         [](TM v) { return (T)v; }, [x](int c) { return (T)x[c]; });
 }
 
-// Slice of this wavefront under the XCD-aware numbering (lb: logical block).
-__device__ __forceinline__ int wave_slice(int lb) {
-    return __builtin_amdgcn_readfirstlane(lb * (BLOCK / SLICE) + (int)(threadIdx.x >> 6));
+// This thread's row in logical block lb; past every row for the threads of a
+// block of 4 * BLOCK (WS == 4) beyond the first BLOCK.
+template <int WS>
+__device__ __forceinline__ int block_row(int lb) {
+    return (WS == 1 || threadIdx.x < BLOCK) ? lb * BLOCK + (int)threadIdx.x : INT_MAX;
 }
 
 // System of logical block lb (block-uniform scalar load).
@@ -149,8 +99,8 @@ __device__ __forceinline__ int block_seg(const SegView& sg, int lb) {
 
 // r = rhs - A~ x; r0 = r; p = v = 0 on a fresh start (mode 0, every system
 // taking part); mode 1 restarts the systems flagged with done == 3.
-template <typename TM, typename T>
-__global__ __launch_bounds__(BLOCK) void k_residual_init(
+template <int WS, typename TM, typename T>
+__global__ __launch_bounds__(BLOCK * WS) void k_residual_init(
     SellView sv, SegView sg, const TM* __restrict__ a, const T* __restrict__ dinv,
     const T* __restrict__ rhs, const T* __restrict__ x, T* __restrict__ r, T* __restrict__ r0,
     T* __restrict__ p, T* __restrict__ v, double* __restrict__ partial, const KScalars* sc,
@@ -163,24 +113,21 @@ __global__ __launch_bounds__(BLOCK) void k_residual_init(
     if (mode == 0 ? dn != 0 : dn != 3) return;
     const Seg S = sg.seg[q];
     const int iend = S.row0 + S.nv;
-    const int i = lb * BLOCK + threadIdx.x;
-    const int s = wave_slice(lb);
+    const int i = block_row<WS>(lb);
     double vals[3] = {0.0, 0.0, 0.0};  // r.r, rhs.rhs, sum D^-1 x
-    if (s < sv.nslices) {
-        T ax = sell_dot<T>(sv, a, x, s, threadIdx.x & 63);
-        if (i < iend) {
-            if (S.border) ax = ax + x[iend];
-            const T ri = rhs[i] - ax;
-            r[i] = ri;
-            r0[i] = ri;
-            if (mode == 0) {
-                p[i] = (T)0;
-                v[i] = (T)0;
-            }
-            vals[0] = (double)ri * (double)ri;
-            vals[1] = (double)rhs[i] * (double)rhs[i];
-            if (S.border) vals[2] = (double)dinv[i] * (double)x[i];
+    T ax = sell_dot<WS, T>(sv, a, x, lb);
+    if (i < iend) {
+        if (S.border) ax = ax + x[iend];
+        const T ri = rhs[i] - ax;
+        r[i] = ri;
+        r0[i] = ri;
+        if (mode == 0) {
+            p[i] = (T)0;
+            v[i] = (T)0;
         }
+        vals[0] = (double)ri * (double)ri;
+        vals[1] = (double)rhs[i] * (double)rhs[i];
+        if (S.border) vals[2] = (double)dinv[i] * (double)x[i];
     }
     block_store<3>(vals, partial, lb, nbk);
 }
@@ -259,8 +206,8 @@ __global__ __launch_bounds__(BLOCK) void k_update_p(SegView sg, const T* __restr
 // v = A~ y (y = p, or M^-1 p with the multigrid preconditioner); partial sums
 // of r0.v and of D^-1 y (border row).  yg: y's node rows, gathered (y itself
 // or its FP32 copy); y: the border unknown.
-template <typename TM, typename T, typename TX>
-__global__ __launch_bounds__(BLOCK) void k_spmv_alpha(SellView sv, SegView sg,
+template <int WS, typename TM, typename T, typename TX>
+__global__ __launch_bounds__(BLOCK * WS) void k_spmv_alpha(SellView sv, SegView sg,
                                                       const TM* __restrict__ a,
                                                       const T* __restrict__ dinv,
                                                       const T* __restrict__ y,
@@ -275,17 +222,14 @@ __global__ __launch_bounds__(BLOCK) void k_spmv_alpha(SellView sv, SegView sg,
     if (sc[q].done) return;
     const Seg S = sg.seg[q];
     const int iend = S.row0 + S.nv;
-    const int i = lb * BLOCK + threadIdx.x;
-    const int s = wave_slice(lb);
+    const int i = block_row<WS>(lb);
     double vals[2] = {0.0, 0.0};
-    if (s < sv.nslices) {
-        T yv = sell_dot<T>(sv, a, yg, s, threadIdx.x & 63);
-        if (i < iend) {
-            if (S.border) yv = yv + y[iend];
-            v[i] = yv;
-            vals[0] = (double)r0[i] * (double)yv;
-            if (S.border) vals[1] = (double)dinv[i] * (double)yg[i];
-        }
+    T yv = sell_dot<WS, T>(sv, a, yg, lb);
+    if (i < iend) {
+        if (S.border) yv = yv + y[iend];
+        v[i] = yv;
+        vals[0] = (double)r0[i] * (double)yv;
+        if (S.border) vals[1] = (double)dinv[i] * (double)yg[i];
     }
     block_store<2>(vals, partial, lb, nbk);
 }
@@ -329,8 +273,8 @@ __global__ __launch_bounds__(BLOCK) void k_update_s(SegView sg, const T* __restr
 
 // t = A~ z (z = s, or M^-1 s with the multigrid preconditioner); partial sums
 // of t.s, t.t and D^-1 z
-template <typename TM, typename T, typename TX>
-__global__ __launch_bounds__(BLOCK) void k_spmv_omega(SellView sv, SegView sg,
+template <int WS, typename TM, typename T, typename TX>
+__global__ __launch_bounds__(BLOCK * WS) void k_spmv_omega(SellView sv, SegView sg,
                                                       const TM* __restrict__ a,
                                                       const T* __restrict__ dinv,
                                                       const T* __restrict__ z,
@@ -345,18 +289,15 @@ __global__ __launch_bounds__(BLOCK) void k_spmv_omega(SellView sv, SegView sg,
     if (sc[q].done) return;
     const Seg S = sg.seg[q];
     const int iend = S.row0 + S.nv;
-    const int i = lb * BLOCK + threadIdx.x;
-    const int sl = wave_slice(lb);
+    const int i = block_row<WS>(lb);
     double vals[3] = {0.0, 0.0, 0.0};
-    if (sl < sv.nslices) {
-        T y = sell_dot<T>(sv, a, zg, sl, threadIdx.x & 63);
-        if (i < iend) {
-            if (S.border) y = y + z[iend];
-            t[i] = y;
-            vals[0] = (double)y * (double)s[i];
-            vals[1] = (double)y * (double)y;
-            if (S.border) vals[2] = (double)dinv[i] * (double)zg[i];
-        }
+    T y = sell_dot<WS, T>(sv, a, zg, lb);
+    if (i < iend) {
+        if (S.border) y = y + z[iend];
+        t[i] = y;
+        vals[0] = (double)y * (double)s[i];
+        vals[1] = (double)y * (double)y;
+        if (S.border) vals[2] = (double)dinv[i] * (double)zg[i];
     }
     block_store<3>(vals, partial, lb, nbk);
 }
@@ -418,7 +359,8 @@ __global__ __launch_bounds__(FIN) void k_finish_xr(SegView sg, const double* __r
 }
 
 // out = b - A~ x (FP64) for every system; partial sums of out.out, b.b, D^-1 x
-__global__ __launch_bounds__(BLOCK) void k_residual64(SellView sv, SegView sg,
+template <int WS>
+__global__ __launch_bounds__(BLOCK * WS) void k_residual64(SellView sv, SegView sg,
                                                       const double* __restrict__ a,
                                                       const double* __restrict__ dinv,
                                                       const double* __restrict__ b,
@@ -430,19 +372,16 @@ __global__ __launch_bounds__(BLOCK) void k_residual64(SellView sv, SegView sg,
     if (lb < 0) return;
     const Seg S = sg.seg[block_seg(sg, lb)];
     const int iend = S.row0 + S.nv;
-    const int i = lb * BLOCK + threadIdx.x;
-    const int s = wave_slice(lb);
+    const int i = block_row<WS>(lb);
     double vals[3] = {0.0, 0.0, 0.0};
-    if (s < sv.nslices) {
-        double ax = sell_dot<double>(sv, a, x, s, threadIdx.x & 63);
-        if (i < iend) {
-            if (S.border) ax = ax + x[iend];
-            const double ri = b[i] - ax;
-            out[i] = ri;
-            vals[0] = ri * ri;
-            vals[1] = b[i] * b[i];
-            if (S.border) vals[2] = dinv[i] * x[i];
-        }
+    double ax = sell_dot<WS, double>(sv, a, x, lb);
+    if (i < iend) {
+        if (S.border) ax = ax + x[iend];
+        const double ri = b[i] - ax;
+        out[i] = ri;
+        vals[0] = ri * ri;
+        vals[1] = b[i] * b[i];
+        if (S.border) vals[2] = dinv[i] * x[i];
     }
     block_store<3>(vals, partial, lb, nbk);
 }
@@ -562,6 +501,15 @@ __global__ __launch_bounds__(BLOCK) void k_diag_inverse(int n, const double* __r
 
 inline int nblk(int n) { return (n + BLOCK - 1) / BLOCK; }
 
+// f(wavefronts per slice) for a product over nbk row blocks
+template <typename F>
+void with_split(int nbk, F&& f) {
+    if (nbk <= SPLIT_MAX_BLOCKS)
+        f(std::integral_constant<int, 4>{});
+    else
+        f(std::integral_constant<int, 1>{});
+}
+
 // ---- GMRES(m), right-preconditioned ----
 // Per system: Arnoldi with classical Gram-Schmidt over FP64 basis vectors V
 // (node rows and the border unknown), the Hessenberg column's Givens
@@ -570,7 +518,8 @@ inline int nblk(int n) { return (n + BLOCK - 1) / BLOCK; }
 // ends with x += Z y (no further V-cycle).  A system's kernels return at
 // entry once it has stopped: converged, at its iteration cap, broken down,
 // or with a full cycle waiting for its restart.  Partials: rows 0..GM_MAX-1
-// of the work array hold the dot products, row GM_MAX the border row of A z.
+// of the work array hold the dot products, row GM_MAX the border row of A z,
+// row GM_MAX + 1 the norm of the next basis vector.
 
 __global__ void k_gm_reset(int nseg, GmState* gm, GmFlags* fl, const SegCtl* ctl) {
     const int q = blockIdx.x * 64 + threadIdx.x;
@@ -595,8 +544,8 @@ __global__ void k_gm_reset(int nseg, GmState* gm, GmFlags* fl, const SegCtl* ctl
 // scaling) over the node rows; partial sums of v0.v0, rhs.rhs and the border
 // row's D^-1 x.  x_zero: x is known to be zero (a defect-correction cycle's
 // start), so A x is not formed.
-template <typename TM, typename TV>
-__global__ __launch_bounds__(BLOCK) void k_gm_residual(SellView sv, SegView sg,
+template <int WS, typename TM, typename TV>
+__global__ __launch_bounds__(BLOCK * WS) void k_gm_residual(SellView sv, SegView sg,
                                                        const TM* __restrict__ a,
                                                        const double* __restrict__ dinv,
                                                        const double* __restrict__ rhs,
@@ -614,21 +563,18 @@ __global__ __launch_bounds__(BLOCK) void k_gm_residual(SellView sv, SegView sg,
     if (mode == 0 ? g->done != 0 : !(g->full && g->done == 0)) return;
     const Seg S = sg.seg[q];
     const int iend = S.row0 + S.nv;
-    const int i = lb * BLOCK + threadIdx.x;
-    const int s = wave_slice(lb);
+    const int i = block_row<WS>(lb);
     double vals[3] = {0.0, 0.0, 0.0};
-    if (s < sv.nslices) {
-        double ax = x_zero ? 0.0 : sell_dot<double>(sv, a, x, s, threadIdx.x & 63);
-        if (i < iend) {
-            if (S.border && !x_zero) ax = ax + x[iend];
-            const double ri = rhs[i] - ax;
-            const TV vi = (TV)ri;
-            v0[i] = vi;
-            if (xs) xs[i] = d0 ? d0[i] * (float)vi : (float)vi;
-            vals[0] = ri * ri;
-            vals[1] = rhs[i] * rhs[i];
-            if (S.border && !x_zero) vals[2] = dinv[i] * x[i];
-        }
+    double ax = x_zero ? 0.0 : sell_dot<WS, double>(sv, a, x, lb);
+    if (i < iend) {
+        if (S.border && !x_zero) ax = ax + x[iend];
+        const double ri = rhs[i] - ax;
+        const TV vi = (TV)ri;
+        v0[i] = vi;
+        if (xs) xs[i] = d0 ? d0[i] * (float)vi : (float)vi;
+        vals[0] = ri * ri;
+        vals[1] = rhs[i] * rhs[i];
+        if (S.border && !x_zero) vals[2] = dinv[i] * x[i];
     }
     block_store<3>(vals, partial, lb, nbk);
 }
@@ -691,14 +637,19 @@ __global__ __launch_bounds__(FIN) void k_gm_residual_finish(SegView sg,
 
 // w = A z: node rows (plus the border unknown's column), partial sums of the
 // border row sum D^-1 z; zg: the gathered copy of z (FP32 when z holds FP32
-// values, the V-cycle's output).
-template <typename TM, typename TX, typename TB>
-__global__ __launch_bounds__(BLOCK) void k_gm_spmv(SellView sv, SegView sg,
+// values, the V-cycle's output).  WS == 4 also forms the partial sums of
+// v_k . w, k < nk, from its w rows in LDS, sixteen wavefronts a vector each
+// (k_gm_dots's sums, order and all): for a small system that saves a launch
+// of 4.6 us; at 1M nodes the two kernels apart are faster (67 + 14 us against
+// 83).
+template <int WS, typename TM, typename TX, typename TB>
+__global__ __launch_bounds__(BLOCK * WS) void k_gm_spmv(SellView sv, SegView sg,
                                                    const TM* __restrict__ a,
                                                    const double* __restrict__ dinv,
                                                    const TB* __restrict__ z,
                                                    const TX* __restrict__ zg,
                                                    double* __restrict__ w,
+                                                   const TB* __restrict__ V, size_t ld, int nk,
                                                    double* __restrict__ partial,
                                                    const GmState* gm) {
     const int nbk = sg.nrows / BLOCK;
@@ -708,18 +659,32 @@ __global__ __launch_bounds__(BLOCK) void k_gm_spmv(SellView sv, SegView sg,
     if (gm[q].stop) return;
     const Seg S = sg.seg[q];
     const int iend = S.row0 + S.nv;
-    const int i = lb * BLOCK + threadIdx.x;
-    const int s = wave_slice(lb);
+    const int i = block_row<WS>(lb);
     double vals[1] = {0.0};
-    if (s < sv.nslices) {
-        double y = sell_dot<double>(sv, a, zg, s, threadIdx.x & 63);
-        if (i < iend) {
-            if (S.border) y = y + (double)z[iend];
-            w[i] = y;
-            if (S.border) vals[0] = dinv[i] * (double)zg[i];
-        }
+    double y = sell_dot<WS, double>(sv, a, zg, lb);
+    if (i < iend) {
+        if (S.border) y = y + (double)z[iend];
+        w[i] = y;
+        if (S.border) vals[0] = dinv[i] * (double)zg[i];
     }
-    block_store<1>(vals, partial + (size_t)GM_MAX * nbk, lb, nbk);
+    if constexpr (WS == 4) {
+        __shared__ double sw[BLOCK];
+        if (threadIdx.x < BLOCK) sw[threadIdx.x] = y;
+        block_store<1>(vals, partial + (size_t)GM_MAX * nbk, lb, nbk);  // (a barrier in it)
+        const int lane = threadIdx.x & 63;
+        const int r0 = lb * BLOCK + lane;
+        for (int k = (int)(threadIdx.x >> 6); k < nk; k += BLOCK * WS / 64) {
+            const TB* vk = V + k * ld + r0;
+            double acc = 0.0;
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                if (r0 + 64 * t < iend) acc = fma((double)vk[64 * t], sw[lane + 64 * t], acc);
+            for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
+            if (lane == 0) partial[(size_t)k * nbk + lb] = acc;
+        }
+    } else {
+        block_store<1>(vals, partial + (size_t)GM_MAX * nbk, lb, nbk);
+    }
 }
 
 // partial sums of v_k . w over the node rows, k < nk (the border row is added
@@ -762,6 +727,10 @@ __global__ __launch_bounds__(BLOCK) void k_gm_dots(SegView sg, const double* __r
 // the border row (every 256th partial per thread, four in flight, then a
 // fixed reduction tree).
 constexpr int GMF = 256;  // threads of the Hessenberg-column kernel
+// Row blocks up to which k_gm_orth_h runs: at 40 blocks it takes 5.2 us where
+// the two launches took 3.4 + 4.3; at 249 blocks 8.4 against 3.5 + 4.3, every
+// block then reading more partials than it saves.
+constexpr int ORTH_H_MAX_BLOCKS = 128;
 __device__ __forceinline__ double gm_row_sum(const double* __restrict__ p, int cnt) {
     double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
     int b = threadIdx.x;
@@ -775,6 +744,30 @@ __device__ __forceinline__ double gm_row_sum(const double* __restrict__ p, int c
     double acc = (a0 + a1) + (a2 + a3);
     for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
     return acc;  // per wavefront
+}
+
+// The same sum by one wavefront, standing in for the block's four in turn.
+__device__ __forceinline__ double gm_row_sum_wave(const double* __restrict__ p, int cnt) {
+    double tot = 0.0;
+#pragma unroll
+    for (int u = 0; u < GMF / 64; ++u) {
+        double acc = 0.0;
+        if (64 * u < cnt) {
+            double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
+            int b = (int)(threadIdx.x & 63) + 64 * u;
+            for (; b + 3 * GMF < cnt; b += 4 * GMF) {
+                a0 += p[b];
+                a1 += p[b + GMF];
+                a2 += p[b + 2 * GMF];
+                a3 += p[b + 3 * GMF];
+            }
+            for (; b < cnt; b += GMF) a0 += p[b];
+            acc = (a0 + a1) + (a2 + a3);
+            for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
+        }
+        tot = u == 0 ? acc : tot + acc;
+    }
+    return tot;
 }
 
 template <typename TV>
@@ -815,13 +808,25 @@ __global__ __launch_bounds__(GMF) void k_gm_finish_h(SegView sg, double* __restr
 // The next basis vector, unnormalised: V'_nk = sig[nk-1] w - sum_k hc[k] V'_k
 // over the node rows and the border unknown (rounded to the basis type), the
 // V-cycle's FP32 input (d0 V'_nk, or V'_nk without the scaling) over the node
-// rows, and partial sums of V'_nk . V'_nk (its 1/norm becomes sig[nk]).
+// rows, and partial sums of V'_nk . V'_nk (its 1/norm becomes sig[nk]).  The
+// sum over k is four fma chains (k modulo 4), added as (0 + 1) + (2 + 3).
+// Row i's part of it: wi = sig[nk-1] w - the sum.
+template <typename TV>
+__device__ __forceinline__ double gm_orth_row(double wi, int i, int iend, TV* __restrict__ V,
+                                              size_t ld, int nk, const float* __restrict__ d0,
+                                              float* __restrict__ xs) {
+    const TV v = (TV)wi;
+    V[(size_t)nk * ld + i] = v;
+    if (xs && i < iend) xs[i] = d0 ? d0[i] * (float)v : (float)v;
+    return (double)v * (double)v;
+}
+
 template <typename TV>
 __global__ __launch_bounds__(BLOCK) void k_gm_orth(SegView sg, const double* __restrict__ w,
                                                    TV* __restrict__ V, size_t ld, int nk,
                                                    const float* __restrict__ d0,
                                                    float* __restrict__ xs,
-                                                   double* __restrict__ partial,
+                                                   double* __restrict__ norm_partial,
                                                    const GmState* gm) {
     const int nbk = sg.nrows / BLOCK;
     const int lb = blockIdx.x;
@@ -832,85 +837,92 @@ __global__ __launch_bounds__(BLOCK) void k_gm_orth(SegView sg, const double* __r
     const int i = lb * BLOCK + threadIdx.x;
     double vals[1] = {0.0};
     if (i < S.row0 + S.nv + S.border) {
-        double wi = g->sig[nk - 1] * w[i];
-        for (int k = 0; k < nk; ++k) wi = fma(-g->hc[k], (double)V[k * ld + i], wi);
-        const TV v = (TV)wi;
-        V[(size_t)nk * ld + i] = v;
-        if (xs && i < S.row0 + S.nv) xs[i] = d0 ? d0[i] * (float)v : (float)v;
-        vals[0] = (double)v * (double)v;
+        double t[4] = {0.0, 0.0, 0.0, 0.0};
+        int k = 0;
+        for (; k + 4 <= nk; k += 4)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) t[c] = fma(g->hc[k + c], (double)V[(k + c) * ld + i], t[c]);
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            if (k + c < nk) t[c] = fma(g->hc[k + c], (double)V[(k + c) * ld + i], t[c]);
+        const double wi = g->sig[nk - 1] * w[i] - ((t[0] + t[1]) + (t[2] + t[3]));
+        vals[0] = gm_orth_row(wi, i, S.row0 + S.nv, V, ld, nk, d0, xs);
     }
-    block_store<1>(vals, partial, lb, nbk);
+    block_store<1>(vals, norm_partial, lb, nbk);
 }
 
-// Givens rotation (c, s) with c a + s b = r, -s a + c b = 0
-__device__ __forceinline__ void gm_givens(double a, double b, double& c, double& s, double& r) {
-    if (b == 0.0) {
-        c = 1.0;
-        s = 0.0;
-        r = a;
-    } else {
-        r = hypot(a, b);
-        c = a / r;
-        s = b / r;
-    }
-}
-
-// h_{j+1,j} = |w|; the column's rotations, the new rotation and the residual
-// estimate; then the stopping tests.
-__global__ __launch_bounds__(FIN) void k_gm_finish_norm(SegView sg,
-                                                        const double* __restrict__ partial,
-                                                        GmState* gm, GmFlags* fl, int m) {
-    GmState* g = gm + blockIdx.x;
+// k_gm_finish_h and k_gm_orth in one launch of 1024 threads per block of
+// BLOCK rows: every block forms its system's Hessenberg column from the
+// partials itself (a wavefront per entry, k_gm_finish_h's sums, order and
+// all), then each quarter of the block runs one of the four chains of its
+// rows.  For at most ORTH_H_MAX_BLOCKS row blocks, whose partials a block reads
+// in a few loads.
+template <typename TV>
+__global__ __launch_bounds__(4 * BLOCK) void k_gm_orth_h(SegView sg, const double* __restrict__ w,
+                                                         TV* __restrict__ V, size_t ld, int nk,
+                                                         const double* __restrict__ partial,
+                                                         const float* __restrict__ d0,
+                                                         float* __restrict__ xs,
+                                                         double* __restrict__ norm_partial,
+                                                         GmState* gm) {
+    const int nbk = sg.nrows / BLOCK;
+    const int lb = blockIdx.x;
+    const int q = block_seg(sg, lb);
+    GmState* g = gm + q;
     if (g->stop) return;
-    const Seg S = sg.seg[blockIdx.x];
-    double tot[1];
-    finish_sum<1>(partial, sg.nrows / BLOCK, S.blk0, S.nblk, tot);
-    // the column and the previous rotations into LDS in one parallel load;
-    // the rotations themselves are sequential (thread 0)
-    __shared__ double h[GM_MAX + 1], cs[GM_MAX], sn[GM_MAX];
-    const int j = g->j;
-    if ((int)threadIdx.x <= j) h[threadIdx.x] = g->h[threadIdx.x];
-    if ((int)threadIdx.x < j) {
-        cs[threadIdx.x] = g->cs[threadIdx.x];
-        sn[threadIdx.x] = g->sn[threadIdx.x];
+    const Seg S = sg.seg[q];
+    const int ib = S.row0 + S.nv;
+    __shared__ double sk[GM_MAX + 1], shc[GM_MAX], red[4][BLOCK];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    // entries 0 .. nk-1, then the border row of w (the last wavefront's first)
+    constexpr int NW = 4 * BLOCK / 64;
+    for (int k = wid; k < nk; k += NW) {
+        const double tk = gm_row_sum_wave(partial + (size_t)k * nbk + S.blk0, S.nblk);
+        if (lane == 0) sk[k] = tk;
+    }
+    if (wid == NW - 1) {
+        const double wb =
+            S.border ? gm_row_sum_wave(partial + (size_t)GM_MAX * nbk + S.blk0, S.nblk) : 0.0;
+        if (lane == 0) sk[GM_MAX] = wb;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int i = 0; i < j; ++i) {
-            const double a = h[i], b = h[i + 1];
-            h[i] = cs[i] * a + sn[i] * b;
-            h[i + 1] = -sn[i] * a + cs[i] * b;
+    if ((int)threadIdx.x < nk) {
+        const int k = threadIdx.x;
+        double tk = sk[k];
+        if (S.border) tk += (double)V[k * ld + ib] * sk[GM_MAX];
+        const double h = g->sig[k] * g->sig[nk - 1] * tk;
+        shc[k] = h * g->sig[k];
+        if (lb == S.blk0) {
+            g->h[k] = h;
+            g->hc[k] = shc[k];
         }
     }
     __syncthreads();
-    if ((int)threadIdx.x < j) g->R[j * GM_MAX + threadIdx.x] = h[threadIdx.x];
-    if (threadIdx.x != 0) return;
-    const double eta = sqrt(tot[0]);
-    double c, s, r;
-    gm_givens(h[j], eta, c, s, r);
-    g->cs[j] = c;
-    g->sn[j] = s;
-    g->R[j * GM_MAX + j] = r;
-    g->g[j + 1] = -s * g->g[j];
-    g->g[j] = c * g->g[j];
-    g->j = j + 1;
-    g->iter += 1;
-    const double res2 = g->g[j + 1] * g->g[j + 1];
-    g->rr = res2;
-    g->inv_eta = 1.0 / eta;
-    g->sig[j + 1] = g->inv_eta;
-    if (!(res2 <= 1.0e300) || !(fabs(r) <= 1.0e300))
-        g->done = 5;
-    else if (res2 <= g->tol2)
-        g->done = 1;
-    else if (r == 0.0)
-        g->done = 5;  // singular Hessenberg column
-    else if (g->iter >= g->maxit)
-        g->done = 2;
-    else if (g->j >= m)
-        g->full = 1;
-    g->stop = (g->done != 0 || g->full) ? 1 : 0;
-    fl[blockIdx.x] = GmFlags{g->done, g->full, g->iter, g->cycles};
+    const int t = threadIdx.x & (BLOCK - 1), part = threadIdx.x >> 8;
+    const int i = lb * BLOCK + t;
+    const bool mine = i < ib + S.border;
+    double c = 0.0;
+    if (mine)
+        for (int k = part; k < nk; k += 4) c = fma(shc[k], (double)V[k * ld + i], c);
+    red[part][t] = c;
+    __syncthreads();
+    double vals[1] = {0.0};
+    if (part == 0 && mine) {
+        const double wv = i == ib ? sk[GM_MAX] : w[i];
+        const double wi =
+            g->sig[nk - 1] * wv - ((red[0][t] + red[1][t]) + (red[2][t] + red[3][t]));
+        vals[0] = gm_orth_row(wi, i, ib, V, ld, nk, d0, xs);
+    }
+    block_store<1>(vals, norm_partial, lb, nbk);
+}
+
+// The norm step of the iteration whose Gram-Schmidt update ran last, in a
+// launch of its own (the last iteration of a chunk, whose flags the host polls
+// next; inside a chunk it runs beside the next V-cycle's first product).
+__global__ __launch_bounds__(FIN) void k_gm_finish_norm(SegView sg,
+                                                        const double* __restrict__ partial,
+                                                        GmState* gm, GmFlags* fl, int m) {
+    gm_norm_step<FIN>(sg, (int)blockIdx.x, partial, gm, fl, m);
 }
 
 // end of a cycle: y = R^-1 g over the cycle's columns (back substitution)
@@ -1059,6 +1071,7 @@ void PpeSolver::setup(hipStream_t st, const SellView& view, const std::vector<Se
     nv = 0;
     n_sys = 0;
     bordered = 0;
+    max_nblk = 0;
     std::vector<int> hb(nrows / BLOCK, 0);
     for (int q = 0; q < nseg; ++q) {
         const Seg& S = segs[q];
@@ -1067,6 +1080,7 @@ void PpeSolver::setup(hipStream_t st, const SellView& view, const std::vector<Se
         for (int b = 0; b < S.nblk; ++b) hb[S.blk0 + b] = q;
         nv += S.nv;
         n_sys += S.nv + S.border;
+        max_nblk = std::max(max_nblk, S.nblk);
         bordered |= S.border;
     }
     seg_d.alloc(nseg);
@@ -1251,13 +1265,17 @@ void PpeSolver::launch_chunk(hipStream_t st, int chunk, const TM* a, const T* di
         // with the V-cycle, the products gather its FP32 output (the same values)
         const T* yin = precondition(st, pp, yv.p, y32.p);
         spmv_timer.begin(st);
-        if (amg)
-            hipLaunchKernelGGL((k_spmv_alpha<TM, T, float>), dim3(grid_xcd(nbk)), dim3(BLOCK), 0,
-                               st, view_of<TM>(), sg, a, di, yin, (const float*)y32.p, vv, rr0,
-                               partial.p, sc.p);
-        else
-            hipLaunchKernelGGL((k_spmv_alpha<TM, T, T>), dim3(grid_xcd(nbk)), dim3(BLOCK), 0, st,
-                               view_of<TM>(), sg, a, di, yin, yin, vv, rr0, partial.p, sc.p);
+        with_split(nbk, [&](auto ws) {
+            constexpr int WS = decltype(ws)::value;
+            if (amg)
+                hipLaunchKernelGGL((k_spmv_alpha<WS, TM, T, float>), dim3(grid_xcd(nbk)),
+                                   dim3(BLOCK * WS), 0, st, view_of<TM>(), sg, a, di, yin,
+                                   (const float*)y32.p, vv, rr0, partial.p, sc.p);
+            else
+                hipLaunchKernelGGL((k_spmv_alpha<WS, TM, T, T>), dim3(grid_xcd(nbk)),
+                                   dim3(BLOCK * WS), 0, st, view_of<TM>(), sg, a, di, yin, yin, vv,
+                                   rr0, partial.p, sc.p);
+        });
         spmv_timer.end(st);
         hipLaunchKernelGGL(k_finish_alpha<T>, dim3(nseg), dim3(FIN), 0, st, sg, vv, rr0, partial.p,
                            sc.p);
@@ -1265,13 +1283,17 @@ void PpeSolver::launch_chunk(hipStream_t st, int chunk, const TM* a, const T* di
                            xs);
         const T* zin = precondition(st, ss, zv.p, z32.p);
         spmv_timer.begin(st);
-        if (amg)
-            hipLaunchKernelGGL((k_spmv_omega<TM, T, float>), dim3(grid_xcd(nbk)), dim3(BLOCK), 0,
-                               st, view_of<TM>(), sg, a, di, zin, (const float*)z32.p, ss, tt,
-                               partial.p, sc.p);
-        else
-            hipLaunchKernelGGL((k_spmv_omega<TM, T, T>), dim3(grid_xcd(nbk)), dim3(BLOCK), 0, st,
-                               view_of<TM>(), sg, a, di, zin, zin, ss, tt, partial.p, sc.p);
+        with_split(nbk, [&](auto ws) {
+            constexpr int WS = decltype(ws)::value;
+            if (amg)
+                hipLaunchKernelGGL((k_spmv_omega<WS, TM, T, float>), dim3(grid_xcd(nbk)),
+                                   dim3(BLOCK * WS), 0, st, view_of<TM>(), sg, a, di, zin,
+                                   (const float*)z32.p, ss, tt, partial.p, sc.p);
+            else
+                hipLaunchKernelGGL((k_spmv_omega<WS, TM, T, T>), dim3(grid_xcd(nbk)),
+                                   dim3(BLOCK * WS), 0, st, view_of<TM>(), sg, a, di, zin, zin, ss,
+                                   tt, partial.p, sc.p);
+        });
         spmv_timer.end(st);
         hipLaunchKernelGGL(k_finish_omega<T>, dim3(nseg), dim3(FIN), 0, st, sg, tt, ss, partial.p,
                            sc.p);
@@ -1330,7 +1352,8 @@ template <typename TM, typename TV>
 void PpeSolver::run_gmres_chunk(hipStream_t st, int j, int c, int m, const TM* a,
                                 const double* di) {
     if (!use_graphs || spmv_timer.enabled || smooth_timer.enabled) {  // (events stay out of graphs)
-        for (int k = j; k < j + c; ++k) gmres_iteration<TM, TV>(st, k, m, a, di);
+        for (int k = j; k < j + c; ++k)
+            gmres_iteration<TM, TV>(st, k, m, a, di, k == j, k == j + c - 1);
         return;
     }
     const uintptr_t key[ChunkGraph::KEY] = {
@@ -1338,7 +1361,8 @@ void PpeSolver::run_gmres_chunk(hipStream_t st, int j, int c, int m, const TM* a
         (uintptr_t)a, (uintptr_t)di, (uintptr_t)gm_v.p, (uintptr_t)gm_d.p,
         (uintptr_t)gm_partial.p, (uintptr_t)gm_w.p, (uintptr_t)amg.get()};
     replay_or_capture(st, key, [&]() {
-        for (int k = j; k < j + c; ++k) gmres_iteration<TM, TV>(st, k, m, a, di);
+        for (int k = j; k < j + c; ++k)
+            gmres_iteration<TM, TV>(st, k, m, a, di, k == j, k == j + c - 1);
     });
 }
 
@@ -1358,9 +1382,15 @@ void PpeSolver::run_bicgstab(hipStream_t st, const TM* a, const T* di, const T* 
     const int nbk = nrows / BLOCK;
     MP_HIP(hipMemcpyAsync(ctl_d.p, host_ctl, sizeof(SegCtl) * nseg, hipMemcpyHostToDevice, st));
     hipLaunchKernelGGL(k_sc_reset, dim3((nseg + 63) / 64), dim3(64), 0, st, nseg, sc.p, ctl_d.p);
-    hipLaunchKernelGGL((k_residual_init<TM, T>), dim3(grid_xcd(nbk)), dim3(BLOCK), 0, st,
-                       view_of<TM>(), sg,
-                       a, di, rhs, x, rr, rr0, pp, vv, partial.p, sc.p, 0);
+    auto residual_init = [&](int mode) {
+        with_split(nbk, [&](auto ws) {
+            constexpr int WS = decltype(ws)::value;
+            hipLaunchKernelGGL((k_residual_init<WS, TM, T>), dim3(grid_xcd(nbk)), dim3(BLOCK * WS),
+                               0, st, view_of<TM>(), sg, a, di, rhs, x, rr, rr0, pp, vv, partial.p,
+                               sc.p, mode);
+        });
+    };
+    residual_init(0);
     hipLaunchKernelGGL(k_finish_init<T>, dim3(nseg), dim3(FIN), 0, st, sg, rhs, rr, rr0, pp, vv,
                        partial.p, sc.p, 0, rel_to_rhs);
     MP_HIP(hipGetLastError());
@@ -1385,9 +1415,7 @@ void PpeSolver::run_bicgstab(hipStream_t st, const TM* a, const T* di, const T* 
                 // run, restart those systems with r0 = r = rhs - A x, as Eigen's
                 // BiCGSTAB does (the kernels act on the systems still at done == 3)
                 MP_HIP(hipEventSynchronize(ev[slot]));
-                hipLaunchKernelGGL((k_residual_init<TM, T>), dim3(grid_xcd(nbk)), dim3(BLOCK), 0,
-                                   st, view_of<TM>(), sg, a, di, rhs, x, rr, rr0, pp, vv,
-                                   partial.p, sc.p, 1);
+                residual_init(1);
                 hipLaunchKernelGGL(k_finish_init<T>, dim3(nseg), dim3(FIN), 0, st, sg, rhs, rr,
                                    rr0, pp, vv, partial.p, sc.p, 1, rel_to_rhs);
                 MP_HIP(hipGetLastError());
@@ -1412,15 +1440,23 @@ void PpeSolver::run_bicgstab(hipStream_t st, const TM* a, const T* di, const T* 
     }
 }
 
-// Per-system FP64 residual |b - A x~|^2 and |b|^2 of xt into tmp; waits.
-void PpeSolver::residual64(hipStream_t st, const double* b_dev, std::vector<double>& rr,
-                           std::vector<double>& bb) {
+// b - A x~ (FP64) of xt into tmp, its norm and b's into the scalars.
+void PpeSolver::launch_residual64(hipStream_t st, const double* b_dev) {
     const int nbk = nrows / BLOCK;
-    hipLaunchKernelGGL(k_residual64, dim3(grid_xcd(nbk)), dim3(BLOCK), 0, st, sv, sg, aval.p,
-                       dinv.p, b_dev, xt.p, tmp.p, partial.p);
+    with_split(nbk, [&](auto ws) {
+        constexpr int WS = decltype(ws)::value;
+        hipLaunchKernelGGL(k_residual64<WS>, dim3(grid_xcd(nbk)), dim3(BLOCK * WS), 0, st, sv, sg,
+                           aval.p, dinv.p, b_dev, xt.p, tmp.p, partial.p);
+    });
     hipLaunchKernelGGL(k_finish_res64, dim3(nseg), dim3(FIN), 0, st, sg, b_dev, tmp.p, partial.p,
                        sc.p, xt.p, dinv.p);
     MP_HIP(hipGetLastError());
+}
+
+// Per-system FP64 residual |b - A x~|^2 and |b|^2 of xt into tmp; waits.
+void PpeSolver::residual64(hipStream_t st, const double* b_dev, std::vector<double>& rr,
+                           std::vector<double>& bb) {
+    launch_residual64(st, b_dev);
     MP_HIP(hipMemcpyAsync(host_sc, sc.p, sizeof(KScalars) * nseg, hipMemcpyDeviceToHost, st));
     MP_HIP(hipStreamSynchronize(st));
     rr.resize(nseg);
@@ -1440,11 +1476,7 @@ double PpeSolver::last_residual_norm2(hipStream_t st) {
 double* PpeSolver::residual_of(hipStream_t st, const double* b_dev, const double* x_dev) {
     const int nbk = nrows / BLOCK;
     hipLaunchKernelGGL(k_scale, dim3(nbk), dim3(BLOCK), 0, st, nrows, dinv.p, x_dev, xt.p, 1);
-    hipLaunchKernelGGL(k_residual64, dim3(grid_xcd(nbk)), dim3(BLOCK), 0, st, sv, sg, aval.p,
-                       dinv.p, b_dev, xt.p, tmp.p, partial.p);
-    hipLaunchKernelGGL(k_finish_res64, dim3(nseg), dim3(FIN), 0, st, sg, b_dev, tmp.p, partial.p,
-                       sc.p, xt.p, dinv.p);
-    MP_HIP(hipGetLastError());
+    launch_residual64(st, b_dev);
     return tmp.p;
 }
 
@@ -1460,7 +1492,7 @@ void PpeSolver::gmres_alloc(hipStream_t st, int m) {
     }
     gm_w.alloc(ld);
     MP_HIP(hipMemsetAsync(gm_w.p, 0, sizeof(double) * ld, st));
-    gm_partial.alloc((size_t)(GM_MAX + 1) * (nrows / BLOCK));
+    gm_partial.alloc((size_t)(GM_MAX + 2) * (nrows / BLOCK));
     gm_d.alloc(nseg);
     MP_HIP(hipMemsetAsync(gm_d.p, 0, sizeof(GmState) * nseg, st));
     gmf_d.alloc(nseg);
@@ -1471,39 +1503,60 @@ void PpeSolver::gmres_alloc(hipStream_t st, int m) {
 }
 
 // Iteration k of a GMRES cycle: z_k = M v_k, w = A z_k, Gram-Schmidt against
-// v_0..v_k, the Hessenberg column's rotations, v_{k+1} = w / |w|.
+// v_0..v_k, the Hessenberg column's rotations, v_{k+1} = w / |w|.  With the
+// V-cycle the norm step (norm, rotations, stopping test) of an iteration that
+// is not the chunk's last runs in the next iteration's first product, which
+// does not need it.
 template <typename TM, typename TV>
-void PpeSolver::gmres_iteration(hipStream_t st, int k, int m, const TM* a, const double* di) {
+void PpeSolver::gmres_iteration(hipStream_t st, int k, int m, const TM* a, const double* di,
+                                bool first, bool last) {
     const int nbk = nrows / BLOCK;
     const size_t ld = (size_t)nrows;
     TV* V = reinterpret_cast<TV*>(gm_v.p);
     TV* vk = V + ld * k;
+    double* norm_partial = gm_partial.p + (size_t)(GM_MAX + 1) * nbk;
+    const bool split = nbk <= SPLIT_MAX_BLOCKS;
+    auto product = [&](const auto* zg) {
+        using TX = std::remove_cv_t<std::remove_pointer_t<decltype(zg)>>;
+        spmv_timer.begin(st);
+        with_split(nbk, [&](auto ws) {
+            constexpr int WS = decltype(ws)::value;
+            hipLaunchKernelGGL((k_gm_spmv<WS, TM, TX, TV>), dim3(grid_xcd(nbk)), dim3(BLOCK * WS),
+                               0, st, view_of<TM>(), sg, a, di, (const TV*)vk, zg, gm_w.p,
+                               (const TV*)V, ld, k + 1, gm_partial.p, gm_d.p);
+        });
+        spmv_timer.end(st);
+    };
     if (amg) {
         // one system: its V-cycle stops with it; a batch runs it while any
         // system iterates (the others ignore the result).  The V-cycle reads
         // the basis vector and writes Z'_k in FP32.
         float* zk = gm_z.p + ld * k;
-        amg->apply_basis<TV>(st, vk, zk, nseg == 1 ? &gm_d.p[0].stop : nullptr);
-        spmv_timer.begin(st);
-        hipLaunchKernelGGL((k_gm_spmv<TM, float, TV>), dim3(grid_xcd(nbk)), dim3(BLOCK), 0, st,
-                           view_of<TM>(), sg, a, di, (const TV*)vk, (const float*)zk, gm_w.p,
-                           gm_partial.p, gm_d.p);
+        GmNorm norm;
+        if (!first) norm = GmNorm{sg, norm_partial, gm_d.p, gmf_d.p, m};
+        amg->apply_basis<TV>(st, vk, zk, nseg == 1 ? &gm_d.p[0].stop : nullptr, norm);
+        product((const float*)zk);
     } else {
-        spmv_timer.begin(st);
-        hipLaunchKernelGGL((k_gm_spmv<TM, TV, TV>), dim3(grid_xcd(nbk)), dim3(BLOCK), 0, st,
-                           view_of<TM>(), sg, a, di, (const TV*)vk, (const TV*)vk, gm_w.p,
-                           gm_partial.p, gm_d.p);
+        product((const TV*)vk);
     }
-    spmv_timer.end(st);
-    hipLaunchKernelGGL(k_gm_dots<TV>, dim3(nbk), dim3(BLOCK), 0, st, sg, gm_w.p, (const TV*)V, ld,
-                       k + 1, gm_partial.p, gm_d.p);
-    hipLaunchKernelGGL(k_gm_finish_h<TV>, dim3(nseg * GM_MAX), dim3(GMF), 0, st, sg, gm_w.p,
-                       (const TV*)V, ld, k + 1, gm_partial.p, gm_d.p);
-    hipLaunchKernelGGL(k_gm_orth<TV>, dim3(nbk), dim3(BLOCK), 0, st, sg, (const double*)gm_w.p,
-                       V, ld, k + 1, amg ? amg->level0_dinv() : nullptr,
-                       amg ? amg->prescaled_input() : nullptr, gm_partial.p, gm_d.p);
-    hipLaunchKernelGGL(k_gm_finish_norm, dim3(nseg), dim3(FIN), 0, st, sg, gm_partial.p, gm_d.p,
-                       gmf_d.p, m);
+    if (!split)
+        hipLaunchKernelGGL(k_gm_dots<TV>, dim3(nbk), dim3(BLOCK), 0, st, sg, gm_w.p, (const TV*)V,
+                           ld, k + 1, gm_partial.p, gm_d.p);
+    const float* d0 = amg ? amg->level0_dinv() : nullptr;
+    float* xs = amg ? amg->prescaled_input() : nullptr;
+    if (nbk <= ORTH_H_MAX_BLOCKS) {
+        hipLaunchKernelGGL(k_gm_orth_h<TV>, dim3(nbk), dim3(4 * BLOCK), 0, st, sg,
+                           (const double*)gm_w.p, V, ld, k + 1, (const double*)gm_partial.p, d0,
+                           xs, norm_partial, gm_d.p);
+    } else {
+        hipLaunchKernelGGL(k_gm_finish_h<TV>, dim3(nseg * GM_MAX), dim3(GMF), 0, st, sg, gm_w.p,
+                           (const TV*)V, ld, k + 1, gm_partial.p, gm_d.p);
+        hipLaunchKernelGGL(k_gm_orth<TV>, dim3(nbk), dim3(BLOCK), 0, st, sg,
+                           (const double*)gm_w.p, V, ld, k + 1, d0, xs, norm_partial, gm_d.p);
+    }
+    if (last || !amg)
+        hipLaunchKernelGGL(k_gm_finish_norm, dim3(nseg), dim3(FIN), 0, st, sg, norm_partial,
+                           gm_d.p, gmf_d.p, m);
     MP_HIP(hipGetLastError());
 }
 
@@ -1524,9 +1577,12 @@ void PpeSolver::run_gmres(hipStream_t st, const TM* a, const double* di, const d
     // V'_0 = rhs - A x, sig[0] = 1 / |rhs - A x| for the systems taking part
     // (mode 0), or for those whose full cycle restarts (mode 1)
     auto start = [&](int mode) {
-        hipLaunchKernelGGL((k_gm_residual<TM, TV>), dim3(grid_xcd(nbk)), dim3(BLOCK), 0, st,
-                           view_of<TM>(), sg, a, di, rhs, x, V, d0, xs, gm_partial.p, gm_d.p,
-                           mode, (mode == 0 && x_zero) ? 1 : 0);
+        with_split(nbk, [&](auto ws) {
+            constexpr int WS = decltype(ws)::value;
+            hipLaunchKernelGGL((k_gm_residual<WS, TM, TV>), dim3(grid_xcd(nbk)), dim3(BLOCK * WS),
+                               0, st, view_of<TM>(), sg, a, di, rhs, x, V, d0, xs, gm_partial.p,
+                               gm_d.p, mode, (mode == 0 && x_zero) ? 1 : 0);
+        });
         hipLaunchKernelGGL(k_gm_residual_finish<TV>, dim3(nseg), dim3(FIN), 0, st, sg, rhs, V,
                            gm_partial.p, gm_d.p, gmf_d.p, mode, rel_to_rhs);
         MP_HIP(hipGetLastError());

@@ -78,6 +78,7 @@ struct PpeSolver {
     int nv = 0;      // real rows of all systems
     int n_sys = 0;   // unknowns: real rows + border unknowns
     int nseg = 1, bordered = 0, dim = 0;
+    int max_nblk = 0;  // row blocks of the largest system
     long nnz = 0;    // real stencil entries of the operator
     SellView sv{};
     // column-sorted slot order (set before setup; slot_perm null: none): the
@@ -192,8 +193,10 @@ struct PpeSolver {
                    double* x, int rel_to_rhs, std::vector<int>& done, std::vector<int>& iters,
                    std::vector<int>& restarts, bool x_zero = false);
     template <typename TM, typename TV>
-    void gmres_iteration(hipStream_t s, int k, int m, const TM* aval_t, const double* dinv_t);
+    void gmres_iteration(hipStream_t s, int k, int m, const TM* aval_t, const double* dinv_t,
+                         bool first, bool last);
     void gmres_alloc(hipStream_t s, int m);
+    void launch_residual64(hipStream_t s, const double* b_dev);
     void residual64(hipStream_t s, const double* b_dev, std::vector<double>& rr,
                     std::vector<double>& bb);
     const double* precondition(hipStream_t s, const double* in, double* out, float* out32);

@@ -6,6 +6,7 @@
 #include <cstdint>
 #include <string>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/memphys_hip.h"
@@ -81,11 +82,12 @@ constexpr int NXCD = 8;
 // logical block (b % 8) * ceil(G/8) + b / 8, so each XCD (and its L2) owns a
 // contiguous range of rows.  Returns -1 for the padding blocks.
 __host__ __device__ inline int grid_xcd(int g) { return ((g + NXCD - 1) / NXCD) * NXCD; }
-__device__ __forceinline__ int xcd_block(int g) {
+__device__ __forceinline__ int xcd_block(int g, int block) {
     const int per = (g + NXCD - 1) / NXCD;
-    const int lb = (int)(blockIdx.x % NXCD) * per + (int)(blockIdx.x / NXCD);
+    const int lb = (block % NXCD) * per + block / NXCD;
     return lb < g ? lb : -1;
 }
+__device__ __forceinline__ int xcd_block(int g) { return xcd_block(g, (int)blockIdx.x); }
 
 // SELL-64x4 slot numbering: slice s holds rows 64s..64s+63; neighbour j of
 // slice row l sits at sptr[s] + 256*(j/4) + 4*l + j%4, so each lane reads its
@@ -123,9 +125,11 @@ __device__ __forceinline__ int col_decode(uint32_t e, const int (&b)[CW_COUNT]) 
     return ((w & 4u) ? u1 : u0) + (int)(e & ((1u << CW_BITS) - 1u));
 }
 
-template <typename V>
-__device__ __forceinline__ V load_values(const V* p) {
-    if constexpr (sizeof(V) > 16)
+// Loads of the matrix: non-temporal (NT) keep the gathered vector in L2; the
+// small systems' matrices stay in L2 themselves between two products.
+template <bool NT, typename V>
+__device__ __forceinline__ V load_stream(const V* p) {
+    if constexpr (!NT || sizeof(V) > 16)
         return *p;
     else
         return __builtin_nontemporal_load(p);
@@ -133,26 +137,32 @@ __device__ __forceinline__ V load_values(const V* p) {
 
 // The neighbour loop of one slice row (groups of four slots from slot b0 +
 // 4 lane, w4 groups): load(g) fetches group g's stored columns and decode()
-// turns them into column ids.  The stored columns and the values of U4
-// groups are all requested before the first decode, so their loads overlap.
-template <int U4, typename T, typename TM, typename LD, typename DC, typename FV, typename FX>
-__device__ __forceinline__ T sell4_loop(int b0, int w4, int lane, const TM* __restrict__ a,
-                                        LD load, DC decode, FV fv, FX fx) {
+// turns them into column ids.  A row's sum is four fma chains, chain p over the
+// groups p, p + 4, ..., added as (0 + 1) + (2 + 3).  WS == 1: one wavefront forms
+// all four; the stored columns and the values of U4 groups are requested
+// before the first decode, so their loads overlap.  WS == 4: this wavefront
+// forms chain `part` alone and returns it (two groups in flight); the caller
+// adds the four.  Either way the row's sum has the same bits.
+template <int WS, int U4, typename T, typename TM, typename LD, typename DC, typename FV,
+          typename FX>
+__device__ __forceinline__ T sell4_loop(int b0, int w4, int lane, int part,
+                                        const TM* __restrict__ a, LD load, DC decode, FV fv,
+                                        FX fx) {
     typedef typename Vec4<TM>::type v4;
     typedef decltype(load(0)) raw4;
     const v4* ap = reinterpret_cast<const v4*>(a + b0) + lane;
-    T acc = (T)0;
-    int g = 0;
-    for (; g + U4 <= w4; g += U4) {
-        raw4 e[U4];
-        v4 v[U4];
-        T xv[4 * U4];
+    // acc += the products of N groups g, g + step, ... (chain by chain)
+    auto groups = [&](auto n, int g, int step, T* acc, int astep) {
+        constexpr int N = decltype(n)::value;
+        raw4 e[N];
+        v4 v[N];
+        T xv[4 * N];
 #pragma unroll
-        for (int u = 0; u < U4; ++u) e[u] = load(g + u);
+        for (int u = 0; u < N; ++u) e[u] = load(g + u * step);
 #pragma unroll
-        for (int u = 0; u < U4; ++u) v[u] = load_values(ap + (g + u) * SLICE);
+        for (int u = 0; u < N; ++u) v[u] = load_stream<WS == 1>(ap + (g + u * step) * SLICE);
 #pragma unroll
-        for (int u = 0; u < U4; ++u) {
+        for (int u = 0; u < N; ++u) {
             const typename Vec4<int>::type c = decode(e[u]);
             xv[4 * u + 0] = fx(c.x);
             xv[4 * u + 1] = fx(c.y);
@@ -160,68 +170,139 @@ __device__ __forceinline__ T sell4_loop(int b0, int w4, int lane, const TM* __re
             xv[4 * u + 3] = fx(c.w);
         }
 #pragma unroll
-        for (int u = 0; u < U4; ++u) {
-            acc = fma(fv(v[u].x), xv[4 * u + 0], acc);
-            acc = fma(fv(v[u].y), xv[4 * u + 1], acc);
-            acc = fma(fv(v[u].z), xv[4 * u + 2], acc);
-            acc = fma(fv(v[u].w), xv[4 * u + 3], acc);
+        for (int u = 0; u < N; ++u) {
+            T& s = acc[u * astep];
+            s = fma(fv(v[u].x), xv[4 * u + 0], s);
+            s = fma(fv(v[u].y), xv[4 * u + 1], s);
+            s = fma(fv(v[u].z), xv[4 * u + 2], s);
+            s = fma(fv(v[u].w), xv[4 * u + 3], s);
         }
+    };
+    if constexpr (WS == 4) {
+        T acc = (T)0;
+        int g = part;
+        for (; g + 4 < w4; g += 8) groups(std::integral_constant<int, 2>{}, g, 4, &acc, 0);
+        if (g < w4) groups(std::integral_constant<int, 1>{}, g, 4, &acc, 0);
+        return acc;
+    } else {
+        // U4 == 2 forms chains 0 and 1, then 2 and 3 (two accumulators live)
+        static_assert(WS == 1 && (U4 == 2 || U4 == 4), "");
+        T sum[4 / U4];
+#pragma unroll
+        for (int h = 0; h < 4; h += U4) {
+            T acc[U4];
+#pragma unroll
+            for (int u = 0; u < U4; ++u) acc[u] = (T)0;
+            int g = h;
+            for (; g + U4 <= w4; g += 4) groups(std::integral_constant<int, U4>{}, g, 1, acc, 1);
+#pragma unroll
+            for (int u = 0; u + 1 < U4; ++u)
+                if (g + u < w4) groups(std::integral_constant<int, 1>{}, g + u, 1, acc + u, 1);
+            if constexpr (U4 == 4)
+                sum[0] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+            else
+                sum[h / 2] = acc[0] + acc[1];
+        }
+        if constexpr (U4 == 4)
+            return sum[0];
+        else
+            return sum[0] + sum[1];
     }
-    for (; g < w4; ++g) {
-        const raw4 e = load(g);
-        const v4 v = load_values(ap + g * SLICE);
-        const typename Vec4<int>::type c = decode(e);
-        const T x0 = fx(c.x), x1 = fx(c.y), x2 = fx(c.z), x3 = fx(c.w);
-        acc = fma(fv(v.x), x0, acc);
-        acc = fma(fv(v.y), x1, acc);
-        acc = fma(fv(v.z), x2, acc);
-        acc = fma(fv(v.w), x3, acc);
+}
+
+// Where a slice's slots start, its groups, and its column windows (base[0] < 0:
+// 32-bit columns).  A slice past the matrix has no groups.
+struct SellHead {
+    int b0, w4;
+    int base[CW_COUNT];
+};
+
+// Sum over the neighbours of one slice row of fv(value) * fx(column) (WS == 4:
+// chain `part` of it; see sell4_loop): the slice of head h, lane = slice row.  The
+// four neighbours of a group come in one vector load of columns (16-bit
+// compressed ones when col16 is given and the slice has them) and one of
+// values; U4 groups are loaded before their gathers.  With WS == 1 columns and
+// values up to 4 bytes use non-temporal loads so the gathered vector stays
+// cached; FP64 values (32 bytes a lane, fetched as two 16-byte halves) use ordinary loads,
+// which keep the line in cache between the halves.
+template <int WS, int U4, typename T, typename TM, typename FV, typename FX>
+__device__ __forceinline__ T sell4_accumulate(const SellHead& h, const int* __restrict__ col,
+                                              const uint16_t* __restrict__ col16,
+                                              const TM* __restrict__ a, int lane, int part,
+                                              FV fv, FX fx) {
+    typedef typename Vec4<int>::type c4;
+    typedef typename Vec4<uint16_t>::type e4;
+    if (h.base[0] >= 0) {
+        const e4* ep = reinterpret_cast<const e4*>(col16 + h.b0) + lane;
+        return sell4_loop<WS, U4, T>(
+            h.b0, h.w4, lane, part, a, [&](int g) { return load_stream<WS == 1>(ep + g * SLICE); },
+            [&](e4 e) {
+                c4 c;
+                c.x = col_decode(e.x, h.base);
+                c.y = col_decode(e.y, h.base);
+                c.z = col_decode(e.z, h.base);
+                c.w = col_decode(e.w, h.base);
+                return c;
+            },
+            fv, fx);
+    }
+    const c4* cp = reinterpret_cast<const c4*>(col + h.b0) + lane;
+    return sell4_loop<WS, U4, T>(
+        h.b0, h.w4, lane, part, a, [&](int g) { return load_stream<WS == 1>(cp + g * SLICE); },
+        [](c4 c) { return c; }, fv, fx);
+}
+
+// The head of this wavefront's slice in logical block lb.
+__device__ __forceinline__ SellHead sell4_head(int nslices, const int* __restrict__ sptr,
+                                               const uint16_t* __restrict__ col16,
+                                               const int* __restrict__ cbase, int lb) {
+    SellHead h{0, 0, {-1, 0, 0, 0, 0, 0, 0, 0}};
+    const int s = __builtin_amdgcn_readfirstlane(lb * (BLOCK / SLICE) +
+                                                 (int)((threadIdx.x >> 6) & 3));
+    if (s < nslices) {
+        h.b0 = sptr[s];
+        h.w4 = (sptr[s + 1] - h.b0) >> 8;
+        if (col16 != nullptr)
+#pragma unroll
+            for (int k = 0; k < CW_COUNT; ++k) h.base[k] = cbase[CW_COUNT * s + k];
+    }
+    return h;
+}
+
+// The row sums of one block of BLOCK rows (four slices, logical block lb): row
+// lb * BLOCK + t goes to thread t < BLOCK (zero past nslices).  WS == 1: a block
+// of BLOCK threads, one wavefront per slice.  WS == 4: a block of 4 * BLOCK
+// threads, four wavefronts per slice, one chain each; every thread must call.
+// Four wavefronts per slice are for systems whose slices leave SIMDs idle: the
+// row's serial chain of loads, a few microseconds of latency, is then a
+// quarter as long.
+template <int WS, int U4, typename T, typename TM, typename FV, typename FX>
+__device__ __forceinline__ T sell4_block(int nslices, const int* __restrict__ sptr,
+                                         const int* __restrict__ col,
+                                         const uint16_t* __restrict__ col16,
+                                         const int* __restrict__ cbase,
+                                         const TM* __restrict__ a, int lb, FV fv, FX fx) {
+    const SellHead h = sell4_head(nslices, sptr, col16, cbase, lb);
+    const int lane = (int)(threadIdx.x & 63);
+    const int part = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8));
+    T acc = sell4_accumulate<WS, U4, T>(h, col, col16, a, lane, part, fv, fx);
+    if constexpr (WS == 4) {
+        __shared__ T red[4][BLOCK];
+        const int t = (int)(threadIdx.x & (BLOCK - 1));
+        red[part][t] = acc;
+        __syncthreads();
+        acc = (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]);
     }
     return acc;
 }
 
-// Sum over the neighbours of one slice row, in neighbour order, of
-// fv(value) * fx(column), as an fma chain: slice s, lane = slice row.  The
-// four neighbours of a group come in one vector load of columns (16-bit
-// compressed ones when col16 is given and the slice has them) and one of
-// values; U4 groups are loaded before their gathers.  Columns and values up
-// to 4 bytes use non-temporal loads so the gathered vector stays cached; FP64
-// values (32 bytes a lane, fetched as two 16-byte halves) use ordinary loads,
-// which keep the line in cache between the halves.
-template <int U4, typename T, typename TM, typename FV, typename FX>
-__device__ __forceinline__ T sell4_accumulate(const int* __restrict__ sptr,
-                                              const int* __restrict__ col,
-                                              const uint16_t* __restrict__ col16,
-                                              const int* __restrict__ cbase,
-                                              const TM* __restrict__ a, int s, int lane, FV fv,
-                                              FX fx) {
-    typedef typename Vec4<int>::type c4;
-    typedef typename Vec4<uint16_t>::type e4;
-    const int b0 = sptr[s];
-    const int w4 = (sptr[s + 1] - b0) >> 8;
-    if (col16 != nullptr) {
-        const int* bp = cbase + CW_COUNT * s;
-        const int base[CW_COUNT] = {bp[0], bp[1], bp[2], bp[3], bp[4], bp[5], bp[6], bp[7]};
-        if (base[0] >= 0) {
-            const e4* ep = reinterpret_cast<const e4*>(col16 + b0) + lane;
-            return sell4_loop<U4, T>(
-                b0, w4, lane, a, [&](int g) { return __builtin_nontemporal_load(ep + g * SLICE); },
-                [&](e4 e) {
-                    c4 c;
-                    c.x = col_decode(e.x, base);
-                    c.y = col_decode(e.y, base);
-                    c.z = col_decode(e.z, base);
-                    c.w = col_decode(e.w, base);
-                    return c;
-                },
-                fv, fx);
-        }
-    }
-    const c4* cp = reinterpret_cast<const c4*>(col + b0) + lane;
-    return sell4_loop<U4, T>(
-        b0, w4, lane, a, [&](int g) { return __builtin_nontemporal_load(cp + g * SLICE); },
-        [](c4 c) { return c; }, fv, fx);
-}
+// Blocks of BLOCK rows up to which a product runs with four wavefronts per
+// slice: 1024 blocks are 4 wavefronts per SIMD with one per slice.  One
+// against four wavefronts per slice: level-0 residual of a 64k-node cube (249
+// blocks) 11.7 and 9.3 us, of a 216k-node cube (843 blocks) 21.4 and 19.2 us;
+// GMRES product and dot products 17.4 (two launches) and 10.6 us, and 38.3 and
+// 29.2 us.
+constexpr int SPLIT_MAX_BLOCKS = 1024;
 
 // SELL-64x4 view of the stencil set in device order.
 struct SellView {

@@ -161,8 +161,9 @@ def steps(db: str, marker: str = "predictor_kernel", last: int = 0) -> str:
             else:
                 if "k_amg" in name:
                     # the finest level's two smoothing products (SELL layout,
-                    # one lane per row: their grid is the marker's)
-                    l0 = ("k_amg_op<0, 2" in name or "k_amg_op<0, 3" in name) and g >= grid
+                    # at least one lane per row: their grid covers the marker's)
+                    l0 = any(k in name for k in ("k_amg_op<0, 2", "k_amg_op<0, 3", "k_amg_pres",
+                                                 "k_amg_op<0, 5")) and g >= grid
                     per["mg l0 smooth" if l0 else "multigrid other"] += e - s
                 else:
                     per["other"] += e - s
