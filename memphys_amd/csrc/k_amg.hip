@@ -51,6 +51,12 @@ enum { OP_PRE = 0, OP_SPMV = 1, OP_POST = 2, OP_RQ = 4, OP_TPOST = 5 };
 
 __host__ __device__ inline int nblk_rows(int nslices) { return (nslices * SLICE + BLOCK - 1) / BLOCK; }
 
+// Blocks of a product of shape WS.
+template <int WS>
+__host__ __device__ inline int ws_blocks(int nslices) {
+    return WS == 4 ? nslices : nblk_rows(nslices);
+}
+
 __device__ __forceinline__ bool stopped(const int* done) { return done && *done; }
 
 struct MatView {
@@ -99,9 +105,9 @@ __device__ __forceinline__ float gathered(int c, const TB* __restrict__ b, const
 //            CSR layouts only)
 //   OP_TPOST: out = D^-1 (b + base) + M xin (M = T_l, base = res_l)
 // Level 0 also copies the border unknown (border_in -> border_out).
-// WS: wavefronts per slice in the SELL layout (sell4_block).
+// WS: the block shape in the SELL layout (1 or 4).
 template <int G, int OP, typename TB, typename TO, int WS = 1>
-__global__ __launch_bounds__(BLOCK * WS) void k_amg_op(MatView m, const float* __restrict__ dinv,
+__global__ __launch_bounds__(BLOCK) void k_amg_op(MatView m, const float* __restrict__ dinv,
                                                   const TB* __restrict__ b, const float* xin,
                                                   const float* base, float* __restrict__ xout,
                                                   float* __restrict__ res, TO* out,
@@ -113,15 +119,15 @@ __global__ __launch_bounds__(BLOCK * WS) void k_amg_op(MatView m, const float* _
     int i;
     if constexpr (G == 0) {
         static_assert(OP != OP_RQ, "two value arrays: CSR layouts only");
-        const int lb = xcd_block(nblk_rows(m.nslices));
+        const int lb = xcd_block(ws_blocks<WS>(m.nslices));
         if (lb < 0) return;
         if (border_out && lb == 0 && threadIdx.x == 0) *border_out = *border_in;
-        i = lb * BLOCK + threadIdx.x;
+        i = block_row<WS>(lb);
         acc = sell4_block<WS, 4, float>(
             m.nslices, m.ptr, m.col, m.col16, m.cbase, m.val, lb,
             [](uint16_t v) { return bf2f(v); },
             [=](int c) { return gathered<OP>(c, b, xin, dinv); });
-        if (threadIdx.x >= BLOCK || i >= m.n) return;
+        if (i >= m.n) return;
     } else {
         constexpr int RPB = BLOCK / G;
         const int lb = xcd_block((m.n + RPB - 1) / RPB);
@@ -208,7 +214,7 @@ __global__ __launch_bounds__(BLOCK * WS) void k_amg_op(MatView m, const float* _
 // being a launch.  The stop flag the step may raise is read once per block;
 // a block that misses it works on a stopped system, whose V-cycle is ignored.
 template <typename TB, int WS>
-__global__ __launch_bounds__(BLOCK * WS) void k_amg_pres(MatView m, const TB* __restrict__ b,
+__global__ __launch_bounds__(BLOCK) void k_amg_pres(MatView m, const TB* __restrict__ b,
                                                          const float* __restrict__ xin,
                                                          float* __restrict__ res,
                                                          const double* __restrict__ border_in,
@@ -216,11 +222,11 @@ __global__ __launch_bounds__(BLOCK * WS) void k_amg_pres(MatView m, const TB* __
                                                          const int* done, GmNorm norm, int nx) {
     if ((int)blockIdx.x < nx) {
         if ((int)blockIdx.x < norm.sg.nseg)
-            gm_norm_step<BLOCK * WS>(norm.sg, (int)blockIdx.x, norm.partial, norm.gm, norm.fl,
+            gm_norm_step<BLOCK>(norm.sg, (int)blockIdx.x, norm.partial, norm.gm, norm.fl,
                                      norm.m);
         return;
     }
-    const int lb = xcd_block(nblk_rows(m.nslices), (int)blockIdx.x - nx);
+    const int lb = xcd_block(ws_blocks<WS>(m.nslices), (int)blockIdx.x - nx);
     if (lb < 0) return;
     __shared__ int stop;
     if (threadIdx.x == 0)
@@ -231,8 +237,8 @@ __global__ __launch_bounds__(BLOCK * WS) void k_amg_pres(MatView m, const TB* __
     const float acc = sell4_block<WS, 4, float>(
         m.nslices, m.ptr, m.col, m.col16, m.cbase, m.val, lb, [](uint16_t v) { return bf2f(v); },
         [xin](int c) { return xin[c]; });
-    const int i = lb * BLOCK + threadIdx.x;
-    if (threadIdx.x >= BLOCK || i >= m.n) return;
+    const int i = block_row<WS>(lb);
+    if (i >= m.n) return;
     res[i] = (float)b[i] - acc;
 }
 
@@ -336,9 +342,9 @@ void launch_g(hipStream_t st, const AmgMat& M, const float* dinv, const TB* b, c
     if constexpr (G == 0) {
         nb = nblk_rows(M.nslices);
         if (nb <= SPLIT_MAX_BLOCKS) {
-            hipLaunchKernelGGL((k_amg_op<0, OP, TB, TO, 4>), dim3(grid_xcd(nb)), dim3(4 * BLOCK),
-                               0, st, v, dinv, b, xin, base, xout, res, out, bin, bout, done,
-                               out32);
+            hipLaunchKernelGGL((k_amg_op<0, OP, TB, TO, 4>), dim3(grid_xcd(M.nslices)),
+                               dim3(BLOCK), 0, st, v, dinv, b, xin, base, xout, res, out, bin,
+                               bout, done, out32);
             return;
         }
     } else {
@@ -373,8 +379,8 @@ void launch_pres(hipStream_t st, const AmgMat& M, const TB* b, const float* xin,
     const MatView v{M.n, M.nslices, M.ptr, M.col, M.val, M.col16, M.cbase, M.val2};
     const int nb = nblk_rows(M.nslices), nx = grid_xcd(norm.sg.nseg);
     if (nb <= SPLIT_MAX_BLOCKS)
-        hipLaunchKernelGGL((k_amg_pres<TB, 4>), dim3(nx + grid_xcd(nb)), dim3(4 * BLOCK), 0, st, v,
-                           b, xin, res, bin, bout, done, norm, nx);
+        hipLaunchKernelGGL((k_amg_pres<TB, 4>), dim3(nx + grid_xcd(M.nslices)), dim3(BLOCK), 0, st,
+                           v, b, xin, res, bin, bout, done, norm, nx);
     else
         hipLaunchKernelGGL((k_amg_pres<TB, 1>), dim3(nx + grid_xcd(nb)), dim3(BLOCK), 0, st, v, b,
                            xin, res, bin, bout, done, norm, nx);

@@ -67,8 +67,8 @@ __device__ void loop_top(KScalars* sc, double rr, double r0r) {
     sc->beta = (sc->rho / sc->rho_old) * (sc->alpha / sc->omega);
 }
 
-// Rows of the SELL-64x4 product A x over logical block lb (thread t < BLOCK:
-// row lb * BLOCK + t; see sell4_block).  Padding slots hold a zero value and a
+// Rows of the SELL-64x4 product A x over logical block lb (row block_row<WS>(lb)
+// to its thread; see sell4_block).  Padding slots hold a zero value and a
 // valid column, which leaves the fma chains unchanged.
 template <int WS, typename T, typename TM, typename TX>
 __device__ __forceinline__ T sell_dot(const SellView& sv, const TM* __restrict__ a,
@@ -85,33 +85,45 @@ __device__ __forceinline__ T sell_dot(const SellView& sv, const TM* __restrict__
         [](TM v) { return (T)v; }, [x](int c) { return (T)x[c]; });
 }
 
-// This thread's row in logical block lb; past every row for the threads of a
-// block of 4 * BLOCK (WS == 4) beyond the first BLOCK.
-template <int WS>
-__device__ __forceinline__ int block_row(int lb) {
-    return (WS == 1 || threadIdx.x < BLOCK) ? lb * BLOCK + (int)threadIdx.x : INT_MAX;
+// The same product with gathered entries made of several vectors' entries
+// (sell4_block_early).
+template <typename T, typename TM, typename PRE, typename MID, typename FIN>
+__device__ __forceinline__ T sell_dot_early(const SellView& sv, const TM* __restrict__ a, int lb,
+                                            PRE pre, MID mid, FIN fin, bool& ok) {
+    return sell4_block_early<T>(sv.nslices, sv.sptr, sv.col,
+                                sizeof(TM) == 8 ? nullptr : sv.col16, sv.cbase, a, lb, pre, mid,
+                                fin, ok);
 }
 
-// System of logical block lb (block-uniform scalar load).
-__device__ __forceinline__ int block_seg(const SegView& sg, int lb) {
-    return __builtin_amdgcn_readfirstlane(sg.bseg[lb]);
+// The product's partial sums come per slice (shape 4).
+__device__ __forceinline__ bool by_slices(const SegView& sg) {
+    return sg.nrows / BLOCK <= SPLIT_MAX_BLOCKS;
+}
+// Blocks of a product of shape WS over sg's rows, and their system.
+template <int WS>
+__device__ __forceinline__ int ws_blocks(const SegView& sg) {
+    return sg.nrows / WS_ROWS<WS>;
+}
+template <int WS>
+__device__ __forceinline__ int ws_seg(const SegView& sg, int lb) {
+    return block_seg(sg, WS == 4 ? lb / (BLOCK / SLICE) : lb);
 }
 
 // r = rhs - A~ x; r0 = r; p = v = 0 on a fresh start (mode 0, every system
 // taking part); mode 1 restarts the systems flagged with done == 3.
 template <int WS, typename TM, typename T>
-__global__ __launch_bounds__(BLOCK * WS) void k_residual_init(
+__global__ __launch_bounds__(WS_THREADS<WS>) void k_residual_init(
     SellView sv, SegView sg, const TM* __restrict__ a, const T* __restrict__ dinv,
     const T* __restrict__ rhs, const T* __restrict__ x, T* __restrict__ r, T* __restrict__ r0,
     T* __restrict__ p, T* __restrict__ v, double* __restrict__ partial, const KScalars* sc,
     int mode) {
-    const int nbk = sg.nrows / BLOCK;
+    const int nbk = ws_blocks<WS>(sg);
     const int lb = xcd_block(nbk);
     if (lb < 0) return;
-    const int q = block_seg(sg, lb);
+    const int q = ws_seg<WS>(sg, lb);
     const int dn = sc[q].done;
     if (mode == 0 ? dn != 0 : dn != 3) return;
-    const Seg S = sg.seg[q];
+    const Seg S = seg_at(sg, q);
     const int iend = S.row0 + S.nv;
     const int i = block_row<WS>(lb);
     double vals[3] = {0.0, 0.0, 0.0};  // r.r, rhs.rhs, sum D^-1 x
@@ -129,7 +141,7 @@ __global__ __launch_bounds__(BLOCK * WS) void k_residual_init(
         vals[1] = (double)rhs[i] * (double)rhs[i];
         if (S.border) vals[2] = (double)dinv[i] * (double)x[i];
     }
-    block_store<3>(vals, partial, lb, nbk);
+    block_store<3, WS>(vals, partial, lb, nbk);
 }
 
 template <typename T>
@@ -141,9 +153,9 @@ __global__ __launch_bounds__(FIN) void k_finish_init(SegView sg, const T* __rest
     KScalars* sc = scs + blockIdx.x;
     const int dn = sc->done;
     if (mode == 0 ? dn != 0 : dn != 3) return;
-    const Seg S = sg.seg[blockIdx.x];
+    const Seg S = seg_at(sg, (int)blockIdx.x);
     double tot[3];
-    finish_sum<3>(partial, sg.nrows / BLOCK, S.blk0, S.nblk, tot);
+    finish_sum<3>(partial, sg.nrows / BLOCK, S.blk0, S.nblk, tot, by_slices(sg));
     if (threadIdx.x != 0) return;
     double rr = tot[0], bb = tot[1];
     if (S.border) {
@@ -200,14 +212,14 @@ __global__ __launch_bounds__(BLOCK) void k_update_p(SegView sg, const T* __restr
     const T beta = (T)sc->beta, w = (T)sc->omega;
     const T pi = r[i] + beta * (p[i] - w * v[i]);
     p[i] = pi;
-    if (xs && i < sg.seg[q].row0 + sg.seg[q].nv) xs[i] = d0[i] * (float)pi;  // V-cycle input
+    if (xs && i < seg_at(sg, q).row0 + seg_at(sg, q).nv) xs[i] = d0[i] * (float)pi;  // V-cycle input
 }
 
 // v = A~ y (y = p, or M^-1 p with the multigrid preconditioner); partial sums
 // of r0.v and of D^-1 y (border row).  yg: y's node rows, gathered (y itself
 // or its FP32 copy); y: the border unknown.
 template <int WS, typename TM, typename T, typename TX>
-__global__ __launch_bounds__(BLOCK * WS) void k_spmv_alpha(SellView sv, SegView sg,
+__global__ __launch_bounds__(WS_THREADS<WS>) void k_spmv_alpha(SellView sv, SegView sg,
                                                       const TM* __restrict__ a,
                                                       const T* __restrict__ dinv,
                                                       const T* __restrict__ y,
@@ -215,12 +227,12 @@ __global__ __launch_bounds__(BLOCK * WS) void k_spmv_alpha(SellView sv, SegView 
                                                       const T* __restrict__ r0,
                                                       double* __restrict__ partial,
                                                       const KScalars* sc) {
-    const int nbk = sg.nrows / BLOCK;
+    const int nbk = ws_blocks<WS>(sg);
     const int lb = xcd_block(nbk);
     if (lb < 0) return;
-    const int q = block_seg(sg, lb);
+    const int q = ws_seg<WS>(sg, lb);
     if (sc[q].done) return;
-    const Seg S = sg.seg[q];
+    const Seg S = seg_at(sg, q);
     const int iend = S.row0 + S.nv;
     const int i = block_row<WS>(lb);
     double vals[2] = {0.0, 0.0};
@@ -231,7 +243,7 @@ __global__ __launch_bounds__(BLOCK * WS) void k_spmv_alpha(SellView sv, SegView 
         vals[0] = (double)r0[i] * (double)yv;
         if (S.border) vals[1] = (double)dinv[i] * (double)yg[i];
     }
-    block_store<2>(vals, partial, lb, nbk);
+    block_store<2, WS>(vals, partial, lb, nbk);
 }
 
 template <typename T>
@@ -241,9 +253,9 @@ __global__ __launch_bounds__(FIN) void k_finish_alpha(SegView sg, T* __restrict_
                                                       KScalars* scs) {
     KScalars* sc = scs + blockIdx.x;
     if (sc->done) return;
-    const Seg S = sg.seg[blockIdx.x];
+    const Seg S = seg_at(sg, (int)blockIdx.x);
     double tot[2];
-    finish_sum<2>(partial, sg.nrows / BLOCK, S.blk0, S.nblk, tot);
+    finish_sum<2>(partial, sg.nrows / BLOCK, S.blk0, S.nblk, tot, by_slices(sg));
     if (threadIdx.x != 0) return;
     double r0v = tot[0];
     if (S.border) {
@@ -268,13 +280,13 @@ __global__ __launch_bounds__(BLOCK) void k_update_s(SegView sg, const T* __restr
     const int i = blockIdx.x * BLOCK + threadIdx.x;
     const T si = r[i] - (T)sc->alpha * v[i];
     s[i] = si;
-    if (xs && i < sg.seg[q].row0 + sg.seg[q].nv) xs[i] = d0[i] * (float)si;  // V-cycle input
+    if (xs && i < seg_at(sg, q).row0 + seg_at(sg, q).nv) xs[i] = d0[i] * (float)si;  // V-cycle input
 }
 
 // t = A~ z (z = s, or M^-1 s with the multigrid preconditioner); partial sums
 // of t.s, t.t and D^-1 z
 template <int WS, typename TM, typename T, typename TX>
-__global__ __launch_bounds__(BLOCK * WS) void k_spmv_omega(SellView sv, SegView sg,
+__global__ __launch_bounds__(WS_THREADS<WS>) void k_spmv_omega(SellView sv, SegView sg,
                                                       const TM* __restrict__ a,
                                                       const T* __restrict__ dinv,
                                                       const T* __restrict__ z,
@@ -282,12 +294,12 @@ __global__ __launch_bounds__(BLOCK * WS) void k_spmv_omega(SellView sv, SegView 
                                                       const T* __restrict__ s, T* __restrict__ t,
                                                       double* __restrict__ partial,
                                                       const KScalars* sc) {
-    const int nbk = sg.nrows / BLOCK;
+    const int nbk = ws_blocks<WS>(sg);
     const int lb = xcd_block(nbk);
     if (lb < 0) return;
-    const int q = block_seg(sg, lb);
+    const int q = ws_seg<WS>(sg, lb);
     if (sc[q].done) return;
-    const Seg S = sg.seg[q];
+    const Seg S = seg_at(sg, q);
     const int iend = S.row0 + S.nv;
     const int i = block_row<WS>(lb);
     double vals[3] = {0.0, 0.0, 0.0};
@@ -299,7 +311,7 @@ __global__ __launch_bounds__(BLOCK * WS) void k_spmv_omega(SellView sv, SegView 
         vals[1] = (double)y * (double)y;
         if (S.border) vals[2] = (double)dinv[i] * (double)zg[i];
     }
-    block_store<3>(vals, partial, lb, nbk);
+    block_store<3, WS>(vals, partial, lb, nbk);
 }
 
 template <typename T>
@@ -309,9 +321,9 @@ __global__ __launch_bounds__(FIN) void k_finish_omega(SegView sg, T* __restrict_
                                                       KScalars* scs) {
     KScalars* sc = scs + blockIdx.x;
     if (sc->done) return;
-    const Seg S = sg.seg[blockIdx.x];
+    const Seg S = seg_at(sg, (int)blockIdx.x);
     double tot[3];
-    finish_sum<3>(partial, sg.nrows / BLOCK, S.blk0, S.nblk, tot);
+    finish_sum<3>(partial, sg.nrows / BLOCK, S.blk0, S.nblk, tot, by_slices(sg));
     if (threadIdx.x != 0) return;
     double ts = tot[0], tt = tot[1];
     if (S.border) {
@@ -346,31 +358,372 @@ __global__ __launch_bounds__(BLOCK) void k_update_xr(SegView sg, T* __restrict__
     block_store<2>(vals, partial, blockIdx.x, gridDim.x);
 }
 
+// (fused: only the systems whose last iteration is pending)
 __global__ __launch_bounds__(FIN) void k_finish_xr(SegView sg, const double* __restrict__ partial,
-                                                   KScalars* scs) {
+                                                   KScalars* scs, int fused) {
     KScalars* sc = scs + blockIdx.x;
-    if (sc->done) return;
-    const Seg S = sg.seg[blockIdx.x];
+    if (sc->done || (fused && !sc->pending)) return;
+    const Seg S = seg_at(sg, (int)blockIdx.x);
     double tot[2];
     finish_sum<2>(partial, sg.nrows / BLOCK, S.blk0, S.nblk, tot);
     if (threadIdx.x != 0) return;
     sc->iter += 1;
+    sc->pending = 0;
     loop_top(sc, tot[0], tot[1]);
+}
+
+// ---- fused iterations ----
+// On a small system every launch is 2-5 us of latency, and eight a BiCGSTAB
+// iteration (28 us at 10k nodes) are most of its time.  Here the finishing
+// reductions run in the kernel that needs their scalars: every block sums its
+// system's partials itself (finish_sum's order, so the scalars have the same
+// bits), and the system's first block writes the new state.  A kernel reads
+// one record of the state and writes another (A -> B -> C -> A), and likewise
+// reads one group of partial sums and writes another, so no block sees a
+// neighbour's update.  The last finish of an iteration (r.r, r0.r and the loop
+// head) waits in the partials for the next iteration's first kernel, or for
+// k_finish_xr at the end of a chunk.
+//
+// Two forms with the eight kernels' arithmetic:
+//  - five launches: p-update, product, s-update, product, x/r-update;
+//  - three, for systems whose operator the L2s hold: the products form p and s
+//    at the gathered columns (three and two gathers instead of one), p and v
+//    alternating between two buffers because neighbours still read the old.
+// rows (of one double per block) of the partial sums: the products' are per slice
+constexpr int BI_XR = 0, BI_ALPHA = 4, BI_OMEGA = 12, BI_ROWS = 24;
+constexpr int FUSE_MAX_BLOCKS = SPLIT_MAX_BLOCKS;  // (the products' partials per slice)
+// Row blocks up to which the three-launch form runs.  An iteration in 8, 5 and
+// 3 launches: 10k 2D nodes (40 blocks) 27.5, - and 15.9 us; 17k (67) -, 19.9 and
+// 18.8; 40k (157) -, 21.8 and 21.8; 37k 3D (146) -, 25.6 and 29.0; 110k 3D (414)
+// 47, 41 and 52: the extra gathers grow with the system, the launches do not.
+constexpr int FUSE3_MAX_BLOCKS = 96;
+
+// The scalars a kernel of a fused iteration works with, and what it changes
+// in the state.
+struct FusedState {
+    double alpha, beta, omega, rr, rho, rho_old;
+    int done, iter, pending, par;
+};
+
+// The new record, by one thread at the end of the system's first block (a
+// wavefront without rows where the block has one: the copy's latency then
+// delays nobody).
+template <int WS>
+__device__ __forceinline__ bool fused_writer(const Seg& S, int lb) {
+    return WS == 4 ? lb == S.blk0 * (BLOCK / SLICE) && threadIdx.x == BLOCK - 64
+                   : lb == S.blk0 && threadIdx.x == 0;
+}
+__device__ __forceinline__ void fused_store(const KScalars* __restrict__ in,
+                                            KScalars* __restrict__ out, const FusedState& k) {
+    *out = *in;
+    out->alpha = k.alpha;
+    out->beta = k.beta;
+    out->omega = k.omega;
+    out->rr = k.rr;
+    out->rho = k.rho;
+    out->rho_old = k.rho_old;
+    out->done = k.done;
+    out->iter = k.iter;
+    out->pending = k.pending;
+    out->par = k.par;
+}
+__device__ __forceinline__ FusedState fused_load(const KScalars* __restrict__ in) {
+    return FusedState{in->alpha, in->beta,    in->omega, in->rr,      in->rho,
+                      in->rho_old, in->done, in->iter,  in->pending, in->par};
+}
+
+// Loop head of the system (record A): loop_top's tests and scalars, by every
+// thread.  flip: the three-launch form's change of buffers.
+template <int NT>
+__device__ __forceinline__ void fused_head(const SegView& sg, const Seg& S,
+                                           const double* __restrict__ partial,
+                                           const KScalars* __restrict__ in, FusedState& k,
+                                           int flip) {
+    const int nbk = sg.nrows / BLOCK;
+    if (!k.done && k.pending) {
+        double tot[2];
+        finish_sum<2, NT>(partial + (size_t)BI_XR * nbk, nbk, S.blk0, S.nblk, tot);
+        k.iter += 1;
+        k.pending = 0;
+        k.rr = tot[0];
+        if (!(k.rr <= 1.0e300))
+            k.done = 5;
+        else if (k.rr <= in->tol2)
+            k.done = 1;
+        else if (k.iter >= in->maxit)
+            k.done = 2;
+        else if (k.omega == 0.0)
+            k.done = 5;
+        else {
+            k.rho_old = k.rho;
+            k.rho = tot[1];
+            if (fabs(k.rho) < in->eps2 * in->r0sq)
+                k.done = 3;
+            else
+                k.beta = (k.rho / k.rho_old) * (k.alpha / k.omega);
+        }
+    }
+    if (!k.done) k.par ^= flip;
+}
+
+// alpha (and v's border entry vb) of a running system (record B).
+template <int NT, typename T>
+__device__ __forceinline__ void fused_alpha(const SegView& sg, const Seg& S,
+                                            const double* __restrict__ partial,
+                                            const T* __restrict__ r0, FusedState& k, T& vb) {
+    const int nbk = sg.nrows / BLOCK;
+    const double r0b = S.border ? (double)r0[S.row0 + S.nv] : 0.0;
+    double tot[2];
+    finish_sum<2, NT>(partial + (size_t)BI_ALPHA * nbk, nbk, S.blk0, S.nblk, tot, true);
+    double r0v = tot[0];
+    vb = (T)0;
+    if (S.border) {
+        vb = (T)tot[1];
+        r0v += r0b * (double)vb;
+    }
+    k.alpha = k.rho / r0v;
+    if (!(fabs(k.alpha) <= 1.0e300)) k.done = 5;
+}
+
+// p-update of the five-launch form (in place).
+template <typename T>
+__global__ __launch_bounds__(BLOCK) void k_fused_p(SegView sg, const T* __restrict__ r,
+                                                   T* __restrict__ p, const T* __restrict__ v,
+                                                   const double* __restrict__ partial,
+                                                   const KScalars* __restrict__ in,
+                                                   KScalars* __restrict__ out) {
+    const int lb = blockIdx.x, q = block_seg(sg, lb);
+    const Seg S = seg_at(sg, q);
+    FusedState k = fused_load(in + q);
+    const int i = lb * BLOCK + threadIdx.x;
+    const T ri = r[i], pi = p[i], vi = v[i];
+    fused_head<BLOCK>(sg, S, partial, in + q, k, 0);
+    if (!k.done) {
+        const T beta = (T)k.beta, w = (T)k.omega;
+        p[i] = ri + beta * (pi - w * vi);
+    }
+    if (fused_writer<1>(S, lb)) fused_store(in + q, out + q, k);
+}
+
+// s-update of the five-launch form; also v's border entry.
+template <typename T>
+__global__ __launch_bounds__(BLOCK) void k_fused_s(SegView sg, const T* __restrict__ r,
+                                                   T* __restrict__ v, T* __restrict__ s,
+                                                   const T* __restrict__ r0,
+                                                   const double* __restrict__ partial,
+                                                   const KScalars* __restrict__ in,
+                                                   KScalars* __restrict__ out) {
+    const int lb = blockIdx.x, q = block_seg(sg, lb);
+    const Seg S = seg_at(sg, q);
+    FusedState k = fused_load(in + q);
+    if (!k.done) {
+        const int i = lb * BLOCK + threadIdx.x;
+        const T ri = r[i], vi = v[i];
+        T vb;
+        fused_alpha<BLOCK>(sg, S, partial, r0, k, vb);
+        if (!k.done) {
+            const bool border = S.border && i == S.row0 + S.nv;
+            if (border) v[i] = vb;
+            s[i] = ri - (T)k.alpha * (border ? vb : vi);
+        }
+    }
+    if (fused_writer<1>(S, lb)) fused_store(in + q, out + q, k);
+}
+
+// Three-launch form, first kernel: p = r + beta (p - omega v) and v = A~ p.
+template <typename TM, typename T>
+__global__ __launch_bounds__(BLOCK) void k_fused_v(SellView sv, SegView sg,
+                                                       const TM* __restrict__ a,
+                                                       const T* __restrict__ dinv,
+                                                       const T* __restrict__ r,
+                                                       const T* __restrict__ r0, T* pa, T* pb,
+                                                       T* va, T* vb, double* partial,
+                                                       const KScalars* __restrict__ in,
+                                                       KScalars* __restrict__ out) {
+    const int nbk = ws_blocks<4>(sg);
+    const int lb = xcd_block(nbk);
+    if (lb < 0) return;
+    const int q = ws_seg<4>(sg, lb);
+    const Seg S = seg_at(sg, q);
+    in += q;
+    out += q;
+    FusedState k = fused_load(in);
+    if (k.done) {
+        if (fused_writer<4>(S, lb)) fused_store(in, out, k);
+        return;
+    }
+    // (a running system's par names the old buffers)
+    const T* __restrict__ po = in->par ? pb : pa;
+    const T* __restrict__ vo = in->par ? vb : va;
+    T* __restrict__ pn = in->par ? pa : pb;
+    T* __restrict__ vn = in->par ? va : vb;
+    T beta = (T)0, w = (T)0;
+    struct Raw {
+        T r, p, v;
+    };
+    auto pre = [=](int c) { return Raw{r[c], po[c], vo[c]}; };
+    auto pnew = [&](const Raw& e) { return e.r + beta * (e.p - w * e.v); };
+    const int iend = S.row0 + S.nv;
+    const int i = block_row<4>(lb);
+    const bool row = i < iend, border = S.border && i == iend;
+    Raw own{}, bord{};
+    if (row || border) own = pre(i);
+    if (S.border) bord = pre(iend);
+    const T r0i = row ? r0[i] : (T)0, di = row && S.border ? dinv[i] : (T)0;
+    bool ok;
+    T yv = sell_dot_early<T>(
+        sv, a, lb, pre,
+        [&]() {
+            fused_head<BLOCK>(sg, S, partial, in, k, 1);
+            beta = (T)k.beta;
+            w = (T)k.omega;
+            return k.done == 0;
+        },
+        pnew, ok);
+    if (!ok) {
+        if (fused_writer<4>(S, lb)) fused_store(in, out, k);
+        return;
+    }
+    double vals[2] = {0.0, 0.0};
+    if (row) {
+        const T pi = pnew(own);
+        pn[i] = pi;
+        if (S.border) yv = yv + pnew(bord);
+        vn[i] = yv;
+        vals[0] = (double)r0i * (double)yv;
+        if (S.border) vals[1] = (double)di * (double)pi;
+    } else if (border) {
+        pn[i] = pnew(own);
+    }
+    block_store<2, 4>(vals, partial + (size_t)BI_ALPHA * (sg.nrows / BLOCK), lb, nbk);
+    if (fused_writer<4>(S, lb)) fused_store(in, out, k);
+}
+
+// Second kernel: s = r - alpha v and t = A~ s; also v's border entry.
+template <typename TM, typename T>
+__global__ __launch_bounds__(BLOCK) void k_fused_t(SellView sv, SegView sg,
+                                                       const TM* __restrict__ a,
+                                                       const T* __restrict__ dinv,
+                                                       const T* __restrict__ r,
+                                                       const T* __restrict__ r0, T* va, T* vb,
+                                                       T* __restrict__ s, T* __restrict__ t,
+                                                       double* partial,
+                                                       const KScalars* __restrict__ in,
+                                                       KScalars* __restrict__ out) {
+    const int nbk = ws_blocks<4>(sg);
+    const int lb = xcd_block(nbk);
+    if (lb < 0) return;
+    const int q = ws_seg<4>(sg, lb);
+    const Seg S = seg_at(sg, q);
+    in += q;
+    out += q;
+    FusedState k = fused_load(in);
+    if (k.done) {
+        if (fused_writer<4>(S, lb)) fused_store(in, out, k);
+        return;
+    }
+    T* v = k.par ? vb : va;  // (its border entry is written here, by one thread)
+    T vbord = (T)0, alpha = (T)0;
+    struct Raw {
+        T r, v;
+    };
+    auto pre = [=](int c) { return Raw{r[c], v[c]}; };
+    auto snew = [&](const Raw& e) { return e.r - alpha * e.v; };
+    const int iend = S.row0 + S.nv;
+    const int i = block_row<4>(lb);
+    const bool row = i < iend;
+    Raw own{};
+    if (row) own = pre(i);
+    const T rb = S.border ? r[iend] : (T)0, di = row && S.border ? dinv[i] : (T)0;
+    bool ok;
+    T y = sell_dot_early<T>(
+        sv, a, lb, pre,
+        [&]() {
+            fused_alpha<BLOCK>(sg, S, partial, r0, k, vbord);
+            alpha = (T)k.alpha;
+            return k.done == 0;
+        },
+        snew, ok);
+    if (!ok) {
+        if (fused_writer<4>(S, lb)) fused_store(in, out, k);
+        return;
+    }
+    double vals[3] = {0.0, 0.0, 0.0};
+    const T sb = S.border ? rb - alpha * vbord : (T)0;
+    if (row) {
+        const T si = snew(own);
+        s[i] = si;
+        if (S.border) y = y + sb;
+        t[i] = y;
+        vals[0] = (double)y * (double)si;
+        vals[1] = (double)y * (double)y;
+        if (S.border) vals[2] = (double)di * (double)si;
+    } else if (S.border && i == iend) {
+        v[i] = vbord;
+        s[i] = sb;
+    }
+    block_store<3, 4>(vals, partial + (size_t)BI_OMEGA * (sg.nrows / BLOCK), lb, nbk);
+    if (fused_writer<4>(S, lb)) fused_store(in, out, k);
+}
+
+// Last kernel of both forms: omega; x += alpha p + omega s, r = s - omega t;
+// partial sums of r.r and r0.r (t's border entry comes from the partials).
+template <typename T>
+__global__ __launch_bounds__(BLOCK) void k_fused_x(SegView sg, T* __restrict__ x,
+                                                   T* __restrict__ r, const T* __restrict__ pa,
+                                                   const T* __restrict__ pb,
+                                                   const T* __restrict__ s,
+                                                   const T* __restrict__ t,
+                                                   const T* __restrict__ r0, double* partial,
+                                                   const KScalars* __restrict__ in,
+                                                   KScalars* __restrict__ out) {
+    const int nbk = sg.nrows / BLOCK;
+    const int lb = blockIdx.x, q = block_seg(sg, lb);
+    const Seg S = seg_at(sg, q);
+    in += q;
+    out += q;
+    FusedState k = fused_load(in);
+    if (k.done) {
+        if (fused_writer<1>(S, lb)) fused_store(in, out, k);
+        return;
+    }
+    const int i = lb * BLOCK + threadIdx.x;
+    const T xi = x[i], pi = (k.par ? pb : pa)[i], si = s[i], r0i = r0[i], ti0 = t[i];
+    const T sb = S.border ? s[S.row0 + S.nv] : (T)0;
+    double tot[3];
+    finish_sum<3, BLOCK>(partial + (size_t)BI_OMEGA * nbk, nbk, S.blk0, S.nblk, tot, true);
+    double ts = tot[0], tt = tot[1];
+    T tb = (T)0;
+    if (S.border) {
+        tb = (T)tot[2];
+        ts += (double)tb * (double)sb;
+        tt += (double)tb * (double)tb;
+    }
+    k.omega = (tt > 0.0) ? ts / tt : 0.0;
+    k.pending = 1;
+    const T al = (T)k.alpha, w = (T)k.omega;
+    const T ti = (S.border && i == S.row0 + S.nv) ? tb : ti0;
+    x[i] = xi + (al * pi + w * si);
+    const T ri = si - w * ti;
+    r[i] = ri;
+    double vals[2] = {(double)ri * (double)ri, (double)r0i * (double)ri};
+    block_store<2>(vals, partial + (size_t)BI_XR * nbk, lb, nbk);
+    if (fused_writer<1>(S, lb)) fused_store(in, out, k);
 }
 
 // out = b - A~ x (FP64) for every system; partial sums of out.out, b.b, D^-1 x
 template <int WS>
-__global__ __launch_bounds__(BLOCK * WS) void k_residual64(SellView sv, SegView sg,
+__global__ __launch_bounds__(WS_THREADS<WS>) void k_residual64(SellView sv, SegView sg,
                                                       const double* __restrict__ a,
                                                       const double* __restrict__ dinv,
                                                       const double* __restrict__ b,
                                                       const double* __restrict__ x,
                                                       double* __restrict__ out,
                                                       double* __restrict__ partial) {
-    const int nbk = sg.nrows / BLOCK;
+    const int nbk = ws_blocks<WS>(sg);
     const int lb = xcd_block(nbk);
     if (lb < 0) return;
-    const Seg S = sg.seg[block_seg(sg, lb)];
+    const Seg S = seg_at(sg, ws_seg<WS>(sg, lb));
     const int iend = S.row0 + S.nv;
     const int i = block_row<WS>(lb);
     double vals[3] = {0.0, 0.0, 0.0};
@@ -383,7 +736,7 @@ __global__ __launch_bounds__(BLOCK * WS) void k_residual64(SellView sv, SegView 
         vals[1] = b[i] * b[i];
         if (S.border) vals[2] = dinv[i] * x[i];
     }
-    block_store<3>(vals, partial, lb, nbk);
+    block_store<3, WS>(vals, partial, lb, nbk);
 }
 
 // (red[2]: the border unknown as the solve returns it, D^-1 x~, so the host
@@ -394,9 +747,9 @@ __global__ __launch_bounds__(FIN) void k_finish_res64(SegView sg, const double* 
                                                       KScalars* scs, const double* __restrict__ x,
                                                       const double* __restrict__ dinv) {
     KScalars* sc = scs + blockIdx.x;
-    const Seg S = sg.seg[blockIdx.x];
+    const Seg S = seg_at(sg, (int)blockIdx.x);
     double tot[3];
-    finish_sum<3>(partial, sg.nrows / BLOCK, S.blk0, S.nblk, tot);
+    finish_sum<3>(partial, sg.nrows / BLOCK, S.blk0, S.nblk, tot, by_slices(sg));
     if (threadIdx.x != 0) return;
     double rr = tot[0], bb = tot[1];
     if (S.border) {
@@ -501,7 +854,7 @@ __global__ __launch_bounds__(BLOCK) void k_diag_inverse(int n, const double* __r
 
 inline int nblk(int n) { return (n + BLOCK - 1) / BLOCK; }
 
-// f(wavefronts per slice) for a product over nbk row blocks
+// f(block shape) for a product over nbk row blocks
 template <typename F>
 void with_split(int nbk, F&& f) {
     if (nbk <= SPLIT_MAX_BLOCKS)
@@ -545,7 +898,7 @@ __global__ void k_gm_reset(int nseg, GmState* gm, GmFlags* fl, const SegCtl* ctl
 // row's D^-1 x.  x_zero: x is known to be zero (a defect-correction cycle's
 // start), so A x is not formed.
 template <int WS, typename TM, typename TV>
-__global__ __launch_bounds__(BLOCK * WS) void k_gm_residual(SellView sv, SegView sg,
+__global__ __launch_bounds__(WS_THREADS<WS>) void k_gm_residual(SellView sv, SegView sg,
                                                        const TM* __restrict__ a,
                                                        const double* __restrict__ dinv,
                                                        const double* __restrict__ rhs,
@@ -555,13 +908,13 @@ __global__ __launch_bounds__(BLOCK * WS) void k_gm_residual(SellView sv, SegView
                                                        float* __restrict__ xs,
                                                        double* __restrict__ partial,
                                                        const GmState* gm, int mode, int x_zero) {
-    const int nbk = sg.nrows / BLOCK;
+    const int nbk = ws_blocks<WS>(sg);
     const int lb = xcd_block(nbk);
     if (lb < 0) return;
-    const int q = block_seg(sg, lb);
+    const int q = ws_seg<WS>(sg, lb);
     const GmState* g = gm + q;
     if (mode == 0 ? g->done != 0 : !(g->full && g->done == 0)) return;
-    const Seg S = sg.seg[q];
+    const Seg S = seg_at(sg, q);
     const int iend = S.row0 + S.nv;
     const int i = block_row<WS>(lb);
     double vals[3] = {0.0, 0.0, 0.0};
@@ -576,7 +929,7 @@ __global__ __launch_bounds__(BLOCK * WS) void k_gm_residual(SellView sv, SegView
         vals[1] = rhs[i] * rhs[i];
         if (S.border && !x_zero) vals[2] = dinv[i] * x[i];
     }
-    block_store<3>(vals, partial, lb, nbk);
+    block_store<3, WS>(vals, partial, lb, nbk);
 }
 
 // (v0 holds the residual rounded to the basis type; its norm is the FP64 one)
@@ -589,9 +942,9 @@ __global__ __launch_bounds__(FIN) void k_gm_residual_finish(SegView sg,
                                                             int rel_to_rhs) {
     GmState* g = gm + blockIdx.x;
     if (mode == 0 ? g->done != 0 : !(g->full && g->done == 0)) return;
-    const Seg S = sg.seg[blockIdx.x];
+    const Seg S = seg_at(sg, (int)blockIdx.x);
     double tot[3];
-    finish_sum<3>(partial, sg.nrows / BLOCK, S.blk0, S.nblk, tot);
+    finish_sum<3>(partial, sg.nrows / BLOCK, S.blk0, S.nblk, tot, by_slices(sg));
     if (threadIdx.x != 0) return;
     double rr = tot[0], bb = tot[1];
     if (S.border) {
@@ -637,13 +990,13 @@ __global__ __launch_bounds__(FIN) void k_gm_residual_finish(SegView sg,
 
 // w = A z: node rows (plus the border unknown's column), partial sums of the
 // border row sum D^-1 z; zg: the gathered copy of z (FP32 when z holds FP32
-// values, the V-cycle's output).  WS == 4 also forms the partial sums of
+// values, the V-cycle's output).  WS == 16 also forms the partial sums of
 // v_k . w, k < nk, from its w rows in LDS, sixteen wavefronts a vector each
 // (k_gm_dots's sums, order and all): for a small system that saves a launch
 // of 4.6 us; at 1M nodes the two kernels apart are faster (67 + 14 us against
 // 83).
 template <int WS, typename TM, typename TX, typename TB>
-__global__ __launch_bounds__(BLOCK * WS) void k_gm_spmv(SellView sv, SegView sg,
+__global__ __launch_bounds__(WS_THREADS<WS>) void k_gm_spmv(SellView sv, SegView sg,
                                                    const TM* __restrict__ a,
                                                    const double* __restrict__ dinv,
                                                    const TB* __restrict__ z,
@@ -657,7 +1010,7 @@ __global__ __launch_bounds__(BLOCK * WS) void k_gm_spmv(SellView sv, SegView sg,
     if (lb < 0) return;
     const int q = block_seg(sg, lb);
     if (gm[q].stop) return;
-    const Seg S = sg.seg[q];
+    const Seg S = seg_at(sg, q);
     const int iend = S.row0 + S.nv;
     const int i = block_row<WS>(lb);
     double vals[1] = {0.0};
@@ -667,13 +1020,13 @@ __global__ __launch_bounds__(BLOCK * WS) void k_gm_spmv(SellView sv, SegView sg,
         w[i] = y;
         if (S.border) vals[0] = dinv[i] * (double)zg[i];
     }
-    if constexpr (WS == 4) {
+    if constexpr (WS == 16) {
         __shared__ double sw[BLOCK];
         if (threadIdx.x < BLOCK) sw[threadIdx.x] = y;
-        block_store<1>(vals, partial + (size_t)GM_MAX * nbk, lb, nbk);  // (a barrier in it)
+        block_store<1, WS>(vals, partial + (size_t)GM_MAX * nbk, lb, nbk);  // (a barrier in it)
         const int lane = threadIdx.x & 63;
         const int r0 = lb * BLOCK + lane;
-        for (int k = (int)(threadIdx.x >> 6); k < nk; k += BLOCK * WS / 64) {
+        for (int k = (int)(threadIdx.x >> 6); k < nk; k += 4 * BLOCK / 64) {
             const TB* vk = V + k * ld + r0;
             double acc = 0.0;
 #pragma unroll
@@ -683,7 +1036,7 @@ __global__ __launch_bounds__(BLOCK * WS) void k_gm_spmv(SellView sv, SegView sg,
             if (lane == 0) partial[(size_t)k * nbk + lb] = acc;
         }
     } else {
-        block_store<1>(vals, partial + (size_t)GM_MAX * nbk, lb, nbk);
+        block_store<1, WS>(vals, partial + (size_t)GM_MAX * nbk, lb, nbk);
     }
 }
 
@@ -701,7 +1054,7 @@ __global__ __launch_bounds__(BLOCK) void k_gm_dots(SegView sg, const double* __r
     const int lb = blockIdx.x;
     const int q = block_seg(sg, lb);
     if (gm[q].stop) return;
-    const Seg S = sg.seg[q];
+    const Seg S = seg_at(sg, q);
     const int iend = S.row0 + S.nv;
     const int lane = threadIdx.x & 63, u = threadIdx.x >> 6;
     const int r0 = lb * BLOCK + lane;
@@ -778,7 +1131,7 @@ __global__ __launch_bounds__(GMF) void k_gm_finish_h(SegView sg, double* __restr
     const int q = blockIdx.x / GM_MAX, k = blockIdx.x % GM_MAX;
     GmState* g = gm + q;
     if (k >= nk || g->stop) return;
-    const Seg S = sg.seg[q];
+    const Seg S = seg_at(sg, q);
     const int nb = sg.nrows / BLOCK;
     __shared__ double sh[2][GMF / 64];
     const double dk = gm_row_sum(partial + (size_t)k * nb + S.blk0, S.nblk);
@@ -833,7 +1186,7 @@ __global__ __launch_bounds__(BLOCK) void k_gm_orth(SegView sg, const double* __r
     const int q = block_seg(sg, lb);
     const GmState* g = gm + q;
     if (g->stop) return;
-    const Seg S = sg.seg[q];
+    const Seg S = seg_at(sg, q);
     const int i = lb * BLOCK + threadIdx.x;
     double vals[1] = {0.0};
     if (i < S.row0 + S.nv + S.border) {
@@ -870,7 +1223,7 @@ __global__ __launch_bounds__(4 * BLOCK) void k_gm_orth_h(SegView sg, const doubl
     const int q = block_seg(sg, lb);
     GmState* g = gm + q;
     if (g->stop) return;
-    const Seg S = sg.seg[q];
+    const Seg S = seg_at(sg, q);
     const int ib = S.row0 + S.nv;
     __shared__ double sk[GM_MAX + 1], shc[GM_MAX], red[4][BLOCK];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -973,7 +1326,7 @@ __global__ __launch_bounds__(BLOCK) void k_gm_update_x(SegView sg, double* __res
     const int q = block_seg(sg, blockIdx.x);
     const GmState* g = gm + q;
     if (!g->apply) return;
-    const Seg S = sg.seg[q];
+    const Seg S = seg_at(sg, q);
     const int i = blockIdx.x * BLOCK + threadIdx.x;
     const int iend = S.row0 + S.nv;
     if (i >= iend + S.border) return;
@@ -1087,7 +1440,7 @@ void PpeSolver::setup(hipStream_t st, const SellView& view, const std::vector<Se
     bseg_d.alloc(hb.size());
     MP_HIP(hipMemcpyAsync(seg_d.p, segs.data(), sizeof(Seg) * nseg, hipMemcpyHostToDevice, st));
     MP_HIP(hipMemcpyAsync(bseg_d.p, hb.data(), sizeof(int) * hb.size(), hipMemcpyHostToDevice, st));
-    sg = SegView{nseg, nrows, seg_d.p, bseg_d.p};
+    sg = SegView{nseg, nrows, seg_d.p, bseg_d.p, segs[0]};
     const size_t vlen = (size_t)nrows + 64;
     DevBuf<double> raw, diag;
     const int total_slots = [&]() {
@@ -1177,9 +1530,14 @@ void PpeSolver::setup(hipStream_t st, const SellView& view, const std::vector<Se
         b->alloc(vlen);
         MP_HIP(hipMemsetAsync(b->p, 0, sizeof(double) * vlen, st));
     }
-    partial.alloc((size_t)(nrows / BLOCK) * 4);
-    sc.alloc(nseg);
-    MP_HIP(hipMemsetAsync(sc.p, 0, sizeof(KScalars) * nseg, st));
+    if (!amg && nrows / BLOCK <= FUSE_MAX_BLOCKS)
+        for (DevBuf<double>* b : {&p2, &v2}) {
+            b->alloc(vlen);
+            MP_HIP(hipMemsetAsync(b->p, 0, sizeof(double) * vlen, st));
+        }
+    partial.alloc((size_t)(nrows / BLOCK) * BI_ROWS);
+    sc.alloc(3 * (size_t)nseg);
+    MP_HIP(hipMemsetAsync(sc.p, 0, sizeof(KScalars) * sc.n, st));
     ctl_d.alloc(nseg);
     if (host_sc) (void)hipHostFree(host_sc);
     if (host_ctl) (void)hipHostFree(host_ctl);
@@ -1251,12 +1609,63 @@ const double* PpeSolver::precondition(hipStream_t st, const double* in, double* 
     return out;
 }
 
+// The fused forms of a chunk (Jacobi, small systems).
+template <typename TM, typename T>
+void PpeSolver::launch_fused_chunk(hipStream_t st, int chunk, const TM* a, const T* di, T* x,
+                                   T* rr, T* rr0, T* pp, T* vv, T* ss, T* tt) {
+    const int nbk = nrows / BLOCK;
+    KScalars *A = sc.p, *B = A + nseg, *C = B + nseg;
+    T *pb = p2.p, *vb = v2.p;
+    const bool three = nbk <= FUSE3_MAX_BLOCKS;
+    for (int c = 0; c < chunk; ++c) {
+        if (three) {
+            spmv_timer.begin(st);
+            hipLaunchKernelGGL((k_fused_v<TM, T>), dim3(grid_xcd(4 * nbk)), dim3(BLOCK), 0, st,
+                               view_of<TM>(), sg, a, di, (const T*)rr, (const T*)rr0, pp, pb, vv,
+                               vb, partial.p, (const KScalars*)A, B);
+            spmv_timer.end(st);
+            spmv_timer.begin(st);
+            hipLaunchKernelGGL((k_fused_t<TM, T>), dim3(grid_xcd(4 * nbk)), dim3(BLOCK), 0, st,
+                               view_of<TM>(), sg, a, di, (const T*)rr, (const T*)rr0, vv, vb, ss,
+                               tt, partial.p, (const KScalars*)B, C);
+            spmv_timer.end(st);
+        } else {
+            hipLaunchKernelGGL(k_fused_p<T>, dim3(nbk), dim3(BLOCK), 0, st, sg, (const T*)rr, pp,
+                               (const T*)vv, (const double*)partial.p, (const KScalars*)A, B);
+            spmv_timer.begin(st);
+            hipLaunchKernelGGL((k_spmv_alpha<4, TM, T, T>), dim3(grid_xcd(4 * nbk)), dim3(BLOCK),
+                               0, st, view_of<TM>(), sg, a, di, (const T*)pp, (const T*)pp, vv,
+                               (const T*)rr0, partial.p + (size_t)BI_ALPHA * nbk,
+                               (const KScalars*)B);
+            spmv_timer.end(st);
+            hipLaunchKernelGGL(k_fused_s<T>, dim3(nbk), dim3(BLOCK), 0, st, sg, (const T*)rr, vv,
+                               ss, (const T*)rr0, (const double*)partial.p, (const KScalars*)B, C);
+            spmv_timer.begin(st);
+            hipLaunchKernelGGL((k_spmv_omega<4, TM, T, T>), dim3(grid_xcd(4 * nbk)), dim3(BLOCK),
+                               0, st, view_of<TM>(), sg, a, di, (const T*)ss, (const T*)ss,
+                               (const T*)ss, tt, partial.p + (size_t)BI_OMEGA * nbk,
+                               (const KScalars*)C);
+            spmv_timer.end(st);
+        }
+        hipLaunchKernelGGL(k_fused_x<T>, dim3(nbk), dim3(BLOCK), 0, st, sg, x, rr, (const T*)pp,
+                           (const T*)pb, (const T*)ss, (const T*)tt, (const T*)rr0, partial.p,
+                           (const KScalars*)C, A);
+    }
+    hipLaunchKernelGGL(k_finish_xr, dim3(nseg), dim3(FIN), 0, st, sg,
+                       (const double*)partial.p, A, 1);
+    MP_HIP(hipGetLastError());
+}
+
 // The chunk of iterations between two convergence polls, launched on the
 // stream (captured into a graph by run_chunk).
 template <typename TM, typename T>
 void PpeSolver::launch_chunk(hipStream_t st, int chunk, const TM* a, const T* di, T* x, T* rr,
                              T* rr0, T* pp, T* vv, T* ss, T* tt) {
     const int nbk = nrows / BLOCK;
+    if (!amg && nbk <= FUSE_MAX_BLOCKS) {
+        launch_fused_chunk<TM, T>(st, chunk, a, di, x, rr, rr0, pp, vv, ss, tt);
+        return;
+    }
     float* xs = amg ? amg->prescaled_input() : nullptr;
     const float* d0 = amg ? amg->level0_dinv() : nullptr;
     for (int c = 0; c < chunk; ++c) {
@@ -1268,12 +1677,12 @@ void PpeSolver::launch_chunk(hipStream_t st, int chunk, const TM* a, const T* di
         with_split(nbk, [&](auto ws) {
             constexpr int WS = decltype(ws)::value;
             if (amg)
-                hipLaunchKernelGGL((k_spmv_alpha<WS, TM, T, float>), dim3(grid_xcd(nbk)),
-                                   dim3(BLOCK * WS), 0, st, view_of<TM>(), sg, a, di, yin,
+                hipLaunchKernelGGL((k_spmv_alpha<WS, TM, T, float>), dim3(grid_xcd(nrows / WS_ROWS<WS>)),
+                                   dim3(WS_THREADS<WS>), 0, st, view_of<TM>(), sg, a, di, yin,
                                    (const float*)y32.p, vv, rr0, partial.p, sc.p);
             else
-                hipLaunchKernelGGL((k_spmv_alpha<WS, TM, T, T>), dim3(grid_xcd(nbk)),
-                                   dim3(BLOCK * WS), 0, st, view_of<TM>(), sg, a, di, yin, yin, vv,
+                hipLaunchKernelGGL((k_spmv_alpha<WS, TM, T, T>), dim3(grid_xcd(nrows / WS_ROWS<WS>)),
+                                   dim3(WS_THREADS<WS>), 0, st, view_of<TM>(), sg, a, di, yin, yin, vv,
                                    rr0, partial.p, sc.p);
         });
         spmv_timer.end(st);
@@ -1286,12 +1695,12 @@ void PpeSolver::launch_chunk(hipStream_t st, int chunk, const TM* a, const T* di
         with_split(nbk, [&](auto ws) {
             constexpr int WS = decltype(ws)::value;
             if (amg)
-                hipLaunchKernelGGL((k_spmv_omega<WS, TM, T, float>), dim3(grid_xcd(nbk)),
-                                   dim3(BLOCK * WS), 0, st, view_of<TM>(), sg, a, di, zin,
+                hipLaunchKernelGGL((k_spmv_omega<WS, TM, T, float>), dim3(grid_xcd(nrows / WS_ROWS<WS>)),
+                                   dim3(WS_THREADS<WS>), 0, st, view_of<TM>(), sg, a, di, zin,
                                    (const float*)z32.p, ss, tt, partial.p, sc.p);
             else
-                hipLaunchKernelGGL((k_spmv_omega<WS, TM, T, T>), dim3(grid_xcd(nbk)),
-                                   dim3(BLOCK * WS), 0, st, view_of<TM>(), sg, a, di, zin, zin, ss,
+                hipLaunchKernelGGL((k_spmv_omega<WS, TM, T, T>), dim3(grid_xcd(nrows / WS_ROWS<WS>)),
+                                   dim3(WS_THREADS<WS>), 0, st, view_of<TM>(), sg, a, di, zin, zin, ss,
                                    tt, partial.p, sc.p);
         });
         spmv_timer.end(st);
@@ -1299,7 +1708,7 @@ void PpeSolver::launch_chunk(hipStream_t st, int chunk, const TM* a, const T* di
                            sc.p);
         hipLaunchKernelGGL(k_update_xr<T>, dim3(nbk), dim3(BLOCK), 0, st, sg, x, rr, yin, zin, ss,
                            tt, rr0, partial.p, sc.p);
-        hipLaunchKernelGGL(k_finish_xr, dim3(nseg), dim3(FIN), 0, st, sg, partial.p, sc.p);
+        hipLaunchKernelGGL(k_finish_xr, dim3(nseg), dim3(FIN), 0, st, sg, partial.p, sc.p, 0);
     }
     MP_HIP(hipGetLastError());
 }
@@ -1385,7 +1794,7 @@ void PpeSolver::run_bicgstab(hipStream_t st, const TM* a, const T* di, const T* 
     auto residual_init = [&](int mode) {
         with_split(nbk, [&](auto ws) {
             constexpr int WS = decltype(ws)::value;
-            hipLaunchKernelGGL((k_residual_init<WS, TM, T>), dim3(grid_xcd(nbk)), dim3(BLOCK * WS),
+            hipLaunchKernelGGL((k_residual_init<WS, TM, T>), dim3(grid_xcd(nrows / WS_ROWS<WS>)), dim3(WS_THREADS<WS>),
                                0, st, view_of<TM>(), sg, a, di, rhs, x, rr, rr0, pp, vv, partial.p,
                                sc.p, mode);
         });
@@ -1445,7 +1854,7 @@ void PpeSolver::launch_residual64(hipStream_t st, const double* b_dev) {
     const int nbk = nrows / BLOCK;
     with_split(nbk, [&](auto ws) {
         constexpr int WS = decltype(ws)::value;
-        hipLaunchKernelGGL(k_residual64<WS>, dim3(grid_xcd(nbk)), dim3(BLOCK * WS), 0, st, sv, sg,
+        hipLaunchKernelGGL(k_residual64<WS>, dim3(grid_xcd(nrows / WS_ROWS<WS>)), dim3(WS_THREADS<WS>), 0, st, sv, sg,
                            aval.p, dinv.p, b_dev, xt.p, tmp.p, partial.p);
     });
     hipLaunchKernelGGL(k_finish_res64, dim3(nseg), dim3(FIN), 0, st, sg, b_dev, tmp.p, partial.p,
@@ -1519,12 +1928,14 @@ void PpeSolver::gmres_iteration(hipStream_t st, int k, int m, const TM* a, const
     auto product = [&](const auto* zg) {
         using TX = std::remove_cv_t<std::remove_pointer_t<decltype(zg)>>;
         spmv_timer.begin(st);
-        with_split(nbk, [&](auto ws) {
-            constexpr int WS = decltype(ws)::value;
-            hipLaunchKernelGGL((k_gm_spmv<WS, TM, TX, TV>), dim3(grid_xcd(nbk)), dim3(BLOCK * WS),
+        if (split)
+            hipLaunchKernelGGL((k_gm_spmv<16, TM, TX, TV>), dim3(grid_xcd(nbk)), dim3(4 * BLOCK),
                                0, st, view_of<TM>(), sg, a, di, (const TV*)vk, zg, gm_w.p,
                                (const TV*)V, ld, k + 1, gm_partial.p, gm_d.p);
-        });
+        else
+            hipLaunchKernelGGL((k_gm_spmv<1, TM, TX, TV>), dim3(grid_xcd(nbk)), dim3(BLOCK), 0, st,
+                               view_of<TM>(), sg, a, di, (const TV*)vk, zg, gm_w.p, (const TV*)V,
+                               ld, k + 1, gm_partial.p, gm_d.p);
         spmv_timer.end(st);
     };
     if (amg) {
@@ -1579,7 +1990,7 @@ void PpeSolver::run_gmres(hipStream_t st, const TM* a, const double* di, const d
     auto start = [&](int mode) {
         with_split(nbk, [&](auto ws) {
             constexpr int WS = decltype(ws)::value;
-            hipLaunchKernelGGL((k_gm_residual<WS, TM, TV>), dim3(grid_xcd(nbk)), dim3(BLOCK * WS),
+            hipLaunchKernelGGL((k_gm_residual<WS, TM, TV>), dim3(grid_xcd(nrows / WS_ROWS<WS>)), dim3(WS_THREADS<WS>),
                                0, st, view_of<TM>(), sg, a, di, rhs, x, V, d0, xs, gm_partial.p,
                                gm_d.p, mode, (mode == 0 && x_zero) ? 1 : 0);
         });

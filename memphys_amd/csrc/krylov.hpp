@@ -114,7 +114,8 @@ struct PpeSolver {
     int gm_cols = 0;                  // columns allocated
     std::unique_ptr<AmgDevice> amg;
     DevBuf<double> partial;
-    DevBuf<KScalars> sc;              // [nseg]
+    DevBuf<KScalars> sc;              // [3 nseg]: the state, and the fused iterations' two more
+    DevBuf<double> p2, v2;            // second p and v of the fused iterations
     DevBuf<SegCtl> ctl_d;             // [nseg]
     KScalars* host_sc = nullptr;      // pinned, 2 x nseg
     SegCtl* host_ctl = nullptr;       // pinned, nseg
@@ -200,6 +201,9 @@ struct PpeSolver {
     void residual64(hipStream_t s, const double* b_dev, std::vector<double>& rr,
                     std::vector<double>& bb);
     const double* precondition(hipStream_t s, const double* in, double* out, float* out32);
+    template <typename TM, typename T>
+    void launch_fused_chunk(hipStream_t s, int chunk, const TM* a, const T* di, T* x, T* rr,
+                            T* rr0, T* pp, T* vv, T* ss, T* tt);
     template <typename TM, typename T>
     void launch_chunk(hipStream_t s, int chunk, const TM* a, const T* di, T* x, T* rr, T* rr0,
                       T* pp, T* vv, T* ss, T* tt);

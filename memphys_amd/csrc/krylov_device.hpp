@@ -7,41 +7,66 @@ namespace mp {
 
 constexpr int FIN = 1024;  // threads of the finishing kernels (one block per system)
 
-// Block sums of the first BLOCK threads' NV values stored at partial[q * nb +
-// lb] (lb: logical block) (plain stores: no atomics, the finishing kernel runs
-// after the grid).  Every thread of the block must call.
-template <int NV>
+// Sums of a block's NV values over its rows (WS: the product's shape), stored
+// at partial[q * nb + lb] (plain stores: no atomics, the finishing kernel runs
+// after the grid): over BLOCK rows, or over one slice (WS == 4, nb and lb then
+// count slices; finish_sum adds a block's four in the same order).  Every
+// thread of the block must call.
+template <int NV, int WS = 1>
 __device__ __forceinline__ void block_store(double (&v)[NV], double* __restrict__ partial, int lb,
                                             int nb) {
-    __shared__ double sh[NV][BLOCK / 64];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    if (wid < BLOCK / 64) {
+    if (wid < WS_ROWS<WS> / 64)
 #pragma unroll
         for (int q = 0; q < NV; ++q)
             for (int off = 32; off > 0; off >>= 1) v[q] += __shfl_xor(v[q], off);
-        if (lane == 0)
+    if constexpr (WS == 4) {
+        if (threadIdx.x == 0)
+#pragma unroll
+            for (int q = 0; q < NV; ++q) partial[(size_t)q * nb + lb] = v[q];
+    } else {
+        __shared__ double sh[NV][BLOCK / 64];
+        if (wid < BLOCK / 64 && lane == 0)
 #pragma unroll
             for (int q = 0; q < NV; ++q) sh[q][wid] = v[q];
-    }
-    __syncthreads();
-    if (threadIdx.x < NV) {
-        const int q = threadIdx.x;
-        double s = sh[q][0];
-        for (int t = 1; t < BLOCK / 64; ++t) s += sh[q][t];
-        partial[(size_t)q * nb + lb] = s;
+        __syncthreads();
+        if (threadIdx.x < NV) {
+            const int q = threadIdx.x;
+            double s = sh[q][0];
+            for (int t = 1; t < BLOCK / 64; ++t) s += sh[q][t];
+            partial[(size_t)q * nb + lb] = s;
+        }
     }
 }
 
 // Sum of the partials of blocks [b0, b0 + cnt) per value (stride nb), in the
 // order of a block of FIN threads whatever the block's size NT: FIN virtual
 // threads each sum every FIN-th partial, their wavefronts reduce by shuffles,
-// and the wavefronts' sums are added in order.  Every thread of the block
+// and the wavefronts' sums are added in order.  slices: the partials are per
+// slice, four adjacent ones a block (stride 4 nb).  Every thread of the block
 // receives the totals.
 template <int NV, int NT = FIN>
 __device__ __forceinline__ void finish_sum(const double* __restrict__ partial, int nb, int b0,
-                                           int cnt, double (&tot)[NV]) {
-    __shared__ double sh[NV][FIN / 64];
+                                           int cnt, double (&tot)[NV], bool slices = false) {
+    typedef double d4 __attribute__((ext_vector_type(4)));
+    auto at = [&](int q, int b) {
+        if (!slices) return partial[(size_t)q * nb + b0 + b];
+        const d4 d = reinterpret_cast<const d4*>(partial)[(size_t)q * nb + b0 + b];
+        return ((d.x + d.y) + d.z) + d.w;
+    };
     const int lane = threadIdx.x & 63;
+    if (cnt <= 64) {
+        // one virtual wavefront holds every partial: each wavefront of the block
+        // forms its sum on its own (the other fifteen are zeros)
+#pragma unroll
+        for (int q = 0; q < NV; ++q) tot[q] = lane < cnt ? at(q, lane) : 0.0;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+            for (int q = 0; q < NV; ++q) tot[q] += __shfl_xor(tot[q], off);
+        return;
+    }
+    __shared__ double sh[NV][FIN / 64];
 #pragma unroll
     for (int u = 0; u < FIN / NT; ++u) {
         const int vt = (int)threadIdx.x + u * NT, wid = vt >> 6;
@@ -51,7 +76,7 @@ __device__ __forceinline__ void finish_sum(const double* __restrict__ partial, i
         if (wid * 64 < cnt) {
             for (int b = vt; b < cnt; b += FIN)
 #pragma unroll
-                for (int q = 0; q < NV; ++q) acc[q] += partial[(size_t)q * nb + b0 + b];
+                for (int q = 0; q < NV; ++q) acc[q] += at(q, b);
 #pragma unroll
             for (int q = 0; q < NV; ++q)
                 for (int off = 32; off > 0; off >>= 1) acc[q] += __shfl_xor(acc[q], off);
@@ -91,7 +116,7 @@ __device__ __forceinline__ void gm_norm_step(const SegView& sg, int q,
                                              GmFlags* fl, int m) {
     GmState* g = gm + q;
     if (g->stop) return;
-    const Seg S = sg.seg[q];
+    const Seg S = seg_at(sg, q);
     double tot[1];
     finish_sum<1, NT>(partial, sg.nrows / BLOCK, S.blk0, S.nblk, tot);
     // the column and the previous rotations into LDS in one parallel load;
@@ -147,7 +172,7 @@ __device__ __forceinline__ void gm_norm_step(const SegView& sg, int q,
 // The norm step of one or more systems, run by extra blocks of another launch
 // (sg.nseg == 0: none).
 struct GmNorm {
-    SegView sg{0, 0, nullptr, nullptr};
+    SegView sg{};
     const double* partial = nullptr;
     GmState* gm = nullptr;
     GmFlags* fl = nullptr;

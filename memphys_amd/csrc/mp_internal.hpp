@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cstdint>
 #include <string>
 #include <thread>
@@ -138,12 +139,12 @@ __device__ __forceinline__ V load_stream(const V* p) {
 // The neighbour loop of one slice row (groups of four slots from slot b0 +
 // 4 lane, w4 groups): load(g) fetches group g's stored columns and decode()
 // turns them into column ids.  A row's sum is four fma chains, chain p over the
-// groups p, p + 4, ..., added as (0 + 1) + (2 + 3).  WS == 1: one wavefront forms
-// all four; the stored columns and the values of U4 groups are requested
-// before the first decode, so their loads overlap.  WS == 4: this wavefront
+// groups p, p + 4, ..., added as (0 + 1) + (2 + 3).  PARTS == 1: one wavefront
+// forms all four; the stored columns and the values of U4 groups are requested
+// before the first decode, so their loads overlap.  PARTS == 4: this wavefront
 // forms chain `part` alone and returns it (two groups in flight); the caller
 // adds the four.  Either way the row's sum has the same bits.
-template <int WS, int U4, typename T, typename TM, typename LD, typename DC, typename FV,
+template <int PARTS, int U4, typename T, typename TM, typename LD, typename DC, typename FV,
           typename FX>
 __device__ __forceinline__ T sell4_loop(int b0, int w4, int lane, int part,
                                         const TM* __restrict__ a, LD load, DC decode, FV fv,
@@ -160,7 +161,7 @@ __device__ __forceinline__ T sell4_loop(int b0, int w4, int lane, int part,
 #pragma unroll
         for (int u = 0; u < N; ++u) e[u] = load(g + u * step);
 #pragma unroll
-        for (int u = 0; u < N; ++u) v[u] = load_stream<WS == 1>(ap + (g + u * step) * SLICE);
+        for (int u = 0; u < N; ++u) v[u] = load_stream<PARTS == 1>(ap + (g + u * step) * SLICE);
 #pragma unroll
         for (int u = 0; u < N; ++u) {
             const typename Vec4<int>::type c = decode(e[u]);
@@ -178,7 +179,7 @@ __device__ __forceinline__ T sell4_loop(int b0, int w4, int lane, int part,
             s = fma(fv(v[u].w), xv[4 * u + 3], s);
         }
     };
-    if constexpr (WS == 4) {
+    if constexpr (PARTS == 4) {
         T acc = (T)0;
         int g = part;
         for (; g + 4 < w4; g += 8) groups(std::integral_constant<int, 2>{}, g, 4, &acc, 0);
@@ -186,7 +187,7 @@ __device__ __forceinline__ T sell4_loop(int b0, int w4, int lane, int part,
         return acc;
     } else {
         // U4 == 2 forms chains 0 and 1, then 2 and 3 (two accumulators live)
-        static_assert(WS == 1 && (U4 == 2 || U4 == 4), "");
+        static_assert(PARTS == 1 && (U4 == 2 || U4 == 4), "");
         T sum[4 / U4];
 #pragma unroll
         for (int h = 0; h < 4; h += U4) {
@@ -217,15 +218,15 @@ struct SellHead {
     int base[CW_COUNT];
 };
 
-// Sum over the neighbours of one slice row of fv(value) * fx(column) (WS == 4:
+// Sum over the neighbours of one slice row of fv(value) * fx(column) (PARTS == 4:
 // chain `part` of it; see sell4_loop): the slice of head h, lane = slice row.  The
 // four neighbours of a group come in one vector load of columns (16-bit
 // compressed ones when col16 is given and the slice has them) and one of
-// values; U4 groups are loaded before their gathers.  With WS == 1 columns and
-// values up to 4 bytes use non-temporal loads so the gathered vector stays
+// values; U4 groups are loaded before their gathers.  With PARTS == 1 columns
+// and values up to 4 bytes use non-temporal loads so the gathered vector stays
 // cached; FP64 values (32 bytes a lane, fetched as two 16-byte halves) use ordinary loads,
 // which keep the line in cache between the halves.
-template <int WS, int U4, typename T, typename TM, typename FV, typename FX>
+template <int PARTS, int U4, typename T, typename TM, typename FV, typename FX>
 __device__ __forceinline__ T sell4_accumulate(const SellHead& h, const int* __restrict__ col,
                                               const uint16_t* __restrict__ col16,
                                               const TM* __restrict__ a, int lane, int part,
@@ -234,8 +235,8 @@ __device__ __forceinline__ T sell4_accumulate(const SellHead& h, const int* __re
     typedef typename Vec4<uint16_t>::type e4;
     if (h.base[0] >= 0) {
         const e4* ep = reinterpret_cast<const e4*>(col16 + h.b0) + lane;
-        return sell4_loop<WS, U4, T>(
-            h.b0, h.w4, lane, part, a, [&](int g) { return load_stream<WS == 1>(ep + g * SLICE); },
+        return sell4_loop<PARTS, U4, T>(
+            h.b0, h.w4, lane, part, a, [&](int g) { return load_stream<PARTS == 1>(ep + g * SLICE); },
             [&](e4 e) {
                 c4 c;
                 c.x = col_decode(e.x, h.base);
@@ -247,18 +248,45 @@ __device__ __forceinline__ T sell4_accumulate(const SellHead& h, const int* __re
             fv, fx);
     }
     const c4* cp = reinterpret_cast<const c4*>(col + h.b0) + lane;
-    return sell4_loop<WS, U4, T>(
-        h.b0, h.w4, lane, part, a, [&](int g) { return load_stream<WS == 1>(cp + g * SLICE); },
+    return sell4_loop<PARTS, U4, T>(
+        h.b0, h.w4, lane, part, a, [&](int g) { return load_stream<PARTS == 1>(cp + g * SLICE); },
         [](c4 c) { return c; }, fv, fx);
 }
 
-// The head of this wavefront's slice in logical block lb.
+// The three shapes of a product's blocks (WS):
+//   1   BLOCK threads over BLOCK rows: a wavefront per slice, four chains each;
+//   4   BLOCK threads over one slice: a wavefront per chain;
+//   16  4 * BLOCK threads over BLOCK rows: a wavefront per chain.
+// The wide shapes are for systems whose slices leave SIMDs idle: the row's
+// serial chain of loads is a quarter as long, and (4) the gathers, which a CU
+// serves one wavefront at a time, spread over four times the CUs.
+template <int WS>
+constexpr int WS_THREADS = WS == 16 ? 4 * BLOCK : BLOCK;
+template <int WS>
+constexpr int WS_ROWS = WS == 4 ? SLICE : BLOCK;
+
+// This wavefront's slice and chain in logical block lb.
+template <int WS>
+__device__ __forceinline__ int ws_slice(int lb) {
+    const int wid = (int)(threadIdx.x >> 6);
+    return __builtin_amdgcn_readfirstlane(WS == 4 ? lb : lb * (BLOCK / SLICE) + (wid & 3));
+}
+template <int WS>
+__device__ __forceinline__ int ws_part() {
+    const int wid = (int)(threadIdx.x >> 6);
+    return __builtin_amdgcn_readfirstlane(WS == 4 ? wid : wid >> 2);
+}
+// This thread's row in logical block lb; past every row for the threads beyond
+// the block's rows.
+template <int WS>
+__device__ __forceinline__ int block_row(int lb) {
+    return (int)threadIdx.x < WS_ROWS<WS> ? lb * WS_ROWS<WS> + (int)threadIdx.x : INT_MAX;
+}
+
 __device__ __forceinline__ SellHead sell4_head(int nslices, const int* __restrict__ sptr,
                                                const uint16_t* __restrict__ col16,
-                                               const int* __restrict__ cbase, int lb) {
+                                               const int* __restrict__ cbase, int s) {
     SellHead h{0, 0, {-1, 0, 0, 0, 0, 0, 0, 0}};
-    const int s = __builtin_amdgcn_readfirstlane(lb * (BLOCK / SLICE) +
-                                                 (int)((threadIdx.x >> 6) & 3));
     if (s < nslices) {
         h.b0 = sptr[s];
         h.w4 = (sptr[s + 1] - h.b0) >> 8;
@@ -269,39 +297,106 @@ __device__ __forceinline__ SellHead sell4_head(int nslices, const int* __restric
     return h;
 }
 
-// The row sums of one block of BLOCK rows (four slices, logical block lb): row
-// lb * BLOCK + t goes to thread t < BLOCK (zero past nslices).  WS == 1: a block
-// of BLOCK threads, one wavefront per slice.  WS == 4: a block of 4 * BLOCK
-// threads, four wavefronts per slice, one chain each; every thread must call.
-// Four wavefronts per slice are for systems whose slices leave SIMDs idle: the
-// row's serial chain of loads, a few microseconds of latency, is then a
-// quarter as long.
+// The four chains of a block's rows, one from each wavefront, added up: row t
+// of the block to the threads of wavefront t / 64 and those that share its rows.
+template <int WS, typename T>
+__device__ __forceinline__ T add_chains(T acc, int part) {
+    __shared__ T red[4][WS_ROWS<WS>];
+    const int t = (int)(threadIdx.x & (WS_ROWS<WS> - 1));
+    red[part][t] = acc;
+    __syncthreads();
+    return (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]);
+}
+
+// The row sums of one block (logical block lb): row block_row<WS>(lb) to its
+// thread (zero past nslices); every thread must call.
 template <int WS, int U4, typename T, typename TM, typename FV, typename FX>
 __device__ __forceinline__ T sell4_block(int nslices, const int* __restrict__ sptr,
                                          const int* __restrict__ col,
                                          const uint16_t* __restrict__ col16,
                                          const int* __restrict__ cbase,
                                          const TM* __restrict__ a, int lb, FV fv, FX fx) {
-    const SellHead h = sell4_head(nslices, sptr, col16, cbase, lb);
-    const int lane = (int)(threadIdx.x & 63);
-    const int part = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8));
-    T acc = sell4_accumulate<WS, U4, T>(h, col, col16, a, lane, part, fv, fx);
-    if constexpr (WS == 4) {
-        __shared__ T red[4][BLOCK];
-        const int t = (int)(threadIdx.x & (BLOCK - 1));
-        red[part][t] = acc;
-        __syncthreads();
-        acc = (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]);
-    }
+    const SellHead h = sell4_head(nslices, sptr, col16, cbase, ws_slice<WS>(lb));
+    const int part = ws_part<WS>();
+    T acc = sell4_accumulate<(WS == 1 ? 1 : 4), U4, T>(h, col, col16, a,
+                                                       (int)(threadIdx.x & 63), part, fv, fx);
+    if constexpr (WS != 1) acc = add_chains<WS>(acc, part);
     return acc;
 }
 
-// Blocks of BLOCK rows up to which a product runs with four wavefronts per
-// slice: 1024 blocks are 4 wavefronts per SIMD with one per slice.  One
-// against four wavefronts per slice: level-0 residual of a 64k-node cube (249
-// blocks) 11.7 and 9.3 us, of a 216k-node cube (843 blocks) 21.4 and 19.2 us;
-// GMRES product and dot products 17.4 (two launches) and 10.6 us, and 38.3 and
-// 29.2 us.
+// sell4_block<4> for gathered entries fin(raw), raw = pre(column) loaded from
+// the vectors: the columns, values and raw entries of the chain's first two
+// groups are requested before mid() runs, which may hold barriers and returns
+// whether to go on (the same on every thread), so mid's latency and theirs
+// overlap.  ok receives mid's answer.
+template <typename T, typename TM, typename PRE, typename MID, typename FIN>
+__device__ __forceinline__ T sell4_block_early(int nslices, const int* __restrict__ sptr,
+                                               const int* __restrict__ col,
+                                               const uint16_t* __restrict__ col16,
+                                               const int* __restrict__ cbase,
+                                               const TM* __restrict__ a, int lb, PRE pre, MID mid,
+                                               FIN fin, bool& ok) {
+    typedef typename Vec4<TM>::type v4;
+    typedef typename Vec4<int>::type c4;
+    typedef typename Vec4<uint16_t>::type e4;
+    typedef decltype(pre(0)) raw;
+    const SellHead h = sell4_head(nslices, sptr, col16, cbase, ws_slice<4>(lb));
+    const int lane = (int)(threadIdx.x & 63), part = ws_part<4>();
+    const v4* ap = reinterpret_cast<const v4*>(a + h.b0) + lane;
+    auto columns = [&](int g) {
+        c4 c;
+        if (h.base[0] >= 0) {
+            const e4 e = (reinterpret_cast<const e4*>(col16 + h.b0) + lane)[g * SLICE];
+            c.x = col_decode(e.x, h.base);
+            c.y = col_decode(e.y, h.base);
+            c.z = col_decode(e.z, h.base);
+            c.w = col_decode(e.w, h.base);
+        } else {
+            c = (reinterpret_cast<const c4*>(col + h.b0) + lane)[g * SLICE];
+        }
+        return c;
+    };
+    T acc = (T)0;
+    auto add = [&](v4 v, raw r0, raw r1, raw r2, raw r3) {
+        acc = fma((T)v.x, fin(r0), acc);
+        acc = fma((T)v.y, fin(r1), acc);
+        acc = fma((T)v.z, fin(r2), acc);
+        acc = fma((T)v.w, fin(r3), acc);
+    };
+    v4 v[2];
+    raw r[2][4];
+    c4 c[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+        if (part + 4 * u < h.w4) {
+            c[u] = columns(part + 4 * u);
+            v[u] = ap[(part + 4 * u) * SLICE];
+        }
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+        if (part + 4 * u < h.w4) {
+            r[u][0] = pre(c[u].x);
+            r[u][1] = pre(c[u].y);
+            r[u][2] = pre(c[u].z);
+            r[u][3] = pre(c[u].w);
+        }
+    ok = mid();
+    if (!ok) return (T)0;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+        if (part + 4 * u < h.w4) add(v[u], r[u][0], r[u][1], r[u][2], r[u][3]);
+    for (int g = part + 8; g < h.w4; g += 4) {
+        const c4 cc = columns(g);
+        const v4 vv = ap[g * SLICE];
+        add(vv, pre(cc.x), pre(cc.y), pre(cc.z), pre(cc.w));
+    }
+    return add_chains<4>(acc, part);
+}
+
+// Blocks of BLOCK rows up to which a product runs with a wavefront per chain.
+// 1024 blocks are 4 wavefronts per SIMD with one per slice.  Shapes 1, 16 and
+// 4: level-0 residual of a 64k-node cube (249 blocks) 11.7, 9.3 and 6.9 us, FP64
+// product of a 110k-node cube (414 blocks) 18.2, 16.0 and 13.6 us.
 constexpr int SPLIT_MAX_BLOCKS = 1024;
 
 // SELL-64x4 view of the stencil set in device order.
@@ -344,6 +439,9 @@ struct KScalars {
     // right-hand side, 5 breakdown / non-finite, 6 not part of this solve
     int done;
     int iter, maxit, restarts;
+    // fused iterations: 1 when the last iteration's r.r and r0.r still wait in
+    // the partial sums; which of the two buffers holds p and v
+    int pending, par;
 };
 
 // One independent system of a batch: real rows [row0, row0 + nv), its border
@@ -358,7 +456,21 @@ struct SegView {
     int nseg, nrows;    // systems; rows of all systems incl. padding (multiple of BLOCK)
     const Seg* seg;     // [nseg]
     const int* bseg;    // [nrows / BLOCK] system of each row block
+    Seg one;            // the system, when there is only one: it comes with the
+                        // kernel's arguments, two dependent loads (about 1 us
+                        // of a small system's kernel) sooner
 };
+#ifdef __HIPCC__
+// System of logical block lb (block-uniform scalar load), and its rows.
+__device__ __forceinline__ int block_seg(const SegView& sg, int lb) {
+    return sg.nseg == 1 ? 0 : __builtin_amdgcn_readfirstlane(sg.bseg[lb]);
+}
+__device__ __forceinline__ Seg seg_at(const SegView& sg, int q) {
+    Seg s = sg.one;
+    if (sg.nseg != 1) s = sg.seg[q];
+    return s;
+}
+#endif
 
 // Per-system controls of one Krylov run (uploaded before it starts).
 struct SegCtl {

@@ -1,0 +1,87 @@
+"""Krylov solves around the sizes where the small-system kernels take over: 64
+rows per block with a wavefront per chain, BiCGSTAB iterations of three, five or
+eight launches, GMRES with its Hessenberg column in the update.  A system's
+iterates do not depend on which of them runs, so a cavity inside a batch large
+enough for the general kernels equals its stand-alone run bit for bit, and
+every size meets the oracle's operator."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _print(*a):
+    print(*a, flush=True)
+
+
+def _run(ctx, cloud, krylov, precision, steps=2):
+    import memphys_amd as M
+    u_dir, p_dir, u0 = M.lid_conditions(cloud)
+    ctx.weights(3, 3, download=False)
+    ctx.fs_create(1.0, 0.01, 1e-5, 2, 1e-10, 4000, u_dir, u_dir, None, p_dir, krylov=krylov,
+                  precision=precision, restart=30)
+    ctx.set_field(M.MP_U, u0)
+    ctx.set_field(M.MP_V, np.zeros(cloud.nv))
+    ctx.set_field(M.MP_P, np.zeros(ctx.n_sys))
+    ctx.step(steps, 0)
+    return [ctx.get_field(f) for f in (M.MP_U, M.MP_V, M.MP_P)]
+
+
+@pytest.mark.parametrize("krylov", [0, 1])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_small_cavity_in_large_batch_is_bit_identical(krylov, precision):
+    """Cavities of 1, 3, 96, 97 and 128 row blocks alone (three- and five-launch
+    BiCGSTAB, both GMRES updates) and in one batch of more than 1024 blocks
+    (the general kernels)."""
+    import memphys_amd as M
+    sizes = [15, 27, 156, 157, 181, 460]
+    clouds = [M.box_cloud(dim=2, n=n, jitter=0.25, seed=n, k_interior=30) for n in sizes]
+    rows = [-(-(c.nv + 1) // 256) for c in clouds]
+    _print("row blocks", rows)
+    assert rows[:5] == [1, 3, 96, 97, 128] and sum(rows) > 1024
+    with M.Context(0) as ctx:
+        cat = ctx.upload_batch(clouds)
+        batch = _run(ctx, cat, krylov, precision)
+        iters = [ctx.batch_stats(q).iterations for q in range(len(clouds))]
+    off = 0
+    for q, c in enumerate(clouds[:5]):
+        with M.Context(0) as ctx:
+            ctx.upload(c)
+            alone = _run(ctx, c, krylov, precision)
+            st = ctx.stats()
+        _print("n", sizes[q], "blocks", rows[q], "iterations", st.iterations, iters[q])
+        assert st.iterations == iters[q]
+        for a, b in zip(alone, batch):
+            assert np.array_equal(a[:c.nv], b[off:off + c.nv])
+        assert alone[2][c.nv] == batch[2][cat.nv + q]  # border unknown
+        off += c.nv
+
+
+@pytest.mark.parametrize("n,k", [(8, 12), (15, 30), (17, 65), (64, 20)])
+def test_small_system_solves_its_operator(n, k):
+    """Stencils of 12 to 65 entries (one to seventeen groups of four: chains of
+    unequal length, tails past the prefetched groups)."""
+    import memphys_amd as M
+    import oracle as O
+    import scipy.sparse as sp
+    cloud = M.box_cloud(dim=2, n=n, jitter=0.25, seed=3, k_interior=k)
+    w = O.stencil_weights(cloud, 3, 3)[:4]
+    p_dir = np.zeros(cloud.nv, dtype=np.uint8)
+    ones = np.ones(cloud.nv, dtype=np.uint8)
+    fs = O.FractionalStep(cloud, w, ones, ones, None, p_dir, 1.0, 0.01, 1e-3, 2, solver_kind=0,
+                          precond=2, tol=1e-14)
+    rp, ci, v = fs.ppe_csr()
+    rng = np.random.default_rng(n)
+    for prec in (0, 1):
+        with M.Context(0) as ctx:
+            ctx.upload(cloud)
+            ctx.set_weights(*w)
+            m = ctx.solver_init(p_dir, 0.0, 0.0, 1.0, tol=1e-10, n_iter=20000, precision=prec)
+            A = sp.csr_matrix((v, ci, rp), shape=(m, m))
+            b = rng.standard_normal(m)
+            b[-1] = 0.0
+            x, _ = ctx.solve(b, np.zeros(m))
+            res = np.linalg.norm(A @ x - b) / np.linalg.norm(b)
+            _print("n", n, "k", k, "prec", prec, "iterations", ctx.stats().iterations, "res", res)
+            # the solver's own FP64 test, plus the rounding of A x on this host
+            assert res <= 1.1e-10
