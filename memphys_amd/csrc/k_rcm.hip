@@ -5,12 +5,20 @@
 // visited stencil neighbours in stencil order and appends them sorted by
 // (degree, index).  A node reached from level L is therefore claimed by the
 // level-L node of lowest queue position whose stencil holds it, and level L+1
-// is the list of claimed nodes sorted by (claiming position, degree, index):
-// one atomicMin per stencil entry and one radix sort per level give the same
-// numbering.  Nodes the start cannot reach restart the search at the
+// is each level-L node's claimed neighbours, in queue order, sorted by (degree,
+// index).  Per level:
+//   claim   a wavefront per node: atomicMin of (queue position, entry) on every
+//           unvisited column, so each column belongs to one stencil entry;
+//   count   the node's columns that kept its claim;
+//   scan    offsets of the nodes' groups, the next level's bounds;
+//   place   a column's rank inside its group by comparing keys across the
+//           wavefront; its queue position.
+// The levels' bounds live on the device, so the host launches several levels
+// between two looks at them.  A 250k-node cube (about 60 levels): 1.1 ms of kernels
+// where one thread per node, a radix sort and a synchronisation per level took
+// 5.9 ms of kernels and about 2 ms of gaps.
+// Nodes the start cannot reach restart the search at the
 // lowest-index unvisited node of minimum degree.  order[old] = new, reversed.
-#include <hipcub/hipcub.hpp>
-
 #include <algorithm>
 #include <climits>
 #include <stdexcept>
@@ -38,56 +46,151 @@ __global__ __launch_bounds__(BLOCK) void k_rcm_start(int nv, const int* __restri
     if ((threadIdx.x & 63) == 0 && k != ~0ull) atomicMin(best, k);
 }
 
-__global__ void k_rcm_place(const unsigned long long* __restrict__ best, unsigned long long mask,
-                            int at, int* __restrict__ numbering, int* __restrict__ pos) {
-    const int v = (int)(*best & mask);
+// The search's progress: the current level is queue positions a .. b-1 (empty
+// once its component is done).
+struct RcmState {
+    int a, b, levels;
+};
+
+__global__ void k_rcm_root(const unsigned long long* __restrict__ best, unsigned long long mask,
+                           int* __restrict__ numbering, int* __restrict__ pos, RcmState* s) {
+    const int v = (int)(*best & mask), at = s->b;
     numbering[at] = v;
     pos[v] = at;
+    s->a = at;
+    s->b = at + 1;
+    s->levels += 1;
 }
 
-// every stencil entry of the level's nodes claims its unvisited column for
-// the lowest queue position; the first claim appends the column to cand
-__global__ __launch_bounds__(BLOCK) void k_rcm_claim(int a, int b, const int* __restrict__ rp,
+// smallest entry whose column is outside 0 .. nv-1 (LLONG_MAX: none)
+__global__ __launch_bounds__(BLOCK) void k_rcm_check(long nnz, int nv, const int* __restrict__ col,
+                                                     unsigned long long* bad) {
+    for (long e = (long)blockIdx.x * BLOCK + threadIdx.x; e < nnz; e += (long)gridDim.x * BLOCK)
+        if (col[e] < 0 || col[e] >= nv) {
+            atomicMin(bad, (unsigned long long)e);
+            return;
+        }
+}
+
+constexpr int RCM_WAVES = BLOCK / 64;
+constexpr int RCM_BLOCKS = 2048;  // grid of the per-level kernels: 8192 nodes at a time
+
+// every stencil entry of the level's nodes claims its unvisited column
+__global__ __launch_bounds__(BLOCK) void k_rcm_claim(const RcmState* s, const int* __restrict__ rp,
                                                      const int* __restrict__ col,
                                                      const int* __restrict__ numbering,
                                                      const int* __restrict__ pos,
-                                                     int* __restrict__ claim,
-                                                     int* __restrict__ cand,
-                                                     int* __restrict__ ncand) {
-    const int t = a + blockIdx.x * BLOCK + threadIdx.x;
-    if (t >= b) return;
-    const int v = numbering[t];
-    for (int e = rp[v]; e < rp[v + 1]; ++e) {
-        const int c = col[e];
-        if (pos[c] >= 0) continue;
-        if (atomicMin(claim + c, t) == INT_MAX) cand[atomicAdd(ncand, 1)] = c;
+                                                     unsigned long long* __restrict__ claim) {
+    const int b = s->b, lane = threadIdx.x & 63;
+    for (int t = s->a + (int)blockIdx.x * RCM_WAVES + (int)(threadIdx.x >> 6); t < b;
+         t += (int)gridDim.x * RCM_WAVES) {
+        const int v = numbering[t], e0 = rp[v], e1 = rp[v + 1];
+        for (int e = e0 + lane; e < e1; e += 64) {
+            const int c = col[e];
+            if (pos[c] < 0)
+                atomicMin(claim + c, ((unsigned long long)t << 32) | (unsigned)(e - e0));
+        }
     }
 }
 
-__global__ __launch_bounds__(BLOCK) void k_rcm_keys(int n, const int* __restrict__ cand,
-                                                    const int* __restrict__ claim,
-                                                    const int* __restrict__ rp, int idx_bits,
-                                                    int deg_bits,
-                                                    unsigned long long* __restrict__ keys) {
-    const int t = blockIdx.x * BLOCK + threadIdx.x;
-    if (t >= n) return;
-    const int c = cand[t];
-    keys[t] = ((unsigned long long)claim[c] << (idx_bits + deg_bits)) |
-              ((unsigned long long)(rp[c + 1] - rp[c]) << idx_bits) | (unsigned long long)c;
+// entry e (of queue position t's row from e0) holds an unvisited column it claimed
+__device__ __forceinline__ bool rcm_owns(int c, int t, int k, const int* __restrict__ pos,
+                                         const unsigned long long* __restrict__ claim) {
+    return pos[c] < 0 && claim[c] == (((unsigned long long)t << 32) | (unsigned)k);
 }
 
-__global__ __launch_bounds__(BLOCK) void k_rcm_append(int n, int at,
-                                                      const unsigned long long* __restrict__ keys,
-                                                      unsigned long long mask,
-                                                      int* __restrict__ numbering,
-                                                      int* __restrict__ pos,
-                                                      int* __restrict__ claim) {
-    const int t = blockIdx.x * BLOCK + threadIdx.x;
-    if (t >= n) return;
-    const int c = (int)(keys[t] & mask);
-    numbering[at + t] = c;
-    pos[c] = at + t;
-    claim[c] = INT_MAX;
+__global__ __launch_bounds__(BLOCK) void k_rcm_count(const RcmState* s, const int* __restrict__ rp,
+                                                     const int* __restrict__ col,
+                                                     const int* __restrict__ numbering,
+                                                     const int* __restrict__ pos,
+                                                     const unsigned long long* __restrict__ claim,
+                                                     int* __restrict__ cnt) {
+    const int a = s->a, b = s->b, lane = threadIdx.x & 63;
+    for (int t = a + (int)blockIdx.x * RCM_WAVES + (int)(threadIdx.x >> 6); t < b;
+         t += (int)gridDim.x * RCM_WAVES) {
+        const int v = numbering[t], e0 = rp[v], e1 = rp[v + 1];
+        int n = 0;
+        for (int e = e0; e < e1; e += 64) {
+            const bool own = e + lane < e1 && rcm_owns(col[e + lane], t, e + lane - e0, pos, claim);
+            n += __popcll(__ballot(own));
+        }
+        if (lane == 0) cnt[t - a] = n;
+    }
+}
+
+// cnt -> exclusive offsets over the level; the next level's bounds go to out
+// (k_rcm_place still reads the current ones)
+__global__ __launch_bounds__(1024) void k_rcm_scan(const RcmState* s, RcmState* out,
+                                                   int* __restrict__ cnt) {
+    __shared__ int wsum[16];
+    const int n = s->b - s->a, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    int carry = 0;
+    for (int i0 = 0; i0 < n; i0 += 1024) {
+        const int i = i0 + (int)threadIdx.x;
+        const int v = i < n ? cnt[i] : 0;
+        int x = v;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(x, o);
+            if (lane >= o) x += y;
+        }
+        if (lane == 63) wsum[wid] = x;
+        __syncthreads();
+        int before = carry, total = carry;
+        for (int w = 0; w < 16; ++w) {
+            before += w < wid ? wsum[w] : 0;
+            total += wsum[w];
+        }
+        if (i < n) cnt[i] = before + x - v;
+        carry = total;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) *out = RcmState{s->b, s->b + carry, s->levels + (carry > 0 ? 1 : 0)};
+}
+
+// numbers each claimed column: its group's offset plus the columns of the
+// group with a smaller (degree, index); grid.y shares out a long row's chunks
+__global__ __launch_bounds__(BLOCK) void k_rcm_place(const RcmState* s, const int* __restrict__ rp,
+                                                     const int* __restrict__ col,
+                                                     int* __restrict__ numbering,
+                                                     int* __restrict__ pos,
+                                                     const unsigned long long* __restrict__ claim,
+                                                     const int* __restrict__ off, int idx_bits) {
+    const int a = s->a, b = s->b, lane = threadIdx.x & 63;
+    for (int t = a + (int)blockIdx.x * RCM_WAVES + (int)(threadIdx.x >> 6); t < b;
+         t += (int)gridDim.x * RCM_WAVES) {
+        const int v = numbering[t], e0 = rp[v], e1 = rp[v + 1];
+        // (a column's claim stays its owner's after it is numbered, so the test
+        // for the others reads the claim alone)
+        auto mine = [&](int e, int& c) {
+            c = e < e1 ? col[e] : 0;
+            return e < e1 && claim[c] == (((unsigned long long)t << 32) | (unsigned)(e - e0));
+        };
+        for (int e = e0 + 64 * (int)blockIdx.y; e < e1; e += 64 * (int)gridDim.y) {
+            int c;
+            const bool own = mine(e + lane, c);
+            const unsigned long long key =
+                own ? ((unsigned long long)(rp[c + 1] - rp[c]) << idx_bits) | (unsigned)c : ~0ull;
+            if (__ballot(own) == 0) continue;
+            int rank = 0;
+            for (int f = e0; f < e1; f += 64) {
+                int d = c;
+                bool other = own;
+                unsigned long long k = key;
+                if (f != e) {
+                    other = mine(f + lane, d);
+                    k = other ? ((unsigned long long)(rp[d + 1] - rp[d]) << idx_bits) | (unsigned)d
+                              : ~0ull;
+                }
+                for (unsigned long long m = __ballot(other); m; m &= m - 1)
+                    rank += __shfl(k, __ffsll(m) - 1) < key ? 1 : 0;
+            }
+            if (own) {
+                const int at = b + off[t - a] + rank;
+                numbering[at] = c;
+                pos[c] = at;
+            }
+        }
+    }
 }
 
 __global__ __launch_bounds__(BLOCK) void k_rcm_reverse(int nv, const int* __restrict__ numbering,
@@ -96,9 +199,19 @@ __global__ __launch_bounds__(BLOCK) void k_rcm_reverse(int nv, const int* __rest
     if (p < nv) order[numbering[p]] = nv - 1 - p;
 }
 
-__global__ __launch_bounds__(BLOCK) void k_fill_int(int* __restrict__ x, int v, int n) {
+// pos = -1 (unvisited), claim = none
+__global__ __launch_bounds__(BLOCK) void k_rcm_init(int nv, int* __restrict__ pos,
+                                                    unsigned long long* __restrict__ claim,
+                                                    RcmState* s, unsigned long long* bad) {
     const int i = blockIdx.x * BLOCK + threadIdx.x;
-    if (i < n) x[i] = v;
+    if (i < nv) {
+        pos[i] = -1;
+        claim[i] = ~0ull;
+    }
+    if (i == 0) {
+        s[0] = s[1] = RcmState{0, 0, 0};
+        *bad = ~0ull;
+    }
 }
 
 int bits_for(long v) {  // bits to hold 0..v
@@ -119,80 +232,75 @@ void rcm_order(hipStream_t st, int nv, const int* row_ptr, const int* col, int* 
         max_deg = std::max(max_deg, row_ptr[i + 1] - row_ptr[i]);
     }
     const long nnz = row_ptr[nv];
-    for (long e = 0; e < nnz; ++e)
-        if (col[e] < 0 || col[e] >= nv)
-            throw std::invalid_argument("rcm: column " + std::to_string(col[e]) +
-                                        " out of range");
     const int idx_bits = bits_for(nv - 1);
     const int deg_bits = bits_for(max_deg);
     if (2 * idx_bits + deg_bits > 64)
         throw std::invalid_argument("rcm: graph too large for 64-bit sort keys");
     const unsigned long long mask = (1ull << idx_bits) - 1ull;
+    // (ranking a row's columns is quadratic in its length: rows of thousands of
+    // entries are shared by up to 64 wavefronts)
+    const int gy = std::min(64, std::max(1, max_deg / MAX_STENCIL));
 
-    DevBuf<int> drp, dcol, numbering, pos, claim, cand, ncand, dorder;
-    DevBuf<unsigned long long> keys, keys_sorted, best;
+    DevBuf<int> drp, dcol, numbering, pos, cnt, dorder;
+    DevBuf<unsigned long long> claim, best;  // best: [0] the start's key, [1] the column check
+    DevBuf<RcmState> state;  // two: the current level and the next
     drp.alloc((size_t)nv + 1);
     dcol.alloc(std::max<long>(nnz, 1));
     numbering.alloc(nv);
     pos.alloc(nv);
     claim.alloc(nv);
-    cand.alloc(nv);
-    ncand.alloc(1);
+    cnt.alloc(nv);
     dorder.alloc(nv);
-    keys.alloc(nv);
-    keys_sorted.alloc(nv);
-    best.alloc(1);
+    best.alloc(2);
+    state.alloc(2);
     MP_HIP(hipMemcpyAsync(drp.p, row_ptr, sizeof(int) * (nv + 1), hipMemcpyHostToDevice, st));
     if (nnz > 0)
         MP_HIP(hipMemcpyAsync(dcol.p, col, sizeof(int) * nnz, hipMemcpyHostToDevice, st));
     const int nb = (nv + BLOCK - 1) / BLOCK;
-    hipLaunchKernelGGL(k_fill_int, dim3(nb), dim3(BLOCK), 0, st, pos.p, -1, nv);
-    hipLaunchKernelGGL(k_fill_int, dim3(nb), dim3(BLOCK), 0, st, claim.p, INT_MAX, nv);
+    hipLaunchKernelGGL(k_rcm_init, dim3(nb), dim3(BLOCK), 0, st, nv, pos.p, claim.p, state.p,
+                       best.p + 1);
+    hipLaunchKernelGGL(k_rcm_check, dim3(RCM_BLOCKS), dim3(BLOCK), 0, st, nnz, nv, dcol.p,
+                       best.p + 1);
     MP_HIP(hipGetLastError());
-    size_t tmp_bytes = 0;
-    MP_HIP(hipcub::DeviceRadixSort::SortKeys(nullptr, tmp_bytes, keys.p, keys_sorted.p, nv, 0,
-                                             2 * idx_bits + deg_bits, st));
-    DevBuf<unsigned char> tmp;
-    tmp.alloc(std::max<size_t>(tmp_bytes, 1));
-    int numbered = 0, levels = 0;
-    int* h_n = nullptr;
-    MP_HIP(hipHostMalloc((void**)&h_n, sizeof(int), 0));
+    struct Polled {
+        RcmState s;
+        unsigned long long bad;
+    };
+    Polled* h = nullptr;
+    MP_HIP(hipHostMalloc((void**)&h, sizeof(Polled), 0));
     try {
-        while (numbered < nv) {
-            MP_HIP(hipMemsetAsync(best.p, 0xFF, sizeof(unsigned long long), st));
-            hipLaunchKernelGGL(k_rcm_start, dim3(nb), dim3(BLOCK), 0, st, nv, drp.p, pos.p,
-                               idx_bits, best.p);
-            hipLaunchKernelGGL(k_rcm_place, dim3(1), dim3(1), 0, st, best.p, mask, numbered,
-                               numbering.p, pos.p);
-            MP_HIP(hipGetLastError());
-            int a = numbered, b = numbered + 1;
-            numbered = b;
-            ++levels;
-            while (b > a) {
-                MP_HIP(hipMemsetAsync(ncand.p, 0, sizeof(int), st));
-                hipLaunchKernelGGL(k_rcm_claim, dim3((b - a + BLOCK - 1) / BLOCK), dim3(BLOCK),
-                                   0, st, a, b, drp.p, dcol.p, numbering.p, pos.p, claim.p,
-                                   cand.p, ncand.p);
-                MP_HIP(hipGetLastError());
-                MP_HIP(hipMemcpyAsync(h_n, ncand.p, sizeof(int), hipMemcpyDeviceToHost, st));
-                MP_HIP(hipStreamSynchronize(st));
-                const int n = *h_n;
-                if (n == 0) break;
-                if (n > nv - numbered) throw std::runtime_error("rcm: level overflow");
-                const int gb = (n + BLOCK - 1) / BLOCK;
-                hipLaunchKernelGGL(k_rcm_keys, dim3(gb), dim3(BLOCK), 0, st, n, cand.p, claim.p,
-                                   drp.p, idx_bits, deg_bits, keys.p);
-                MP_HIP(hipcub::DeviceRadixSort::SortKeys(tmp.p, tmp_bytes, keys.p,
-                                                         keys_sorted.p, n, 0,
-                                                         2 * idx_bits + deg_bits, st));
-                hipLaunchKernelGGL(k_rcm_append, dim3(gb), dim3(BLOCK), 0, st, n, numbered,
-                                   keys_sorted.p, mask, numbering.p, pos.p, claim.p);
-                MP_HIP(hipGetLastError());
-                a = numbered;
-                numbered += n;
-                b = numbered;
-                ++levels;
+        MP_HIP(hipMemcpyAsync(&h->bad, best.p + 1, sizeof(h->bad), hipMemcpyDeviceToHost, st));
+        MP_HIP(hipStreamSynchronize(st));
+        if (h->bad != ~0ull)
+            throw std::invalid_argument("rcm: column " + std::to_string(col[h->bad]) +
+                                        " out of range");
+        int cur = 0;
+        h->s = RcmState{0, 0, 0};
+        while (h->s.b < nv) {
+            if (h->s.a == h->s.b) {  // (no level left: the next component's root)
+                MP_HIP(hipMemsetAsync(best.p, 0xFF, sizeof(unsigned long long), st));
+                hipLaunchKernelGGL(k_rcm_start, dim3(nb), dim3(BLOCK), 0, st, nv, drp.p, pos.p,
+                                   idx_bits, best.p);
+                hipLaunchKernelGGL(k_rcm_root, dim3(1), dim3(1), 0, st, best.p, mask, numbering.p,
+                                   pos.p, state.p + cur);
             }
+            // 16 levels between two looks: those past the component's last are
+            // empty (four launches of about 2 us each)
+            for (int l = 0; l < 16; ++l) {
+                RcmState *s = state.p + cur, *next = state.p + (cur ^ 1);
+                hipLaunchKernelGGL(k_rcm_claim, dim3(RCM_BLOCKS), dim3(BLOCK), 0, st, s, drp.p,
+                                   dcol.p, numbering.p, pos.p, claim.p);
+                hipLaunchKernelGGL(k_rcm_count, dim3(RCM_BLOCKS), dim3(BLOCK), 0, st, s, drp.p,
+                                   dcol.p, numbering.p, pos.p, claim.p, cnt.p);
+                hipLaunchKernelGGL(k_rcm_scan, dim3(1), dim3(1024), 0, st, s, next, cnt.p);
+                hipLaunchKernelGGL(k_rcm_place, dim3(RCM_BLOCKS, gy), dim3(BLOCK), 0, st, s, drp.p,
+                                   dcol.p, numbering.p, pos.p, claim.p, cnt.p, idx_bits);
+                cur ^= 1;
+            }
+            MP_HIP(hipGetLastError());
+            MP_HIP(hipMemcpyAsync(&h->s, state.p + cur, sizeof(RcmState), hipMemcpyDeviceToHost,
+                                  st));
+            MP_HIP(hipStreamSynchronize(st));
         }
         hipLaunchKernelGGL(k_rcm_reverse, dim3(nb), dim3(BLOCK), 0, st, nv, numbering.p,
                            dorder.p);
@@ -200,10 +308,11 @@ void rcm_order(hipStream_t st, int nv, const int* row_ptr, const int* col, int* 
         MP_HIP(hipMemcpyAsync(order, dorder.p, sizeof(int) * nv, hipMemcpyDeviceToHost, st));
         MP_HIP(hipStreamSynchronize(st));
     } catch (...) {
-        (void)hipHostFree(h_n);
+        (void)hipHostFree(h);
         throw;
     }
-    (void)hipHostFree(h_n);
+    const int levels = h->s.levels;
+    (void)hipHostFree(h);
     if (levels_out) *levels_out = levels;
 }
 

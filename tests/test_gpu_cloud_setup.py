@@ -165,3 +165,34 @@ def test_rcm_rejects_bad_graph():
             ctx.rcm_order(rp, np.array([0, 5, 1], dtype=np.int32))
         with pytest.raises(M.MemphysError):
             ctx.rcm_order(rp, np.array([0, -1, 1], dtype=np.int32))
+
+
+@pytest.mark.parametrize("seed,nv,deg", [(1, 1, 1), (2, 65, 3), (3, 700, 130), (4, 5000, 20)])
+def test_rcm_random_graphs_match_host(seed, nv, deg):
+    """Random CSR rows (not symmetric, with repeated columns, empty rows, rows
+    of one to several wavefront chunks, several components)."""
+    import memphys_amd as M
+    rng = np.random.default_rng(seed)
+    length = rng.integers(0, deg + 1, nv)
+    rp = np.concatenate([[0], np.cumsum(length)]).astype(np.int32)
+    # columns near the row, so that some seeds fall into many components
+    col = (np.repeat(np.arange(nv), length) + rng.integers(-deg, deg + 1, rp[-1])) % nv
+    col = col.astype(np.int32)
+    with M.Context(0) as ctx:
+        assert np.array_equal(ctx.rcm_order(rp, col), _host_rcm(rp, col))
+
+
+@pytest.mark.parametrize("nv", [900, 3000])
+def test_rcm_star_matches_host(nv):
+    """One row that holds every node (its columns ranked by several wavefronts),
+    the others holding the hub and themselves."""
+    import memphys_amd as M
+    rows = [np.arange(nv)] + [np.array([i, 0]) for i in range(1, nv)]
+    rp = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    col = np.concatenate(rows).astype(np.int32)
+    with M.Context(0) as ctx:
+        assert np.array_equal(ctx.rcm_order(rp, col), _host_rcm(rp, col))
+        bad = col.copy()
+        bad[[7, nv]] = nv, -1
+        with pytest.raises(M.MemphysError, match=f"column {nv} out of range"):
+            ctx.rcm_order(rp, bad)
