@@ -26,7 +26,6 @@ __device__ __forceinline__ uint16_t f2bf(float f) {
 
 constexpr int H = GNN_H;
 constexpr int F = GNN_F;
-constexpr int RG = 4;  // rows per block iteration of the dense kernels (4 x 64 threads)
 
 // sum of squares of (p1 - p2) over the node block -> block partials
 __global__ __launch_bounds__(256) void k_sq_partial(int nv, const double* __restrict__ p1,
@@ -44,14 +43,20 @@ __global__ __launch_bounds__(256) void k_sq_partial(int nv, const double* __rest
     if (threadIdx.x == 0) part[blockIdx.x] = sh[0] + sh[1] + sh[2] + sh[3];
 }
 
-// s = sqrt(mean) with a floor, into scal[0]
-__global__ void k_scale_finish(int nb, int nv, const double* __restrict__ part,
-                               double* __restrict__ scal) {
-    if (threadIdx.x != 0) return;
+// sum of nb partials by one wavefront
+__device__ __forceinline__ double wave_sum(int nb, const double* __restrict__ part) {
     double s = 0.0;
-    for (int b = 0; b < nb; ++b) s += part[b];
-    s = sqrt(s / (double)nv);
-    scal[0] = (s > 1e-300) ? s : 1.0;
+    for (int b = threadIdx.x; b < nb; b += 64) s += part[b];
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    return s;
+}
+
+// s = sqrt(mean) with a floor, into scal[0] (one wavefront)
+__global__ __launch_bounds__(64) void k_scale_finish(int nb, int nv,
+                                                     const double* __restrict__ part,
+                                                     double* __restrict__ scal) {
+    const double s = sqrt(wave_sum(nb, part) / (double)nv);
+    if (threadIdx.x == 0) scal[0] = (s > 1e-300) ? s : 1.0;
 }
 
 __global__ __launch_bounds__(256) void k_features(int nv, const double* __restrict__ p1,
@@ -238,22 +243,85 @@ __global__ __launch_bounds__(256) void k_dense_mfma(int nv, const float* __restr
     }
 }
 
-// out[i][k] = sum_c dZ[i][c] W[k][c] (+ out[i][k] if accumulate); W: [K][H]
-template <int K>
-__global__ __launch_bounds__(256) void k_dense_t(int nv, const float* __restrict__ dZ,
-                                                 const uint16_t* __restrict__ W,
-                                                 float* __restrict__ out, int accumulate) {
-    __shared__ float w[K * H];
-    for (int t = threadIdx.x; t < K * H; t += 256) w[t] = bf2f(W[t]);
+// Backward through a hidden layer on the matrix cores: dZ = dH * (Z > 0), out_n =
+// dZ Wn^T and out_s = dZ Ws^T (Wn, Ws: [H][H], out[i][k] = sum_c dZ[i][c] W[k][c]).
+// dH null: the output layer's, dH[i][c] = dd_i wo[c].  out_s may be dH (a wavefront
+// reads its tile's rows before it writes them).  Tiles, fragments and precision
+// as in k_dense_mfma: the 64 reduction indices c in 16 steps of 4, lane l at c =
+// 16 j + 4 (l / 16) + e; the two transposed weights side by side, eight blocks
+// of 16 columns.  A 64k-node layer: 30 us, where the ReLU pass and one thread per
+// output and product took 12 + 2 x 118 us.
+__global__ __launch_bounds__(256) void k_back_mfma(int nv, const float* dH,
+                                                   const float* __restrict__ dd,
+                                                   const uint16_t* __restrict__ wo,
+                                                   const float* __restrict__ Z,
+                                                   const uint16_t* __restrict__ Wn,
+                                                   const uint16_t* __restrict__ Ws,
+                                                   float* __restrict__ dZ,
+                                                   float* __restrict__ out_n, float* out_s) {
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    __shared__ f4 wf[4 * 8 * 64];
+    for (int t = threadIdx.x; t < 4 * 8 * 64; t += 256) {
+        const int lane = t & 63, nb = (t >> 6) & 7, j = t >> 9;
+        const int n = 16 * (nb & 3) + (lane & 15);
+        const uint16_t* W = nb < 4 ? Wn : Ws;
+        f4 v;
+        for (int e = 0; e < 4; ++e) v[e] = bf2f(W[n * H + 16 * j + 4 * (lane >> 4) + e]);
+        wf[t] = v;
+    }
     __syncthreads();
-    const int k = threadIdx.x & 63;
-    if (k >= K) return;
-    for (int row = blockIdx.x * RG + (threadIdx.x >> 6); row < nv; row += gridDim.x * RG) {
-        const float* d = dZ + (size_t)row * H;
-        float acc = accumulate ? out[(size_t)row * K + k] : 0.0f;
-#pragma unroll 8
-        for (int c = 0; c < H; ++c) acc = fmaf(d[c], w[k * H + c], acc);
-        out[(size_t)row * K + k] = acc;
+    const int lane = threadIdx.x & 63;
+    const int q = lane >> 4, c = lane & 15;
+    const int ntiles = (nv + MROWS - 1) / MROWS;
+    for (int tile = blockIdx.x * 4 + (threadIdx.x >> 6); tile < ntiles; tile += gridDim.x * 4) {
+        const int r0 = tile * MROWS;
+        const int row = r0 + c;
+        f4 a[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) a[j] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (row < nv) {
+            const float ddi = dH ? 0.0f : dd[row];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int k = 16 * j + 4 * q;
+                const size_t o = (size_t)row * H + k;
+                f4 g;
+                if (dH)
+                    g = *reinterpret_cast<const f4*>(dH + o);
+                else
+                    for (int e = 0; e < 4; ++e) g[e] = ddi * bf2f(wo[k + e]);
+                const f4 z = *reinterpret_cast<const f4*>(Z + o);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) a[j][e] = z[e] > 0.0f ? g[e] : 0.0f;
+                *reinterpret_cast<f4*>(dZ + o) = a[j];
+            }
+        }
+        f4 acc[8];
+#pragma unroll
+        for (int nb = 0; nb < 8; ++nb) acc[nb] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+#pragma unroll
+            for (int nb = 0; nb < 8; ++nb) {
+                const f4 w = wf[(j * 8 + nb) * 64 + lane];
+                acc[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j].x, w.x, acc[nb], 0, 0, 0);
+                acc[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j].y, w.y, acc[nb], 0, 0, 0);
+                acc[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j].z, w.z, acc[nb], 0, 0, 0);
+                acc[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j].w, w.w, acc[nb], 0, 0, 0);
+            }
+        }
+        // lane holds rows r0 + 4q + i, columns 16 nb + c
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = r0 + 4 * q + i;
+            if (r >= nv) break;
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb) {
+                const size_t o = (size_t)r * H + 16 * nb + c;
+                out_n[o] = acc[nb][i];
+                out_s[o] = acc[nb + 4][i];
+            }
+        }
     }
 }
 
@@ -370,97 +438,174 @@ __global__ __launch_bounds__(256) void k_loss(int nv, const float* __restrict__ 
     if (threadIdx.x == 0) part[blockIdx.x] = sh[0] + sh[1] + sh[2] + sh[3];
 }
 
-__global__ void k_loss_finish(int nb, int nv, const double* __restrict__ part,
-                              double* __restrict__ scal) {
-    if (threadIdx.x != 0) return;
-    double s = 0.0;
-    for (int b = 0; b < nb; ++b) s += part[b];
-    scal[1] = s / (double)nv;
+__global__ __launch_bounds__(64) void k_loss_finish(int nb, int nv,
+                                                    const double* __restrict__ part,
+                                                    double* __restrict__ scal) {
+    const double s = wave_sum(nb, part);
+    if (threadIdx.x == 0) scal[1] = s / (double)nv;
 }
 
-// dH[i][c] = dd_i wo[c]
-__global__ __launch_bounds__(256) void k_outer_wo(int nv, const float* __restrict__ dd,
-                                                  const uint16_t* __restrict__ wo,
-                                                  float* __restrict__ dH) {
-    const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (t >= (size_t)nv * H) return;
-    dH[t] = dd[t / H] * bf2f(wo[t % H]);
-}
-
-// dZ = dH * (Z > 0)
-__global__ __launch_bounds__(256) void k_relu_back(size_t n, const float* __restrict__ dH,
-                                                   const float* __restrict__ Z,
-                                                   float* __restrict__ dZ) {
-    const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (t < n) dZ[t] = (Z[t] > 0.0f) ? dH[t] : 0.0f;
-}
-
-// Weight gradients: part[b][k][c] = sum over this block's rows of A[i][k] B[i][c]
-// for k < KA, plus row KA = sum B[i][c] (bias) when BIAS.  256 threads own the
-// (KA+BIAS) x KB outputs; rows are staged through LDS 16 at a time.
-template <int KA, int KB, bool BIAS>
-__global__ __launch_bounds__(256) void k_wgrad_partial(int nv, const float* __restrict__ A,
-                                                       const float* __restrict__ B,
-                                                       float* __restrict__ part) {
-    constexpr int KR = KA + (BIAS ? 1 : 0);
-    constexpr int NOUT = KR * KB;
-    constexpr int PER = (NOUT + 255) / 256;
-    constexpr int TR = 16;
-    __shared__ float sa[TR][KA > 0 ? KA : 1];
-    __shared__ float sb[TR][KB];
-    float acc[PER];
+// Weight gradients of a hidden layer: block b's sums over its rows of h^T dZ,
+// m^T dZ (64 x 64 each) and of dZ (the bias) into part[b][8256], in that order
+// (the layer's order in the packed gradient).  Contractions over the rows on
+// the FP32 matrix cores (v_mfma_f32_16x16x4f32, four rows a step): lane l loads
+// features 4 (l % 16) .. + 3 of row l / 16 of the step, one 16-byte load per
+// matrix, and element e of the loads feeds the blocks of features 4 i + e and
+// columns 4 j + e.  The block's four wavefronts add up in LDS.  A 64k-node
+// layer: 28 us for both products, where LDS tiles and one thread per 16
+// outputs took 83 + 78 us.
+constexpr int WG_OUT = 2 * H * H + H;
+__global__ __launch_bounds__(256) void k_wgrad_mfma(int nv, const float* __restrict__ h,
+                                                    const float* __restrict__ m,
+                                                    const float* __restrict__ dZ,
+                                                    float* __restrict__ part) {
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    __shared__ float sum[WG_OUT];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int q = lane >> 4, c = lane & 15;
+    f4 a1[4][4], a2[4][4], bias = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int q = 0; q < PER; ++q) acc[q] = 0.0f;
-    const int rows_per_block = (nv + gridDim.x - 1) / gridDim.x;
-    const int r0 = blockIdx.x * rows_per_block;
-    const int r1 = min(nv, r0 + rows_per_block);
-    for (int t0 = r0; t0 < r1; t0 += TR) {
-        const int nr = min(TR, r1 - t0);
-        for (int t = threadIdx.x; t < TR * KA; t += 256) {
-            const int rr = t / KA, kk = t - rr * KA;
-            sa[rr][kk] = (rr < nr) ? A[(size_t)(t0 + rr) * KA + kk] : 0.0f;
-        }
-        for (int t = threadIdx.x; t < TR * KB; t += 256) {
-            const int rr = t / KB, kk = t - rr * KB;
-            sb[rr][kk] = (rr < nr) ? B[(size_t)(t0 + rr) * KB + kk] : 0.0f;
-        }
-        __syncthreads();
+    for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int q = 0; q < PER; ++q) {
-            const int o = threadIdx.x + q * 256;
-            if (o < NOUT) {
-                const int k = o / KB, c = o - k * KB;
-                float a = acc[q];
-                for (int rr = 0; rr < TR; ++rr) {
-                    const float av = (k < KA) ? sa[rr][k] : 1.0f;
-                    a = fmaf(av, sb[rr][c], a);
+        for (int f = 0; f < 4; ++f) a1[e][f] = a2[e][f] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    const f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    // steps of four rows, dealt out to the grid's wavefronts in turn
+    const int nw = gridDim.x * 4;
+    for (int r = (blockIdx.x * 4 + wid) * 4; r < nv; r += nw * 4) {
+        const int row = r + q;
+        const bool ok = row < nv;
+        const size_t o = (size_t)(ok ? row : 0) * H + 4 * c;
+        f4 x = *reinterpret_cast<const f4*>(h + o);
+        f4 y = *reinterpret_cast<const f4*>(m + o);
+        f4 d = *reinterpret_cast<const f4*>(dZ + o);
+        if (!ok) x = y = d = zero;
+        bias += d;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int f = 0; f < 4; ++f) {
+                a1[e][f] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], d[f], a1[e][f], 0, 0, 0);
+                a2[e][f] = __builtin_amdgcn_mfma_f32_16x16x4f32(y[e], d[f], a2[e][f], 0, 0, 0);
+            }
+    }
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {  // over the four rows of a step
+        bias[f] += __shfl_xor(bias[f], 16);
+        bias[f] += __shfl_xor(bias[f], 32);
+    }
+    // element i of block (e, f): feature 4 (4 q + i) + e, column 4 c + f
+    for (int w = 0; w < 4; ++w) {
+        if (wid == w) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int o = (4 * (4 * q + i) + e) * H + 4 * c;
+                    f4 *s1 = reinterpret_cast<f4*>(sum + o),
+                       *s2 = reinterpret_cast<f4*>(sum + H * H + o);
+                    const f4 v1 = {a1[e][0][i], a1[e][1][i], a1[e][2][i], a1[e][3][i]};
+                    const f4 v2 = {a2[e][0][i], a2[e][1][i], a2[e][2][i], a2[e][3][i]};
+                    *s1 = w ? *s1 + v1 : v1;
+                    *s2 = w ? *s2 + v2 : v2;
                 }
-                acc[q] = a;
+            if (q == 0) {
+                f4* sb = reinterpret_cast<f4*>(sum + 2 * H * H + 4 * c);
+                *sb = w ? *sb + bias : bias;
             }
         }
         __syncthreads();
     }
-#pragma unroll
-    for (int q = 0; q < PER; ++q) {
-        const int o = threadIdx.x + q * 256;
-        if (o < NOUT) part[(size_t)blockIdx.x * NOUT + o] = acc[q];
-    }
+    for (int t = threadIdx.x; t < WG_OUT; t += 256) part[(size_t)blockIdx.x * WG_OUT + t] = sum[t];
 }
 
-// grad[off + o] = sum_b part[b][o] (block order); bias row goes to bias_off
-__global__ __launch_bounds__(256) void k_wgrad_finish(int nb, int nout, int kb, int ka,
+// Weight gradients of the input layer, through its ReLU (dZ0 = dH * (Z0 > 0)):
+// block b's sums of X^T dZ0 and dZ0 into part[b][6 * 64]; thread c of a row
+// group owns column c.
+constexpr int WIN_OUT = (F + 1) * H;
+__global__ __launch_bounds__(256) void k_wgrad_in(int nv, const float* __restrict__ X,
+                                                  const float* __restrict__ dH,
+                                                  const float* __restrict__ Z,
+                                                  float* __restrict__ part) {
+    __shared__ float sum[4][WIN_OUT];
+    const int c = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    float acc[F + 1] = {};
+    const int step = gridDim.x * 4;
+    auto add = [&](float z, float g, const float* x) {
+        const float d = z > 0.0f ? g : 0.0f;
+#pragma unroll
+        for (int f = 0; f < F; ++f) acc[f] = fmaf(x[f], d, acc[f]);
+        acc[F] += d;
+    };
+    // (eight rows' loads in flight)
+    int row = __builtin_amdgcn_readfirstlane((int)blockIdx.x * 4 + wid);
+    for (; row + 7 * step < nv; row += 8 * step) {
+        float z[8], g[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            z[u] = Z[(size_t)(row + u * step) * H + c];
+            g[u] = dH[(size_t)(row + u * step) * H + c];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) add(z[u], g[u], X + (size_t)(row + u * step) * F);
+    }
+    for (; row < nv; row += step)
+        add(Z[(size_t)row * H + c], dH[(size_t)row * H + c], X + (size_t)row * F);
+#pragma unroll
+    for (int f = 0; f <= F; ++f) sum[wid][f * H + c] = acc[f];
+    __syncthreads();
+    for (int t = threadIdx.x; t < WIN_OUT; t += 256)
+        part[(size_t)blockIdx.x * WIN_OUT + t] = (sum[0][t] + sum[1][t]) + (sum[2][t] + sum[3][t]);
+}
+
+// Weight gradients of the output layer: block b's sums of h^T dd and dd into
+// part[b][65].
+constexpr int WOUT_OUT = H + 1;
+__global__ __launch_bounds__(256) void k_wgrad_out(int nv, const float* __restrict__ h,
+                                                   const float* __restrict__ dd,
+                                                   float* __restrict__ part) {
+    __shared__ float sum[4][WOUT_OUT];
+    const int c = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    float acc = 0.0f, b = 0.0f;
+    const int step = gridDim.x * 4;
+    int row = __builtin_amdgcn_readfirstlane((int)blockIdx.x * 4 + wid);
+    for (; row + 7 * step < nv; row += 8 * step) {  // (eight rows' loads in flight)
+        float x[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) x[u] = h[(size_t)(row + u * step) * H + c];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            acc = fmaf(x[u], dd[row + u * step], acc);
+            b += dd[row + u * step];
+        }
+    }
+    for (; row < nv; row += step) {
+        acc = fmaf(h[(size_t)row * H + c], dd[row], acc);
+        b += dd[row];
+    }
+    sum[wid][c] = acc;
+    if (c == 0) sum[wid][H] = b;
+    __syncthreads();
+    for (int t = threadIdx.x; t < WOUT_OUT; t += 256)
+        part[(size_t)blockIdx.x * WOUT_OUT + t] = (sum[0][t] + sum[1][t]) + (sum[2][t] + sum[3][t]);
+}
+
+// grad[o] = sum_b part[b][o]: a block takes 64 outputs, four groups of threads
+// every fourth partial each.
+__global__ __launch_bounds__(256) void k_wgrad_finish(int nb, int nout,
                                                       const float* __restrict__ part,
-                                                      float* __restrict__ grad, int w_off,
-                                                      int bias_off) {
-    const int o = blockIdx.x * 256 + threadIdx.x;
-    if (o >= nout) return;
+                                                      float* __restrict__ grad) {
+    __shared__ float sum[4][64];
+    const int lane = threadIdx.x & 63, g = threadIdx.x >> 6;
+    const int o = blockIdx.x * 64 + lane;
     float s = 0.0f;
-    for (int b = 0; b < nb; ++b) s += part[(size_t)b * nout + o];
-    const int k = o / kb, c = o - k * kb;
-    if (k < ka)
-        grad[w_off + o] = s;
-    else
-        grad[bias_off + c] = s;
+    if (o < nout) {
+#pragma unroll 8
+        for (int b = g; b < nb; b += 4) s += part[(size_t)b * nout + o];
+    }
+    sum[g][lane] = s;
+    __syncthreads();
+    if (g == 0 && o < nout)
+        grad[o] = (sum[0][lane] + sum[1][lane]) + (sum[2][lane] + sum[3][lane]);
 }
 
 __global__ __launch_bounds__(256) void k_adam(int n, float* __restrict__ th,
@@ -488,7 +633,7 @@ __global__ __launch_bounds__(256) void k_to_bf(int n, const float* __restrict__ 
 
 inline int blocks(size_t n) { return (int)((n + 255) / 256); }
 constexpr int DENSE_GRID = 2048;
-constexpr int WG_GRID = 256;
+constexpr int WG_GRID = 256;  // blocks (partials) of the weight-gradient kernels
 
 }  // namespace
 
@@ -570,7 +715,7 @@ void GuessNet::setup(hipStream_t st, const SellView& view, const float* a32_slot
     scal.alloc(8);
     partial.alloc(4096);
     wpart_blocks = WG_GRID;
-    wpart.alloc((size_t)WG_GRID * (H + 1) * H);
+    wpart.alloc((size_t)WG_GRID * WG_OUT);
     MP_HIP(hipMemsetAsync(adam_m.p, 0, sizeof(float) * GNN_NPARAM, st));
     MP_HIP(hipMemsetAsync(adam_v.p, 0, sizeof(float) * GNN_NPARAM, st));
     MP_HIP(hipMemsetAsync(grad.p, 0, sizeof(float) * GNN_NPARAM, st));
@@ -650,41 +795,35 @@ void GuessNet::guess(hipStream_t st, const double* base, double* dst) {
 void GuessNet::backward(hipStream_t st, const double* base, const double* pt) {
     const uint16_t* P = theta_bf.p;
     const int nb = 256;
-    const size_t nh = (size_t)nv * H;
     hipLaunchKernelGGL(k_loss, dim3(nb), dim3(256), 0, st, nv, out.p, base, pt, scal.p, dbuf.p,
                        partial.p);
     hipLaunchKernelGGL(k_loss_finish, dim3(1), dim3(64), 0, st, nb, nv, partial.p, scal.p);
-    // output layer: grad wo, bo; dH3
-    hipLaunchKernelGGL((k_wgrad_partial<H, 1, true>), dim3(WG_GRID), dim3(256), 0, st, nv,
-                       Hh[GNN_L].p, dbuf.p, wpart.p);
-    hipLaunchKernelGGL(k_wgrad_finish, dim3(blocks(H + 1)), dim3(256), 0, st, WG_GRID, H + 1, 1, H,
-                       wpart.p, grad.p, GNN_WO, GNN_BO);
-    hipLaunchKernelGGL(k_outer_wo, dim3(blocks(nh)), dim3(256), 0, st, nv, dbuf.p, P + GNN_WO, dH.p);
-    const int g = std::min(DENSE_GRID, (nv + RG - 1) / RG);
+    auto finish = [&](int nout, int off) {
+        hipLaunchKernelGGL(k_wgrad_finish, dim3((nout + 63) / 64), dim3(256), 0, st, WG_GRID, nout,
+                           (const float*)wpart.p, grad.p + off);
+    };
+    // output layer: grad wo, bo
+    hipLaunchKernelGGL(k_wgrad_out, dim3(WG_GRID), dim3(256), 0, st, nv, Hh[GNN_L].p, dbuf.p,
+                       wpart.p);
+    finish(WOUT_OUT, GNN_WO);
+    const int g = std::min(DENSE_GRID, (nv + 4 * MROWS - 1) / (4 * MROWS));
     for (int l = GNN_L; l >= 1; --l) {
         const int o = GNN_LAYER + (l - 1) * GNN_LAYER_SIZE;
-        hipLaunchKernelGGL(k_relu_back, dim3(blocks(nh)), dim3(256), 0, st, nh, dH.p, Z[l].p, dZ.p);
-        // dWs = h_{l-1}^T dZ (+ db), dWn = m_l^T dZ
-        hipLaunchKernelGGL((k_wgrad_partial<H, H, true>), dim3(WG_GRID), dim3(256), 0, st, nv,
-                           Hh[l - 1].p, dZ.p, wpart.p);
-        hipLaunchKernelGGL(k_wgrad_finish, dim3(blocks((H + 1) * H)), dim3(256), 0, st, WG_GRID,
-                           (H + 1) * H, H, H, wpart.p, grad.p, o, o + 2 * H * H);
-        hipLaunchKernelGGL((k_wgrad_partial<H, H, false>), dim3(WG_GRID), dim3(256), 0, st, nv,
-                           Mm[l].p, dZ.p, wpart.p);
-        hipLaunchKernelGGL(k_wgrad_finish, dim3(blocks(H * H)), dim3(256), 0, st, WG_GRID, H * H,
-                           H, H, wpart.p, grad.p, o + H * H, 0);
+        // dZ through the ReLU; dTmp = dZ Wn^T, dH = dZ Ws^T
+        hipLaunchKernelGGL(k_back_mfma, dim3(g), dim3(256), 0, st, nv,
+                           l == GNN_L ? (const float*)nullptr : (const float*)dH.p,
+                           (const float*)dbuf.p, P + GNN_WO, (const float*)Z[l].p, P + o + H * H,
+                           P + o, dZ.p, dTmp.p, dH.p);
+        // dWs = h_{l-1}^T dZ, dWn = m_l^T dZ, db
+        hipLaunchKernelGGL(k_wgrad_mfma, dim3(WG_GRID), dim3(256), 0, st, nv, Hh[l - 1].p, Mm[l].p,
+                           dZ.p, wpart.p);
+        finish(WG_OUT, o);
         // dH_{l-1} = dZ Ws^T + A~^T (dZ Wn^T)
-        hipLaunchKernelGGL((k_dense_t<H>), dim3(g), dim3(256), 0, st, nv, dZ.p, P + o + H * H,
-                           dTmp.p, 0);
-        hipLaunchKernelGGL((k_dense_t<H>), dim3(g), dim3(256), 0, st, nv, dZ.p, P + o, dH.p, 0);
         hipLaunchKernelGGL(k_aggregate<float>, dim3((nv + 15) / 16), dim3(256), 0, st, tsv, tval.p,
                            (const float*)dTmp.p, dH.p, 1);
     }
-    hipLaunchKernelGGL(k_relu_back, dim3(blocks(nh)), dim3(256), 0, st, nh, dH.p, Z[0].p, dZ.p);
-    hipLaunchKernelGGL((k_wgrad_partial<F, H, true>), dim3(WG_GRID), dim3(256), 0, st, nv, X.p,
-                       dZ.p, wpart.p);
-    hipLaunchKernelGGL(k_wgrad_finish, dim3(blocks((F + 1) * H)), dim3(256), 0, st, WG_GRID,
-                       (F + 1) * H, H, F, wpart.p, grad.p, GNN_W0, GNN_B0);
+    hipLaunchKernelGGL(k_wgrad_in, dim3(WG_GRID), dim3(256), 0, st, nv, X.p, dH.p, Z[0].p, wpart.p);
+    finish(WIN_OUT, GNN_W0);
     MP_HIP(hipGetLastError());
 }
 

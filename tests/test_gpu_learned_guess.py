@@ -99,6 +99,41 @@ def test_guess_forward_and_gradient_match_oracle(cube3d_small):
         assert rel_err(grad_gpu[a:bnd], grad_or[a:bnd]) <= 1e-3, (a, bnd)
 
 
+@pytest.mark.parametrize("n", [6, 7, 9, 12])
+def test_gradient_row_remainders_match_oracle(n):
+    """Small 2D clouds of 32 to 140 nodes: row counts off the kernels' tiles of
+    16 rows and steps of 4, and fewer rows than wavefronts.  One dropped or
+    doubled row moves a block of the gradient by at least 1 / sqrt(nodes), 8 %;
+    the bound allows one BF16 rounding boundary crossed by an aggregated state
+    (2^-8 on one of the sums)."""
+    import scipy.sparse as sp
+
+    import memphys_amd as M
+    import oracle as O
+    from oracle import gnn as G
+    c = M.box_cloud(dim=2, n=n, jitter=0.2, seed=n, k_interior=12)
+    with M.Context(0) as ctx:
+        w, u_dir, p_dir, _ = _fs(ctx, c)
+        rng = np.random.default_rng(n)
+        theta = (rng.standard_normal(G.NPARAM) * 0.1).astype(np.float32)
+        ctx.guess_params(theta)
+        m = ctx.n_sys
+        p1, p2, b, pt = (rng.standard_normal(m) for _ in range(4))
+        g_gpu, grad_gpu, loss_gpu = ctx.guess_eval(p1, p2, b, pt)
+    fs = O.FractionalStep(c, w, u_dir, u_dir, None, p_dir, 1.0, 0.0025, 5e-4, 2)
+    rp, ci, v = fs.ppe_csr()
+    A = sp.csr_matrix((v, ci, rp), shape=(m, m))
+    g_or, grad_or, loss_or = G.evaluate(theta, A, c.nv, p1, p2, b, c.xyz, pt)
+    _print("nv", c.nv, "guess", rel_err(g_gpu, g_or), "grad", rel_err(grad_gpu, grad_or))
+    assert rel_err(g_gpu, g_or) <= 5e-3
+    assert abs(loss_gpu - loss_or) <= 5e-3 * abs(loss_or)
+    for a, bnd in [(G.W0, G.B0), (G.B0, G.LAYER)] + \
+            [(G.LAYER + l * G.LAYER_SIZE + o, G.LAYER + l * G.LAYER_SIZE + e)
+             for l in range(G.L) for o, e in ((0, 4096), (4096, 8192), (8192, G.LAYER_SIZE))] + \
+            [(G.WO, G.BO), (G.BO, G.NPARAM)]:
+        assert rel_err(grad_gpu[a:bnd], grad_or[a:bnd]) <= 5e-3, (a, bnd)
+
+
 def test_trained_guess_saves_iterations():
     """Train on episodes with random lid speeds, then run a fresh cavity with
     the previous-pressure guess (the reference's solveWithGuess(rhs, p_old)),
