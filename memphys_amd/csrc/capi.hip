@@ -1383,7 +1383,7 @@ int mp_guess_eval(mp_ctx* c, const double* p1, const double* p2, const double* b
         download(c, dg.p, h);
         from_device_order(c, h, guess);
         if (p_true) {
-            to_device_order(c, p_true, h, S);
+            to_device_order(c, p_true, h);  // (the loss sees the node rows only)
             upload(c, dt.p, h);
             c->net->backward(c->stream, dx.p, dt.p);
             double ls = c->net->loss_host(c->stream);
