@@ -27,12 +27,19 @@ struct AmgMat {
     DevBuf<uint16_t> val2_b; // a second value array in the same slots (composed restriction)
     DevBuf<uint16_t> col16_b;  // compressed columns of its own (T_0)
     DevBuf<int> cbase_b;
-    long slots = 0, nnz16 = 0; // T_0: slots, those of slices with 16-bit columns
+    DevBuf<int> uptr_b, ucol_b;  // distinct columns per row block of its own (T_0)
+    DevBuf<uint16_t> loc_b;
+    long slots = 0, nnz16 = 0, nuniq = 0;  // T_0: slots, those of slices with 16-bit
+                                           // columns, entries of ucol
     const int* ptr = nullptr;
     const int* col = nullptr;
     const uint16_t* val = nullptr;
     const uint16_t* col16 = nullptr;  // compressed columns of level 0 (the solver's)
     const int* cbase = nullptr;
+    const int* uptr = nullptr;  // distinct columns per row block (level 0; see Slots)
+    const int* ucol = nullptr;
+    const uint16_t* loc = nullptr;
+    int max_u = 0;
     const uint16_t* val2 = nullptr;
 };
 

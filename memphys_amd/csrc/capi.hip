@@ -53,6 +53,9 @@ struct mp_ctx {
     // 16-bit columns, window bases, and slot_perm[sorted slot] = stencil slot
     DevBuf<int> col_s, cbase_s, slot_perm;
     DevBuf<uint16_t> col16_s;
+    // distinct columns per row block and the slots' places (large clouds)
+    DevBuf<int> uptr, ucol;
+    DevBuf<uint16_t> loc, loc_s;
     int nb = 0;
     DevBuf<double> xyz, normal;
     DevBuf<uint8_t> bnd;
@@ -606,14 +609,28 @@ int upload_clouds(mp_ctx* c, const char* fn, int nprob, const int* nvp, int dim,
             });
         for (auto& t : pool) t.join();
     }
-    std::vector<uint16_t> hcol16;
-    std::vector<int> hcb;
-    compress_columns(hsptr, hcol_s, c->nslices, hcol16, hcb);
+    // large clouds: the distinct columns of each row block and the slots' places
+    // among them, in both slot orders; else 16-bit columns of the sorted order
+    std::vector<uint16_t> hcol16, hloc;
+    std::vector<int> hcb, huptr, hucol;
+    int max_u = 0;
+    if (rows / BLOCK <= SPLIT_MAX_BLOCKS ||
+        !stage_columns(hsptr, hcol, c->nslices, huptr, hucol, hloc, max_u))
+        compress_columns(hsptr, hcol_s, c->nslices, hcol16, hcb);
+    std::vector<uint16_t> hloc_s(hloc.size());
+    if (max_u > 0)
+        parallel_for(c->nslices, [&](int sl) {
+            for (int t = hsptr[sl]; t < hsptr[sl + 1]; ++t) hloc_s[t] = hloc[hperm[t]];
+        });
     c->col.alloc(hcol.size());
     c->col_s.alloc(hcol_s.size());
     c->slot_perm.alloc(hperm.size());
     c->col16_s.alloc(hcol16.size());
     c->cbase_s.alloc(hcb.size());
+    c->uptr.alloc(huptr.size());
+    c->ucol.alloc(hucol.size());
+    c->loc.alloc(hloc.size());
+    c->loc_s.alloc(hloc_s.size());
     c->len.alloc(hlen.size());
     c->brows.alloc(std::max<size_t>(1, hb.size()));
     c->xyz.alloc(hx.size());
@@ -626,9 +643,21 @@ int upload_clouds(mp_ctx* c, const char* fn, int nprob, const int* nvp, int dim,
                      hipMemcpyHostToDevice));
     MP_HIP(hipMemcpy(c->slot_perm.p, hperm.data(), sizeof(int) * hperm.size(),
                      hipMemcpyHostToDevice));
-    MP_HIP(hipMemcpy(c->col16_s.p, hcol16.data(), sizeof(uint16_t) * hcol16.size(),
-                     hipMemcpyHostToDevice));
-    MP_HIP(hipMemcpy(c->cbase_s.p, hcb.data(), sizeof(int) * hcb.size(), hipMemcpyHostToDevice));
+    if (max_u > 0) {
+        MP_HIP(hipMemcpy(c->uptr.p, huptr.data(), sizeof(int) * huptr.size(),
+                         hipMemcpyHostToDevice));
+        MP_HIP(hipMemcpy(c->ucol.p, hucol.data(), sizeof(int) * hucol.size(),
+                         hipMemcpyHostToDevice));
+        MP_HIP(hipMemcpy(c->loc.p, hloc.data(), sizeof(uint16_t) * hloc.size(),
+                         hipMemcpyHostToDevice));
+        MP_HIP(hipMemcpy(c->loc_s.p, hloc_s.data(), sizeof(uint16_t) * hloc_s.size(),
+                         hipMemcpyHostToDevice));
+    } else {
+        MP_HIP(hipMemcpy(c->col16_s.p, hcol16.data(), sizeof(uint16_t) * hcol16.size(),
+                         hipMemcpyHostToDevice));
+        MP_HIP(hipMemcpy(c->cbase_s.p, hcb.data(), sizeof(int) * hcb.size(),
+                         hipMemcpyHostToDevice));
+    }
     MP_HIP(hipMemcpy(c->len.p, hlen.data(), sizeof(int) * hlen.size(), hipMemcpyHostToDevice));
     if (!hb.empty())
         MP_HIP(hipMemcpy(c->brows.p, hb.data(), sizeof(int) * hb.size(), hipMemcpyHostToDevice));
@@ -640,10 +669,16 @@ int upload_clouds(mp_ctx* c, const char* fn, int nprob, const int* nvp, int dim,
     c->sv.nslices = c->nslices;
     c->sv.sptr = c->sptr.p;
     c->sv.col = c->col.p;
+    c->sv.uptr = max_u > 0 ? c->uptr.p : nullptr;
+    c->sv.ucol = max_u > 0 ? c->ucol.p : nullptr;
+    c->sv.loc = max_u > 0 ? c->loc.p : nullptr;
+    c->sv.max_u = max_u;
+    c->sv.nuniq = (long)hucol.size();
     c->svs = c->sv;
     c->svs.col = c->col_s.p;
-    c->svs.col16 = c->col16_s.p;
-    c->svs.cbase = c->cbase_s.p;
+    c->svs.loc = max_u > 0 ? c->loc_s.p : nullptr;
+    c->svs.col16 = max_u > 0 ? nullptr : c->col16_s.p;
+    c->svs.cbase = max_u > 0 ? nullptr : c->cbase_s.p;
     c->sv.len = c->len.p;
     for (auto& wb : c->w) {
         wb.alloc(c->total_slots);

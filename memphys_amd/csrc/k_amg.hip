@@ -64,10 +64,14 @@ struct MatView {
     const int* ptr;
     const int* col;
     const uint16_t* val;    // BF16
-    const uint16_t* col16;  // compressed columns (SELL-64x4 only; may be null)
-    const int* cbase;
+    Slots sl;               // SELL-64x4: the slots' columns
     const uint16_t* val2;   // second BF16 value array in the same slots (OP_RQ)
 };
+MatView mat_view(const AmgMat& M) {
+    return MatView{M.n, M.nslices, M.ptr, M.col, M.val,
+                   Slots{M.nslices, M.ptr, M.col, M.col16, M.cbase, M.uptr, M.ucol, M.loc, M.max_u},
+                   M.val2};
+}
 
 __device__ __forceinline__ float bf2f(uint16_t v) { return __uint_as_float((uint32_t)v << 16); }
 
@@ -105,7 +109,7 @@ __device__ __forceinline__ float gathered(int c, const TB* __restrict__ b, const
 //            CSR layouts only)
 //   OP_TPOST: out = D^-1 (b + base) + M xin (M = T_l, base = res_l)
 // Level 0 also copies the border unknown (border_in -> border_out).
-// WS: the block shape in the SELL layout (1 or 4).
+// WS: the block shape in the SELL layout (1, 2 or 4).
 template <int G, int OP, typename TB, typename TO, int WS = 1>
 __global__ __launch_bounds__(BLOCK) void k_amg_op(MatView m, const float* __restrict__ dinv,
                                                   const TB* __restrict__ b, const float* xin,
@@ -124,8 +128,7 @@ __global__ __launch_bounds__(BLOCK) void k_amg_op(MatView m, const float* __rest
         if (border_out && lb == 0 && threadIdx.x == 0) *border_out = *border_in;
         i = block_row<WS>(lb);
         acc = sell4_block<WS, 4, float>(
-            m.nslices, m.ptr, m.col, m.col16, m.cbase, m.val, lb,
-            [](uint16_t v) { return bf2f(v); },
+            m.sl, m.val, lb, [](uint16_t v) { return bf2f(v); },
             [=](int c) { return gathered<OP>(c, b, xin, dinv); });
         if (i >= m.n) return;
     } else {
@@ -235,8 +238,7 @@ __global__ __launch_bounds__(BLOCK) void k_amg_pres(MatView m, const TB* __restr
     if (stop) return;
     if (border_out && lb == 0 && threadIdx.x == 0) *border_out = *border_in;
     const float acc = sell4_block<WS, 4, float>(
-        m.nslices, m.ptr, m.col, m.col16, m.cbase, m.val, lb, [](uint16_t v) { return bf2f(v); },
-        [xin](int c) { return xin[c]; });
+        m.sl, m.val, lb, [](uint16_t v) { return bf2f(v); }, [xin](int c) { return xin[c]; });
     const int i = block_row<WS>(lb);
     if (i >= m.n) return;
     res[i] = (float)b[i] - acc;
@@ -337,7 +339,7 @@ template <int G, int OP, typename TB, typename TO>
 void launch_g(hipStream_t st, const AmgMat& M, const float* dinv, const TB* b, const float* xin,
               const float* base, float* xout, float* res, TO* out, const double* bin,
               double* bout, const int* done, float* out32) {
-    const MatView v{M.n, M.nslices, M.ptr, M.col, M.val, M.col16, M.cbase, M.val2};
+    const MatView v = mat_view(M);
     int nb;
     if constexpr (G == 0) {
         nb = nblk_rows(M.nslices);
@@ -345,6 +347,12 @@ void launch_g(hipStream_t st, const AmgMat& M, const float* dinv, const TB* b, c
             hipLaunchKernelGGL((k_amg_op<0, OP, TB, TO, 4>), dim3(grid_xcd(M.nslices)),
                                dim3(BLOCK), 0, st, v, dinv, b, xin, base, xout, res, out, bin,
                                bout, done, out32);
+            return;
+        }
+        if (M.max_u > 0) {
+            hipLaunchKernelGGL((k_amg_op<0, OP, TB, TO, 2>), dim3(grid_xcd(nb)), dim3(BLOCK),
+                               sizeof(float) * M.max_u, st, v, dinv, b, xin, base, xout, res, out,
+                               bin, bout, done, out32);
             return;
         }
     } else {
@@ -376,11 +384,14 @@ void launch_op(hipStream_t st, const AmgMat& M, const float* dinv, const TB* b, 
 template <typename TB>
 void launch_pres(hipStream_t st, const AmgMat& M, const TB* b, const float* xin, float* res,
                  const double* bin, double* bout, const int* done, const GmNorm& norm) {
-    const MatView v{M.n, M.nslices, M.ptr, M.col, M.val, M.col16, M.cbase, M.val2};
+    const MatView v = mat_view(M);
     const int nb = nblk_rows(M.nslices), nx = grid_xcd(norm.sg.nseg);
     if (nb <= SPLIT_MAX_BLOCKS)
         hipLaunchKernelGGL((k_amg_pres<TB, 4>), dim3(nx + grid_xcd(M.nslices)), dim3(BLOCK), 0, st,
                            v, b, xin, res, bin, bout, done, norm, nx);
+    else if (M.max_u > 0)
+        hipLaunchKernelGGL((k_amg_pres<TB, 2>), dim3(nx + grid_xcd(nb)), dim3(BLOCK),
+                           sizeof(float) * M.max_u, st, v, b, xin, res, bin, bout, done, norm, nx);
     else
         hipLaunchKernelGGL((k_amg_pres<TB, 1>), dim3(nx + grid_xcd(nb)), dim3(BLOCK), 0, st, v, b,
                            xin, res, bin, bout, done, norm, nx);
@@ -509,19 +520,36 @@ void upload_t0(AmgMat& d, const std::vector<mp_amg::Hierarchy>& hs,
             for (; j < w; ++j) col[base + sell_off(j)] = pad;
         }
     });
-    compress_columns(sptr, col, ns, c16, cb);
+    if (nblk_rows(ns) <= SPLIT_MAX_BLOCKS) {
+        compress_columns(sptr, col, ns, c16, cb);
+    } else {
+        std::vector<int> up, uc;
+        std::vector<uint16_t> loc;
+        if (stage_columns(sptr, col, ns, up, uc, loc, d.max_u)) {
+            d.nuniq = (long)uc.size();
+            put(d.uptr_b, up, st);
+            put(d.ucol_b, uc, st);
+            put(d.loc_b, loc, st);
+            MP_HIP(hipStreamSynchronize(st));
+            d.uptr = d.uptr_b.p;
+            d.ucol = d.ucol_b.p;
+            d.loc = d.loc_b.p;
+        }
+    }
     d.n = n;
     d.g = 0;
     d.nslices = ns;
     d.nnz16 = 0;
-    for (int s = 0; s < ns; ++s)
+    for (int s = 0; s < ns && !cb.empty(); ++s)
         if (cb[(size_t)s * CW_COUNT] >= 0) d.nnz16 += sptr[s + 1] - sptr[s];
     d.slots = sptr[ns];
     put(d.ptr_b, sptr, st);
     put(d.col_b, col, st);
     put(d.val_b, val, st);
-    put(d.col16_b, c16, st);
-    put(d.cbase_b, cb, st);
+    if (!cb.empty()) {
+        put(d.col16_b, c16, st);
+        put(d.cbase_b, cb, st);
+    }
     MP_HIP(hipStreamSynchronize(st));  // (the host arrays end here)
     d.ptr = d.ptr_b.p;
     d.col = d.col_b.p;
@@ -709,6 +737,42 @@ mp_amg::Csr minus_scaled(const mp_amg::Csr& X, const std::vector<float>* d, cons
 
 }  // namespace
 
+bool stage_columns(const std::vector<int>& sptr, const std::vector<int>& col, int nslices,
+                   std::vector<int>& uptr, std::vector<int>& ucol, std::vector<uint16_t>& loc,
+                   int& max_u) {
+    const int per = BLOCK / SLICE, nb = (nslices + per - 1) / per;
+    std::vector<std::vector<int>> u(nb);
+    auto range = [&](int b) {
+        return std::make_pair(sptr[b * per], sptr[std::min(nslices, (b + 1) * per)]);
+    };
+    parallel_for(nb, [&](int b) {
+        const auto r = range(b);
+        u[b].assign(col.begin() + r.first, col.begin() + r.second);
+        std::sort(u[b].begin(), u[b].end());
+        u[b].erase(std::unique(u[b].begin(), u[b].end()), u[b].end());
+        u[b].shrink_to_fit();
+    });
+    uptr.assign(nb + 1, 0);
+    max_u = 0;
+    for (int b = 0; b < nb; ++b) {
+        uptr[b + 1] = uptr[b] + (int)u[b].size();
+        max_u = std::max(max_u, (int)u[b].size());
+    }
+    if (max_u > STAGE_MAX) {
+        max_u = 0;
+        return false;
+    }
+    ucol.assign(uptr[nb], 0);
+    loc.assign(col.size(), 0);
+    parallel_for(nb, [&](int b) {
+        std::copy(u[b].begin(), u[b].end(), ucol.begin() + uptr[b]);
+        const auto r = range(b);
+        for (int t = r.first; t < r.second; ++t)
+            loc[t] = (uint16_t)(std::lower_bound(u[b].begin(), u[b].end(), col[t]) - u[b].begin());
+    });
+    return true;
+}
+
 void compress_columns(const std::vector<int>& sptr, const std::vector<int>& col, int nslices,
                       std::vector<uint16_t>& c16, std::vector<int>& cb) {
     // per slice, the sorted distinct columns are covered greedily by windows of
@@ -869,6 +933,10 @@ void AmgDevice::setup(hipStream_t st, const SellView& sv, const double* val64_de
             d.A.col = sv_apply.col;
             d.A.col16 = sv_apply.col16;
             d.A.cbase = sv_apply.cbase;
+            d.A.uptr = sv_apply.uptr;
+            d.A.ucol = sv_apply.ucol;
+            d.A.loc = sv_apply.loc;
+            d.A.max_u = sv_apply.max_u;
             // BF16 copy of the solver's FP32 slots (padding slots stay 0)
             d.A.val_b.alloc((size_t)slots);
             hipLaunchKernelGGL(k_to_bf16, dim3((unsigned)((slots + BLOCK - 1) / BLOCK)),

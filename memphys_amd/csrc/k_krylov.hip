@@ -67,6 +67,14 @@ __device__ void loop_top(KScalars* sc, double rr, double r0r) {
     sc->beta = (sc->rho / sc->rho_old) * (sc->alpha / sc->omega);
 }
 
+// The slots of an operator with values of type TM (FP64: 32-bit columns).
+template <typename TM>
+__device__ __forceinline__ Slots op_slots(const SellView& sv) {
+    Slots m = sv.slots();
+    if (sizeof(TM) == 8) m.col16 = nullptr;
+    return m;
+}
+
 // Rows of the SELL-64x4 product A x over logical block lb (row block_row<WS>(lb)
 // to its thread; see sell4_block).  Padding slots hold a zero value and a
 // valid column, which leaves the fma chains unchanged.
@@ -80,9 +88,9 @@ __device__ __forceinline__ T sell_dot(const SellView& sv, const TM* __restrict__
     // and the 16-bit columns of the view.  x may be an FP32 copy of a vector
     // whose values are FP32 numbers (the V-cycle's output): same sums.
     constexpr bool wide = sizeof(TM) == 8;
-    return sell4_block<WS, (wide ? 2 : 4), T>(
-        sv.nslices, sv.sptr, sv.col, wide ? nullptr : sv.col16, sv.cbase, a, lb,
-        [](TM v) { return (T)v; }, [x](int c) { return (T)x[c]; });
+    return sell4_block<WS, (wide ? 2 : 4), T>(op_slots<TM>(sv), a, lb,
+                                              [](TM v) { return (T)v; },
+                                              [x](int c) { return x[c]; });
 }
 
 // The same product with gathered entries made of several vectors' entries
@@ -90,9 +98,7 @@ __device__ __forceinline__ T sell_dot(const SellView& sv, const TM* __restrict__
 template <typename T, typename TM, typename PRE, typename MID, typename FIN>
 __device__ __forceinline__ T sell_dot_early(const SellView& sv, const TM* __restrict__ a, int lb,
                                             PRE pre, MID mid, FIN fin, bool& ok) {
-    return sell4_block_early<T>(sv.nslices, sv.sptr, sv.col,
-                                sizeof(TM) == 8 ? nullptr : sv.col16, sv.cbase, a, lb, pre, mid,
-                                fin, ok);
+    return sell4_block_early<T>(op_slots<TM>(sv), a, lb, pre, mid, fin, ok);
 }
 
 // The product's partial sums come per slice (shape 4).
@@ -854,13 +860,16 @@ __global__ __launch_bounds__(BLOCK) void k_diag_inverse(int n, const double* __r
 
 inline int nblk(int n) { return (n + BLOCK - 1) / BLOCK; }
 
-// f(block shape) for a product over nbk row blocks
+// f(block shape, dynamic LDS bytes) for a product over nbk row blocks of view sv
+// that gathers entries of xb bytes
 template <typename F>
-void with_split(int nbk, F&& f) {
+void with_shape(int nbk, const SellView& sv, size_t xb, F&& f) {
     if (nbk <= SPLIT_MAX_BLOCKS)
-        f(std::integral_constant<int, 4>{});
+        f(std::integral_constant<int, 4>{}, (size_t)0);
+    else if (sv.max_u > 0)
+        f(std::integral_constant<int, 2>{}, xb * sv.max_u);
     else
-        f(std::integral_constant<int, 1>{});
+        f(std::integral_constant<int, 1>{}, (size_t)0);
 }
 
 // ---- GMRES(m), right-preconditioned ----
@@ -1555,7 +1564,7 @@ void PpeSolver::setup(hipStream_t st, const SellView& view, const std::vector<Se
     for (int i = 0; i < nrows; ++i) nnz += hl[i];
     nnz16 = 0;
     nslices16 = 0;
-    if (svk.col16) {
+    if (svk.col16 && svk.cbase) {
         std::vector<int> cb((size_t)svk.nslices * CW_COUNT);
         MP_HIP(hipMemcpy(cb.data(), svk.cbase, sizeof(int) * cb.size(), hipMemcpyDeviceToHost));
         for (int sl = 0; sl < svk.nslices; ++sl)
@@ -1568,33 +1577,40 @@ void PpeSolver::setup(hipStream_t st, const SellView& view, const std::vector<Se
 }
 
 double PpeSolver::smooth_bytes() const {
-    // T_0's slots: BF16 value + column (2 B in slices with 16-bit columns, plus
-    // their window bases, else 4 B); per row: b, the residual and D^-1 read,
+    // T_0's slots: BF16 value + column (with staged entries a 2 B place, plus 4 B
+    // per distinct column of a row block; else 2 B in slices with 16-bit columns,
+    // plus their window bases, or 4 B); per row: b, the residual and D^-1 read,
     // the output written (GMRES: b is the FP32 basis vector and the output the
     // FP32 direction; BiCGSTAB: b FP64, the output in FP64 and FP32); the
     // level-1 vector gathered once
     if (!amg) return 0.0;
     const AmgMat& T = amg->lv[0].T;
-    const double n16 = (double)T.nnz16;
     const double per_row = krylov == 1 ? 4.0 + 4.0 + 4.0 + 4.0 : 8.0 + 4.0 + 4.0 + 8.0 + 4.0;
+    const double rest = (double)nv * per_row + 4.0 * (double)amg->lv[1].n;
+    if (T.max_u > 0) return (double)T.slots * 4.0 + 4.0 * (double)T.nuniq + rest;
+    const double n16 = (double)T.nnz16;
     return (double)T.slots * 2.0 + 2.0 * n16 + 4.0 * ((double)T.slots - n16) +
-           (double)T.nslices * 4.0 * CW_COUNT + (double)nv * per_row + 4.0 * (double)amg->lv[1].n;
+           (double)T.nslices * 4.0 * CW_COUNT + rest;
 }
 
 double PpeSolver::spmv_bytes(int fp32) const {
-    // per entry: value (8 B, or 4 B for the FP32 operator) + column (4 B; the
-    // FP32 operator: 2 B in slices with 16-bit columns, plus their window
+    // per entry: value (8 B, or 4 B for the FP32 operator) + column (with staged
+    // entries a 2 B place, plus 4 B per distinct column of a row block; else 4 B,
+    // the FP32 operator 2 B in slices with 16-bit columns, plus their window
     // bases); per row: gathered x once (FP32 with the V-cycle, else FP64),
     // the product written, r0 read (BiCGSTAB's fused dot; FP64), length,
     // D^-1 for the border row
     const double vb = fp32 ? 4.0 : 8.0;
-    const double n16 = fp32 ? (double)nnz16 : 0.0;
     // the V-cycle's output, and an FP32 GMRES basis vector, are gathered in FP32
     const double xb = (amg || (krylov == 1 && fp32)) ? 4.0 : 8.0;
     const double vec = (krylov == 1 ? 1.0 : 2.0) + (bordered ? 1.0 : 0.0);
+    const SellView& w = fp32 ? svk : sv;
+    const double rows = (double)nv * (xb + 8.0 * vec + 4.0);
+    if (nrows / BLOCK > SPLIT_MAX_BLOCKS && w.max_u > 0)  // (places and distinct columns)
+        return (double)nnz * (vb + 2.0) + 4.0 * (double)w.nuniq + rows;
+    const double n16 = fp32 ? (double)nnz16 : 0.0;
     return (double)nnz * vb + 2.0 * n16 + 4.0 * ((double)nnz - n16) +
-           (fp32 ? (double)nslices16 * 4.0 * CW_COUNT : 0.0) +
-           (double)nv * (xb + 8.0 * vec + 4.0);
+           (fp32 ? (double)nslices16 * 4.0 * CW_COUNT : 0.0) + rows;
 }
 
 // y = M^-1 p with the multigrid V-cycle; without it the direction itself.
@@ -1674,15 +1690,15 @@ void PpeSolver::launch_chunk(hipStream_t st, int chunk, const TM* a, const T* di
         // with the V-cycle, the products gather its FP32 output (the same values)
         const T* yin = precondition(st, pp, yv.p, y32.p);
         spmv_timer.begin(st);
-        with_split(nbk, [&](auto ws) {
+        with_shape(nbk, view_of<TM>(), amg ? 4 : sizeof(T), [&](auto ws, size_t shm) {
             constexpr int WS = decltype(ws)::value;
             if (amg)
                 hipLaunchKernelGGL((k_spmv_alpha<WS, TM, T, float>), dim3(grid_xcd(nrows / WS_ROWS<WS>)),
-                                   dim3(WS_THREADS<WS>), 0, st, view_of<TM>(), sg, a, di, yin,
+                                   dim3(WS_THREADS<WS>), shm, st, view_of<TM>(), sg, a, di, yin,
                                    (const float*)y32.p, vv, rr0, partial.p, sc.p);
             else
                 hipLaunchKernelGGL((k_spmv_alpha<WS, TM, T, T>), dim3(grid_xcd(nrows / WS_ROWS<WS>)),
-                                   dim3(WS_THREADS<WS>), 0, st, view_of<TM>(), sg, a, di, yin, yin, vv,
+                                   dim3(WS_THREADS<WS>), shm, st, view_of<TM>(), sg, a, di, yin, yin, vv,
                                    rr0, partial.p, sc.p);
         });
         spmv_timer.end(st);
@@ -1692,15 +1708,15 @@ void PpeSolver::launch_chunk(hipStream_t st, int chunk, const TM* a, const T* di
                            xs);
         const T* zin = precondition(st, ss, zv.p, z32.p);
         spmv_timer.begin(st);
-        with_split(nbk, [&](auto ws) {
+        with_shape(nbk, view_of<TM>(), amg ? 4 : sizeof(T), [&](auto ws, size_t shm) {
             constexpr int WS = decltype(ws)::value;
             if (amg)
                 hipLaunchKernelGGL((k_spmv_omega<WS, TM, T, float>), dim3(grid_xcd(nrows / WS_ROWS<WS>)),
-                                   dim3(WS_THREADS<WS>), 0, st, view_of<TM>(), sg, a, di, zin,
+                                   dim3(WS_THREADS<WS>), shm, st, view_of<TM>(), sg, a, di, zin,
                                    (const float*)z32.p, ss, tt, partial.p, sc.p);
             else
                 hipLaunchKernelGGL((k_spmv_omega<WS, TM, T, T>), dim3(grid_xcd(nrows / WS_ROWS<WS>)),
-                                   dim3(WS_THREADS<WS>), 0, st, view_of<TM>(), sg, a, di, zin, zin, ss,
+                                   dim3(WS_THREADS<WS>), shm, st, view_of<TM>(), sg, a, di, zin, zin, ss,
                                    tt, partial.p, sc.p);
         });
         spmv_timer.end(st);
@@ -1792,10 +1808,10 @@ void PpeSolver::run_bicgstab(hipStream_t st, const TM* a, const T* di, const T* 
     MP_HIP(hipMemcpyAsync(ctl_d.p, host_ctl, sizeof(SegCtl) * nseg, hipMemcpyHostToDevice, st));
     hipLaunchKernelGGL(k_sc_reset, dim3((nseg + 63) / 64), dim3(64), 0, st, nseg, sc.p, ctl_d.p);
     auto residual_init = [&](int mode) {
-        with_split(nbk, [&](auto ws) {
+        with_shape(nbk, view_of<TM>(), sizeof(T), [&](auto ws, size_t shm) {
             constexpr int WS = decltype(ws)::value;
             hipLaunchKernelGGL((k_residual_init<WS, TM, T>), dim3(grid_xcd(nrows / WS_ROWS<WS>)), dim3(WS_THREADS<WS>),
-                               0, st, view_of<TM>(), sg, a, di, rhs, x, rr, rr0, pp, vv, partial.p,
+                               shm, st, view_of<TM>(), sg, a, di, rhs, x, rr, rr0, pp, vv, partial.p,
                                sc.p, mode);
         });
     };
@@ -1852,9 +1868,9 @@ void PpeSolver::run_bicgstab(hipStream_t st, const TM* a, const T* di, const T* 
 // b - A x~ (FP64) of xt into tmp, its norm and b's into the scalars.
 void PpeSolver::launch_residual64(hipStream_t st, const double* b_dev) {
     const int nbk = nrows / BLOCK;
-    with_split(nbk, [&](auto ws) {
+    with_shape(nbk, sv, sizeof(double), [&](auto ws, size_t shm) {
         constexpr int WS = decltype(ws)::value;
-        hipLaunchKernelGGL(k_residual64<WS>, dim3(grid_xcd(nrows / WS_ROWS<WS>)), dim3(WS_THREADS<WS>), 0, st, sv, sg,
+        hipLaunchKernelGGL(k_residual64<WS>, dim3(grid_xcd(nrows / WS_ROWS<WS>)), dim3(WS_THREADS<WS>), shm, st, sv, sg,
                            aval.p, dinv.p, b_dev, xt.p, tmp.p, partial.p);
     });
     hipLaunchKernelGGL(k_finish_res64, dim3(nseg), dim3(FIN), 0, st, sg, b_dev, tmp.p, partial.p,
@@ -1933,9 +1949,12 @@ void PpeSolver::gmres_iteration(hipStream_t st, int k, int m, const TM* a, const
                                0, st, view_of<TM>(), sg, a, di, (const TV*)vk, zg, gm_w.p,
                                (const TV*)V, ld, k + 1, gm_partial.p, gm_d.p);
         else
-            hipLaunchKernelGGL((k_gm_spmv<1, TM, TX, TV>), dim3(grid_xcd(nbk)), dim3(BLOCK), 0, st,
-                               view_of<TM>(), sg, a, di, (const TV*)vk, zg, gm_w.p, (const TV*)V,
-                               ld, k + 1, gm_partial.p, gm_d.p);
+            with_shape(nbk, view_of<TM>(), sizeof(TX), [&](auto ws, size_t shm) {
+                constexpr int WS = decltype(ws)::value == 4 ? 1 : decltype(ws)::value;
+                hipLaunchKernelGGL((k_gm_spmv<WS, TM, TX, TV>), dim3(grid_xcd(nbk)), dim3(BLOCK),
+                                   shm, st, view_of<TM>(), sg, a, di, (const TV*)vk, zg, gm_w.p,
+                                   (const TV*)V, ld, k + 1, gm_partial.p, gm_d.p);
+            });
         spmv_timer.end(st);
     };
     if (amg) {
@@ -1988,10 +2007,10 @@ void PpeSolver::run_gmres(hipStream_t st, const TM* a, const double* di, const d
     // V'_0 = rhs - A x, sig[0] = 1 / |rhs - A x| for the systems taking part
     // (mode 0), or for those whose full cycle restarts (mode 1)
     auto start = [&](int mode) {
-        with_split(nbk, [&](auto ws) {
+        with_shape(nbk, view_of<TM>(), sizeof(double), [&](auto ws, size_t shm) {
             constexpr int WS = decltype(ws)::value;
             hipLaunchKernelGGL((k_gm_residual<WS, TM, TV>), dim3(grid_xcd(nrows / WS_ROWS<WS>)), dim3(WS_THREADS<WS>),
-                               0, st, view_of<TM>(), sg, a, di, rhs, x, V, d0, xs, gm_partial.p,
+                               shm, st, view_of<TM>(), sg, a, di, rhs, x, V, d0, xs, gm_partial.p,
                                gm_d.p, mode, (mode == 0 && x_zero) ? 1 : 0);
         });
         hipLaunchKernelGGL(k_gm_residual_finish<TV>, dim3(nseg), dim3(FIN), 0, st, sg, rhs, V,

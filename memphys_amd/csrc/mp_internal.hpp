@@ -253,11 +253,37 @@ __device__ __forceinline__ T sell4_accumulate(const SellHead& h, const int* __re
         [](c4 c) { return c; }, fv, fx);
 }
 
-// The three shapes of a product's blocks (WS):
+// Where a SELL-64x4 matrix keeps its slots' columns: 32-bit, compressed to 16
+// bits where a slice allows (col16, cbase; may be null), and, for large
+// matrices, per block of BLOCK rows: uptr[b] .. uptr[b+1]-1 index the block's
+// distinct columns ucol (ascending), loc holds each slot's place among them,
+// max_u their largest number (0: not built).
+struct Slots {
+    int nslices = 0;
+    const int* sptr = nullptr;
+    const int* col = nullptr;
+    const uint16_t* col16 = nullptr;
+    const int* cbase = nullptr;
+    const int* uptr = nullptr;
+    const int* ucol = nullptr;
+    const uint16_t* loc = nullptr;
+    int max_u = 0;
+};
+
+// The shapes of a product's blocks (WS):
 //   1   BLOCK threads over BLOCK rows: a wavefront per slice, four chains each;
+//   2   as 1, with the block's distinct gathered entries staged in LDS first
+//       (dynamic LDS: max_u of them);
 //   4   BLOCK threads over one slice: a wavefront per chain;
 //   16  4 * BLOCK threads over BLOCK rows: a wavefront per chain.
-// The wide shapes are for systems whose slices leave SIMDs idle: the row's
+// Shape 2 is for large systems: a CU serves a gather of 64 entries from L2 in
+// about 50 cycles, and a row block of a compact cluster reads each of its
+// distinct columns (4-6 per row of 42) about nine times; gathered once, in
+// ascending order, and read back from LDS, the product streams its matrix.
+// One against staged: 1M-node cube, GMRES product 66.8 and 53.1 us (5.3 TB/s),
+// level-0 residual 58.9 and 42.5, T_0 35 and 24, FP64 residual 126 and 92; 64 2D
+// cavities of 665k nodes 31.5, 26.6, 15.5, 58 and 26.5, 21.3, 12.8, 47 us.
+// The wide shapes (4, 16) are for systems whose slices leave SIMDs idle: the row's
 // serial chain of loads is a quarter as long, and (4) the gathers, which a CU
 // serves one wavefront at a time, spread over four times the CUs.
 template <int WS>
@@ -311,17 +337,41 @@ __device__ __forceinline__ T add_chains(T acc, int part) {
 // The row sums of one block (logical block lb): row block_row<WS>(lb) to its
 // thread (zero past nslices); every thread must call.
 template <int WS, int U4, typename T, typename TM, typename FV, typename FX>
-__device__ __forceinline__ T sell4_block(int nslices, const int* __restrict__ sptr,
-                                         const int* __restrict__ col,
-                                         const uint16_t* __restrict__ col16,
-                                         const int* __restrict__ cbase,
-                                         const TM* __restrict__ a, int lb, FV fv, FX fx) {
-    const SellHead h = sell4_head(nslices, sptr, col16, cbase, ws_slice<WS>(lb));
-    const int part = ws_part<WS>();
-    T acc = sell4_accumulate<(WS == 1 ? 1 : 4), U4, T>(h, col, col16, a,
-                                                       (int)(threadIdx.x & 63), part, fv, fx);
-    if constexpr (WS != 1) acc = add_chains<WS>(acc, part);
-    return acc;
+__device__ __forceinline__ T sell4_block(const Slots& m, const TM* __restrict__ a, int lb, FV fv,
+                                         FX fx) {
+    const int lane = (int)(threadIdx.x & 63);
+    if constexpr (WS == 2) {
+        typedef decltype(fx(0)) TX;
+        typedef typename Vec4<uint16_t>::type e4;
+        typedef typename Vec4<int>::type c4;
+        extern __shared__ __align__(16) char stage_lds[];
+        TX* xs = reinterpret_cast<TX*>(stage_lds);
+        const int s = ws_slice<1>(lb);
+        const int b0 = s < m.nslices ? m.sptr[s] : 0;
+        const int w4 = s < m.nslices ? (m.sptr[s + 1] - b0) >> 8 : 0;
+        const int u0 = m.uptr[lb], nu = m.uptr[lb + 1] - u0;
+        for (int t = (int)threadIdx.x; t < nu; t += 4 * BLOCK) {
+            int c[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (t + q * BLOCK < nu) c[q] = m.ucol[u0 + t + q * BLOCK];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (t + q * BLOCK < nu) xs[t + q * BLOCK] = fx(c[q]);
+        }
+        __syncthreads();
+        const e4* ep = reinterpret_cast<const e4*>(m.loc + b0) + lane;
+        return sell4_loop<1, U4, T>(
+            b0, w4, lane, 0, a, [&](int g) { return load_stream<true>(ep + g * SLICE); },
+            [](e4 e) { return c4{e.x, e.y, e.z, e.w}; }, fv, [xs](int i) { return (T)xs[i]; });
+    } else {
+        const SellHead h = sell4_head(m.nslices, m.sptr, m.col16, m.cbase, ws_slice<WS>(lb));
+        const int part = ws_part<WS>();
+        T acc = sell4_accumulate<(WS == 1 ? 1 : 4), U4, T>(
+            h, m.col, m.col16, a, lane, part, fv, [&](int c) { return (T)fx(c); });
+        if constexpr (WS != 1) acc = add_chains<WS>(acc, part);
+        return acc;
+    }
 }
 
 // sell4_block<4> for gathered entries fin(raw), raw = pre(column) loaded from
@@ -330,29 +380,25 @@ __device__ __forceinline__ T sell4_block(int nslices, const int* __restrict__ sp
 // whether to go on (the same on every thread), so mid's latency and theirs
 // overlap.  ok receives mid's answer.
 template <typename T, typename TM, typename PRE, typename MID, typename FIN>
-__device__ __forceinline__ T sell4_block_early(int nslices, const int* __restrict__ sptr,
-                                               const int* __restrict__ col,
-                                               const uint16_t* __restrict__ col16,
-                                               const int* __restrict__ cbase,
-                                               const TM* __restrict__ a, int lb, PRE pre, MID mid,
-                                               FIN fin, bool& ok) {
+__device__ __forceinline__ T sell4_block_early(const Slots& m, const TM* __restrict__ a, int lb,
+                                               PRE pre, MID mid, FIN fin, bool& ok) {
     typedef typename Vec4<TM>::type v4;
     typedef typename Vec4<int>::type c4;
     typedef typename Vec4<uint16_t>::type e4;
     typedef decltype(pre(0)) raw;
-    const SellHead h = sell4_head(nslices, sptr, col16, cbase, ws_slice<4>(lb));
+    const SellHead h = sell4_head(m.nslices, m.sptr, m.col16, m.cbase, ws_slice<4>(lb));
     const int lane = (int)(threadIdx.x & 63), part = ws_part<4>();
     const v4* ap = reinterpret_cast<const v4*>(a + h.b0) + lane;
     auto columns = [&](int g) {
         c4 c;
         if (h.base[0] >= 0) {
-            const e4 e = (reinterpret_cast<const e4*>(col16 + h.b0) + lane)[g * SLICE];
+            const e4 e = (reinterpret_cast<const e4*>(m.col16 + h.b0) + lane)[g * SLICE];
             c.x = col_decode(e.x, h.base);
             c.y = col_decode(e.y, h.base);
             c.z = col_decode(e.z, h.base);
             c.w = col_decode(e.w, h.base);
         } else {
-            c = (reinterpret_cast<const c4*>(col + h.b0) + lane)[g * SLICE];
+            c = (reinterpret_cast<const c4*>(m.col + h.b0) + lane)[g * SLICE];
         }
         return c;
     };
@@ -394,10 +440,12 @@ __device__ __forceinline__ T sell4_block_early(int nslices, const int* __restric
 }
 
 // Blocks of BLOCK rows up to which a product runs with a wavefront per chain.
-// 1024 blocks are 4 wavefronts per SIMD with one per slice.  Shapes 1, 16 and
-// 4: level-0 residual of a 64k-node cube (249 blocks) 11.7, 9.3 and 6.9 us, FP64
-// product of a 110k-node cube (414 blocks) 18.2, 16.0 and 13.6 us.
-constexpr int SPLIT_MAX_BLOCKS = 1024;
+// Shapes 1, 16 and 4: level-0 residual of a 64k-node cube (249 blocks) 11.7, 9.3
+// and 6.9 us, FP64 product of a 110k-node cube (414 blocks) 18.2, 16.0 and 13.6.
+// Steps with a wavefront per chain against staged entries: 110k nodes (mixed
+// multigrid) 28.1 and 29.3 ms, FP64 solve 4.55 and 4.93; 216k nodes (843 blocks)
+// 41.2 and 40.0, FP64 multigrid 19.2 and 19.1: the line lies between.
+constexpr int SPLIT_MAX_BLOCKS = 640;
 
 // SELL-64x4 view of the stencil set in device order.
 struct SellView {
@@ -408,12 +456,26 @@ struct SellView {
     const int* len;    // [nslices*64] row lengths (0 on ghost rows)
     const uint16_t* col16 = nullptr;  // [slots] compressed column ids (or null)
     const int* cbase = nullptr;       // [nslices*CW_COUNT] window bases
+    const int* uptr = nullptr;        // distinct columns per row block (see Slots; or null)
+    const int* ucol = nullptr;
+    const uint16_t* loc = nullptr;
+    int max_u = 0;
+    long nuniq = 0;  // entries of ucol
+    __host__ __device__ Slots slots() const { return Slots{nslices, sptr, col, col16, cbase, uptr, ucol, loc, max_u}; }
 };
 
 // Host: the compressed columns of slots sptr/col (see CW_BITS above): c16 per
 // slot, cb CW_COUNT window bases per slice (-1: the slice keeps 32-bit columns).
 void compress_columns(const std::vector<int>& sptr, const std::vector<int>& col, int nslices,
                       std::vector<uint16_t>& c16, std::vector<int>& cb);
+
+// Host: the distinct columns of every block of BLOCK rows and each slot's place
+// among them (see Slots); false when a block has more than STAGE_MAX, which the
+// LDS form is not for.
+constexpr int STAGE_MAX = 6144;
+bool stage_columns(const std::vector<int>& sptr, const std::vector<int>& col, int nslices,
+                   std::vector<int>& uptr, std::vector<int>& ucol, std::vector<uint16_t>& loc,
+                   int& max_u);
 
 // Host: f(i) for i in [0, n) on up to 16 threads, contiguous ranges.
 template <typename F>

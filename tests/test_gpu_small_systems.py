@@ -31,14 +31,14 @@ def _run(ctx, cloud, krylov, precision, steps=2):
 @pytest.mark.parametrize("precision", [0, 1])
 def test_small_cavity_in_large_batch_is_bit_identical(krylov, precision):
     """Cavities of 1, 3, 96, 97 and 128 row blocks alone (three- and five-launch
-    BiCGSTAB, both GMRES updates) and in one batch of more than 1024 blocks
+    BiCGSTAB, both GMRES updates) and in one batch of more than 640 blocks
     (the general kernels)."""
     import memphys_amd as M
     sizes = [15, 27, 156, 157, 181, 460]
     clouds = [M.box_cloud(dim=2, n=n, jitter=0.25, seed=n, k_interior=30) for n in sizes]
     rows = [-(-(c.nv + 1) // 256) for c in clouds]
     _print("row blocks", rows)
-    assert rows[:5] == [1, 3, 96, 97, 128] and sum(rows) > 1024
+    assert rows[:5] == [1, 3, 96, 97, 128] and sum(rows) > 640
     with M.Context(0) as ctx:
         cat = ctx.upload_batch(clouds)
         batch = _run(ctx, cat, krylov, precision)
@@ -85,3 +85,41 @@ def test_small_system_solves_its_operator(n, k):
             _print("n", n, "k", k, "prec", prec, "iterations", ctx.stats().iterations, "res", res)
             # the solver's own FP64 test, plus the rounding of A x on this host
             assert res <= 1.1e-10
+
+
+@pytest.mark.parametrize("spread", [40, 10 ** 9])
+@pytest.mark.parametrize("prec", [0, 1])
+def test_large_system_with_local_and_scattered_columns(spread, prec):
+    """170k rows (above the small systems' sizes) whose columns lie near their
+    row (each row block's distinct entries staged in LDS) or anywhere (more
+    distinct entries than are staged: gathered directly), with rows of 3 to 35
+    entries and a block of padding rows."""
+    import memphys_amd as M
+    import scipy.sparse as sp
+    rng = np.random.default_rng(8)
+    nv = 170_011
+    x = np.sort(rng.random(nv))
+    length = rng.integers(3, 36, nv)
+    length[:4096] = 35
+    rp = np.concatenate([[0], np.cumsum(length)]).astype(np.int32)
+    row = np.repeat(np.arange(nv), length)
+    off = rng.integers(1, min(spread, nv // 2), rp[-1]) * rng.choice([-1, 1], rp[-1])
+    col = ((row + off) % nv).astype(np.int32)
+    col[rp[:-1]] = np.arange(nv)
+    cloud = M.Cloud(dim=2, xyz=np.c_[x, np.zeros(nv)], boundary=np.zeros(nv, np.uint8),
+                    normal=np.zeros((nv, 2)), row_ptr=rp, col=col, ksize=length.astype(np.int32),
+                    layer=np.zeros(nv, np.int32))
+    lap = 0.4 * rng.uniform(-1, 1, rp[-1]) / length[row]
+    with M.Context(0) as ctx:
+        ctx.upload(cloud)
+        ctx.set_weights(lap, lap, None, lap)
+        n = ctx.solver_init(np.zeros(nv, np.uint8), 1.0, 0.0, 1.0, tol=1e-11, n_iter=500,
+                            precision=prec)
+        assert n == nv + 1
+        A = sp.csr_matrix((lap, col, rp), shape=(nv, nv)) + sp.identity(nv)
+        b = rng.standard_normal(n)
+        sol, _ = ctx.solve(b, np.zeros(n))
+        r = np.r_[A @ sol[:nv] + sol[nv], sol[:nv].sum()] - b
+        res = np.linalg.norm(r) / np.linalg.norm(b)
+        _print("spread", spread, "prec", prec, "iterations", ctx.stats().iterations, "res", res)
+        assert res <= 1.1e-11  # the solver's FP64 test, plus this host's rounding
