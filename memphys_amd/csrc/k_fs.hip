@@ -47,6 +47,87 @@ __device__ __forceinline__ d4 packed_at(const double* __restrict__ a, int c) {
     }
 }
 
+// Row kernels over staged entries: large clouds whose row blocks' distinct
+// columns are listed (see Slots), when DIM vectors of them fit 64 KB of LDS; the
+// gathers of one entry per weight otherwise bound these kernels.  1M-node cube,
+// gathered and staged: predictor 460 (plus 15 for the interleaved copy it
+// gathers from) and 323 us, right-hand side 296 and 198, corrector 275 and 241.
+template <int DIM>
+bool staged_steps(const SellView& sv) {
+    return sv.max_u > 0 && DIM * sv.max_u <= 8192;
+}
+
+// The row block's distinct columns' entries of NF vectors into LDS: vector f's
+// entry of place i at xs[f * max_u + i].  Ends with a barrier.
+template <int NF>
+__device__ __forceinline__ const double* stage_fields(const SellView& sv, int lb,
+                                                      const double* const (&x)[3]) {
+    extern __shared__ __align__(16) char stage_lds[];
+    double* xs = reinterpret_cast<double*>(stage_lds);
+    const int u0 = sv.uptr[lb], nu = sv.uptr[lb + 1] - u0;
+    for (int t = (int)threadIdx.x; t < nu; t += 2 * BLOCK) {
+        const bool two = t + BLOCK < nu;
+        const int c0 = sv.ucol[u0 + t], c1 = two ? sv.ucol[u0 + t + BLOCK] : c0;
+        double a[NF], b[NF];
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+            a[f] = x[f][c0];
+            b[f] = x[f][c1];
+        }
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+            xs[f * sv.max_u + t] = a[f];
+            if (two) xs[f * sv.max_u + t + BLOCK] = b[f];
+        }
+    }
+    __syncthreads();
+    return xs;
+}
+typedef uint16_t us4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ us4 places4(const SellView& sv, int s4) {
+    return *reinterpret_cast<const us4*>(sv.loc + s4);
+}
+
+// Gradient sums of a row over staged entries, in stencil order: acc[f][o] = sum
+// of operator o's weights (W[0..NO-1]) times vector f.  DIAG: operator f with
+// vector f alone (a divergence), into acc[f][0].  The next group's weights are
+// loaded while the current one is added.
+template <int NF, int NO, bool DIAG>
+__device__ __forceinline__ void staged_row(const SellView& sv, int base, int len,
+                                           const double* const (&W)[4], const double* xs,
+                                           double (&acc)[NF][DIAG ? 1 : NO]) {
+    d4 A[NO], B[NO];
+    us4 l, ln;
+    auto load = [&](int j0, d4 (&v)[NO], us4& p) {
+        const int s4 = base + (j0 << 6);
+        p = places4(sv, s4);
+#pragma unroll
+        for (int o = 0; o < NO; ++o) v[o] = vals4(W[o], s4);
+    };
+    auto add = [&](int j0, const d4 (&v)[NO], us4 p) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (j0 + e >= len) continue;
+#pragma unroll
+            for (int f = 0; f < NF; ++f) {
+                const double x = xs[f * sv.max_u + p[e]];
+                if constexpr (DIAG)
+                    acc[f][0] = fma(v[f][e], x, acc[f][0]);
+                else
+#pragma unroll
+                    for (int o = 0; o < NO; ++o) acc[f][o] = fma(v[o][e], x, acc[f][o]);
+            }
+        }
+    };
+    if (len > 0) load(0, A, l);
+    for (int j0 = 0; j0 < len; j0 += 8) {
+        if (j0 + 4 < len) load(j0 + 4, B, ln);
+        add(j0, A, l);
+        if (j0 + 8 < len) load(j0 + 8, A, l);
+        if (j0 + 4 < len) add(j0 + 4, B, ln);
+    }
+}
+
 template <int DIM>
 __global__ __launch_bounds__(BLOCK) void pack_kernel(int n, const double* __restrict__ u,
                                                      const double* __restrict__ v,
@@ -60,10 +141,12 @@ __global__ __launch_bounds__(BLOCK) void pack_kernel(int n, const double* __rest
         *reinterpret_cast<d2*>(out + 2 * (size_t)r) = d2{u[r], v[r]};
 }
 
-template <int DIM>
+// STAGED: gathers u, v, w through LDS (upk and uhpk unused).
+template <int DIM, bool STAGED>
 __global__ __launch_bounds__(BLOCK) void predictor_kernel(
     SellView sv, const double* __restrict__ gx, const double* __restrict__ gy,
     const double* __restrict__ gz, const double* __restrict__ lap,
+    const double* __restrict__ u, const double* __restrict__ v, const double* __restrict__ w,
     const double* __restrict__ upk, double* __restrict__ uh, double* __restrict__ vh,
     double* __restrict__ wh, double* __restrict__ uhpk, double* __restrict__ S_new,
     const double* __restrict__ S_oo, int npad, double rho_all, double mu_all, double dt_all,
@@ -74,6 +157,8 @@ __global__ __launch_bounds__(BLOCK) void predictor_kernel(
     const int lb = xcd_block((sv.nv + BLOCK - 1) / BLOCK);
     if (lb < 0) return;
     const int r = lb * BLOCK + threadIdx.x;
+    const double* xs = nullptr;
+    if constexpr (STAGED) xs = stage_fields<DIM>(sv, lb, {u, v, w});
     if (r >= sv.nv) return;
     double rho = rho_all, mu = mu_all, dt = dt_all;
     if (bprob) {  // batch: parameters of this block's problem
@@ -89,30 +174,47 @@ __global__ __launch_bounds__(BLOCK) void predictor_kernel(
     for (int f = 0; f < DIM; ++f)
 #pragma unroll
         for (int o = 0; o < 4; ++o) acc[f][o] = 0.0;
-    for (int j0 = 0; j0 < len; j0 += 4) {
-        const int s4 = base + (j0 << 6);
-        const i4 c4 = cols4(sv, s4);
-        const d4 A0 = vals4(gx, s4), A1 = vals4(gy, s4), A3 = vals4(lap, s4);
-        const d4 A2 = (DIM == 3) ? vals4(gz, s4) : d4{0.0, 0.0, 0.0, 0.0};
-        // the four gathers are issued together (slots past the row's length
-        // read the row's own node, and their terms are skipped)
-        d4 fg[4];
+    if constexpr (STAGED) {
+        // (2D: the Laplacian takes the third place, copied to the fourth below)
+        double sum[DIM][DIM + 1] = {};
+        const double* const W[4] = {gx, gy, DIM == 3 ? gz : lap, lap};
+        staged_row<DIM, DIM + 1, false>(sv, base, len, W, xs, sum);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) fg[e] = packed_at<DIM>(upk, j0 + e < len ? c4[e] : r);
+        for (int f = 0; f < DIM; ++f) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            if (j0 + e >= len) continue;
-            const d4 f = fg[e];
+            for (int o = 0; o < DIM; ++o) acc[f][o] = sum[f][o];
+            acc[f][3] = sum[f][DIM];
+        }
+    } else {
+        for (int j0 = 0; j0 < len; j0 += 4) {
+            const int s4 = base + (j0 << 6);
+            const i4 c4 = cols4(sv, s4);
+            const d4 A0 = vals4(gx, s4), A1 = vals4(gy, s4), A3 = vals4(lap, s4);
+            const d4 A2 = (DIM == 3) ? vals4(gz, s4) : d4{0.0, 0.0, 0.0, 0.0};
+            // the four gathers are issued together (slots past the row's length
+            // read the row's own node, and their terms are skipped)
+            d4 fg[4];
 #pragma unroll
-            for (int q = 0; q < DIM; ++q) {
-                acc[q][0] = fma(A0[e], f[q], acc[q][0]);
-                acc[q][1] = fma(A1[e], f[q], acc[q][1]);
-                if (DIM == 3) acc[q][2] = fma(A2[e], f[q], acc[q][2]);
-                acc[q][3] = fma(A3[e], f[q], acc[q][3]);
+            for (int e = 0; e < 4; ++e) fg[e] = packed_at<DIM>(upk, j0 + e < len ? c4[e] : r);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (j0 + e >= len) continue;
+                const d4 f = fg[e];
+#pragma unroll
+                for (int q = 0; q < DIM; ++q) {
+                    acc[q][0] = fma(A0[e], f[q], acc[q][0]);
+                    acc[q][1] = fma(A1[e], f[q], acc[q][1]);
+                    if (DIM == 3) acc[q][2] = fma(A2[e], f[q], acc[q][2]);
+                    acc[q][3] = fma(A3[e], f[q], acc[q][3]);
+                }
             }
         }
     }
-    const d4 own = packed_at<DIM>(upk, r);
+    d4 own;
+    if constexpr (STAGED)
+        own = d4{u[r], v[r], DIM == 3 ? w[r] : 0.0, 0.0};
+    else
+        own = packed_at<DIM>(upk, r);
     double* out[3] = {uh, vh, wh};
     d4 hat = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
@@ -132,13 +234,14 @@ __global__ __launch_bounds__(BLOCK) void predictor_kernel(
         out[q][r] = res;
         hat[q] = res;
     }
+    if constexpr (STAGED) return;  // (nobody gathers the interleaved copy)
     if constexpr (DIM == 3)
         *reinterpret_cast<d4*>(uhpk + 4 * (size_t)r) = hat;
     else
         *reinterpret_cast<d2*>(uhpk + 2 * (size_t)r) = d2{hat[0], hat[1]};
 }
 
-template <int DIM>
+template <int DIM, bool STAGED>
 __global__ __launch_bounds__(BLOCK) void ppe_rhs_kernel(
     SellView sv, const double* __restrict__ gx, const double* __restrict__ gy,
     const double* __restrict__ gz, const double* __restrict__ uh, const double* __restrict__ vh,
@@ -152,6 +255,8 @@ __global__ __launch_bounds__(BLOCK) void ppe_rhs_kernel(
     const int lb = xcd_block((sv.nv + BLOCK - 1) / BLOCK);
     if (lb < 0) return;
     const int r = lb * BLOCK + threadIdx.x;
+    const double* xs = nullptr;
+    if constexpr (STAGED) xs = stage_fields<DIM>(sv, lb, {uh, vh, wh});
     if (r >= sv.nv) return;  // rows without a stencil (border unknowns, padding) get b = 0
     double rho = rho_all, dt = dt_all;
     if (bprob) {
@@ -172,21 +277,30 @@ __global__ __launch_bounds__(BLOCK) void ppe_rhs_kernel(
         const int base = row_base(sv, r);
         const int len = sv.len[r];
         double ax = 0.0, ay = 0.0, az = 0.0;
-        for (int j0 = 0; j0 < len; j0 += 4) {
-            const int s4 = base + (j0 << 6);
-            const i4 c4 = cols4(sv, s4);
-            const d4 X = vals4(gx, s4), Y = vals4(gy, s4);
-            const d4 Z = (DIM == 3) ? vals4(gz, s4) : d4{0.0, 0.0, 0.0, 0.0};
-            d4 fg[4];
+        if constexpr (STAGED) {
+            double sum[DIM][1] = {};
+            const double* const W[4] = {gx, gy, gz, nullptr};
+            staged_row<DIM, DIM, true>(sv, base, len, W, xs, sum);
+            ax = sum[0][0];
+            ay = sum[1][0];
+            if constexpr (DIM == 3) az = sum[2][0];
+        } else {
+            for (int j0 = 0; j0 < len; j0 += 4) {
+                const int s4 = base + (j0 << 6);
+                const i4 c4 = cols4(sv, s4);
+                const d4 X = vals4(gx, s4), Y = vals4(gy, s4);
+                const d4 Z = (DIM == 3) ? vals4(gz, s4) : d4{0.0, 0.0, 0.0, 0.0};
+                d4 fg[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) fg[e] = packed_at<DIM>(uhpk, j0 + e < len ? c4[e] : r);
+                for (int e = 0; e < 4; ++e) fg[e] = packed_at<DIM>(uhpk, j0 + e < len ? c4[e] : r);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                if (j0 + e >= len) continue;
-                const d4 f = fg[e];
-                ax = fma(X[e], f[0], ax);
-                ay = fma(Y[e], f[1], ay);
-                if (DIM == 3) az = fma(Z[e], f[2], az);
+                for (int e = 0; e < 4; ++e) {
+                    if (j0 + e >= len) continue;
+                    const d4 f = fg[e];
+                    ax = fma(X[e], f[0], ax);
+                    ay = fma(Y[e], f[1], ay);
+                    if (DIM == 3) az = fma(Z[e], f[2], az);
+                }
             }
         }
         out = ax + ay;
@@ -196,7 +310,7 @@ __global__ __launch_bounds__(BLOCK) void ppe_rhs_kernel(
     b[r] = out;
 }
 
-template <int DIM>
+template <int DIM, bool STAGED>
 __global__ __launch_bounds__(BLOCK) void corrector_kernel(
     SellView sv, const double* __restrict__ gx, const double* __restrict__ gy,
     const double* __restrict__ gz, const double* __restrict__ p, const double* __restrict__ uh,
@@ -208,6 +322,8 @@ __global__ __launch_bounds__(BLOCK) void corrector_kernel(
     const int lb = xcd_block((sv.nv + BLOCK - 1) / BLOCK);
     if (lb < 0) return;
     const int r = lb * BLOCK + threadIdx.x;
+    const double* xs = nullptr;
+    if constexpr (STAGED) xs = stage_fields<1>(sv, lb, {p, p, p});
     if (r >= sv.nv) return;
     double rho = rho_all, dt = dt_all;
     if (bprob) {
@@ -218,21 +334,30 @@ __global__ __launch_bounds__(BLOCK) void corrector_kernel(
     const int base = row_base(sv, r);
     const int len = sv.len[r];
     double ax = 0.0, ay = 0.0, az = 0.0;
-    for (int j0 = 0; j0 < len; j0 += 4) {
-        const int s4 = base + (j0 << 6);
-        const i4 c4 = cols4(sv, s4);
-        const d4 X = vals4(gx, s4), Y = vals4(gy, s4);
-        const d4 Z = (DIM == 3) ? vals4(gz, s4) : d4{0.0, 0.0, 0.0, 0.0};
-        double pg[4];
+    if constexpr (STAGED) {
+        double sum[1][DIM] = {};
+        const double* const W[4] = {gx, gy, gz, nullptr};
+        staged_row<1, DIM, false>(sv, base, len, W, xs, sum);
+        ax = sum[0][0];
+        ay = sum[0][1];
+        if constexpr (DIM == 3) az = sum[0][2];
+    } else {
+        for (int j0 = 0; j0 < len; j0 += 4) {
+            const int s4 = base + (j0 << 6);
+            const i4 c4 = cols4(sv, s4);
+            const d4 X = vals4(gx, s4), Y = vals4(gy, s4);
+            const d4 Z = (DIM == 3) ? vals4(gz, s4) : d4{0.0, 0.0, 0.0, 0.0};
+            double pg[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) pg[e] = p[j0 + e < len ? c4[e] : r];
+            for (int e = 0; e < 4; ++e) pg[e] = p[j0 + e < len ? c4[e] : r];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            if (j0 + e >= len) continue;
-            const double pc = pg[e];
-            ax = fma(X[e], pc, ax);
-            ay = fma(Y[e], pc, ay);
-            if (DIM == 3) az = fma(Z[e], pc, az);
+            for (int e = 0; e < 4; ++e) {
+                if (j0 + e >= len) continue;
+                const double pc = pg[e];
+                ax = fma(X[e], pc, ax);
+                ay = fma(Y[e], pc, ay);
+                if (DIM == 3) az = fma(Z[e], pc, az);
+            }
         }
     }
     un[r] = uh[r] - (dt * ax) / rho;
@@ -432,9 +557,17 @@ void launch_predictor(hipStream_t s, const SellView& sv, const double* gx, const
                       double* upk, double* uhpk, const int* bprob, const double* prm,
                       const double* force) {
     const int g = (sv.nv + BLOCK - 1) / BLOCK;
-    hipLaunchKernelGGL(pack_kernel<DIM>, dim3(g), dim3(BLOCK), 0, s, sv.nv, u, v, w, upk);
-    hipLaunchKernelGGL(predictor_kernel<DIM>, dim3(grid_xcd(g)), dim3(BLOCK), 0, s, sv, gx, gy, gz, lap, upk,
-                       uh, vh, wh, uhpk, S_new, S_oo, npad, rho, mu, dt, euler, bprob, prm, force);
+    if (staged_steps<DIM>(sv)) {
+        hipLaunchKernelGGL((predictor_kernel<DIM, true>), dim3(grid_xcd(g)), dim3(BLOCK),
+                           sizeof(double) * DIM * sv.max_u, s, sv, gx, gy, gz, lap, u, v, w, upk,
+                           uh, vh, wh, uhpk, S_new, S_oo, npad, rho, mu, dt, euler, bprob, prm,
+                           force);
+    } else {
+        hipLaunchKernelGGL(pack_kernel<DIM>, dim3(g), dim3(BLOCK), 0, s, sv.nv, u, v, w, upk);
+        hipLaunchKernelGGL((predictor_kernel<DIM, false>), dim3(grid_xcd(g)), dim3(BLOCK), 0, s,
+                           sv, gx, gy, gz, lap, u, v, w, upk, uh, vh, wh, uhpk, S_new, S_oo, npad,
+                           rho, mu, dt, euler, bprob, prm, force);
+    }
     MP_HIP(hipGetLastError());
 }
 
@@ -446,8 +579,12 @@ void launch_ppe_rhs(hipStream_t s, const SellView& sv, const double* gx, const d
                     const double* normal_soa, int npad, double rho, double dt, double* b,
                     const int* bprob, const double* prm) {
     const int g = (sv.nv + BLOCK - 1) / BLOCK;
-    hipLaunchKernelGGL(ppe_rhs_kernel<DIM>, dim3(grid_xcd(g)), dim3(BLOCK), 0, s, sv, gx, gy, gz, uh, vh, wh,
-                       uhpk, u, v, w, p_old, bnd, pdir, normal_soa, npad, rho, dt, b, bprob, prm);
+    const bool st = staged_steps<DIM>(sv);
+    auto kernel = st ? ppe_rhs_kernel<DIM, true> : ppe_rhs_kernel<DIM, false>;
+    hipLaunchKernelGGL(kernel, dim3(grid_xcd(g)), dim3(BLOCK),
+                       st ? sizeof(double) * DIM * sv.max_u : 0, s,
+                       sv, gx, gy, gz, uh, vh, wh, uhpk, u, v, w, p_old, bnd, pdir, normal_soa,
+                       npad, rho, dt, b, bprob, prm);
     MP_HIP(hipGetLastError());
 }
 
@@ -458,8 +595,11 @@ void launch_corrector(hipStream_t s, const SellView& sv, const double* gx, const
                       double dt, const int* bprob, const double* prm) {
     (void)npad;
     const int g = (sv.nv + BLOCK - 1) / BLOCK;
-    hipLaunchKernelGGL(corrector_kernel<DIM>, dim3(grid_xcd(g)), dim3(BLOCK), 0, s, sv, gx, gy, gz, p, uh,
-                       vh, wh, un, vn, wn, rho, dt, bprob, prm);
+    const bool st = staged_steps<DIM>(sv);
+    auto kernel = st ? corrector_kernel<DIM, true> : corrector_kernel<DIM, false>;
+    hipLaunchKernelGGL(kernel, dim3(grid_xcd(g)), dim3(BLOCK), st ? sizeof(double) * sv.max_u : 0,
+                       s, sv,
+                       gx, gy, gz, p, uh, vh, wh, un, vn, wn, rho, dt, bprob, prm);
     MP_HIP(hipGetLastError());
 }
 

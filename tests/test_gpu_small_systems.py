@@ -123,3 +123,54 @@ def test_large_system_with_local_and_scattered_columns(spread, prec):
         res = np.linalg.norm(r) / np.linalg.norm(b)
         _print("spread", spread, "prec", prec, "iterations", ctx.stats().iterations, "res", res)
         assert res <= 1.1e-11  # the solver's FP64 test, plus this host's rounding
+
+
+@pytest.mark.parametrize("dim,n,k", [(2, 411, 30), (3, 56, 40), (3, 56, 150)])
+def test_large_cloud_step_matches_its_operators(dim, n, k):
+    """One Euler step of a cloud above 640 row blocks, whose predictor, right-hand
+    side and corrector read staged entries (with 150-node stencils a row block
+    has too many for three vectors: the gathering kernels), against the
+    operator products, which gather: the predictor's source and the corrected
+    velocity bit for bit, the pressure by its residual."""
+    import memphys_amd as M
+    kw = dict(k_layers=(60, 55, 50)) if k == 40 else {}
+    cloud = M.box_cloud(dim=dim, n=n, jitter=0.25, seed=5, k_interior=k, **kw)
+    rng = np.random.default_rng(1)
+    u_dir, p_dir, _ = M.lid_conditions(cloud)
+    wall = cloud.boundary == 1
+    rho, mu, dt, tol = 1.0, 0.01, 1e-5, 1e-9
+    with M.Context(0) as ctx:
+        ctx.upload(cloud)
+        ctx.weights(3, 3, download=False)
+        ctx.fs_create(rho, mu, dt, 2, tol, 4000, u_dir, u_dir, u_dir if dim == 3 else None, p_dir,
+                      precision=M.MP_PREC_MIXED, precond=M.MP_PRECOND_AMG,
+                      krylov=M.MP_KRYLOV_GMRES)
+        u = [np.where(wall, 0.0, rng.standard_normal(cloud.nv)) for _ in range(dim)]
+        for q in range(dim):
+            ctx.set_field(q, u[q])
+        ctx.set_field(M.MP_P, np.zeros(ctx.n_sys))
+        ctx.step(1, 0)
+        src = [ctx.get_field(M.MP_SU + q) for q in range(dim)]
+        new = [ctx.get_field(q) for q in range(dim)]
+        p = ctx.get_field(M.MP_P)
+        grad = lambda f: [ctx.apply(o, f) for o in range(dim)]
+        hat = []
+        for q in range(dim):
+            g = grad(u[q])
+            conv = -(u[0] * g[0]) - u[1] * g[1]
+            if dim == 3:
+                conv = conv - u[2] * g[2]
+            s = rho * conv + mu * ctx.apply(M.MP_LAP, u[q])
+            assert np.array_equal(s, src[q])
+            hat.append(u[q] + (dt / rho) * s)
+        gp = grad(p[:cloud.nv])
+        for q in range(dim):
+            assert np.array_equal(np.where(wall, u[q], hat[q] - (dt * gp[q]) / rho), new[q])
+        div = sum(ctx.apply(o, hat[o]) for o in range(dim))
+        flux = sum((u[a] - hat[a]) * cloud.normal[:, a] for a in range(dim))
+        b = np.where(wall, -rho * flux / dt, div * rho / dt)
+        ap = np.where(wall, sum(cloud.normal[:, a] * gp[a] for a in range(dim)),
+                      ctx.apply(M.MP_LAP, p[:cloud.nv])) + p[cloud.nv]
+        res = np.linalg.norm(ap - b) / np.linalg.norm(b)
+        _print("dim", dim, "k", k, "residual", res, ctx.stats().rel_res)
+        assert res <= 1.5 * tol  # the solver's FP64 test, and the sums' own rounding
