@@ -52,21 +52,22 @@ __device__ __forceinline__ void rhs_entries(bool is_pt, int dim, int phs, const 
             double d = xi[a] - xc[a];
             r2 = r2 + d * d;
         }
+        const double q2 = rpow_d(r2, phs - 2);
         for (int a = 0; a < dim; ++a) {
             double v = (-p) * (xi[a] - xc[a]);
-            v = v * rpow_d(r2, phs - 2);
+            v = v * q2;
             out[a] = v / sc[a];
         }
         double lp = 0.0;
         if (fabs(r2) > 1e-14) {
             double g[3] = {0.0, 0.0, 0.0};
+            const double q4 = rpow_d(r2, phs - 4);
             for (int a = 0; a < dim; ++a) {
                 double d = xi[a] - xc[a];
                 double d2 = d * d;
-                double q4 = rpow_d(r2, phs - 4);
                 double v = (p * p) * d2 * q4;
                 v = v - (2.0 * p) * d2 * q4;
-                v = v + p * rpow_d(r2, phs - 2);
+                v = v + p * q2;
                 g[a] = v / (sc[a] * sc[a]);
             }
             lp = g[0] + g[1];
@@ -394,15 +395,23 @@ __global__ __launch_bounds__(256) void weights_fp64_kernel(
 // row keeps its columns c..M-1 in a[0..M-1-c]: the trailing update writes a[j]
 // from a[j+1], so the row shifts by one column per step and every register
 // index is a compile-time constant.  The update width is rounded up to a
-// multiple of 8 (the entries past the row's end are never read back).  The
-// pivot row is published through LDS, where it stays as row c of U (packed,
-// row c at c*M - c(c-1)/2) for the back substitution, and its forward-
-// eliminated right-hand sides stay in Y[c].  Every entry sees the oracle's
-// roundings in the oracle's order: the same division for each multiplier,
-// fma(-l, u, a) for each update, the pivot chosen as the first maximum in
-// position order (a NaN on the diagonal position keeps it), and the column-
-// oriented back substitution.  The weights are therefore bit-identical to the
-// oracle's and to the LDS kernel's.
+// multiple of 8 (the entries past the row's end are never read back).  Only the
+// rows below the pivot are updated, so a finished row keeps its row of U in
+// registers; U and the forward-eliminated right-hand sides go to LDS for the
+// back substitution.  Every entry sees the oracle's roundings in the oracle's
+// order: the same division for each multiplier, fma(-l, u, a) for each update,
+// the pivot chosen as the first maximum in position order (a NaN on the
+// diagonal position keeps it), and the column-oriented back substitution.  The
+// weights are therefore bit-identical to the oracle's and to the LDS kernel's.
+//
+// One wavefront is bound by its vector instructions (about 80 % busy at three
+// wavefronts per SIMD).  183k stencils of 60 rows: 7.3 ms, 10.7 ms with the
+// whole of U in LDS (two wavefronts per SIMD), the monomials by loops over their
+// exponents, the matrix column by column and the back substitution with four
+// divisions per column.  64k stencils of 70 to 80 rows on two wavefronts: 10.3 ms
+// (11.1 ms); their steps wait for LDS and the barrier.  A row must not spill:
+// readlane takes entries of the pivot's lane where that lane is masked off, and
+// a reload there would leave its registers stale.
 
 __device__ __forceinline__ double readlane_d(double v, int l) {
     const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
@@ -417,6 +426,13 @@ __device__ __forceinline__ double readlane_d(double v, int l) {
 __device__ __forceinline__ double fma3(double a, double b, double c) {
     double d;
     asm("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
+    return d;
+}
+
+// The same with b in scalar registers (a value that readlane has just fetched).
+__device__ __forceinline__ double fma3s(double a, double b, double c) {
+    double d;
+    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(a), "s"(b), "v"(c));
     return d;
 }
 
@@ -444,6 +460,37 @@ __device__ __forceinline__ double wave_max_d(double v) {
     return __hiloint2double(__builtin_amdgcn_readlane(hi, 63), __builtin_amdgcn_readlane(lo, 63));
 }
 
+// Maximum of an unsigned over the wavefront, the same way (one instruction per
+// step: 0 stands in where no lane is read).
+__device__ __forceinline__ unsigned wave_max_u(unsigned v) {
+#define MP_DPP_MAXU(ctrl, rows)                                                              \
+    v = max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xf, false));
+    MP_DPP_MAXU(0x111, 0xf)
+    MP_DPP_MAXU(0x112, 0xf)
+    MP_DPP_MAXU(0x114, 0xf)
+    MP_DPP_MAXU(0x118, 0xf)
+    MP_DPP_MAXU(0x142, 0xa)
+    MP_DPP_MAXU(0x143, 0xc)
+#undef MP_DPP_MAXU
+    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// Lanes whose |v| is the largest among those with act (none of them NaN): the
+// bits of non-negative doubles order as integers, so the high words decide, and
+// only lanes that tie there compare their low words.
+__device__ __forceinline__ unsigned long long wave_argmax(double v, bool act) {
+    const unsigned hi = (unsigned)__double2hiint(v) & 0x7FFFFFFFu;
+    const unsigned mh = wave_max_u(act ? hi + 1u : 0u);  // (0: no lane takes part)
+    bool top = act && hi + 1u == mh;
+    unsigned long long b = __ballot(top);
+    if (b & (b - 1)) {  // several lanes: uniform branch
+        const unsigned lo = (unsigned)__double2loint(v);
+        const unsigned ml = wave_max_u(top ? lo : 0u);
+        b = __ballot(top && lo == ml);
+    }
+    return b;
+}
+
 // Minimum and maximum over the lanes that hold a point, each equal to the
 // oracle's left-to-right scan (a later value replaces the current one only when
 // strictly smaller / larger): the extreme value by DPP reductions, then the
@@ -462,11 +509,24 @@ __device__ __forceinline__ void ordered_minmax(double& mn, double& mx, int& has,
     has = __ballot(has) != 0ull;
 }
 
+// First column of U's right strip: the single-wavefront kernel of up to 64 rows
+// puts its columns 48.. and then its columns 0..47 in LDS for the back
+// substitution, so that a stencil needs about 12 KB and the registers, not LDS,
+// set the number of wavefronts in flight (the whole triangle: 18 KB, 8 blocks
+// per CU instead of 12).
+constexpr int wave_split(int NW, int AW) { return NW == 1 && AW > 48 ? 48 : AW; }
+
 // LDS doubles the register-resident kernel needs for a stencil of M = k + m.
-__host__ __device__ inline int wave_lds_doubles(int M, int k, int m) {
-    const int lu = M * (M + 1) / 2 + 8 + 4 * M;  // packed U (+ overflow) and Y
-    const int asm_ = 4 * k + m * k;             // scaled coordinates and monomials
-    return lu > asm_ ? lu : asm_;
+template <int NW, int AW>
+constexpr int wave_lds_doubles(int m) {
+    const int M = AW, k = AW - m, H = wave_split(NW, AW);
+    const int left = H * (H + 1) / 2, right = M * ((M - H) | 1);
+    const int cand = NW == 2 ? 4 * (AW + 6) : AW + 2;  // published pivot rows
+    const int asm_ = 4 * k + m * k;                    // scaled coordinates and monomials
+    int n = 4 * M + left;
+    if (H < M && right > left) n = 4 * M + right;
+    if (n < cand) n = cand;
+    return n > asm_ ? n : asm_;
 }
 
 // The pivot steps of one wavefront's rows.  phase<W> runs the steps whose
@@ -477,36 +537,29 @@ template <int NW, int AW>
 struct WaveLu {
     double (&a)[AW + 1];
     double (&r)[4];
-    double* U;
-    double* Y;
+    double* pub;         // published pivot rows
     const double* zero;  // AW + 1 zeros
     double* s_cv;
     int* s_cp;
-    int* s_cn;
     int M, pos, lane, wv;
     bool valid;
-    int ub = 0;         // start of U row c
     bool zero_pivot = false;  // a single wavefront met an exactly zero pivot (stencil redone)
 
-    // One wavefront (M <= 64): no LDS inside the factorisation.  The pivot is
-    // found with a DPP maximum and a ballot, its row is broadcast with
-    // readlane, and only the rows below the pivot are updated (exec mask), so
-    // a pivot row keeps its U row in registers until the end (store_u).
+    // One wavefront (M <= 64).  The pivot is found with a DPP maximum and a
+    // ballot, and only the rows below the pivot are updated (exec mask), so a
+    // pivot row keeps its U row in registers until the end (store_u).
     template <int W>
     __device__ __forceinline__ void step1(int c) {
-        const double av = fabs(a[0]);
         const bool act = valid && pos >= c;
-        const bool isn = !(av == av);
-        const double cv = (act && !isn) ? av : -1.0;
-        const double mxv = wave_max_d(cv);
-        const unsigned long long tie = __ballot(act && cv == mxv && mxv >= 0.0);
+        const bool isn = !(a[0] == a[0]);
+        const unsigned long long tie = wave_argmax(a[0], act && !isn);
         int piv;
         if (__ballot(valid && pos == c && isn) != 0ull || tie == 0ull) {
             piv = c;  // a NaN on the diagonal position keeps it (nothing compares greater)
         } else if (__popcll(tie) == 1) {
             piv = __builtin_amdgcn_readlane(pos, __ffsll((long long)tie) - 1);
         } else {  // exact ties: the first in position order
-            int cp = (act && cv == mxv) ? pos : INT_MAX;
+            int cp = ((tie >> lane) & 1ull) ? pos : INT_MAX;
             for (int off = 32; off > 0; off >>= 1) cp = min(cp, __shfl_xor(cp, off));
             piv = __builtin_amdgcn_readfirstlane(cp);
         }
@@ -514,16 +567,18 @@ struct WaveLu {
         else if (pos == piv) pos = c;
         const int pl = __ffsll((long long)__ballot(pos == c)) - 1;  // the pivot row's lane
         // The pivot row reaches the other rows two ways at once: its first
-        // L+1 entries through LDS (one lane writes, every lane reads the same
-        // address), the rest by readlane, which balances the LDS and vector
-        // pipes (LDS alone or readlane alone each take about 1.5x longer).
-        constexpr int L = (3 * W / 4) & ~1;
-        if (pos == c) {
+        // quarter through LDS (one lane writes, every lane reads the same
+        // address), the rest by readlane into scalar operands.  7.3 ms for 183k
+        // stencils of 60 rows with a quarter, 7.4 with a half, 7.8 with three.
+        constexpr int L = (W / 4) & ~1;
+        if (L > 0) {
+            if (pos == c) {
 #pragma unroll
-            for (int j = 0; j <= L; ++j) U[ub + j] = a[j];
+                for (int j = 1; j <= L; ++j) pub[j + 1] = a[j];  // (a[1] 16-byte aligned)
+            }
+            __syncthreads();
         }
-        __syncthreads();
-        const double* u = U + ub;
+        const double* u = pub + 1;
         const double d = readlane_d(a[0], pl);
         if (d == 0.0) {  // a singular column (the oracle skips it): left to the LDS kernel
             zero_pivot = true;
@@ -534,94 +589,231 @@ struct WaveLu {
 #pragma unroll
             for (int j = 0; j < L; ++j) a[j] = fma3(nl, u[j + 1], a[j + 1]);
 #pragma unroll
-            for (int j = L; j < W; ++j) a[j] = fma3(nl, readlane_d(a[j + 1], pl), a[j + 1]);
+            for (int j = L; j < W; ++j) a[j] = fma3s(nl, readlane_d(a[j + 1], pl), a[j + 1]);
 #pragma unroll
-            for (int q = 0; q < 4; ++q) r[q] = fma3(nl, readlane_d(r[q], pl), r[q]);
+            for (int q = 0; q < 4; ++q) r[q] = fma3s(nl, readlane_d(r[q], pl), r[q]);
         }
-        ub += M - c;
     }
 
-    // After the last step every row holds its U row (columns pos..M-1 in
-    // a[0..M-1-pos]) and its forward-eliminated right-hand sides.
-    __device__ __forceinline__ void store_u() {
-        if (!valid) return;
-        const int b = pos * M - pos * (pos - 1) / 2;
-#pragma unroll
-        for (int j = 0; j < AW; ++j)
-            if (j < M - pos) U[b + j] = a[j];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) Y[4 * pos + q] = r[q];
-    }
-
+    // Two wavefronts: each publishes the candidate among its own rows, whole,
+    // and one barrier later both read the winner's, so a step has a single
+    // barrier (two buffers in turn: a wavefront one step ahead writes the other).
     template <int W>
-    __device__ __forceinline__ void step(int c) {
-        if constexpr (NW == 1) {
-            step1<W>(c);
-            return;
-        }
-        // pivot: the first maximum of |column c| in position order
-        const double av = fabs(a[0]);
+    __device__ __forceinline__ void step2(int c) {
         const bool act = valid && pos >= c;
-        const bool isn = !(av == av);
-        const double cv = (act && !isn) ? av : -1.0;
-        double mxv = cv;
-        for (int off = 32; off > 0; off >>= 1) mxv = fmax(mxv, __shfl_xor(mxv, off));
-        int cp = (cv == mxv && mxv >= 0.0) ? pos : INT_MAX;
-        const unsigned long long tie = __ballot(cp != INT_MAX);
-        if (__popcll(tie) == 1) {
-            cp = __builtin_amdgcn_readlane(cp, __ffsll((long long)tie) - 1);
-        } else {
-            for (int off = 32; off > 0; off >>= 1) cp = min(cp, __shfl_xor(cp, off));
-        }
-        int nanc = __any(valid && pos == c && isn) ? 1 : 0;
-        if (NW == 2) {
-            if (lane == 0) {
-                s_cv[wv] = mxv;
-                s_cp[wv] = cp;
-                s_cn[wv] = nanc;
+        const bool isn = !(a[0] == a[0]);
+        const unsigned long long diag_nan = __ballot(valid && pos == c && isn);
+        unsigned long long tie = wave_argmax(a[0], act && !isn);
+        double key = -1.0;  // |candidate|; a NaN on the diagonal position wins over all
+        int cp = INT_MAX, cl = 64;
+        if (diag_nan) {
+            cl = __ffsll((long long)diag_nan) - 1;
+            key = __builtin_inf();
+            cp = -1;
+        } else if (tie) {
+            cl = __ffsll((long long)tie) - 1;
+            key = fabs(readlane_d(a[0], cl));
+            cp = __builtin_amdgcn_readlane(pos, cl);
+            if (__popcll(tie) > 1) {  // exact ties: the first in position order
+                cp = ((tie >> lane) & 1ull) ? pos : INT_MAX;
+                for (int off = 32; off > 0; off >>= 1) cp = min(cp, __shfl_xor(cp, off));
+                cp = __builtin_amdgcn_readfirstlane(cp);
+                cl = __ffsll((long long)__ballot(act && pos == cp)) - 1;
             }
-            __syncthreads();
-            const double v0 = s_cv[0], v1 = s_cv[1];
-            const int p0 = s_cp[0], p1 = s_cp[1];
-            nanc = s_cn[0] | s_cn[1];
-            mxv = v0 > v1 ? v0 : v1;
-            cp = (v0 == v1) ? min(p0, p1) : (v0 > v1 ? p0 : p1);
         }
-        const int piv = (nanc || mxv < 0.0) ? c : cp;
-        if (pos == c) pos = piv;
-        else if (pos == piv) pos = c;
-        // the pivot row becomes row c of U (entries past its end are overwritten later)
-        if (pos == c) {
+        const int buf = 2 * (c & 1);
+        if (lane == cl) {
+            double* o = pub + (buf + wv) * (AW + 6);
 #pragma unroll
-            for (int j = 0; j <= W; ++j) U[ub + j] = a[j];
+            for (int j = 0; j <= W; ++j) o[j + 1] = a[j];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) Y[4 * c + q] = r[q];
+            for (int q = 0; q < 4; ++q) o[AW + 2 + q] = r[q];
+        }
+        if (lane == 0) {
+            s_cv[buf + wv] = key;
+            s_cp[buf + wv] = cp;
         }
         __syncthreads();
+        const double v0 = s_cv[buf], v1 = s_cv[buf + 1];
+        const int p0 = s_cp[buf], p1 = s_cp[buf + 1];
+        const bool one = v0 == v1 ? p1 < p0 : v1 > v0;  // wavefront 1 holds the pivot
+        const int best = one ? p1 : p0;
+        const int piv = best < 0 ? c : best;
+        if (pos == c) pos = piv;
+        else if (pos == piv) pos = c;
         // A zero pivot leaves the rows below untouched (the oracle skips the
         // column): multiplier -0 against a row of +0 gives x + (-0) = x exactly
         // for every x, so the same instructions run in both cases.
-        const double d = U[ub];
+        const double* u = pub + (buf + (one ? 1 : 0)) * (AW + 6) + 1;
+        const double* y = u + AW + 1;
+        const double d = u[0];
         const bool sing = (d == 0.0);
-        const double nl = sing ? -0.0 : -(a[0] / d);
-        const double* u = sing ? zero : U + ub;
-        const double* y = sing ? zero : Y + 4 * c;
+        if (sing) u = y = zero;
+        if (pos > c) {
+            const double nl = sing ? -0.0 : -(a[0] / d);
 #pragma unroll
-        for (int j = 0; j < W; ++j) a[j] = fma3(nl, u[j + 1], a[j + 1]);
+            for (int j = 0; j < W; ++j) a[j] = fma3(nl, u[j + 1], a[j + 1]);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) r[q] = fma3(nl, y[q], r[q]);
-        ub += M - c;
+            for (int q = 0; q < 4; ++q) r[q] = fma3(nl, y[q], r[q]);
+        }
+    }
+
+    // After the last step every row holds its U row (columns pos..M-1 in
+    // a[0..M-1-pos]) and its forward-eliminated right-hand sides.  Columns
+    // [0, H) go to LDS packed (row p at p*H - p(p-1)/2), columns [H, M) with a
+    // row stride of rs.
+    __device__ __forceinline__ void store_left(double* U, int H) const {
+        if (!valid || pos >= H) return;
+        const int b = pos * H - pos * (pos - 1) / 2;
+#pragma unroll
+        for (int j = 0; j < AW; ++j)
+            if (j < H - pos) U[b + j] = a[j];
+    }
+    __device__ __forceinline__ void store_right(double* U, int H, int rs) const {
+        if (!valid) return;
+        const int b = pos * rs + pos - H;
+#pragma unroll
+        for (int j = 0; j < AW; ++j)
+            if ((unsigned)(j + pos - H) < (unsigned)(M - H)) U[b + j] = a[j];
     }
 
     template <int W>
     __device__ __forceinline__ void phase(int& c) {
-        for (; c < M && M - 1 - c > W - 8 && !zero_pivot; ++c) step<W>(c);
+        for (; c < M && M - 1 - c > W - 8 && !zero_pivot; ++c) {
+            if constexpr (NW == 1) step1<W>(c);
+            else step2<W>(c);
+        }
         if constexpr (W > 0) phase<W - 8>(c);
     }
 };
 
+// Back substitution, column oriented.  16 lanes per right-hand side, lane l of
+// a group holding its rows 16*b + l, so a column takes one division and its
+// quotient reaches the group through one DPP broadcast; the four right-hand
+// sides go side by side.  (One lane per row with the four one after the other
+// took 38k cycles for 60 rows.)
+//
+// y / d from the correctly rounded reciprocal of the row's diagonal (Markstein
+// 1990): q1 is within one ulp, the remainder y - d*q1 is then exact, and its
+// correction with RN(1/d) gives the correctly rounded quotient.  That holds
+// while nothing under- or overflows; outside [2^-400, 2^400], for infinities
+// and NaN the division itself runs.
+struct BackRow {
+    double y, d, rd;
+    bool dok;  // the diagonal is in range
+};
+
+__device__ __forceinline__ double back_quotient(const BackRow& b, bool ask) {
+    const double q0 = b.y * b.rd;
+    double e = fma(-b.d, q0, b.y);
+    const double q1 = fma(e, b.rd, q0);
+    e = fma(-b.d, q1, b.y);
+    double q = fma(e, b.rd, q1);
+    const double ay = fabs(b.y);
+    const bool zero = ay == 0.0;
+    q = zero ? q0 : q;
+    const bool ok = b.dok && (zero || (ay >= 0x1p-400 && ay <= 0x1p400));
+    if (__ballot(ask && !ok)) q = b.y / b.d;  // uniform
+    return q;
+}
+
+// Columns c = 16*B + C .. 16*B (C counts down) of the rows 0..16*B+15: at(p, c)
+// is the LDS index of U's entry.
+template <int B, int C, int NB, class At>
+__device__ __forceinline__ void back_columns(BackRow (&row)[NB], const double* U, int M, int l,
+                                             const At& at) {
+    constexpr int c = 16 * B + C;
+    if (c < M) {
+        double u[B + 1];
+#pragma unroll
+        for (int b = 0; b <= B; ++b) u[b] = b < B || l < C ? U[at(16 * b + l, c)] : 0.0;
+        const double q = back_quotient(row[B], l == C);
+        const int qh = __double2hiint(q), ql = __double2loint(q);
+        const double x = __hiloint2double(
+            __builtin_amdgcn_update_dpp(0, qh, 0x150 + C, 0xf, 0xf, true),   // row_newbcast:C
+            __builtin_amdgcn_update_dpp(0, ql, 0x150 + C, 0xf, 0xf, true));
+#pragma unroll
+        for (int b = 0; b < B; ++b) row[b].y = fma(-u[b], x, row[b].y);
+        if (l < C) row[B].y = fma(-u[B], x, row[B].y);
+        else if (l == C) row[B].y = x;
+    }
+    if constexpr (C > 0) back_columns<B, C - 1>(row, U, M, l, at);
+}
+
+// Column blocks B .. LO.
+template <int B, int LO, int NB, class At>
+__device__ __forceinline__ void back_blocks(BackRow (&row)[NB], const double* U, int M, int l,
+                                            const At& at) {
+    back_columns<B, 15>(row, U, M, l, at);
+    if constexpr (B > LO) back_blocks<B - 1, LO>(row, U, M, l, at);
+}
+
+// Row i of the saddle-point matrix, from the assembly tables in LDS.
+struct SaddleRow {
+    const double *xs, *P;
+    int i, it, ip, k, M, dim, phs;
+    double x0, x1, x2;
+
+    // Columns J .. J+T-1, all of them stencil points: their square roots side by side.
+    template <int J, int T, int N>
+    __device__ __forceinline__ void points(double (&a)[N]) const {
+        double sq[T], v[T];
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            const double d0 = x0 - xs[4 * (J + t)], d1 = x1 - xs[4 * (J + t) + 1];
+            double s = 0.0;
+            s = s + d0 * d0;
+            s = s + d1 * d1;
+            sq[t] = s;
+        }
+        if (dim == 3) {
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                const double d2 = x2 - xs[4 * (J + t) + 2];
+                sq[t] = sq[t] + d2 * d2;
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < T; ++t) v[t] = sqrt(sq[t]);
+        for (int e = 0; e < (phs - 1) / 2; ++e) {
+#pragma unroll
+            for (int t = 0; t < T; ++t) v[t] = v[t] * sq[t];
+        }
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+            a[J + t] = i < k ? (i == J + t ? 0.0 : v[t]) : P[it * k + J + t];
+    }
+
+    __device__ __forceinline__ double entry(int j) const {
+        if (j >= M) return 0.0;
+        if (j >= k) return i < k ? P[(j - k) * k + ip] : 0.0;
+        const double d0 = x0 - xs[j * 4], d1 = x1 - xs[j * 4 + 1];
+        double s = 0.0;
+        s = s + d0 * d0;
+        s = s + d1 * d1;
+        if (dim == 3) {
+            const double d2 = x2 - xs[j * 4 + 2];
+            s = s + d2 * d2;
+        }
+        const double rb = (i == j) ? 0.0 : rpow_d(s, phs);
+        return i < k ? rb : P[it * k + j];
+    }
+
+    template <int J, int AW, int N>
+    __device__ __forceinline__ void fill(double (&a)[N]) const {
+        constexpr int T = J + 24 <= AW ? 4 : 2;  // (the row itself fills the registers by then)
+        if (J + T <= k && phs >= 1) {
+            points<J, T>(a);
+        } else {
+#pragma unroll
+            for (int t = 0; t < T; ++t) a[J + t] = entry(J + t);
+        }
+        if constexpr (J + T < AW) fill<J + T, AW>(a);
+    }
+};
+
 template <int NW, int AW>
-__global__ __launch_bounds__(64 * NW) void weights_wave_kernel(
+__global__ __launch_bounds__(64 * NW, AW <= 32 ? 4 : AW <= 64 ? 3 : 2) void weights_wave_kernel(
     int dim, int phs, int m, const int* __restrict__ exps, SellView sv,
     const double* __restrict__ xyz, int npad, double* __restrict__ gx, double* __restrict__ gy,
     double* __restrict__ gz, double* __restrict__ lap, const int* __restrict__ rows,
@@ -630,18 +822,18 @@ __global__ __launch_bounds__(64 * NW) void weights_wave_kernel(
     __shared__ double s_mm[NW][6];
     __shared__ int s_has[NW];
     __shared__ double s_sc[3], s_mn[3];
-    __shared__ double s_cv[NW];
-    __shared__ int s_cp[NW], s_cn[NW];
+    __shared__ double s_cv[4];
+    __shared__ int s_cp[4];
     __shared__ int s_e[WAVE_MAX_POLY * 3];
-    __shared__ double s_zero[AW + 1];
+    __shared__ double s_zero[NW == 2 ? AW + 1 : 1];
 
     const int r = rows[blockIdx.x];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int k = sv.len[r];
     const int M = k + m;
     const int base = sell_base(sv.sptr, r);
-    double* U = lds;                          // packed rows of U
-    double* Y = lds + M * (M + 1) / 2 + 8;    // forward-eliminated right-hand sides [M][4]
+    double* Y = lds;                          // forward-eliminated right-hand sides [M][4]
+    double* U = lds + 4 * M;                  // rows of U (a strip of columns at a time)
     double* xs = lds;                         // assembly: scaled coordinates [k][4]
     double* P = lds + 4 * k;                  // assembly: monomial t at point j, P[t*k + j]
 
@@ -682,10 +874,21 @@ __global__ __launch_bounds__(64 * NW) void weights_wave_kernel(
             xp[a] = (xp[a] - s_mn[a]) / s_sc[a];
             xs[tid * 4 + a] = xp[a];
         }
+        // x^e as 1*x*x*..., the first three powers at hand: a loop over each
+        // exponent's multiplications cost 25k of the stencil's 250k cycles
+        const double p0[2] = {xp[0] * xp[0], xp[0] * xp[0] * xp[0]};
+        const double p1[2] = {xp[1] * xp[1], xp[1] * xp[1] * xp[1]};
+        const double p2[2] = {xp[2] * xp[2], xp[2] * xp[2] * xp[2]};
+        auto pw = [](double x, const double (&p)[2], int e) {
+            double v = e <= 0 ? 1.0 : e == 1 ? x : e == 2 ? p[0] : p[1];
+            for (int s = 3; s < e; ++s) v = v * x;
+            return v;
+        };
         for (int t = 0; t < m; ++t) {
             const int* e = s_e + t * dim;
-            double v = ipow_d(xp[0], e[0]);
-            for (int a = 1; a < dim; ++a) v = v * ipow_d(xp[a], e[a]);
+            double v = pw(xp[0], p0, __builtin_amdgcn_readfirstlane(e[0]));
+            v = v * pw(xp[1], p1, __builtin_amdgcn_readfirstlane(e[1]));
+            if (dim == 3) v = v * pw(xp[2], p2, __builtin_amdgcn_readfirstlane(e[2]));
             P[t * k + tid] = v;
         }
     }
@@ -697,94 +900,82 @@ __global__ __launch_bounds__(64 * NW) void weights_wave_kernel(
     const int ip = i < k ? i : 0;                     // the row's point (stencil rows)
     const int it = (i >= k && i < M) ? i - k : 0;     // the row's monomial (polynomial rows)
     const double xi0 = xs[ip * 4], xi1 = xs[ip * 4 + 1], xi2 = xs[ip * 4 + 2];
-    double a[AW + 1];
-#pragma unroll
-    for (int j = 0; j < AW; ++j) {
-        double v = 0.0;
-        if (j < M) {
-            if (j < k) {
-                const double d0 = xi0 - xs[j * 4], d1 = xi1 - xs[j * 4 + 1];
-                double s = 0.0;
-                s = s + d0 * d0;
-                s = s + d1 * d1;
-                if (dim == 3) {
-                    const double d2 = xi2 - xs[j * 4 + 2];
-                    s = s + d2 * d2;
-                }
-                const double rb = (i == j) ? 0.0 : rpow_d(s, phs);
-                v = (i < k) ? rb : P[it * k + j];
-            } else {
-                v = (i < k) ? P[(j - k) * k + ip] : 0.0;
-            }
-        }
-        a[j] = v;
-    }
-    a[AW] = 0.0;
+    // (the right-hand sides first, while the row is not in registers yet)
     double rr[4] = {0.0, 0.0, 0.0, 0.0};
     if (valid) rhs_entries(i < k, dim, phs, xs + 4 * ip, xs, s_sc, s_e + it * dim, rr);
+    double a[AW + 1];
+    // Four columns at a time, their square roots side by side: column by column
+    // the chain of each left the vector units idle (50k cycles for 60 rows).
+    const SaddleRow sr{xs, P, i, it, ip, k, M, dim, phs, xi0, xi1, xi2};
+    sr.fill<0, AW>(a);
+    a[AW] = 0.0;
     __syncthreads();  // the assembly tables are overwritten by U from here on
 
     // ---- LU with partial pivoting, right-looking ----
-    for (int j = tid; j <= AW; j += 64 * NW) s_zero[j] = 0.0;
-    __syncthreads();
-    WaveLu<NW, AW> lu{a, rr, U, Y, s_zero, s_cv, s_cp, s_cn, M, valid ? i : (1 << 20), lane, wv, valid};
+    if constexpr (NW == 2) {
+        for (int j = tid; j <= AW; j += 64 * NW) s_zero[j] = 0.0;
+        __syncthreads();
+    }
+    WaveLu<NW, AW> lu{a, rr, lds, s_zero, s_cv, s_cp, M, valid ? i : (1 << 20), lane, wv, valid};
     int c = 0;
     lu.template phase<AW>(c);
     if (lu.zero_pivot) {  // uniform: the whole wavefront saw the zero pivot
         if (tid == 0) redo[blockIdx.x] = 1;
         return;
     }
-    if (NW == 1) lu.store_u();
-    __syncthreads();
+    __syncthreads();  // (the published rows are overwritten)
+    if (valid) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) Y[4 * lu.pos + q] = rr[q];
+    }
 
-    // ---- back substitution, column oriented (wavefront 0, positions lane and lane+64) ----
+    // ---- back substitution (wavefront 0) ----
+    constexpr int SPLIT = wave_split(NW, AW), NB = AW / 16;
+    const int q = lane >> 4, l = lane & 15;
+    BackRow row[NB];
+    auto load = [&](int b, double d) {  // row 16*b + l, its diagonal entry d
+        const int p = 16 * b + l;
+        row[b].y = p < M ? Y[4 * p + q] : 0.0;
+        row[b].d = p < M ? d : 1.0;
+        row[b].rd = 1.0 / row[b].d;
+        const double ad = fabs(row[b].d);
+        row[b].dok = ad >= 0x1p-400 && ad <= 0x1p400;
+    };
+    const int H = M < SPLIT ? M : SPLIT;
+    if constexpr (SPLIT < AW) {
+        const int rs = (M - H) | 1;
+        lu.store_right(U, H, rs);
+        __syncthreads();
+        auto at = [&](int p, int cc) { return p < M ? p * rs + cc - H : 0; };
+        row[SPLIT / 16].d = 1.0;
+        load(SPLIT / 16, U[at(SPLIT + l, SPLIT + l)]);
+#pragma unroll
+        for (int b = 0; b < SPLIT / 16; ++b) load(b, 1.0);
+        back_blocks<NB - 1, SPLIT / 16>(row, U, M, l, at);
+        __syncthreads();
+    }
+    lu.store_left(U, H);
+    __syncthreads();
     if (wv != 0) return;
-    const int t0 = lane, t1 = lane + 64;
-    double y0[4] = {0.0, 0.0, 0.0, 0.0}, y1[4] = {0.0, 0.0, 0.0, 0.0};
-    if (t0 < M)
-        for (int q = 0; q < 4; ++q) y0[q] = Y[4 * t0 + q];
-    if (NW == 2 && t1 < M)
-        for (int q = 0; q < 4; ++q) y1[q] = Y[4 * t1 + q];
-    const int b0 = t0 * M - t0 * (t0 - 1) / 2 - t0;  // U[t][c] = U[b_t + c]
-    const int b1 = t1 * M - t1 * (t1 - 1) / 2 - t1;
-    for (int c = M - 1; c >= 0; --c) {
-        const double d = U[c * M - c * (c - 1) / 2];
-        double x[4];
-        if (NW == 1 || c < 64) {
+    {
+        auto at = [&](int p, int cc) { return p <= cc ? p * H - p * (p - 1) / 2 + cc - p : 0; };
 #pragma unroll
-            for (int q = 0; q < 4; ++q) x[q] = readlane_d(y0[q], c & 63) / d;
-        } else {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) x[q] = readlane_d(y1[q], c & 63) / d;
+        for (int b = 0; b < SPLIT / 16; ++b) {
+            const int p = 16 * b + l;
+            const double y = row[b].y;
+            load(b, p < H ? U[at(p, p)] : 1.0);
+            if (SPLIT < AW) row[b].y = y;
         }
-        if (t0 < c) {
-            const double u = U[b0 + c];
+        back_blocks<SPLIT / 16 - 1, 0>(row, U, M, l, at);
+    }
+    double* out = q == 0 ? gx : q == 1 ? gy : q == 2 && dim == 3 ? gz : lap;
+    if (q <= dim) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) y0[q] = fma(-u, x[q], y0[q]);
-        } else if (t0 == c) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) y0[q] = x[q];
-        }
-        if (NW == 2) {
-            if (t1 < c) {
-                const double u = U[b1 + c];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) y1[q] = fma(-u, x[q], y1[q]);
-            } else if (t1 == c) {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) y1[q] = x[q];
-            }
+        for (int b = 0; b < NB; ++b) {
+            const int p = 16 * b + l;
+            if (p < k) out[(size_t)base + (size_t)sell_off(p)] = row[b].y;
         }
     }
-    auto put = [&](int t, const double (&y)[4]) {
-        const size_t slot = (size_t)base + (size_t)sell_off(t);
-        gx[slot] = y[0];
-        gy[slot] = y[1];
-        if (dim == 3) gz[slot] = y[2];
-        lap[slot] = y[dim];
-    };
-    if (t0 < k) put(t0, y0);
-    if (NW == 2 && t1 < k) put(t1, y1);
 }
 
 // Entry (i, j) of the saddle-point matrix from the scaled coordinates, with the
@@ -1083,7 +1274,7 @@ void launch_wave(hipStream_t s, int dim, int phs, int m, const int* exps_dev, co
                  const double* xyz_soa, int npad, double* gx, double* gy, double* gz, double* lap,
                  const int* rows, int nrows, int* redo) {
     if (nrows == 0) return;
-    const size_t lds = sizeof(double) * (size_t)wave_lds_doubles(AW, AW - m, m);
+    const size_t lds = sizeof(double) * (size_t)wave_lds_doubles<NW, AW>(m);
     if (lds > 64 * 1024)
         MP_HIP(hipFuncSetAttribute((const void*)weights_wave_kernel<NW, AW>,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));

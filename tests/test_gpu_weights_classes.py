@@ -80,6 +80,17 @@ def test_weights_bit_identical_to_oracle(ctx, label, args, phs, poly):
     _check(ctx, cloud, phs, poly, label)
 
 
+@pytest.mark.parametrize("dim,k,poly,M_rows", [
+    (3, 12, 2, 22), (3, 23, 2, 33), (3, 28, 3, 48), (3, 29, 3, 49), (3, 43, 3, 63), (3, 44, 3, 64),
+    (3, 45, 3, 65), (3, 61, 3, 81), (2, 43, 5, 64), (2, 48, 5, 69)])
+def test_class_edges_bit_identical_to_oracle(ctx, dim, k, poly, M_rows):
+    """First and last row counts of each register class (up to 32, 48, 64, 80, 96 rows) and
+    exponents past the tabulated powers."""
+    import memphys_amd as M
+    cloud = M.box_cloud(dim=dim, n=16 if dim == 2 else 8, jitter=0.25, seed=11, k_interior=k)
+    _check(ctx, cloud, 3, poly, f"{dim}D k={k} degree {poly}, {M_rows} rows")
+
+
 def test_weights_with_condition_estimates(ctx):
     """Condition estimates requested: the LDS kernel, same weights."""
     import memphys_amd as M
