@@ -30,9 +30,10 @@
 // the separate restriction and pre-smoothing (Q_1 would be about 25 times
 // denser than A_1).  T_0 has half as many entries as A_0 (9 against 30 per row
 // on 2D stencils, 20-22 against 43-46 on 3D ones) and gathers from the 12 times
-// smaller level-1 vector: at 1M nodes it takes 36 us, where the separate
-// prolongation and post-smoothing by A_0 took 17 + 56 us (64 2D cavities of 665k
-// nodes: 16 against 10 + 26 us).
+// smaller level-1 vector: at 1M nodes it takes 24 us with staged
+// entries (36 us gathering from L2), where the separate prolongation and
+// post-smoothing by A_0 took 17 + 56 us (64 2D cavities of 665k nodes: 16
+// against 10 + 26 us, gathering from L2).
 // A matrix is SELL-64x4 (one wavefront per slice of 64 rows, four neighbours
 // of a row side by side, padding slots with value 0) or CSR with several lanes
 // per row, whichever suits its row lengths.

@@ -14,13 +14,17 @@
 // stops on its own; a block looks up its system once and returns at entry
 // when that system is done.  A single system is the one-system batch.
 //
-// Per iteration: p-update, SpMV + partial r0.v, finish(alpha), s-update,
-// SpMV + partial (t.s, t.t), finish(omega), x/r-update + partial (r.r, r0.r),
-// finish(loop head).  Reductions are two-stage and deterministic: every block
-// stores its partial sums (plain stores, no same-address atomics), then one
-// 1024-thread block per system sums that system's partials in block order and
-// updates its scalars in device memory.  The host launches iterations in
-// chunks (replayed from a hipGraph) and polls the flags asynchronously.
+// Per iteration of a large system: p-update, SpMV + partial r0.v, finish(alpha),
+// s-update, SpMV + partial (t.s, t.t), finish(omega), x/r-update + partial (r.r,
+// r0.r), finish(loop head).  Small systems without a preconditioner, whose
+// launches cost more than their work, fuse these into three or five kernels
+// (k_fused_*): every block forms the scalars it needs from the partial sums
+// itself.  Reductions are two-stage and deterministic: every block stores its
+// partial sums (plain stores, no same-address atomics), and one fixed order sums
+// them, in one 1024-thread block per system or in every block of a fused kernel
+// (finish_sum), so a system takes the same iterates whichever kernels run it.
+// The host launches iterations in chunks (replayed from a hipGraph) and polls
+// the flags asynchronously.
 //
 // The full-Neumann border (solver.cpp:205-213) is applied as a rank-one
 // term: the rows of a system add x[b] (b = row0 + nv, its border unknown);
