@@ -409,9 +409,16 @@ __global__ __launch_bounds__(256) void weights_fp64_kernel(
 // whole of U in LDS (two wavefronts per SIMD), the monomials by loops over their
 // exponents, the matrix column by column and the back substitution with four
 // divisions per column.  64k stencils of 70 to 80 rows on two wavefronts: 10.3 ms
-// (11.1 ms); their steps wait for LDS and the barrier.  A row must not spill:
-// readlane takes entries of the pivot's lane where that lane is masked off, and
-// a reload there would leave its registers stale.
+// (11.1 ms); their steps wait for LDS and the barrier.
+
+// f(integral_constant i) for i in [I, N).
+template <int I, int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        static_for<I + 1, N>(f);
+    }
+}
 
 __device__ __forceinline__ double readlane_d(double v, int l) {
     const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
@@ -584,14 +591,35 @@ struct WaveLu {
             zero_pivot = true;
             return;
         }
-        if (pos > c) {
-            const double nl = -(a[0] / d);
+        // Every readlane runs with the whole wavefront active, in front of the
+        // masked fmas that use it: inside the mask the pivot's lane is off, and
+        // a spill, a reload or a register move there would leave its copy stale.
+        // (Eight columns at a time, or 16 or 24: 18.3 ms for 250k 3D stencils,
+        // the time of one masked block with the readlanes inside.)
+        const bool below = pos > c;
+        const double nl = -(a[0] / d);
+        if (below) {
 #pragma unroll
             for (int j = 0; j < L; ++j) a[j] = fma3(nl, u[j + 1], a[j + 1]);
+        }
+        constexpr int T = 8;
+        static_for<0, (W - L + T - 1) / T>([&](auto g) {
+            constexpr int j0 = L + T * decltype(g)::value;
+            constexpr int n = W - j0 < T ? W - j0 : T;
+            double s[n];
 #pragma unroll
-            for (int j = L; j < W; ++j) a[j] = fma3s(nl, readlane_d(a[j + 1], pl), a[j + 1]);
+            for (int t = 0; t < n; ++t) s[t] = readlane_d(a[j0 + t + 1], pl);
+            if (below) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) r[q] = fma3s(nl, readlane_d(r[q], pl), r[q]);
+                for (int t = 0; t < n; ++t) a[j0 + t] = fma3s(nl, s[t], a[j0 + t + 1]);
+            }
+        });
+        double s[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s[q] = readlane_d(r[q], pl);
+        if (below) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) r[q] = fma3s(nl, s[q], r[q]);
         }
     }
 
