@@ -110,3 +110,12 @@ def test_single_wavefront_weights_read_lanes_unmasked(tmp_path, rows):
             assert asm.count("v_readlane") > 4 * rows  # (the broadcasts are in it)
             assert masked_readlanes(asm) == 0
     assert found == 1
+
+
+@pytest.mark.parametrize("kernel", ["weights_mixed_kernel", "weights_fp64_kernel"])
+def test_lds_weight_kernels_keep_eight_wavefronts(kernel):
+    """The weight kernels that hold their systems in LDS hide its latency with
+    eight wavefronts per SIMD: at most 64 vector registers, none spilled."""
+    k, = [v for elf in _code_objects() for n, v in _kernels(elf).items() if kernel in n]
+    assert k[".vgpr_count"] <= 64
+    assert k[".vgpr_spill_count"] == 0 and k[".private_segment_fixed_size"] == 0
