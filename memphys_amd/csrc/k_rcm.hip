@@ -18,7 +18,9 @@
 // where one thread per node, a radix sort and a synchronisation per level took
 // 5.9 ms of kernels and about 2 ms of gaps.
 // Nodes the start cannot reach restart the search at the
-// lowest-index unvisited node of minimum degree.  order[old] = new, reversed.
+// lowest-index unvisited node of minimum degree: while components are short,
+// the device finds their roots itself between levels (see rcm_order).
+// order[old] = new, reversed.
 #include <algorithm>
 #include <climits>
 #include <stdexcept>
@@ -31,10 +33,19 @@ namespace mp {
 
 namespace {
 
-// key of the lowest (degree, index) unvisited node, reduced into *best
-__global__ __launch_bounds__(BLOCK) void k_rcm_start(int nv, const int* __restrict__ rp,
+// The search's progress: the current level is queue positions a .. b-1 (empty
+// once its component is done); roots: components begun.
+struct RcmState {
+    int a, b, levels, roots;
+};
+
+// key of the lowest (degree, index) unvisited node, reduced into *best, when the
+// current level is empty and nodes are left
+__global__ __launch_bounds__(BLOCK) void k_rcm_start(const RcmState* s, int nv,
+                                                     const int* __restrict__ rp,
                                                      const int* __restrict__ pos, int idx_bits,
                                                      unsigned long long* best) {
+    if (s->a != s->b || s->b >= nv) return;
     const int i = blockIdx.x * BLOCK + threadIdx.x;
     unsigned long long k = ~0ull;
     if (i < nv && pos[i] < 0)
@@ -46,20 +57,20 @@ __global__ __launch_bounds__(BLOCK) void k_rcm_start(int nv, const int* __restri
     if ((threadIdx.x & 63) == 0 && k != ~0ull) atomicMin(best, k);
 }
 
-// The search's progress: the current level is queue positions a .. b-1 (empty
-// once its component is done).
-struct RcmState {
-    int a, b, levels;
-};
-
-__global__ void k_rcm_root(const unsigned long long* __restrict__ best, unsigned long long mask,
+// The node k_rcm_start found becomes the next component's root (*best: ~0 when it
+// did not run, and again afterwards).
+__global__ void k_rcm_root(unsigned long long* best, unsigned long long mask,
                            int* __restrict__ numbering, int* __restrict__ pos, RcmState* s) {
-    const int v = (int)(*best & mask), at = s->b;
+    const unsigned long long k = *best;
+    if (k == ~0ull) return;
+    *best = ~0ull;
+    const int v = (int)(k & mask), at = s->b;
     numbering[at] = v;
     pos[v] = at;
     s->a = at;
     s->b = at + 1;
     s->levels += 1;
+    s->roots += 1;
 }
 
 // smallest entry whose column is outside 0 .. nv-1 (LLONG_MAX: none)
@@ -74,6 +85,7 @@ __global__ __launch_bounds__(BLOCK) void k_rcm_check(long nnz, int nv, const int
 
 constexpr int RCM_WAVES = BLOCK / 64;
 constexpr int RCM_BLOCKS = 2048;  // grid of the per-level kernels: 8192 nodes at a time
+constexpr int RCM_FEW_BLOCKS = 256;  // and while components are short
 
 // every stencil entry of the level's nodes claims its unvisited column
 __global__ __launch_bounds__(BLOCK) void k_rcm_claim(const RcmState* s, const int* __restrict__ rp,
@@ -144,11 +156,14 @@ __global__ __launch_bounds__(1024) void k_rcm_scan(const RcmState* s, RcmState* 
         carry = total;
         __syncthreads();
     }
-    if (threadIdx.x == 0) *out = RcmState{s->b, s->b + carry, s->levels + (carry > 0 ? 1 : 0)};
+    if (threadIdx.x == 0)
+        *out = RcmState{s->b, s->b + carry, s->levels + (carry > 0 ? 1 : 0), s->roots};
 }
 
 // numbers each claimed column: its group's offset plus the columns of the
-// group with a smaller (degree, index); grid.y shares out a long row's chunks
+// group with a smaller (degree, index).  A row of more than MAX_STENCIL entries
+// comes in that order already (comparing its columns pairwise would take its
+// length squared): there it is the number of claimed columns in front.
 __global__ __launch_bounds__(BLOCK) void k_rcm_place(const RcmState* s, const int* __restrict__ rp,
                                                      const int* __restrict__ col,
                                                      int* __restrict__ numbering,
@@ -165,7 +180,22 @@ __global__ __launch_bounds__(BLOCK) void k_rcm_place(const RcmState* s, const in
             c = e < e1 ? col[e] : 0;
             return e < e1 && claim[c] == (((unsigned long long)t << 32) | (unsigned)(e - e0));
         };
-        for (int e = e0 + 64 * (int)blockIdx.y; e < e1; e += 64 * (int)gridDim.y) {
+        if (e1 - e0 > MAX_STENCIL) {
+            int at = b + off[t - a];
+            for (int e = e0; e < e1; e += 64) {
+                int c;
+                const bool own = mine(e + lane, c);
+                const unsigned long long m = __ballot(own);
+                if (own) {
+                    const int p = at + __popcll(m & ((1ull << lane) - 1ull));
+                    numbering[p] = c;
+                    pos[c] = p;
+                }
+                at += __popcll(m);
+            }
+            continue;
+        }
+        for (int e = e0; e < e1; e += 64) {
             int c;
             const bool own = mine(e + lane, c);
             const unsigned long long key =
@@ -202,15 +232,15 @@ __global__ __launch_bounds__(BLOCK) void k_rcm_reverse(int nv, const int* __rest
 // pos = -1 (unvisited), claim = none
 __global__ __launch_bounds__(BLOCK) void k_rcm_init(int nv, int* __restrict__ pos,
                                                     unsigned long long* __restrict__ claim,
-                                                    RcmState* s, unsigned long long* bad) {
+                                                    RcmState* s, unsigned long long* best) {
     const int i = blockIdx.x * BLOCK + threadIdx.x;
     if (i < nv) {
         pos[i] = -1;
         claim[i] = ~0ull;
     }
     if (i == 0) {
-        s[0] = s[1] = RcmState{0, 0, 0};
-        *bad = ~0ull;
+        s[0] = s[1] = RcmState{0, 0, 0, 0};
+        best[0] = best[1] = ~0ull;
     }
 }
 
@@ -237,9 +267,23 @@ void rcm_order(hipStream_t st, int nv, const int* row_ptr, const int* col, int* 
     if (2 * idx_bits + deg_bits > 64)
         throw std::invalid_argument("rcm: graph too large for 64-bit sort keys");
     const unsigned long long mask = (1ull << idx_bits) - 1ull;
-    // (ranking a row's columns is quadratic in its length: rows of thousands of
-    // entries are shared by up to 64 wavefronts)
-    const int gy = std::min(64, std::max(1, max_deg / MAX_STENCIL));
+    // rows of more than MAX_STENCIL entries in (degree, index) order (the order
+    // inside a row does not change the numbering; see k_rcm_place)
+    std::vector<int> sorted;
+    if (max_deg > MAX_STENCIL) {
+        sorted.assign(col, col + nnz);
+        for (int i = 0; i < nv; ++i) {
+            int *c0 = sorted.data() + row_ptr[i], *c1 = sorted.data() + row_ptr[i + 1];
+            if (c1 - c0 <= MAX_STENCIL) continue;
+            // (a row with a bad column stays as it is for k_rcm_check)
+            if (std::any_of(c0, c1, [nv](int c) { return c < 0 || c >= nv; })) continue;
+            std::sort(c0, c1, [row_ptr](int x, int y) {
+                const int dx = row_ptr[x + 1] - row_ptr[x], dy = row_ptr[y + 1] - row_ptr[y];
+                return dx != dy ? dx < dy : x < y;
+            });
+        }
+    }
+    const int* const up_col = sorted.empty() ? col : sorted.data();
 
     DevBuf<int> drp, dcol, numbering, pos, cnt, dorder;
     DevBuf<unsigned long long> claim, best;  // best: [0] the start's key, [1] the column check
@@ -255,10 +299,10 @@ void rcm_order(hipStream_t st, int nv, const int* row_ptr, const int* col, int* 
     state.alloc(2);
     MP_HIP(hipMemcpyAsync(drp.p, row_ptr, sizeof(int) * (nv + 1), hipMemcpyHostToDevice, st));
     if (nnz > 0)
-        MP_HIP(hipMemcpyAsync(dcol.p, col, sizeof(int) * nnz, hipMemcpyHostToDevice, st));
+        MP_HIP(hipMemcpyAsync(dcol.p, up_col, sizeof(int) * nnz, hipMemcpyHostToDevice, st));
     const int nb = (nv + BLOCK - 1) / BLOCK;
     hipLaunchKernelGGL(k_rcm_init, dim3(nb), dim3(BLOCK), 0, st, nv, pos.p, claim.p, state.p,
-                       best.p + 1);
+                       best.p);
     hipLaunchKernelGGL(k_rcm_check, dim3(RCM_BLOCKS), dim3(BLOCK), 0, st, nnz, nv, dcol.p,
                        best.p + 1);
     MP_HIP(hipGetLastError());
@@ -275,32 +319,43 @@ void rcm_order(hipStream_t st, int nv, const int* row_ptr, const int* col, int* 
             throw std::invalid_argument("rcm: column " + std::to_string(col[h->bad]) +
                                         " out of range");
         int cur = 0;
-        h->s = RcmState{0, 0, 0};
+        auto root = [&]() {
+            hipLaunchKernelGGL(k_rcm_start, dim3(nb), dim3(BLOCK), 0, st,
+                               (const RcmState*)(state.p + cur), nv, drp.p, pos.p, idx_bits,
+                               best.p);
+            hipLaunchKernelGGL(k_rcm_root, dim3(1), dim3(1), 0, st, best.p, mask, numbering.p,
+                               pos.p, state.p + cur);
+        };
+        h->s = RcmState{0, 0, 0, 0};
+        // 16 levels between two looks: those past the component's last are
+        // empty (four launches of 2 to 4 us each).  After a component of at most
+        // 8 levels the device looks for a root in front of every level (two
+        // launches more), for as long as components keep ending that soon: 4000
+        // single nodes take 85 ms, 1000 cliques of 30 nodes 45, where a look for
+        // every component took 980 and 260 ms.
+        bool many = false;
         while (h->s.b < nv) {
-            if (h->s.a == h->s.b) {  // (no level left: the next component's root)
-                MP_HIP(hipMemsetAsync(best.p, 0xFF, sizeof(unsigned long long), st));
-                hipLaunchKernelGGL(k_rcm_start, dim3(nb), dim3(BLOCK), 0, st, nv, drp.p, pos.p,
-                                   idx_bits, best.p);
-                hipLaunchKernelGGL(k_rcm_root, dim3(1), dim3(1), 0, st, best.p, mask, numbering.p,
-                                   pos.p, state.p + cur);
-            }
-            // 16 levels between two looks: those past the component's last are
-            // empty (four launches of about 2 us each)
+            const RcmState before = h->s;
+            if (!many && before.a == before.b) root();
+            const dim3 grid(many ? RCM_FEW_BLOCKS : RCM_BLOCKS);
             for (int l = 0; l < 16; ++l) {
+                if (many) root();
                 RcmState *s = state.p + cur, *next = state.p + (cur ^ 1);
-                hipLaunchKernelGGL(k_rcm_claim, dim3(RCM_BLOCKS), dim3(BLOCK), 0, st, s, drp.p,
-                                   dcol.p, numbering.p, pos.p, claim.p);
-                hipLaunchKernelGGL(k_rcm_count, dim3(RCM_BLOCKS), dim3(BLOCK), 0, st, s, drp.p,
-                                   dcol.p, numbering.p, pos.p, claim.p, cnt.p);
+                hipLaunchKernelGGL(k_rcm_claim, grid, dim3(BLOCK), 0, st, s, drp.p, dcol.p,
+                                   numbering.p, pos.p, claim.p);
+                hipLaunchKernelGGL(k_rcm_count, grid, dim3(BLOCK), 0, st, s, drp.p, dcol.p,
+                                   numbering.p, pos.p, claim.p, cnt.p);
                 hipLaunchKernelGGL(k_rcm_scan, dim3(1), dim3(1024), 0, st, s, next, cnt.p);
-                hipLaunchKernelGGL(k_rcm_place, dim3(RCM_BLOCKS, gy), dim3(BLOCK), 0, st, s, drp.p,
-                                   dcol.p, numbering.p, pos.p, claim.p, cnt.p, idx_bits);
+                hipLaunchKernelGGL(k_rcm_place, grid, dim3(BLOCK), 0, st, s, drp.p, dcol.p,
+                                   numbering.p, pos.p, claim.p, cnt.p, idx_bits);
                 cur ^= 1;
             }
             MP_HIP(hipGetLastError());
             MP_HIP(hipMemcpyAsync(&h->s, state.p + cur, sizeof(RcmState), hipMemcpyDeviceToHost,
                                   st));
             MP_HIP(hipStreamSynchronize(st));
+            many = h->s.roots - before.roots > 1 ||
+                   (h->s.a == h->s.b && h->s.levels - before.levels <= 8);
         }
         hipLaunchKernelGGL(k_rcm_reverse, dim3(nb), dim3(BLOCK), 0, st, nv, numbering.p,
                            dorder.p);

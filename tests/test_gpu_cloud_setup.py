@@ -196,3 +196,69 @@ def test_rcm_star_matches_host(nv):
         bad[[7, nv]] = nv, -1
         with pytest.raises(M.MemphysError, match=f"column {nv} out of range"):
             ctx.rcm_order(rp, bad)
+
+
+def _csr(rows):
+    rp = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    return rp, np.concatenate(rows).astype(np.int32)
+
+
+def _best_ms(f, n=3):
+    import time
+    out = []
+    for _ in range(n):
+        t = time.perf_counter()
+        f()
+        out.append(1e3 * (time.perf_counter() - t))
+    return min(out)
+
+
+@pytest.mark.parametrize("sizes", [
+    [1] * 2000,                                  # single nodes
+    [30] * 200,                                  # cliques: two levels each
+    [1, 1, 700, 1, 40, 40, 2, 700, 1, 1, 1, 3],  # short and long searches in turn
+])
+def test_rcm_many_components(sizes):
+    """The host's numbering; and a component costs the kernels of its own levels: 200 us
+    each covers several times that (a few launches of about 4 us a level), where
+    sixteen levels and a look from the host for every component took 250 us."""
+    import memphys_amd as M
+    rows, at = [], 0
+    for n in sizes:
+        if n == 700:  # a path: 700 levels
+            rows += [np.array([at + i] + [at + j for j in (i - 1, i + 1) if 0 <= j < n])
+                     for i in range(n)]
+        else:
+            rows += [at + np.roll(np.arange(n), -i) for i in range(n)]
+        at += n
+    rp, col = _csr(rows)
+    with M.Context(0) as ctx:
+        assert np.array_equal(ctx.rcm_order(rp, col), _host_rcm(rp, col))
+        if len(sizes) >= 200:
+            ms = _best_ms(lambda: ctx.rcm_order(rp, col))
+            _print("components", len(sizes), "ms", ms)
+            assert ms <= 0.2 * len(sizes)
+
+
+def test_rcm_long_rows_linear():
+    """Hubs of 15,000 and 60,000 columns, their columns' degrees differing and some of
+    them twice: the host's numbering, in a time that grows with the length (four
+    times; twice that allowed) and not with its square."""
+    import memphys_amd as M
+    ms = []
+    rng = np.random.default_rng(4)
+    with M.Context(0) as ctx:
+        for nv in (15_000, 60_000):
+            hub = np.concatenate([np.arange(nv), rng.integers(0, nv, 500)])
+            rng.shuffle(hub)
+            rows = [hub] + [np.concatenate([[i, 0], rng.integers(1, nv, rng.integers(0, 3))])
+                            for i in range(1, nv)]
+            rp, col = _csr(rows)
+            assert np.array_equal(ctx.rcm_order(rp, col), _host_rcm(rp, col))
+            ms.append(_best_ms(lambda: ctx.rcm_order(rp, col)))
+            _print("hub", len(hub), "ms", ms[-1])
+            bad = col.copy()
+            bad[[9, rp[-1] - 1]] = nv, -1
+            with pytest.raises(M.MemphysError, match=f"column {nv} out of range"):
+                ctx.rcm_order(rp, bad)
+    assert ms[1] <= 8 * ms[0]
