@@ -9,6 +9,8 @@
 #include <thread>
 #include <utility>
 
+#include "parallel.hpp"
+
 namespace mp_amg {
 
 namespace {
@@ -18,21 +20,6 @@ int thread_count(int requested, long work) {
     if (t < 1) t = 1;
     if (work < 20000) t = 1;
     return std::min(t, 32);
-}
-
-// Runs body(r0, r1, tid) over [0, n) split into `t` contiguous ranges.
-template <typename F>
-void parallel_rows(int n, int t, F&& body) {
-    if (t <= 1) {
-        body(0, n, 0);
-        return;
-    }
-    std::vector<std::thread> pool;
-    for (int q = 0; q < t; ++q) {
-        const int r0 = (int)((long)n * q / t), r1 = (int)((long)n * (q + 1) / t);
-        pool.emplace_back([&, r0, r1, q]() { body(r0, r1, q); });
-    }
-    for (auto& th : pool) th.join();
 }
 
 }  // namespace
@@ -209,7 +196,7 @@ Csr multiply(const Csr& A, const Csr& B, int threads) {
     std::vector<std::vector<int>> cols(t);
     std::vector<std::vector<double>> vals(t);
     std::vector<int> rowlen(n, 0);
-    parallel_rows(n, t, [&](int r0, int r1, int q) {
+    mp::parallel_ranges(n, t, [&](int r0, int r1, int q) {
         std::vector<int> mark(B.ncols, -1);
         std::vector<double> acc(B.ncols, 0.0);
         std::vector<int> touched;

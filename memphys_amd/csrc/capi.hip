@@ -587,27 +587,25 @@ int upload_clouds(mp_ctx* c, const char* fn, int nprob, const int* nvp, int dim,
     std::iota(hperm.begin(), hperm.end(), 0);
     {
         const int nthr = (int)std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
-        std::vector<std::thread> pool;
-        for (int tn = 0; tn < nthr; ++tn)
-            pool.emplace_back([&, tn]() {
-                std::vector<std::pair<int, int>> e;
-                for (int d = tn; d < rows; d += nthr) {
-                    const int L = hlen[d];
-                    if (L == 0) continue;
-                    const int base = sell_base(hsptr.data(), d);
-                    e.clear();
-                    for (int j = 0; j < L; ++j)
-                        e.emplace_back(hcol[base + sell_off(j)], base + sell_off(j));
-                    std::stable_sort(e.begin(), e.end(),
-                                     [](const std::pair<int, int>& a,
-                                        const std::pair<int, int>& b) { return a.first < b.first; });
-                    for (int j = 0; j < L; ++j) {
-                        hcol_s[base + sell_off(j)] = e[j].first;
-                        hperm[base + sell_off(j)] = e[j].second;
-                    }
+        parallel_ranges(nthr, nthr, [&](int tn, int, int) {
+            std::vector<std::pair<int, int>> e;
+            for (int d = tn; d < rows; d += nthr) {
+                const int L = hlen[d];
+                if (L == 0) continue;
+                const int base = sell_base(hsptr.data(), d);
+                e.clear();
+                for (int j = 0; j < L; ++j)
+                    e.emplace_back(hcol[base + sell_off(j)], base + sell_off(j));
+                std::stable_sort(e.begin(), e.end(),
+                                 [](const std::pair<int, int>& a, const std::pair<int, int>& b) {
+                                     return a.first < b.first;
+                                 });
+                for (int j = 0; j < L; ++j) {
+                    hcol_s[base + sell_off(j)] = e[j].first;
+                    hperm[base + sell_off(j)] = e[j].second;
                 }
-            });
-        for (auto& t : pool) t.join();
+            }
+        });
     }
     // large clouds: the distinct columns of each row block and the slots' places
     // among them, in both slot orders; else 16-bit columns of the sorted order

@@ -6,11 +6,11 @@
 #include <climits>
 #include <cstdint>
 #include <string>
-#include <thread>
 #include <type_traits>
 #include <vector>
 
 #include "../../include/memphys_hip.h"
+#include "parallel.hpp"
 
 namespace mp {
 
@@ -476,20 +476,6 @@ constexpr int STAGE_MAX = 6144;
 bool stage_columns(const std::vector<int>& sptr, const std::vector<int>& col, int nslices,
                    std::vector<int>& uptr, std::vector<int>& ucol, std::vector<uint16_t>& loc,
                    int& max_u);
-
-// Host: f(i) for i in [0, n) on up to 16 threads, contiguous ranges.
-template <typename F>
-void parallel_for(int n, F&& f) {
-    const int t = (int)std::max(1u, std::min({16u, std::thread::hardware_concurrency(),
-                                              (unsigned)(n / 64 + 1)}));
-    std::vector<std::thread> pool;
-    for (int q = 1; q < t; ++q)
-        pool.emplace_back([&, q]() {
-            for (int i = (int)((long)n * q / t); i < (int)((long)n * (q + 1) / t); ++i) f(i);
-        });
-    for (int i = 0; i < (int)((long)n / t); ++i) f(i);
-    for (auto& w : pool) w.join();
-}
 
 // Device-side Krylov scalars (FP64) of one system.  Written only by the
 // single-block finishing kernels, read by every block of the following kernels.
