@@ -314,14 +314,17 @@ int mp_precond_apply(mp_ctx* ctx, int cycle, int n, const double* in, double* ou
 int mp_graph_mode(mp_ctx* ctx, int enable);
 
 /* Per-kernel timing with HIP events on the library's stream.
- * which: 0 = PPE SpMV, 1 = predictor, 2 = pressure RHS, 3 = corrector,
- *        4 = stencil weights, 5 = the multigrid's level-0 post-smoothing
- *        product, prolongation included (with MP_PRECOND_AMG).  Reports the launches that did the work and
- * their mean milliseconds: Krylov launches of a system that converged inside
- * a chunk of iterations return at once and are left out (a launch counts
- * when it takes at least a quarter of the longest launch's time).  all_launches (may
- * be NULL) receives every timed launch.  bytes_per_launch: the kernel's
- * algorithmic HBM bytes per working launch. */
+ * which: 0 = the Krylov launches that hold a product with the PPE operator (on
+ *        small systems GMRES's dot products, or BiCGSTAB's vector updates and
+ *        loop head, run in the same launch), 1 = predictor, 2 = pressure RHS,
+ *        3 = corrector, 4 = stencil weights, 5 = the multigrid's level-0
+ *        post-smoothing product, prolongation included (with MP_PRECOND_AMG).
+ * Reports the launches that did the work and their mean milliseconds: Krylov
+ * launches of a system that converged inside a chunk of iterations return at
+ * once and are left out (a launch counts when it takes at least a quarter of
+ * the longest launch's time).  all_launches (may be NULL) receives every timed
+ * launch.  bytes_per_launch: the algorithmic HBM bytes of a working launch
+ * (which = 0: their mean, everything the launch does included). */
 int mp_kernel_timing(mp_ctx* ctx, int enable);
 int mp_kernel_timing_get(mp_ctx* ctx, int which, long* launches, double* mean_ms,
                          double* bytes_per_launch, long* all_launches);

@@ -1024,12 +1024,19 @@ int mp_fs_create(mp_ctx* c, const mp_fs_params* prm, const uint8_t* u_dir, const
         c->s_cur = 0;
         c->stats = mp_step_stats{};
         c->prob_total_iters.assign(c->nprob, 0);
-        // algorithmic bytes per launch (real entries only)
+        // algorithmic bytes per launch (real entries only): weights, columns (staged
+        // entries: 2 B places and 4 B per distinct column of a row block; else 4 B
+        // each) and per row its length and vectors, each once (V: the gathered
+        // velocity, one array per component when staged, else the packed copy)
         const double W = (double)c->nnz, N = (double)c->nv, D = (double)c->dim;
-        c->bytes[1] = W * (4.0 + 8.0 * (D + 1.0)) + N * (4.0 + 8.0 * (D /*own*/ + D /*gather*/ +
-                                                                  D /*uh*/ + D /*S*/ + D /*S_oo*/));
-        c->bytes[2] = W * (4.0 + 8.0 * D) + N * (4.0 + 8.0 * (D /*uh*/ + 1.0 /*b*/));
-        c->bytes[3] = W * (4.0 + 8.0 * D) + N * (4.0 + 8.0 * (1.0 + D /*uh*/ + D /*un*/));
+        const bool staged = c->dim == 3 ? staged_steps<3>(c->sv) : staged_steps<2>(c->sv);
+        const double cols = staged ? 2.0 * W + 4.0 * (double)c->sv.nuniq : 4.0 * W;
+        const double V = staged ? D : D == 3.0 ? 4.0 : 2.0;
+        c->bytes[1] = cols + W * 8.0 * (D + 1.0) +
+                      N * (4.0 + 8.0 * (V + D /*uh*/ + (staged ? 0.0 : V) /*its packed copy*/ +
+                                        D /*S*/ + D /*S_oo*/));
+        c->bytes[2] = cols + W * 8.0 * D + N * (4.0 + 8.0 * (V + 1.0 /*b*/));
+        c->bytes[3] = cols + W * 8.0 * D + N * (4.0 + 8.0 * (1.0 /*p*/ + D /*uh*/ + D /*un*/));
         c->has_fs = true;
         return MP_OK;
     });
@@ -1653,14 +1660,20 @@ int mp_kernel_timing_get(mp_ctx* c, int which, long* launches, double* mean_ms,
             PpeSolver* s = c->ppe ? c->ppe.get() : c->solver.get();
             if (!s) return fail(c, MP_ERR_STATE, "mp_kernel_timing_get: no solver");
             long all = 0;
-            (which == 0 ? s->spmv_timer : s->smooth_timer).summary(launches, mean_ms, &all);
+            double bytes = 0.0;
+            (which == 0 ? s->spmv_timer : s->smooth_timer).summary(launches, mean_ms, &bytes, &all);
             if (all_launches) *all_launches = all;
-            *bytes_per_launch = which == 0 ? s->spmv_bytes(s->precision == MP_PREC_MIXED ? 1 : 0)
-                                           : s->smooth_bytes();
+            const bool fp32 = s->precision == MP_PREC_MIXED;
+            if (which == 5)
+                bytes = s->smooth_bytes();
+            else if (all == 0)  // (no launch yet: the product's alone)
+                bytes = s->spmv_bytes(fp32, s->spmv_row_bytes(fp32, s->krylov == 1 ? 0 : 1));
+            *bytes_per_launch = bytes;
         } else {
             KernelTimer& t = c->timers[which];
             long all = 0;
-            t.summary(launches, mean_ms, &all);
+            double bytes = 0.0;
+            t.summary(launches, mean_ms, &bytes, &all);
             if (all_launches) *all_launches = all;
             *bytes_per_launch = c->bytes[which];
         }

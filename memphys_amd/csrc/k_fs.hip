@@ -47,16 +47,6 @@ __device__ __forceinline__ d4 packed_at(const double* __restrict__ a, int c) {
     }
 }
 
-// Row kernels over staged entries: large clouds whose row blocks' distinct
-// columns are listed (see Slots), when DIM vectors of them fit 64 KB of LDS; the
-// gathers of one entry per weight otherwise bound these kernels.  1M-node cube,
-// gathered and staged: predictor 460 (plus 15 for the interleaved copy it
-// gathers from) and 323 us, right-hand side 296 and 198, corrector 275 and 241.
-template <int DIM>
-bool staged_steps(const SellView& sv) {
-    return sv.max_u > 0 && DIM * sv.max_u <= 8192;
-}
-
 // The row block's distinct columns' entries of NF vectors into LDS: vector f's
 // entry of place i at xs[f * max_u + i].  Ends with a barrier.
 template <int NF>

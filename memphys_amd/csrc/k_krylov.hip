@@ -1365,13 +1365,15 @@ void launch_copy(hipStream_t s, double* dst, const double* src, int n) {
     MP_HIP(hipGetLastError());
 }
 
-void KernelTimer::begin(hipStream_t s) {
+void KernelTimer::begin(hipStream_t s, double bytes) {
     if (!enabled) return;
     if (used + 2 > ev.size()) {
         size_t old = ev.size();
         ev.resize(std::max<size_t>(64, old * 2));
         for (size_t i = old; i < ev.size(); ++i) MP_HIP(hipEventCreate(&ev[i]));
+        ev_bytes.resize(ev.size() / 2);
     }
+    ev_bytes[used / 2] = bytes;
     MP_HIP(hipEventRecord(ev[used], s));
 }
 void KernelTimer::end(hipStream_t s) {
@@ -1383,26 +1385,30 @@ void KernelTimer::harvest() {
     for (size_t i = 0; i + 1 < used; i += 2) {
         float ms = 0.f;
         if (hipEventElapsedTime(&ms, ev[i], ev[i + 1]) == hipSuccess && ms > 0.0f)
-            samples.push_back(ms);
+            samples.push_back(Sample{ms, ev_bytes[i / 2]});
     }
     used = 0;
 }
-void KernelTimer::summary(long* working, double* mean_ms, long* all) const {
+void KernelTimer::summary(long* working, double* mean_ms, double* mean_bytes, long* all) const {
     *working = 0;
     *mean_ms = 0.0;
+    *mean_bytes = 0.0;
     *all = (long)samples.size();
     if (samples.empty()) return;
     // (a quarter of the longest launch: launches that returned at once are
     // a few microseconds, working ones tens; the median fails to separate
     // them when most launches of a short solve return at once)
-    const float cut = 0.25f * *std::max_element(samples.begin(), samples.end());
-    double tot = 0.0;
-    for (float ms : samples)
-        if (ms >= cut) {
-            tot += ms;
+    float cut = 0.0f;
+    for (const Sample& s : samples) cut = std::max(cut, 0.25f * s.ms);
+    double tot = 0.0, bytes = 0.0;
+    for (const Sample& s : samples)
+        if (s.ms >= cut) {
+            tot += s.ms;
+            bytes += s.bytes;
             ++*working;
         }
     *mean_ms = tot / (double)*working;
+    *mean_bytes = bytes / (double)*working;
 }
 void KernelTimer::release() {
     for (auto e : ev) (void)hipEventDestroy(e);
@@ -1597,19 +1603,20 @@ double PpeSolver::smooth_bytes() const {
            (double)T.nslices * 4.0 * CW_COUNT + rest;
 }
 
-double PpeSolver::spmv_bytes(int fp32) const {
+double PpeSolver::spmv_row_bytes(bool fp32, int others) const {
+    // the V-cycle's output, and an FP32 GMRES basis vector, are gathered in FP32
+    const double xb = (amg || (krylov == 1 && fp32)) ? 4.0 : 8.0;
+    return xb + 8.0 * (1.0 + others + (bordered ? 1.0 : 0.0));
+}
+
+double PpeSolver::spmv_bytes(bool fp32, double row_bytes) const {
     // per entry: value (8 B, or 4 B for the FP32 operator) + column (with staged
     // entries a 2 B place, plus 4 B per distinct column of a row block; else 4 B,
     // the FP32 operator 2 B in slices with 16-bit columns, plus their window
-    // bases); per row: gathered x once (FP32 with the V-cycle, else FP64),
-    // the product written, r0 read (BiCGSTAB's fused dot; FP64), length,
-    // D^-1 for the border row
+    // bases); per row: its vectors and its length
     const double vb = fp32 ? 4.0 : 8.0;
-    // the V-cycle's output, and an FP32 GMRES basis vector, are gathered in FP32
-    const double xb = (amg || (krylov == 1 && fp32)) ? 4.0 : 8.0;
-    const double vec = (krylov == 1 ? 1.0 : 2.0) + (bordered ? 1.0 : 0.0);
     const SellView& w = fp32 ? svk : sv;
-    const double rows = (double)nv * (xb + 8.0 * vec + 4.0);
+    const double rows = (double)nv * (row_bytes + 4.0);
     if (nrows / BLOCK > SPLIT_MAX_BLOCKS && w.max_u > 0)  // (places and distinct columns)
         return (double)nnz * (vb + 2.0) + 4.0 * (double)w.nuniq + rows;
     const double n16 = fp32 ? (double)nnz16 : 0.0;
@@ -1636,15 +1643,18 @@ void PpeSolver::launch_fused_chunk(hipStream_t st, int chunk, const TM* a, const
     const int nbk = nrows / BLOCK;
     KScalars *A = sc.p, *B = A + nseg, *C = B + nseg;
     T *pb = p2.p, *vb = v2.p;
-    const bool three = nbk <= FUSE3_MAX_BLOCKS;
+    const bool three = nbk <= FUSE3_MAX_BLOCKS, f32 = sizeof(TM) == 4;
+    const double db = bordered ? 8.0 : 0.0;
     for (int c = 0; c < chunk; ++c) {
         if (three) {
-            spmv_timer.begin(st);
+            // r, p and v gathered, p and v written, r0 read, D^-1
+            spmv_timer.begin(st, spmv_bytes(f32, 48.0 + db));
             hipLaunchKernelGGL((k_fused_v<TM, T>), dim3(grid_xcd(4 * nbk)), dim3(BLOCK), 0, st,
                                view_of<TM>(), sg, a, di, (const T*)rr, (const T*)rr0, pp, pb, vv,
                                vb, partial.p, (const KScalars*)A, B);
             spmv_timer.end(st);
-            spmv_timer.begin(st);
+            // r and v gathered, s and t written, D^-1
+            spmv_timer.begin(st, spmv_bytes(f32, 32.0 + db));
             hipLaunchKernelGGL((k_fused_t<TM, T>), dim3(grid_xcd(4 * nbk)), dim3(BLOCK), 0, st,
                                view_of<TM>(), sg, a, di, (const T*)rr, (const T*)rr0, vv, vb, ss,
                                tt, partial.p, (const KScalars*)B, C);
@@ -1652,7 +1662,7 @@ void PpeSolver::launch_fused_chunk(hipStream_t st, int chunk, const TM* a, const
         } else {
             hipLaunchKernelGGL(k_fused_p<T>, dim3(nbk), dim3(BLOCK), 0, st, sg, (const T*)rr, pp,
                                (const T*)vv, (const double*)partial.p, (const KScalars*)A, B);
-            spmv_timer.begin(st);
+            spmv_timer.begin(st, spmv_bytes(f32, spmv_row_bytes(f32, 1)));
             hipLaunchKernelGGL((k_spmv_alpha<4, TM, T, T>), dim3(grid_xcd(4 * nbk)), dim3(BLOCK),
                                0, st, view_of<TM>(), sg, a, di, (const T*)pp, (const T*)pp, vv,
                                (const T*)rr0, partial.p + (size_t)BI_ALPHA * nbk,
@@ -1660,7 +1670,7 @@ void PpeSolver::launch_fused_chunk(hipStream_t st, int chunk, const TM* a, const
             spmv_timer.end(st);
             hipLaunchKernelGGL(k_fused_s<T>, dim3(nbk), dim3(BLOCK), 0, st, sg, (const T*)rr, vv,
                                ss, (const T*)rr0, (const double*)partial.p, (const KScalars*)B, C);
-            spmv_timer.begin(st);
+            spmv_timer.begin(st, spmv_bytes(f32, spmv_row_bytes(f32, 0)));
             hipLaunchKernelGGL((k_spmv_omega<4, TM, T, T>), dim3(grid_xcd(4 * nbk)), dim3(BLOCK),
                                0, st, view_of<TM>(), sg, a, di, (const T*)ss, (const T*)ss,
                                (const T*)ss, tt, partial.p + (size_t)BI_OMEGA * nbk,
@@ -1693,7 +1703,7 @@ void PpeSolver::launch_chunk(hipStream_t st, int chunk, const TM* a, const T* di
                            xs);
         // with the V-cycle, the products gather its FP32 output (the same values)
         const T* yin = precondition(st, pp, yv.p, y32.p);
-        spmv_timer.begin(st);
+        spmv_timer.begin(st, spmv_bytes(sizeof(TM) == 4, spmv_row_bytes(sizeof(TM) == 4, 1)));
         with_shape(nbk, view_of<TM>(), amg ? 4 : sizeof(T), [&](auto ws, size_t shm) {
             constexpr int WS = decltype(ws)::value;
             if (amg)
@@ -1711,7 +1721,8 @@ void PpeSolver::launch_chunk(hipStream_t st, int chunk, const TM* a, const T* di
         hipLaunchKernelGGL(k_update_s<T>, dim3(nbk), dim3(BLOCK), 0, st, sg, rr, vv, ss, sc.p, d0,
                            xs);
         const T* zin = precondition(st, ss, zv.p, z32.p);
-        spmv_timer.begin(st);
+        spmv_timer.begin(  // (without the V-cycle s itself is gathered)
+            st, spmv_bytes(sizeof(TM) == 4, spmv_row_bytes(sizeof(TM) == 4, amg ? 1 : 0)));
         with_shape(nbk, view_of<TM>(), amg ? 4 : sizeof(T), [&](auto ws, size_t shm) {
             constexpr int WS = decltype(ws)::value;
             if (amg)
@@ -1947,7 +1958,10 @@ void PpeSolver::gmres_iteration(hipStream_t st, int k, int m, const TM* a, const
     const bool split = nbk <= SPLIT_MAX_BLOCKS;
     auto product = [&](const auto* zg) {
         using TX = std::remove_cv_t<std::remove_pointer_t<decltype(zg)>>;
-        spmv_timer.begin(st);
+        // (the dot products inside read the k + 1 basis vectors)
+        spmv_timer.begin(st, spmv_bytes(sizeof(TM) == 4,
+                                        spmv_row_bytes(sizeof(TM) == 4, 0) +
+                                            (split ? (double)sizeof(TV) * (k + 1) : 0.0)));
         if (split)
             hipLaunchKernelGGL((k_gm_spmv<16, TM, TX, TV>), dim3(grid_xcd(nbk)), dim3(4 * BLOCK),
                                0, st, view_of<TM>(), sg, a, di, (const TV*)vk, zg, gm_w.p,

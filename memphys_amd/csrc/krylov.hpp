@@ -16,18 +16,25 @@ struct SolveStats {
 
 // HIP-event timing of one kernel's launches.  Krylov kernels of a system that
 // has converged inside a chunk return at once; the summary counts only the
-// launches that did the work: duration at least half the median launch's.
+// launches that did the work: duration at least a quarter of the longest
+// launch's.
 struct KernelTimer {
     bool enabled = false;
     std::vector<hipEvent_t> ev;  // pairs
+    std::vector<double> ev_bytes;  // per pair
     size_t used = 0;
-    std::vector<float> samples;  // milliseconds per launch
-    void begin(hipStream_t s);
+    struct Sample {
+        float ms;
+        double bytes;
+    };
+    std::vector<Sample> samples;  // per launch
+    // bytes: what the launch has to move (where launches differ in it)
+    void begin(hipStream_t s, double bytes = 0.0);
     void end(hipStream_t s);
     void harvest();  // after a synchronize: collect and recycle the events
     void reset() { samples.clear(); }
-    // working launches, their mean duration (ms), and all launches
-    void summary(long* working, double* mean_ms, long* all) const;
+    // working launches, their mean duration (ms) and bytes, and all launches
+    void summary(long* working, double* mean_ms, double* mean_bytes, long* all) const;
     void release();
 };
 
@@ -150,7 +157,12 @@ struct PpeSolver {
     // statistics of a single system, or the worst over a batch (per system in
     // seg_stats).
     SolveStats solve(hipStream_t s, const double* b_dev, double* x_dev);
-    double spmv_bytes(int fp32) const;
+    // algorithmic bytes of a product's launch: the operator (fp32: its FP32 copy)
+    // and row_bytes per row
+    double spmv_bytes(bool fp32, double row_bytes) const;
+    // row_bytes of a product alone: x gathered, the product written, D^-1 of the
+    // border row, the other vectors read
+    double spmv_row_bytes(bool fp32, int others) const;
     // algorithmic bytes of the level-0 prolongation and post-smoothing product (T_0)
     double smooth_bytes() const;
     // r = b - A x (FP64, unscaled operator incl. border) into `tmp`; returns tmp.p

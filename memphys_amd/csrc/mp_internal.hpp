@@ -464,6 +464,17 @@ struct SellView {
     __host__ __device__ Slots slots() const { return Slots{nslices, sptr, col, col16, cbase, uptr, ucol, loc, max_u}; }
 };
 
+// The predictor, right-hand side and corrector read staged entries: large clouds
+// whose row blocks' distinct columns are listed (see Slots), when DIM vectors of
+// them fit 64 KB of LDS; the gathers of one entry per weight otherwise bound
+// these kernels.  1M-node cube, gathered and staged: predictor 460 (plus 15 for
+// the interleaved copy it gathers from) and 323 us, right-hand side 296 and 198,
+// corrector 275 and 241.
+template <int DIM>
+bool staged_steps(const SellView& sv) {
+    return sv.max_u > 0 && DIM * sv.max_u <= 8192;
+}
+
 // Host: the compressed columns of slots sptr/col (see CW_BITS above): c16 per
 // slot, cb CW_COUNT window bases per slice (-1: the slice keeps 32-bit columns).
 void compress_columns(const std::vector<int>& sptr, const std::vector<int>& col, int nslices,

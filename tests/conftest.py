@@ -51,3 +51,32 @@ def rel_err(a, b):
     b = np.asarray(b, dtype=np.float64)
     den = np.linalg.norm(b)
     return np.linalg.norm(a - b) / (den if den > 0 else 1.0)
+
+
+def row_block_columns(cloud):
+    """Distinct columns per block of 256 device rows, as the upload lists them: rows in
+    Morton order of the coordinates, then by decreasing stencil length inside windows
+    of 4096; a padding slot holds its own row."""
+    dim, nv = cloud.dim, cloud.nv
+    bits = 10 if dim == 3 else 16
+    lo, hi = cloud.xyz.min(axis=0), cloud.xyz.max(axis=0)
+    span = np.where(hi > lo, hi - lo, 1.0)
+    g = np.minimum(2.0 ** bits - 1, np.floor((cloud.xyz - lo) / span * 2.0 ** bits))
+    g = g.astype(np.uint64)
+    key = np.zeros(nv, np.uint64)
+    for b in range(bits):
+        for a in range(dim):
+            bit = (g[:, a] >> np.uint64(b)) & np.uint64(1)
+            key |= bit << np.uint64(b * dim + a)
+    order = np.argsort(key, kind="stable")
+    length = np.diff(cloud.row_ptr)
+    for w in range(0, nv, 4096):
+        part = order[w:w + 4096]
+        order[w:w + 4096] = part[np.argsort(-length[part], kind="stable")]
+    out = []
+    for b in range(0, nv + 1, 256):  # (nv + 1: the border unknown's row)
+        rows = order[b:b + 256]
+        cols = [cloud.col[cloud.row_ptr[r]:cloud.row_ptr[r + 1]] for r in rows]
+        n = len(np.unique(np.concatenate(cols))) if len(rows) else 0
+        out.append(n + (-len(rows)) % 64)  # padding rows of the last row's slice
+    return np.array(out)
