@@ -672,6 +672,7 @@ int upload_clouds(mp_ctx* c, const char* fn, int nprob, const int* nvp, int dim,
     c->sv.loc = max_u > 0 ? c->loc.p : nullptr;
     c->sv.max_u = max_u;
     c->sv.nuniq = (long)hucol.size();
+    c->sv.reuse = max_u > 0 ? (double)c->total_slots / (double)c->sv.nuniq : 0.0;
     c->svs = c->sv;
     c->svs.col = c->col_s.p;
     c->svs.loc = max_u > 0 ? c->loc_s.p : nullptr;

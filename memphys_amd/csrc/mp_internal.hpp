@@ -460,19 +460,25 @@ struct SellView {
     const int* ucol = nullptr;
     const uint16_t* loc = nullptr;
     int max_u = 0;
-    long nuniq = 0;  // entries of ucol
+    long nuniq = 0;     // entries of ucol
+    double reuse = 0;   // slots per entry of ucol
     __host__ __device__ Slots slots() const { return Slots{nslices, sptr, col, col16, cbase, uptr, ucol, loc, max_u}; }
 };
 
 // The predictor, right-hand side and corrector read staged entries: large clouds
 // whose row blocks' distinct columns are listed (see Slots), when DIM vectors of
-// them fit 64 KB of LDS; the gathers of one entry per weight otherwise bound
-// these kernels.  1M-node cube, gathered and staged: predictor 460 (plus 15 for
-// the interleaved copy it gathers from) and 323 us, right-hand side 296 and 198,
-// corrector 275 and 241.
+// them fit 64 KB of LDS (the limit without an attribute) and a staged entry
+// serves at least 1.25 slots; the gathers of one entry per weight otherwise
+// bound these kernels.  1M-node cube (reuse 9), gathered and staged: predictor
+// 460 (plus 15 for the interleaved copy it gathers from) and 323 us, right-hand
+// side 296 and 198, corrector 275 and 241.  At the LDS limit, 600k 2D rows of 20
+// and 32 entries, 4,092 and 2,952 columns in the largest block, reuse 1.27 and
+// 2.8: 123, 84, 89 and 114, 87, 70 us; 174, 126, 117 and 130, 92, 86.  600k rows
+// of 12 and 16 entries whose columns lie anywhere, reuse 1.0: 81, 47, 55 and 96,
+// 75, 51; 106, 67, 76 and 127, 102, 71.
 template <int DIM>
 bool staged_steps(const SellView& sv) {
-    return sv.max_u > 0 && DIM * sv.max_u <= 8192;
+    return sv.max_u > 0 && DIM * sv.max_u <= 8192 && sv.reuse >= 1.25;
 }
 
 // Host: the compressed columns of slots sptr/col (see CW_BITS above): c16 per
@@ -481,8 +487,14 @@ void compress_columns(const std::vector<int>& sptr, const std::vector<int>& col,
                       std::vector<uint16_t>& c16, std::vector<int>& cb);
 
 // Host: the distinct columns of every block of BLOCK rows and each slot's place
-// among them (see Slots); false when a block has more than STAGE_MAX, which the
-// LDS form is not for.
+// among them (see Slots); false when a block has more than STAGE_MAX (48 KB of
+// FP64 entries), which the LDS form is not for.  Up to there it is the faster
+// one for the products, whatever the reuse and also when a single block sets
+// every block's LDS.  600k rows, FP64, FP32 operator in BiCGSTAB and in GMRES,
+// gathered and staged: 32 entries, 5,892 columns in the largest block, reuse
+// 1.4: 83, 68, 49 and 55, 50, 41 us; reuse 22 with one block of 5,869: 42, 38, 33
+// and 37, 30, 31; 20 entries anywhere (5,049, reuse 1.0): 68, 65, 60 and 62, 57,
+// 48.
 constexpr int STAGE_MAX = 6144;
 bool stage_columns(const std::vector<int>& sptr, const std::vector<int>& col, int nslices,
                    std::vector<int>& uptr, std::vector<int>& ucol, std::vector<uint16_t>& loc,

@@ -37,8 +37,9 @@ def _steps(ctx, cloud, krylov=0, precision=0, precond=0, steps=2, restart=0, tol
     for f in range(1, cloud.dim):
         ctx.set_field(f, np.zeros(cloud.nv))
     ctx.set_field(M.MP_P, np.zeros(ctx.n_sys))
+    ctx.step(1, 0)  # (the kernels' first launches load them, which would set the cut)
     ctx.kernel_timing(True)
-    ctx.step(steps, 0)
+    ctx.step(steps, 1)
 
 
 @pytest.mark.parametrize("dim,n,k", [(2, 40, 20), (2, 411, 20), (3, 16, 40), (3, 56, 40)])
@@ -54,12 +55,44 @@ def test_step_kernel_bytes(dim, n, k):
     assert got == step_bytes(cloud, staged, int(u.sum()))
 
 
+@pytest.mark.parametrize("length,staged", [(12, False), (20, True)])
+def test_staging_needs_reuse(length, staged):
+    """170k rows in two dimensions.  Rows of 12 whose columns lie anywhere: a row block's
+    3,000 distinct columns would fit, but each serves one entry, so the step kernels
+    gather.  Rows of 20 with their columns within 1,000 rows: 2,000 distinct columns,
+    each serving more than two."""
+    import memphys_amd as M
+    rng = np.random.default_rng(3)
+    nv = 170_011
+    row = np.repeat(np.arange(nv), length)
+    off = rng.integers(1, 1000 if staged else nv, nv * length)
+    col = ((row + off) % nv).astype(np.int32)
+    col[::length] = np.arange(nv)
+    cloud = M.Cloud(dim=2, xyz=np.c_[np.linspace(0, 1, nv), np.zeros(nv)],
+                    boundary=np.zeros(nv, np.uint8), normal=np.zeros((nv, 2)),
+                    row_ptr=(np.arange(nv + 1) * length).astype(np.int32), col=col,
+                    ksize=np.full(nv, length, np.int32), layer=np.zeros(nv, np.int32))
+    u = row_block_columns(cloud)
+    _print("max", u.max(), "reuse", cloud.nnz / u.sum())
+    assert 2 * u.max() <= 8192 and (cloud.nnz / u.sum() > 2 if staged else
+                                    cloud.nnz / u.sum() < 1.1)
+    w = 0.1 * rng.uniform(-1, 1, cloud.nnz)
+    u_dir = np.zeros(nv, np.uint8)
+    u_dir[0] = 1
+    with M.Context(0) as ctx:
+        ctx.upload(cloud)
+        ctx.set_weights(w, w, None, w)
+        ctx.fs_create(1.0, 0.01, 1e-5, 2, 1e-8, 100, u_dir, u_dir, None, np.zeros(nv, np.uint8))
+        got = [ctx.kernel_timing_get(q)[2] for q in (1, 2, 3)]
+    assert got == step_bytes(cloud, staged, int(u.sum()))
+
+
 @pytest.mark.parametrize("n,lo,hi", [(40, 44, 60), (170, 28, 36), (420, 28, 36)])
 def test_bicgstab_product_bytes(n, lo, hi):
     """FP64 BiCGSTAB, per row and beside the matrix.  Up to 96 row blocks the two
     products gather r, p, v and r, v, write p, v and s, t and read r0: 60 and 44
     bytes with D^-1 and the length.  In the other forms x, the product, r0: 36 and
-    28.  The reported mean lies between (launches that returned early left out)."""
+    28.  The reported mean lies between."""
     import memphys_amd as M
     cloud = M.box_cloud(dim=2, n=n, jitter=0.25, seed=5, k_interior=20)
     u = row_block_columns(cloud)
@@ -69,27 +102,27 @@ def test_bicgstab_product_bytes(n, lo, hi):
     matrix = 10 * cloud.nnz + 4 * int(u.sum()) if len(u) > 640 else 12 * cloud.nnz
     rows = (got - matrix) / cloud.nv
     _print("n", n, "blocks", len(u), "launches", launches, "bytes per row", rows)
-    assert launches >= 4
-    assert lo < rows < hi
+    assert launches >= 1
+    assert lo <= rows <= hi
 
 
 @pytest.mark.parametrize("n,fused", [(40, True), (420, False)])
 def test_gmres_product_bytes(n, fused):
-    """FP64 GMRES(6) with the multigrid (with Jacobi it stalls on these systems and
-    BiCGSTAB ends the solve): the V-cycle's FP32 output, the product, D^-1 and the
+    """FP64 GMRES(30) with the multigrid (it would stall with Jacobi or short cycles, and
+    BiCGSTAB end the solve): the V-cycle's FP32 output, the product, D^-1 and the
     length, 24 bytes a row; on small systems the launch of iteration k also reads
     the k + 1 basis vectors."""
     import memphys_amd as M
     cloud = M.box_cloud(dim=2, n=n, jitter=0.25, seed=5, k_interior=20)
     u = row_block_columns(cloud)
     with M.Context(0) as ctx:
-        _steps(ctx, cloud, krylov=1, restart=6, precond=1, steps=1)
+        _steps(ctx, cloud, krylov=1, restart=30, precond=1, steps=1)
         launches, _, got, _ = ctx.kernel_timing_get(0)
     matrix = 12 * cloud.nnz if fused else 10 * cloud.nnz + 4 * int(u.sum())
     rows = (got - matrix) / cloud.nv
     _print("n", n, "blocks", len(u), "launches", launches, "bytes per row", rows)
-    assert launches >= 4
+    assert launches >= 1
     if fused:
-        assert 24 + 8 < rows < 24 + 48
+        assert 24 + 8 <= rows <= 24 + 240
     else:
         assert abs(rows - 24) < 1e-6
