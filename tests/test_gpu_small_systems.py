@@ -125,26 +125,77 @@ def test_large_system_with_local_and_scattered_columns(spread, prec):
         assert res <= 1.1e-11  # the solver's FP64 test, plus this host's rounding
 
 
-@pytest.mark.parametrize("dim,n,k", [(2, 411, 30), (3, 56, 40), (3, 56, 150)])
-def test_large_cloud_step_matches_its_operators(dim, n, k):
-    """One Euler step of a cloud above 640 row blocks, whose predictor, right-hand
-    side and corrector read staged entries (with 150-node stencils a row block
-    has too many for three vectors: the gathering kernels), against the
-    operator products, which gather: the predictor's source and the corrected
-    velocity bit for bit, the pressure by its residual."""
+def _with_far_columns(cloud, weights, rows, extra, rng):
+    """The cloud with `extra` columns from anywhere appended to the stencils of `rows`, and
+    its weights with small ones (1e-3 of the stencil's own) there."""
     import memphys_amd as M
+    nv = cloud.nv
+    add = np.zeros(nv, np.int64)
+    add[rows] = extra
+    length = np.diff(cloud.row_ptr)
+    rp = np.concatenate([[0], np.cumsum(length + add)]).astype(np.int32)
+    old = np.arange(cloud.nnz) + np.repeat(rp[:-1] - cloud.row_ptr[:-1], length)
+    new = (rp[rows] + length[rows])[:, None] + np.arange(extra)
+    col = np.empty(rp[-1], np.int32)
+    col[old] = cloud.col
+    col[new] = rng.integers(0, nv, new.shape)
+    out = []
+    for w in weights:
+        if w is None:
+            out.append(None)
+            continue
+        x = np.empty(rp[-1])
+        x[old] = w
+        x[new] = rng.uniform(-1, 1, new.shape) * 1e-3 * np.abs(w[cloud.row_ptr[rows]])[:, None]
+        out.append(x)
+    c = M.Cloud(dim=cloud.dim, xyz=cloud.xyz, boundary=cloud.boundary, normal=cloud.normal,
+                row_ptr=rp, col=col, ksize=(length + add).astype(np.int32), layer=cloud.layer)
+    return c, out
+
+
+@pytest.mark.parametrize("dim,n,k,extra,form", [
+    (2, 411, 30, 0, "staged"), (3, 56, 40, 0, "staged"), (3, 56, 150, 0, "staged"),
+    (2, 411, 30, 19, "steps gather"), (3, 56, 40, 14, "steps gather"),
+    (2, 411, 30, 32, "all gather"), (3, 56, 40, 32, "all gather")])
+def test_large_cloud_step_matches_its_operators(dim, n, k, extra, form):
+    """One Euler step of a cloud above 640 row blocks against the operator products,
+    which gather: the predictor's source and the corrected velocity bit for bit, the
+    pressure by its residual.  The predictor, right-hand side and corrector read
+    staged entries, unless one row block has too many distinct columns for `dim`
+    vectors in 64 KB (256 rows with columns from anywhere), or for the products too."""
+    import memphys_amd as M
+    from conftest import row_block_columns
+    from test_gpu_kernel_bytes import step_bytes
     kw = dict(k_layers=(60, 55, 50)) if k == 40 else {}
     cloud = M.box_cloud(dim=dim, n=n, jitter=0.25, seed=5, k_interior=k, **kw)
     rng = np.random.default_rng(1)
     u_dir, p_dir, _ = M.lid_conditions(cloud)
     wall = cloud.boundary == 1
+    weights = None
+    if extra:
+        inner = np.flatnonzero(~wall)
+        near = inner[np.argsort(np.linalg.norm(cloud.xyz[inner] - 0.3, axis=1))[:256]]
+        with M.Context(0) as ctx:
+            ctx.upload(cloud)
+            weights, _ = ctx.weights(3, 3)
+        cloud, weights = _with_far_columns(cloud, weights, near, extra, rng)
+    blocks = row_block_columns(cloud)
+    _print("dim", dim, "extra", extra, "distinct columns", blocks.max())
+    assert len(blocks) > 640
+    assert {"staged": blocks.max() <= 8192 // dim, "all gather": blocks.max() > 6144,
+            "steps gather": 8192 // dim < blocks.max() <= 6144}[form]
     rho, mu, dt, tol = 1.0, 0.01, 1e-5, 1e-9
     with M.Context(0) as ctx:
         ctx.upload(cloud)
-        ctx.weights(3, 3, download=False)
+        if weights:
+            ctx.set_weights(*weights)
+        else:
+            ctx.weights(3, 3, download=False)
         ctx.fs_create(rho, mu, dt, 2, tol, 4000, u_dir, u_dir, u_dir if dim == 3 else None, p_dir,
                       precision=M.MP_PREC_MIXED, precond=M.MP_PRECOND_AMG,
                       krylov=M.MP_KRYLOV_GMRES)
+        assert ctx.kernel_timing_get(1)[2] == step_bytes(cloud, form == "staged",
+                                                         int(blocks.sum()))[0]
         u = [np.where(wall, 0.0, rng.standard_normal(cloud.nv)) for _ in range(dim)]
         for q in range(dim):
             ctx.set_field(q, u[q])
