@@ -225,3 +225,136 @@ def test_large_cloud_step_matches_its_operators(dim, n, k, extra, form):
         res = np.linalg.norm(ap - b) / np.linalg.norm(b)
         _print("dim", dim, "k", k, "residual", res, ctx.stats().rel_res)
         assert res <= 1.5 * tol  # the solver's FP64 test, and the sums' own rounding
+
+
+def _chain_system(nv, m=12):
+    """A cloud whose operator is the identity plus x_{i-1} in row i for the m nodes 2 .. m+1.
+    With b = e_1, one BiCGSTAB iteration from x = 0 leaves a residual exactly
+    orthogonal to the first one (alpha = 1, omega = 1/2, r = (e_3 - e_2) / 2): the
+    solver has to restart.  The solution is 1, -1, 1, ... along the chain."""
+    import memphys_amd as M
+    length = np.ones(nv, np.int32)
+    length[2:2 + m] = 2
+    rp = np.concatenate([[0], np.cumsum(length)]).astype(np.int32)
+    col = np.empty(rp[-1], np.int32)
+    col[rp[:-1]] = np.arange(nv)
+    col[rp[2:2 + m] + 1] = np.arange(1, 1 + m)
+    lap = np.zeros(rp[-1])
+    lap[rp[2:2 + m] + 1] = 1.0
+    boundary = np.zeros(nv, np.uint8)
+    boundary[0] = 1  # (Dirichlet: no border unknown)
+    cloud = M.Cloud(dim=2, xyz=np.c_[np.linspace(0, 1, nv), np.zeros(nv)], boundary=boundary,
+                    normal=np.tile([1.0, 0.0], (nv, 1)), row_ptr=rp, col=col, ksize=length,
+                    layer=np.zeros(nv, np.int32))
+    b, x = np.zeros(nv), np.zeros(nv)
+    b[1] = 1.0
+    x[1:2 + m] = (-1.0) ** np.arange(m + 1)
+    return cloud, lap, b, x
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+def test_bicgstab_restart_is_the_same_in_every_form(prec):
+    """The breakdown of r0.r and its restart in iterations of three, five and eight
+    launches, alone and in batches beside a system that runs on and one that is done
+    from the start: the solution, and the same bits in every form (the rest of each
+    system is zero, so its size does not enter the sums)."""
+    import memphys_amd as M
+    rng = np.random.default_rng(6)
+    first = None
+
+    def solve(parts):
+        """Solutions of [(cloud, lap, b)] as one context's systems, and the restarts."""
+        with M.Context(0) as ctx:
+            cat = parts[0][0] if len(parts) == 1 else ctx.upload_batch([p[0] for p in parts])
+            if len(parts) == 1:
+                ctx.upload(cat)
+            lap = np.concatenate([p[1] for p in parts])
+            zero = np.zeros_like(lap)
+            ctx.set_weights(zero, zero, None, lap)
+            n = ctx.solver_init(cat.boundary, 1.0, 0.0, 1.0, tol=1e-13, n_iter=300,
+                                precision=prec)
+            assert n == cat.nv
+            x, _ = ctx.solve(np.concatenate([p[2] for p in parts]), np.zeros(n))
+            at = np.cumsum([0] + [p[0].nv for p in parts])
+            return [x[a:e] for a, e in zip(at[:-1], at[1:])], ctx.stats().restarts
+
+    for nv in (200, 25_100, 170_011):  # 1, 99 and 665 row blocks
+        cloud, lap, b, x = _chain_system(nv)
+        (got,), restarts = solve([(cloud, lap, b)])
+        _print("nv", nv, "restarts", restarts, "error", np.abs(got - x).max())
+        assert restarts >= 1
+        assert np.abs(got - x).max() <= 1e-11
+        first = got[:14] if first is None else first
+        assert np.array_equal(got[:14], first)
+    small = _chain_system(200)
+    for nv in (3_000, 170_011):  # a batch of fused iterations, and one of eight launches
+        cloud = _chain_system(nv, m=nv - 2)[0]
+        lap = 0.3 * rng.uniform(-1, 1, cloud.nnz)
+        lap[cloud.row_ptr[:-1]] = 0.0
+        other = (cloud, lap, rng.standard_normal(nv))
+        idle = (small[0], small[1], np.zeros(200))
+        (a, o, z, c), _ = solve([small[:3], other, idle, small[:3]])
+        assert np.array_equal(a[:14], first) and np.array_equal(c[:14], first)
+        assert not z.any()
+        r = o.copy()
+        r[2:] += lap[cloud.row_ptr[2:-1] + 1] * o[1:-1]
+        assert np.linalg.norm(r - other[2]) <= 1.1e-13 * np.linalg.norm(other[2])
+
+
+def test_middle_size_in_large_batch_is_bit_identical():
+    """A cavity of 352 row blocks, between the sizes that the Hessenberg column runs in the
+    update (128) and those of the general kernels (640): alone and in a batch."""
+    import memphys_amd as M
+    clouds = [M.box_cloud(dim=2, n=n, jitter=0.25, seed=n, k_interior=30) for n in (300, 290)]
+    assert [-(-(c.nv + 1) // 256) for c in clouds] == [352, 329]
+    for krylov in (0, 1):
+        with M.Context(0) as ctx:
+            cat = ctx.upload_batch(clouds)
+            batch = _run(ctx, cat, krylov, 1, steps=1)
+            iters = ctx.batch_stats(0).iterations
+        with M.Context(0) as ctx:
+            ctx.upload(clouds[0])
+            alone = _run(ctx, clouds[0], krylov, 1, steps=1)
+            assert ctx.stats().iterations == iters
+        for a, b in zip(alone, batch):
+            assert np.array_equal(a[:clouds[0].nv], b[:clouds[0].nv])
+
+
+@pytest.mark.parametrize("krylov,precision", [(0, 1), (1, 0), (1, 1)])
+def test_large_batch_with_multigrid(krylov, precision):
+    """Cavities of 1 to 513 row blocks in a batch of 650: staged V-cycle products over
+    several systems and their padding rows, several norm steps beside one product, and
+    systems that stop before the others.  The fields match the stand-alone runs to the
+    solver's accuracy (the solves run to 1e-12, which fixes a full-Neumann pressure to
+    about 1e-10; the hierarchies of a batch share one depth, so not bit for bit)."""
+    import memphys_amd as M
+    from conftest import rel_err
+    sizes = [15, 362, 40, 150, 100]
+    clouds = [M.box_cloud(dim=2, n=n, jitter=0.25, seed=n, k_interior=30) for n in sizes]
+    assert sum(-(-(c.nv + 1) // 256) for c in clouds) > 640
+
+    def run(ctx, cloud):
+        u_dir, p_dir, u0 = M.lid_conditions(cloud)
+        ctx.weights(3, 3, download=False)
+        ctx.fs_create(1.0, 0.01, 1e-5, 2, 1e-12, 4000, u_dir, u_dir, None, p_dir,
+                      krylov=krylov, precision=precision, precond=M.MP_PRECOND_AMG)
+        ctx.set_field(M.MP_U, u0)
+        ctx.set_field(M.MP_V, np.zeros(cloud.nv))
+        ctx.set_field(M.MP_P, np.zeros(ctx.n_sys))
+        ctx.step(2, 0)
+        return [ctx.get_field(f) for f in (M.MP_U, M.MP_V, M.MP_P)]
+
+    with M.Context(0) as ctx:
+        cat = ctx.upload_batch(clouds)
+        batch = run(ctx, cat)
+        stats = [ctx.batch_stats(q) for q in range(len(clouds))]
+    at = 0
+    for q, c in enumerate(clouds):
+        with M.Context(0) as ctx:
+            ctx.upload(c)
+            alone = run(ctx, c)
+            its = ctx.stats().iterations
+        err = [rel_err(b[at:at + c.nv], a[:c.nv]) for a, b in zip(alone, batch)]
+        _print("n", sizes[q], "iterations", its, stats[q].iterations, "err", err)
+        assert stats[q].converged and max(err) <= 1e-8
+        at += c.nv
