@@ -66,18 +66,24 @@ def lid_bc(cloud):
     return u_dir, p_dir, u0
 
 
-def measured_traffic(n: int, kernel_index: int = 0,
+def measured_traffic(n: int, bytes_l: float,
                      summary: str = "ppe_spmv_traffic_cavity3d_1M.md"):
     """HBM bytes per launch measured with rocprofv3 FETCH_SIZE and WRITE_SIZE runs on
-    the 100^3 workload, read from a committed summary: the `kernel_index`-th
-    `traffic_bytes_per_launch` line (PPE SpMV summary: 0 the headline form's
-    FP32-operator GMRES product, 1 the FP64 form's product); None for other workloads."""
+    the 100^3 workload, read from a committed summary: the figure of the product
+    whose algorithmic bytes per launch (given in the summary before each figure)
+    are bytes_l within 1 %; None for other products and workloads."""
     path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles", summary)
     if n != 100 or not os.path.exists(path):
         return None
-    vals = [float(line.split("=")[1]) for line in open(path)
-            if line.startswith("traffic_bytes_per_launch")]
-    return vals[kernel_index] if len(vals) > kernel_index else None
+    alg = None
+    for line in open(path):
+        if line.startswith("algorithmic_bytes_per_launch"):
+            alg = float(line.split("=")[1])
+        elif line.startswith("traffic_bytes_per_launch") and alg:
+            if abs(bytes_l / alg - 1.0) < 0.01:
+                return float(line.split("=")[1])
+            alg = None
+    return None
 
 
 def run_form(M, ctx, cloud, prm, precision, steps, warmup, label, guess=None, precond=0,
@@ -181,7 +187,7 @@ def run_form(M, ctx, cloud, prm, precision, steps, warmup, label, guess=None, pr
 
 
 def step_kernels(form, copy_gbps):
-    """Predictor (with its packing of u, v, w), right-hand side and corrector of
+    """Predictor (with its packing of u, v, w where it gathers), right-hand side and corrector of
     the form's timing steps: mean ms per launch (HIP events) and the
     algorithmic bytes per launch over that time, against the 8 TB/s peak."""
     out = {}
@@ -327,24 +333,6 @@ def cavity2d_c1(M, O, steps=20, warmup=5, with_cpu=True):
     return out
 
 
-def level0_traffic(n: int, bytes_l: float, summary: str = "amg_level0_traffic_cavity3d_1M.md"):
-    """Measured HBM bytes per launch of the multigrid level-0 product whose
-    algorithmic bytes per launch (given in the summary before each figure) are
-    bytes_l within 1 %; None for other products and workloads."""
-    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles", summary)
-    if n != 100 or not os.path.exists(path):
-        return None
-    alg = None
-    for line in open(path):
-        if line.startswith("algorithmic_bytes_per_launch"):
-            alg = float(line.split("=")[1])
-        elif line.startswith("traffic_bytes_per_launch") and alg:
-            if abs(bytes_l / alg - 1.0) < 0.01:
-                return float(line.split("=")[1])
-            alg = None
-    return None
-
-
 def smooth_roofline(t, copy_gbps, n_lattice: int = 0, gmres: bool = True):
     """Roofline entry of the multigrid's level-0 prolongation and post-smoothing
     (the composed T_0 product): algorithmic bytes per launch over its mean
@@ -361,7 +349,8 @@ def smooth_roofline(t, copy_gbps, n_lattice: int = 0, gmres: bool = True):
             "bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": ach / HBM_PEAK_GBS, "frac_of_copy": ach / copy_gbps, "bytes_per_launch": bytes_l,
             "mean_ms": ms, "launches": n, "launches_returned_early": all_l - n,
-            "traffic": level0_traffic(n_lattice, bytes_l) if gmres else None}
+            "traffic": measured_traffic(n_lattice, bytes_l, "amg_level0_traffic_cavity3d_1M.md")
+            if gmres else None}
 
 
 def stream_copy_gbps(mib: int = 1024, reps: int = 10) -> float:
@@ -777,7 +766,7 @@ def main():
         "roofline": {
             "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS,
-            "traffic": measured_traffic(args.n, 0) if kry else None,
+            "traffic": measured_traffic(args.n, bytes_l) if kry else None,
             "kernel": ("k_gm_spmv<float,float,float> (PPE SpMV of GMRES, FP32 operator, FP32 "
                        "gathers of the V-cycle output)" if kry else
                        "k_spmv_alpha/k_spmv_omega<float,double,float> (PPE SpMV, FP32 "
@@ -808,7 +797,7 @@ def main():
                                "frac_of_copy": ach64 / copy_gbps,
                                "bytes_per_launch": b64, "mean_ms": ms64, "launches": n64,
                                "launches_returned_early": all64 - n64,
-                               "traffic": measured_traffic(args.n, 1)},
+                               "traffic": measured_traffic(args.n, b64)},
         "amg_level0_roofline": smooth_roofline(head.get("smooth"), copy_gbps, args.n, bool(kry)),
         "step_kernels": step_kernels(head, copy_gbps),
         "cloud_setup": setup,

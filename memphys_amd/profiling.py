@@ -50,7 +50,8 @@ def _short(name: str) -> str:
 def _working(durs: list) -> list:
     """Launches that did the work: duration at least half the median launch's
     (Krylov kernels launched after their system converged return at once).
-    The same rule as the library's HIP-event kernel timer."""
+    The library's HIP-event kernel timer, with fewer launches to go by, takes a
+    quarter of the longest."""
     srt = sorted(durs)
     cut = 0.5 * srt[len(srt) // 2]
     return [d for d in durs if d >= cut]

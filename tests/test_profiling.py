@@ -83,25 +83,31 @@ def test_traffic_scales_counters_by_the_copy_kernel(tmp_path):
 
 def test_bench_reads_committed_traffic_summaries():
     # The bench's `traffic` fields come from the committed rocprofv3 summaries;
-    # each must be the measured figure of its own kernel, within 1 % of that
-    # kernel's algorithmic bytes per launch (SpMV FP32 279,638,428; FP64
-    # 545,879,136; multigrid level-0 post-smoothing of the GMRES form, which
-    # reads the FP32 basis vector and writes the FP32 direction, 190,656,204),
-    # and absent on other workloads and for the BiCGSTAB form's product.
+    # each must be the measured figure of the kernel whose algorithmic bytes per
+    # launch were timed: of the staged products (SpMV FP32 296,297,104; FP64, mean
+    # of BiCGSTAB's two, 474,261,552; multigrid T_0 131,211,488) and of those that
+    # gather from L2 (279,638,428; 545,879,136; level-0 post-smoothing 190,656,204),
+    # and absent for other bytes, on other workloads and for the BiCGSTAB form's
+    # level-0 product.
     import importlib.util
     import os
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     spec = importlib.util.spec_from_file_location("bench_mod", os.path.join(root, "bench.py"))
     bench = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(bench)
-    for got, alg in [(bench.measured_traffic(100, 0), 279_638_428),
-                     (bench.measured_traffic(100, 1), 545_879_136),
-                     (bench.smooth_roofline((381, 0.06, 190_656_204.0, 393), 6000.0,
-                                            100)["traffic"], 190_656_204)]:
+    for alg, within in [(296_297_104, 0.01), (474_261_552, 0.03), (279_638_428, 0.01),
+                        (545_879_136, 0.01)]:
+        got = bench.measured_traffic(100, alg)
+        assert got is not None and abs(got / alg - 1) < within
+    for alg in (131_211_488, 190_656_204):
+        got = bench.smooth_roofline((381, 0.06, float(alg), 393), 6000.0, 100)["traffic"]
         assert got is not None and abs(got / alg - 1) < 0.01
-    assert bench.measured_traffic(50, 0) is None
-    assert bench.smooth_roofline((381, 0.06, 2e8, 393), 6000.0, 50)["traffic"] is None
-    assert bench.smooth_roofline((381, 0.06, 2e8, 393), 6000.0, 100, gmres=False)["traffic"] is None
+    assert bench.measured_traffic(100, 350e6) is None
+    assert bench.measured_traffic(50, 296_297_104) is None
+    assert bench.smooth_roofline((381, 0.06, 2e8, 393), 6000.0, 100)["traffic"] is None
+    assert bench.smooth_roofline((381, 0.06, 131_211_488.0, 393), 6000.0, 50)["traffic"] is None
+    assert bench.smooth_roofline((381, 0.06, 131_211_488.0, 393), 6000.0, 100,
+                                 gmres=False)["traffic"] is None
 
 
 def test_steps_splits_time_and_idle(tmp_path):
