@@ -68,9 +68,9 @@ struct AmgDevice {
     std::vector<long> nnz;
     std::string layout;  // chosen layout per matrix, for reports
     double setup_seconds = 0.0;
-    // host copies of the hierarchy (A[0] stays empty) and of the T_l, l >= 1,
-    // for re-tuning layouts
-    std::vector<mp_amg::Csr> hA, hP, hR, hT;
+    // host copies of the A_l (A[0] stays empty), the R_l and the T_l, l >= 1, for
+    // re-tuning layouts
+    std::vector<mp_amg::Csr> hA, hR, hT;
     // The cycle runs from the composed matrices (T_l on the way up; with three
     // or more levels, deep, also Q_l and the coarsest solve times R_{L-2},
     // row-dense BF16 in cr_val: row r's size[r] entries at cr_data[r] act on

@@ -1037,7 +1037,6 @@ void AmgDevice::setup(hipStream_t st, const SellView& sv, const double* val64_de
     }
     MP_HIP(hipStreamSynchronize(st));
     hA = std::move(Ab);
-    hP = std::move(Pb);
     hR = std::move(Rb);
     for (int l = 0; l + 1 < L; ++l) {
         char buf[96];

@@ -1443,7 +1443,6 @@ void PpeSolver::setup(hipStream_t st, const SellView& view, const std::vector<Se
     nv = 0;
     n_sys = 0;
     bordered = 0;
-    max_nblk = 0;
     std::vector<int> hb(nrows / BLOCK, 0);
     for (int q = 0; q < nseg; ++q) {
         const Seg& S = segs[q];
@@ -1452,7 +1451,6 @@ void PpeSolver::setup(hipStream_t st, const SellView& view, const std::vector<Se
         for (int b = 0; b < S.nblk; ++b) hb[S.blk0 + b] = q;
         nv += S.nv;
         n_sys += S.nv + S.border;
-        max_nblk = std::max(max_nblk, S.nblk);
         bordered |= S.border;
     }
     seg_d.alloc(nseg);

@@ -85,7 +85,6 @@ struct PpeSolver {
     int nv = 0;      // real rows of all systems
     int n_sys = 0;   // unknowns: real rows + border unknowns
     int nseg = 1, bordered = 0, dim = 0;
-    int max_nblk = 0;  // row blocks of the largest system
     long nnz = 0;    // real stencil entries of the operator
     SellView sv{};
     // column-sorted slot order (set before setup; slot_perm null: none): the
