@@ -442,9 +442,19 @@ __device__ __forceinline__ T sell4_block_early(const Slots& m, const TM* __restr
 // Blocks of BLOCK rows up to which a product runs with a wavefront per chain.
 // Shapes 1, 16 and 4: level-0 residual of a 64k-node cube (249 blocks) 11.7, 9.3
 // and 6.9 us, FP64 product of a 110k-node cube (414 blocks) 18.2, 16.0 and 13.6.
-// Steps with a wavefront per chain against staged entries: 110k nodes (mixed
-// multigrid) 28.1 and 29.3 ms, FP64 solve 4.55 and 4.93; 216k nodes (843 blocks)
-// 41.2 and 40.0, FP64 multigrid 19.2 and 19.1: the line lies between.
+// Whole iterations with a wavefront per chain (and the fused launches that go
+// with it) against staged entries, us:
+//                    FP64 Jacobi BiCGSTAB   mixed multigrid   FP64 multigrid
+//   3D  249 blocks      34.3    38.2           53.9   61.4       57.3   65.0
+//   3D  430             45.7    50.1           74.4   75.9       78.3   81.0
+//   3D  648             59.3    60.4           87.4   85.0       90.9   91.3
+//   3D  842             74.2    68.6           99.7   94.4      104.2  102.5
+//   2D  265             27.9    30.8           63.8   64.1       57.8   62.2
+//   2D  426             37.5    38.1           63.7   62.9       62.1   66.4
+//   2D  625             47.5    47.1           74.5   68.4       72.9   72.1
+//   2D  723             52.2    49.1           75.1   68.7       75.8   74.2
+// The line lies where most of them cross (the 2D mixed multigrid would cross at
+// about 430 blocks).
 constexpr int SPLIT_MAX_BLOCKS = 640;
 
 // SELL-64x4 view of the stencil set in device order.
