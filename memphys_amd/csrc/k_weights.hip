@@ -607,29 +607,28 @@ struct WaveLu {
         // the time of one masked block with the readlanes inside.)
         const bool below = pos > c;
         const double nl = -(a[0] / d);
-        if (below) {
-#pragma unroll
-            for (int j = 0; j < L; ++j) a[j] = fma3(nl, u[j + 1], a[j + 1]);
-        }
-        constexpr int T = 8;
-        static_for<0, (W - L + T - 1) / T>([&](auto g) {
-            constexpr int j0 = L + T * decltype(g)::value;
+        constexpr int T = 8, G = W > L ? (W - L + T - 1) / T : 1;
+        static_for<0, G>([&](auto g) {
+            constexpr int i = decltype(g)::value, j0 = L + T * i;
             constexpr int n = W - j0 < T ? W - j0 : T;
-            double s[n];
+            double s[T], sr[4];
 #pragma unroll
             for (int t = 0; t < n; ++t) s[t] = readlane_d(a[j0 + t + 1], pl);
+            if (i == 0) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) sr[q] = readlane_d(r[q], pl);
+            }
             if (below) {
+                if (i == 0) {
+#pragma unroll
+                    for (int j = 0; j < L; ++j) a[j] = fma3(nl, u[j + 1], a[j + 1]);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) r[q] = fma3s(nl, sr[q], r[q]);
+                }
 #pragma unroll
                 for (int t = 0; t < n; ++t) a[j0 + t] = fma3s(nl, s[t], a[j0 + t + 1]);
             }
         });
-        double s[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) s[q] = readlane_d(r[q], pl);
-        if (below) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) r[q] = fma3s(nl, s[q], r[q]);
-        }
     }
 
     // Two wavefronts: each publishes the candidate among its own rows, whole,
